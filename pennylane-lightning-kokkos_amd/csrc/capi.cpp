@@ -167,8 +167,17 @@ bool to_pauli(const ObsNode &o, int n, std::vector<PauliTerm> &out,
 // ---------------------------------------------------------------------------
 // Gate application.
 // ---------------------------------------------------------------------------
+// A trainable gate of a fused run: its Jacobian column and coefficient, and
+// the operator V^dag G V (V the run's gates before it) as m0 X + m1 Y + m2 Z.
+struct RunTerm {
+    int col;
+    double coef;
+    double m[3];
+};
+
 struct PlanOp {
     CompiledOp U;
+    std::vector<RunTerm> run; // register-tile plans: the trainable gates of a one-wire run
     bool trainable = false;
     CompiledGen G;
     int col = -1;
@@ -233,7 +242,7 @@ struct Pass {
     std::vector<Bundle> bundles;
     std::vector<PlanOp> ops; // register-tile passes: the ops in program order
     bool rt = false;         // a register-tile pass (ops) rather than LDS bundles
-    int nslots = 0;
+    int nslots = 0;            // sums (LDS passes: one per trainable op)
     std::vector<int> cols;     // Jacobian column of each trainable op, in order
     std::vector<double> coefs; // and its coefficient
 };
@@ -383,11 +392,92 @@ bool mixes_bit(const std::vector<cd> &M, int dim, int lb) {
     return false;
 }
 
+// Pauli parts the gates of a run need: bit 0 X, bit 1 Y, bit 2 Z.
+int run_parts(const PlanOp &p) {
+    int parts = 0;
+    for (const auto &t : p.run) {
+        for (int k = 0; k < 3; k++) {
+            parts |= t.m[k] != 0.0 ? 1 << k : 0;
+        }
+    }
+    return parts;
+}
+
+// Sums a register-tile pass keeps for an op.
+int rt_slots(const PlanOp &p) {
+    if (p.run.empty()) {
+        return p.trainable ? 1 : 0;
+    }
+    const int parts = run_parts(p);
+    return (parts & (parts - 1)) ? 3 : 1;
+}
+
+// 2x2 product A B.
+std::vector<cd> mul2(const std::vector<cd> &A, const std::vector<cd> &B) {
+    return {A[0] * B[0] + A[1] * B[2], A[0] * B[1] + A[1] * B[3], A[2] * B[0] + A[3] * B[2],
+            A[2] * B[1] + A[3] * B[3]};
+}
+
+// Fuses the one-wire ops that follow each other on a wire into one 2x2
+// matrix, at the place of the first (ops on other wires commute with them).
+// Trainable ops join when their generator is traceless (X, Y, Z and real
+// combinations of them); anything else on the wire ends the run.
+std::vector<PlanOp> fuse_runs(std::vector<PlanOp> &&ops) {
+    std::vector<PlanOp> out;
+    out.reserve(ops.size());
+    std::vector<long> open(64, -1);
+    for (auto &p : ops) {
+        if (p.U.kind == OpKind::Identity && !p.trainable) {
+            continue;
+        }
+        prepare(p);
+        bool one = p.U.kind == OpKind::Dense && p.U.wires.size() == 1;
+        if (one && p.trainable) {
+            one = p.G.kind == OpKind::Dense && p.G.wires == p.U.wires && p.G.mat[0] + p.G.mat[3] == cd(0.0, 0.0);
+        }
+        if (!one) {
+            for (auto w : p.U.wires) {
+                open[w] = -1;
+            }
+            out.push_back(std::move(p));
+            continue;
+        }
+        const size_t w = p.U.wires[0];
+        const bool first = open[w] < 0;
+        if (p.trainable) {
+            std::vector<cd> g = p.G.mat;
+            if (!first) {
+                const std::vector<cd> &V = out[open[w]].U.mat;
+                const std::vector<cd> Vd = {std::conj(V[0]), std::conj(V[2]), std::conj(V[1]), std::conj(V[3])};
+                g = mul2(Vd, mul2(g, V));
+            }
+            const RunTerm t{p.col, p.coef,
+                            {0.5 * (g[1] + g[2]).real(), 0.5 * (g[2].imag() - g[1].imag()),
+                             0.5 * (g[0] - g[3]).real()}};
+            PlanOp &into = first ? p : out[open[w]];
+            into.run.push_back(t);
+            into.trainable = true;
+        }
+        if (first) {
+            open[w] = static_cast<long>(out.size());
+            out.push_back(std::move(p));
+        } else {
+            PlanOp &o = out[open[w]];
+            o.U.mat = mul2(p.U.mat, o.U.mat);
+        }
+    }
+    return out;
+}
+
 // Global state bits an op mixes (its U or, when trainable, its generator has
 // an entry between indices that differ in the bit).
 uint64_t mixing_mask(const PlanOp &p, int n) {
     const int m = static_cast<int>(p.U.wires.size());
     uint64_t mask = 0;
+    if (!p.run.empty()) {
+        const bool mixes = mixes_bit(p.U.mat, 2, 0) || run_parts(p) != 4;
+        return mixes ? uint64_t{1} << (n - 1 - static_cast<int>(p.U.wires[0])) : 0;
+    }
     for (int k = 0; k < m; k++) {
         const int lb = m - 1 - k;
         if (mixes_bit(p.U.mat, 1 << m, lb) || (p.trainable && mixes_bit(p.G.mat, 1 << m, lb))) {
@@ -401,16 +491,21 @@ uint64_t mixing_mask(const PlanOp &p, int n) {
 // lowest L bits. Operations on disjoint wires commute, so an operation may be
 // taken ahead of skipped ones it shares no wire with; an unfusable operation
 // is a barrier and runs on its own. With bundled == false (register-tile
-// passes) at most maxmix distinct bits may be mixed per pass.
+// passes) one-wire runs are fused first, and a pass needs in its tile only
+// the bits its operations mix.
 std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
-                             int pmax = TILE_PMAX, bool bundled = true, int maxmix = 64) {
+                             int pmax = TILE_PMAX, bool bundled = true) {
     std::vector<PlanOp> all;
-    for (auto &p : ops_in) {
-        if (p.U.kind == OpKind::Identity && !p.trainable) {
-            continue;
+    if (bundled) {
+        for (auto &p : ops_in) {
+            if (p.U.kind == OpKind::Identity && !p.trainable) {
+                continue;
+            }
+            prepare(p);
+            all.push_back(std::move(p));
         }
-        prepare(p);
-        all.push_back(std::move(p));
+    } else {
+        all = fuse_runs(std::move(ops_in));
     }
     // Wire and state-bit masks (wires and bits < 64).
     std::vector<uint64_t> wmask(all.size()), bmask(all.size());
@@ -443,7 +538,7 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
             continue;
         }
         uint64_t bits = L > 0 ? (uint64_t{1} << L) - 1 : 0;
-        uint64_t blocked = 0, mixed = 0;
+        uint64_t blocked = 0;
         taken.clear();
         rest.clear();
         int nslots = 0;
@@ -453,18 +548,16 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
             if (!fus[i] || k >= kLookahead) {
                 break;
             }
-            const bool tr = all[i].trainable;
+            const int sums = bundled ? (all[i].trainable ? 1 : 0) : rt_slots(all[i]);
             // Register-tile passes need only the bits an op mixes in the
             // tile: its other bits may lie outside, where they are fixed per
             // tile and select the op's block.
             const uint64_t nb = bits | (bundled ? bmask[i] : mmask[i]);
-            const bool ok = taken.size() < kPassMaxOps && (!tr || nslots < pmax) &&
-                            !(blocked & wmask[i]) && __builtin_popcountll(nb) <= T &&
-                            __builtin_popcountll(mixed | mmask[i]) <= maxmix;
+            const bool ok = taken.size() < kPassMaxOps && nslots + sums <= pmax &&
+                            !(blocked & wmask[i]) && __builtin_popcountll(nb) <= T;
             if (ok) {
                 bits = nb;
-                mixed |= mmask[i];
-                nslots += tr ? 1 : 0;
+                nslots += sums;
                 taken.push_back(i);
             } else {
                 blocked |= wmask[i];
@@ -491,13 +584,7 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
         if (bundled) {
             make_bundles(s.pass, std::move(ops), n);
         } else {
-            for (auto &p : ops) {
-                if (p.trainable) {
-                    s.pass.cols.push_back(p.col);
-                    s.pass.coefs.push_back(p.coef);
-                    s.pass.nslots++;
-                }
-            }
+            s.pass.nslots = nslots;
             s.pass.ops = std::move(ops);
             s.pass.rt = true;
         }
@@ -869,9 +956,17 @@ void build_pass(const Pass &ps, int n, std::vector<unsigned char> &table,
 // Host images of a plan's device tables: op groups of register segments and
 // LDS bundles, the bundle table, and register-tile programs, with the
 // launch metadata that points into them.
+// An entry of the Jacobian formed from the sums of a register-tile pass.
+struct RtTerm {
+    int col;
+    int slot[3]; // -1: none
+    double m[3]; // coefficients, the gate's own included
+};
+
 struct RtProgram {
     RtLaunch L{};
     size_t off = 0; // byte offset of the program in the plan blob
+    std::vector<RtTerm> terms;
 };
 
 // A single-op step run by the step kernels (kernels_step.hip): its launch
@@ -893,6 +988,7 @@ struct PlanImage {
     std::vector<RtProgram> progs;
     std::vector<unsigned char> mats; // U and G of the step-kernel steps (FP64 complex)
     std::vector<StepMeta> singles;
+    std::vector<RtEntry> entries; // reverse plans: see place_partials
 };
 
 // Device addresses of an image's tables.
@@ -901,6 +997,7 @@ struct PlanPlace {
     const TileBundle *bundles = nullptr;
     const unsigned char *rt = nullptr;
     const unsigned char *mats = nullptr;
+    const RtEntry *entries = nullptr;
 };
 
 // The 2^m x 2^m matrix, over the wires uw (uw[0] most significant), of an
@@ -1085,20 +1182,31 @@ void build_seg_tables(const std::vector<Step> &steps, int n, PlanImage &img) {
 // its generator, has an entry between different values); its other bits may
 // sit on lanes, where each lane applies the block its lane bits select. The
 // builder picks the load layout (the first mixing bits in registers, the
-// next two on lane positions 5 and 4, whose exchanges are single
-// v_permlane swaps), then walks the ops and brings each missing mixing bit
-// into a register by exchanging it with the register whose next use is
-// farthest away (Belady). The final layout is the store layout.
+// next on the lane positions from 5 down, the two cheapest to exchange
+// first), then walks the ops and brings each missing mixing bit into a
+// register by exchanging it with the register whose next use is farthest
+// away (Belady). The final layout is the store layout.
 // ---------------------------------------------------------------------------
-int rt_register_bits(int dtype) { return dtype == PLK_C64 ? 4 : 3; }
-
 template <typename T> struct RtBuilder {
+    struct Slot {
+        RtInstr h;
+        T u[8];
+    };
+    static_assert(sizeof(Slot) == rt_stride<T>(), "instruction stride");
     std::vector<unsigned char> &blob;
-    size_t base = 0;
-    std::vector<RtInstr> ins;
+    std::vector<Slot> ins;
     std::vector<unsigned char> pay;
 
     explicit RtBuilder(std::vector<unsigned char> &b) : blob(b) {}
+
+    void add(const RtInstr &h, const std::vector<double> &u) {
+        Slot s{};
+        s.h = h;
+        for (size_t k = 0; k < u.size() && k < 8; k++) {
+            s.u[k] = static_cast<T>(u[k]);
+        }
+        ins.push_back(s);
+    }
 
     int32_t put(const std::vector<double> &vals) {
         pay.resize((pay.size() + 15) & ~size_t{15}, 0);
@@ -1111,11 +1219,14 @@ template <typename T> struct RtBuilder {
         return static_cast<int32_t>(off); // relative to the payload start; rebased in finish()
     }
 
+    // Appends the program to the blob. One empty instruction follows the
+    // last: the kernel fetches one ahead.
     size_t finish() {
-        const size_t head = ins.size() * sizeof(RtInstr);
+        ins.push_back(Slot{});
+        const size_t head = ins.size() * sizeof(Slot);
         for (auto &i : ins) {
-            i.uoff += static_cast<int32_t>(head);
-            i.goff += static_cast<int32_t>(head);
+            i.h.uoff += static_cast<int32_t>(head);
+            i.h.goff += static_cast<int32_t>(head);
         }
         blob.resize((blob.size() + 255) & ~size_t{255}, 0);
         const size_t off = blob.size();
@@ -1169,41 +1280,47 @@ bool is_x2(const std::vector<cd> &B) {
     return B[0] == cd(0, 0) && B[3] == cd(0, 0) && B[1] == cd(1, 0) && B[2] == cd(1, 0);
 }
 
-// Encodes the U (and, for a trainable op, G) parts of a one-register-bit op.
-template <typename T>
-void rt_encode_reg1(RtBuilder<T> &b, RtInstr &in, const std::vector<cd> &U, const std::vector<cd> *G) {
+// Encodes the U part of a one-register-bit op; returns its reals.
+std::vector<double> rt_encode_u1(RtInstr &in, const std::vector<cd> &U) {
+    if (is_ident2(U)) {
+        in.ukind = U_NONE;
+        return {};
+    }
     if (is_diag2(U)) {
         in.ukind = U_DIAG;
-        in.uoff = b.put(cplx({U[0], U[3]}));
-    } else if (is_x2(U)) {
+        return cplx({U[0], U[3]});
+    }
+    if (is_x2(U)) {
         in.ukind = U_SWAP;
-    } else if (is_real(U)) {
+        return {};
+    }
+    if (is_real(U)) {
         in.ukind = U_REAL;
-        in.uoff = b.put({U[0].real(), U[1].real(), U[2].real(), U[3].real()});
-    } else {
-        in.ukind = U_DENSE;
-        in.uoff = b.put(cplx(U));
+        return {U[0].real(), U[1].real(), U[2].real(), U[3].real()};
     }
-    if (G) {
-        const auto &g = *G;
-        if (is_diag2(g) && is_real(g) && g[0] == cd(1, 0) && g[3] == cd(-1, 0)) {
-            in.gkind = G_Z;
-        } else if (is_diag2(g) && is_real(g)) {
-            in.gkind = G_DIAG;
-            in.goff = b.put({g[0].real(), g[3].real()});
-        } else if (is_x2(g)) {
-            in.gkind = G_X;
-        } else if (g[0] == cd(0, 0) && g[3] == cd(0, 0) && g[1] == cd(0, -1) && g[2] == cd(0, 1)) {
-            in.gkind = G_Y;
-        } else {
-            in.gkind = G_DENSE;
-            in.goff = b.put(cplx(g));
-        }
+    in.ukind = U_DENSE;
+    return cplx(U);
+}
+
+// complex64 programs round every matrix to FP32, which changes the norm of
+// the whole state by a few 1e-8 per gate: the one rounding error that does not
+// average out over the amplitudes (its random walk over a circuit's gates is
+// the bulk of an FP32 expectation value's error). `norm` is the product of
+// these factors so far; a one-wire matrix is divided by it before it is
+// rounded, so the product stays within one rounding of 1.
+std::vector<double> keep_norm(std::vector<double> u, int dim, double &norm) {
+    double sum = 0.0;
+    for (double &x : u) {
+        x /= norm;
+        const double r = static_cast<double>(static_cast<float>(x));
+        sum += r * r;
     }
+    norm *= std::sqrt(sum / dim);
+    return u;
 }
 
 template <typename T>
-RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned char> &blob) {
+RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned char> &blob, double &norm) {
     RtProgram out;
     RtLaunch &L = out.L;
     L.n = n;
@@ -1219,13 +1336,11 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
     std::vector<std::vector<int>> gbits(nops), mix(nops);
     for (size_t i = 0; i < nops; i++) {
         const PlanOp &p = ps.ops[i];
-        const int m = static_cast<int>(p.U.wires.size());
-        const int dim = 1 << m;
-        for (int k = 0; k < m; k++) {
-            const int gb = n - 1 - static_cast<int>(p.U.wires[k]);
+        const uint64_t mm = mixing_mask(p, n);
+        for (auto w : p.U.wires) {
+            const int gb = n - 1 - static_cast<int>(w);
             gbits[i].push_back(gb);
-            const int lb = m - 1 - k;
-            if (mixes_bit(p.U.mat, dim, lb) || (p.trainable && mixes_bit(p.G.mat, dim, lb))) {
+            if (mm >> gb & 1) {
                 mix[i].push_back(gb);
             }
         }
@@ -1244,29 +1359,20 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
     // covers runs of at least 32 bytes. With the three lowest bits all in
     // registers each instruction touches 64 cache lines 16 bytes at a time,
     // and an in-place pass streams at 4.4 TB/s instead of 5.1 (MI355X,
-    // 1-4 GiB states). A keep bit the pass mixes loads on lane position 5
-    // or 4 and is swapped into a register when an op needs it.
+    // 1-4 GiB states). A keep bit the pass mixes is swapped into a register
+    // when an op needs it.
     const int keep = std::is_same<T, double>::value ? 1 : 2;
     auto is_keep = [&](int q) { return q < keep; };
     auto has = [](const std::vector<int> &v, int q) { return std::find(v.begin(), v.end(), q) != v.end(); };
-    std::vector<int> reg, lane(RT_LANE_BITS, -1);
-    std::vector<int> rest;
-    for (size_t k = 0; k < order.size() && static_cast<int>(reg.size()) < R; k++) {
-        if (!is_keep(order[k])) {
-            reg.push_back(order[k]);
-        }
-    }
-    std::vector<int> hot; // mixing bits not in registers: lane positions 5, 4
+    std::vector<int> reg, lane(RT_LANE_BITS, -1), hot;
     for (int q : order) {
-        if (is_keep(q) && hot.size() < 2) {
+        if (!is_keep(q) && static_cast<int>(reg.size()) < R) {
+            reg.push_back(q);
+        } else {
             hot.push_back(q);
         }
     }
-    for (size_t k = 0; k < order.size() && hot.size() < 2; k++) {
-        if (!is_keep(order[k]) && !has(reg, order[k])) {
-            hot.push_back(order[k]);
-        }
-    }
+    std::vector<int> rest;
     for (int q : ps.tb) {
         if (!has(reg, q) && !has(hot, q)) {
             rest.push_back(q); // ascending global bits
@@ -1330,12 +1436,27 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
         }
         return nops + 1;
     };
+    auto add_remap = [&](RtInstr &in, int r, int p) {
+        if (in.nremap >= 2) {
+            raise(PLK_ERR_INVALID, "register-tile instruction needs more than two remaps");
+        }
+        if (in.nremap == 0) {
+            in.rq0 = static_cast<int8_t>(r);
+            in.rp0 = static_cast<int8_t>(p);
+        } else {
+            in.rq1 = static_cast<int8_t>(r);
+            in.rp1 = static_cast<int8_t>(p);
+        }
+        in.nremap++;
+        std::swap(lane[p], reg[r]);
+    };
     int slot = 0;
     for (size_t i = 0; i < nops; i++) {
         const PlanOp &p = ps.ops[i];
         RtInstr in{};
         in.slot = -1;
         in.s0 = in.s1 = -1;
+        std::vector<double> u;
         for (int q : mix[i]) {
             if (reg_of(q) >= 0) {
                 continue;
@@ -1346,48 +1467,70 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
                 if (std::find(mix[i].begin(), mix[i].end(), reg[r]) != mix[i].end()) {
                     continue;
                 }
-                const size_t u = next_use(reg[r], i);
-                if (victim < 0 || u > far) {
+                const size_t use = next_use(reg[r], i);
+                if (victim < 0 || use > far) {
                     victim = r;
-                    far = u;
+                    far = use;
                 }
             }
-            const int l = lane_of(q);
-            if (l < 4 || in.nremap >= 2) {
-                raise(PLK_ERR_INVALID, "register-tile pass needs more mixing bits than it can remap");
-            }
-            if (in.nremap == 0) {
-                in.rq0 = static_cast<int8_t>(victim);
-                in.rp0 = static_cast<int8_t>(l);
-            } else {
-                in.rq1 = static_cast<int8_t>(victim);
-                in.rp1 = static_cast<int8_t>(l);
-            }
-            in.nremap++;
-            lane[l] = reg[victim];
-            reg[victim] = q;
-        }
-        const std::vector<cd> *G = nullptr;
-        if (p.trainable) {
-            if (p.G.wires != p.U.wires || p.G.kind != OpKind::Dense) {
-                raise(PLK_ERR_INVALID, "generator wires differ from gate wires");
-            }
-            G = &p.G.mat;
-            in.slot = slot++;
+            add_remap(in, victim, lane_of(q));
         }
         const int m = static_cast<int>(gbits[i].size());
+        const std::vector<cd> *G = nullptr;
+        if (p.trainable) {
+            in.slot = slot;
+            if (p.run.empty()) {
+                if (p.G.wires != p.U.wires || p.G.kind != OpKind::Dense) {
+                    raise(PLK_ERR_INVALID, "generator wires differ from gate wires");
+                }
+                G = &p.G.mat;
+                out.terms.push_back({p.col, {slot, -1, -1}, {p.coef, 0.0, 0.0}});
+            } else {
+                const int parts = run_parts(p);
+                const bool all = rt_slots(p) == 3;
+                const int only = parts == 1 ? 0 : parts == 2 ? 1 : 2;
+                in.gkind = static_cast<int8_t>(all ? G_XYZ : only == 0 ? G_X : only == 1 ? G_Y : G_Z);
+                for (const RunTerm &t : p.run) {
+                    if (all) {
+                        out.terms.push_back({t.col, {slot, slot + 1, slot + 2},
+                                             {t.coef * t.m[0], t.coef * t.m[1], t.coef * t.m[2]}});
+                    } else {
+                        out.terms.push_back({t.col, {slot, -1, -1}, {t.coef * t.m[only], 0.0, 0.0}});
+                    }
+                }
+            }
+            slot += rt_slots(p);
+        }
         if (m == 1) {
             const int r = reg_of(gbits[i][0]);
             if (r >= 0) {
                 in.code = RT_REG1;
                 in.a = static_cast<int8_t>(r);
-                rt_encode_reg1<T>(b, in, p.U.mat, G);
+                u = rt_encode_u1(in, p.U.mat);
+                if (sizeof(T) == 4 && !u.empty()) {
+                    u = keep_norm(std::move(u), 2, norm);
+                }
+                if (G) {
+                    const auto &g = *G;
+                    if (is_diag2(g) && is_real(g)) {
+                        in.gkind = G_DIAG;
+                        in.goff = b.put({g[0].real(), g[3].real()});
+                    } else {
+                        in.gkind = G_DENSE;
+                        in.goff = b.put(cplx(g));
+                    }
+                }
             } else {
                 in.code = RT_LANE;
                 in.s0 = static_cast<int8_t>(sel_of(gbits[i][0]));
-                in.uoff = b.put(cplx({p.U.mat[0], p.U.mat[3]}));
+                u = cplx({p.U.mat[0], p.U.mat[3]});
+                if (sizeof(T) == 4) {
+                    u = keep_norm(std::move(u), 2, norm);
+                }
                 if (G) {
                     in.goff = b.put({(*G)[0].real(), (*G)[3].real()});
+                } else if (p.trainable) {
+                    in.goff = b.put({1.0, -1.0}); // a diagonal run: Z
                 }
             }
         } else {
@@ -1396,7 +1539,7 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
                 in.code = RT_REG2;
                 in.a = static_cast<int8_t>(std::max(r0, r1));
                 in.b = static_cast<int8_t>(std::min(r0, r1));
-                SegOp<T> d{};
+                SegOp<double> d{};
                 d.slot = G ? 0 : -1;
                 put_mat(d.U, p.U.mat, r0 < r1);
                 if (G) {
@@ -1405,20 +1548,20 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
                 classify(d, 2);
                 in.ukind = static_cast<int8_t>(d.ukind);
                 in.swap = static_cast<int8_t>(d.swap);
-                std::vector<double> u;
                 if (d.ukind == U_DIAG) {
                     for (int k = 0; k < 4; k++) {
                         u.push_back(d.U[2 * (5 * k)]);
                         u.push_back(d.U[2 * (5 * k) + 1]);
                     }
                 } else if (d.ukind == U_REAL) {
+                    std::vector<double> v;
                     for (int e = 0; e < 16; e++) {
-                        u.push_back(d.U[2 * e]);
+                        v.push_back(d.U[2 * e]);
                     }
+                    in.uoff = b.put(v);
                 } else if (d.ukind == U_DENSE) {
-                    u.assign(d.U, d.U + 32);
+                    in.uoff = b.put(std::vector<double>(d.U, d.U + 32));
                 }
-                in.uoff = b.put(u);
                 if (G) {
                     in.gkind = static_cast<int8_t>(d.gkind);
                     std::vector<double> g;
@@ -1441,19 +1584,19 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
                 const std::vector<cd> B0 = block2(p.U.mat, lr, 0), B1 = block2(p.U.mat, lr, 1);
                 if (is_diag2(B0) && is_diag2(B1)) {
                     in.ukind = U_DIAG;
-                    in.uoff = b.put(cplx({B0[0], B0[3], B1[0], B1[3]}));
+                    u = cplx({B0[0], B0[3], B1[0], B1[3]});
                 } else if ((is_ident2(B0) || is_x2(B0)) && (is_ident2(B1) || is_x2(B1))) {
                     in.ukind = U_SWAP;
-                    in.uoff = b.put({is_x2(B0) ? 1.0 : 0.0, is_x2(B1) ? 1.0 : 0.0});
+                    u = {is_x2(B0) ? 1.0 : 0.0, is_x2(B1) ? 1.0 : 0.0};
                 } else if (is_real(B0) && is_real(B1)) {
                     in.ukind = U_REAL;
-                    in.uoff = b.put({B0[0].real(), B0[1].real(), B0[2].real(), B0[3].real(),
-                                     B1[0].real(), B1[1].real(), B1[2].real(), B1[3].real()});
+                    u = {B0[0].real(), B0[1].real(), B0[2].real(), B0[3].real(),
+                         B1[0].real(), B1[1].real(), B1[2].real(), B1[3].real()};
                 } else {
                     in.ukind = U_DENSE;
-                    std::vector<double> u = cplx(B0), u1 = cplx(B1);
-                    u.insert(u.end(), u1.begin(), u1.end());
-                    in.uoff = b.put(u);
+                    std::vector<double> v = cplx(B0), v1 = cplx(B1);
+                    v.insert(v.end(), v1.begin(), v1.end());
+                    in.uoff = b.put(v);
                 }
                 if (G) {
                     const std::vector<cd> G0 = block2(*G, lr, 0), G1 = block2(*G, lr, 1);
@@ -1477,7 +1620,7 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
                 for (int k = 0; k < 4; k++) {
                     f.push_back(p.U.mat[5 * k]);
                 }
-                in.uoff = b.put(cplx(f));
+                u = cplx(f);
                 if (G) {
                     std::vector<double> g;
                     for (int k = 0; k < 4; k++) {
@@ -1487,24 +1630,25 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
                 }
             }
         }
-        b.ins.push_back(in);
+        b.add(in, u);
     }
-    // Store layout: keep bits left in registers go back to lane positions 5
-    // or 4 (whichever holds a bit that is not a keep bit).
-    L.nfin = 0;
+    // Store layout: keep bits left in registers go back to lanes, to the
+    // highest position (the cheapest exchange) that holds no keep bit.
+    RtInstr fin{};
+    fin.slot = -1;
     for (int q = 0; q < keep; q++) {
         const int r = reg_of(q);
         if (r < 0) {
             continue;
         }
-        const int p = !is_keep(lane[5]) ? 5 : 4;
-        if (is_keep(lane[p])) {
-            raise(PLK_ERR_INVALID, "register-tile store layout: no lane position for a low bit");
+        int p = RT_LANE_BITS - 1;
+        while (is_keep(lane[p])) {
+            p--;
         }
-        L.fin_rq[L.nfin] = r;
-        L.fin_rp[L.nfin] = p;
-        L.nfin++;
-        std::swap(reg[r], lane[p]);
+        add_remap(fin, r, p);
+    }
+    if (fin.nremap > 0) {
+        b.add(fin, {});
     }
     for (int r = 0; r < R; r++) {
         L.reg_out[r] = reg[r];
@@ -1514,12 +1658,16 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
     }
     L.ninstr = static_cast<int>(b.ins.size());
     L.nslots = slot;
+    if (slot > RT_SLOTS_MAX) {
+        raise(PLK_ERR_INVALID, "register-tile pass with too many sums");
+    }
     out.off = b.finish();
     return out;
 }
 
 // Programs of every register-tile pass of a plan, uploaded as one blob.
-PlanImage build_image(const std::vector<Step> &steps, const State &s) {
+// nj: observable states per chunk (0: forward).
+PlanImage build_image(const std::vector<Step> &steps, const State &s, int nj) {
     PlanImage img;
     if (s.dtype == PLK_C64) {
         build_seg_tables<float>(steps, s.n, img);
@@ -1533,11 +1681,12 @@ PlanImage build_image(const std::vector<Step> &steps, const State &s) {
         }
     }
     img.progs.resize(steps.size());
-    const int R = rt_register_bits(s.dtype);
+    const int R = rt_reg_bits(s.dtype, nj);
+    double norm = 1.0;
     for (size_t i = 0; i < steps.size(); i++) {
         if (steps[i].tiled && steps[i].pass.rt) {
-            img.progs[i] = s.dtype == PLK_C64 ? build_rt_program<float>(steps[i].pass, s.n, R, img.rt)
-                                              : build_rt_program<double>(steps[i].pass, s.n, R, img.rt);
+            img.progs[i] = s.dtype == PLK_C64 ? build_rt_program<float>(steps[i].pass, s.n, R, img.rt, norm)
+                                              : build_rt_program<double>(steps[i].pass, s.n, R, img.rt, norm);
         }
     }
     return img;
@@ -1546,7 +1695,7 @@ PlanImage build_image(const std::vector<Step> &steps, const State &s) {
 size_t image_bytes(const PlanImage &img) {
     auto up = [](size_t x) { return (x + 255) & ~size_t{255}; };
     return up(img.ops.size()) + up(img.bundles.size() * sizeof(TileBundle)) + up(img.rt.size()) +
-           up(img.mats.size());
+           up(img.mats.size()) + up(img.entries.size() * sizeof(RtEntry));
 }
 
 // Copies the image's tables to base (image_bytes(img) bytes) on the device's
@@ -1568,6 +1717,7 @@ PlanPlace copy_image(Device &dev, const PlanImage &img, unsigned char *base) {
         put(img.bundles.data(), img.bundles.size() * sizeof(TileBundle)));
     pl.rt = put(img.rt.data(), img.rt.size());
     pl.mats = put(img.mats.data(), img.mats.size());
+    pl.entries = reinterpret_cast<const RtEntry *>(put(img.entries.data(), img.entries.size() * sizeof(RtEntry)));
     return pl;
 }
 
@@ -1579,6 +1729,7 @@ PlanPlace place_addresses(const PlanImage &img, unsigned char *base) {
     pl.bundles = reinterpret_cast<const TileBundle *>(base + up(img.ops.size()));
     pl.rt = base + up(img.ops.size()) + up(img.bundles.size() * sizeof(TileBundle));
     pl.mats = pl.rt + up(img.rt.size());
+    pl.entries = reinterpret_cast<const RtEntry *>(pl.mats + up(img.mats.size()));
     return pl;
 }
 
@@ -1594,7 +1745,8 @@ void append_signature(const PlanImage &img, std::vector<unsigned char> &sig) {
         const auto *b = static_cast<const unsigned char *>(p);
         sig.insert(sig.end(), b, b + bytes);
     };
-    const uint64_t sizes[4] = {img.ops.size(), img.bundles.size(), img.rt.size(), img.mats.size()};
+    const uint64_t sizes[5] = {img.ops.size(), img.bundles.size(), img.rt.size(), img.mats.size(),
+                               img.entries.size()};
     put(sizes, sizeof sizes);
     for (const StepMeta &m : img.singles) {
         put(&m.ok, sizeof m.ok);
@@ -1618,7 +1770,7 @@ void append_signature(const PlanImage &img, std::vector<unsigned char> &sig) {
 }
 
 // Observable states per register-tile chunk: 3 keeps phi plus three states
-// and the spare buffer at two wavefronts per SIMD. When a pass has fewer
+// in the registers of three wavefronts per SIMD. When a pass has fewer
 // tiles than the device has CUs, chunks of one state give the launch more
 // blocks (12 qubits complex128, 12 observables: 0.63 ms per Jacobian against
 // 0.74 with chunks of 3). PLK_RTILE_NJ overrides, up to RT_NJMAX.
@@ -1627,9 +1779,14 @@ int rtile_chunk(int dtype, int n, int num_cus) {
     if (e > 0) {
         return std::min(RT_NJMAX, e);
     }
-    const int T = (dtype == PLK_C64 ? 4 : 3) + RT_LANE_BITS;
+    const int T = rt_reg_bits(dtype, 3) + RT_LANE_BITS;
     const bool few_tiles = n - T < 30 && (int64_t{1} << std::max(0, n - T)) < num_cus;
     return few_tiles ? 1 : 3;
+}
+
+// Observable states of the widest chunk of a sweep.
+int sweep_chunk(int dtype, int n, size_t n_obs, int num_cus) {
+    return chunk_sizes(n_obs, rtile_chunk(dtype, n, num_cus)).front();
 }
 
 // Register-tile passes serve every state of at least one register tile:
@@ -1637,9 +1794,8 @@ int rtile_chunk(int dtype, int n, int num_cus) {
 // LDS tile passes at every size from 10 to 21 qubits in both precisions
 // (6-layer adjoint, 9 observables, complex128: 0.70 vs 2.52 ms at 10 qubits,
 // 1.32 vs 2.12 at 16, 8.35 vs 11.26 at 21). PLK_RTILE=0 turns them off.
-bool use_rtile(int n, int dtype) {
-    const int T = rt_register_bits(dtype) + RT_LANE_BITS;
-    return env_int("PLK_RTILE", -1) != 0 && n >= T;
+bool use_rtile(int n, int dtype, int nj) {
+    return env_int("PLK_RTILE", -1) != 0 && n >= rt_reg_bits(dtype, nj) + RT_LANE_BITS;
 }
 
 void apply_single(Device &dev, const State &s, const CompiledOp &op);
@@ -1652,9 +1808,10 @@ void enqueue_forward(Device &dev, const State &s, const std::vector<Step> &steps
         if (steps[i].tiled && steps[i].pass.rt) {
             RtLaunch L = img.progs[i].L;
             L.nj = 0;
+            L.nc = L.nbig = 1;
             L.write_phi = 1;
             L.nslots = 0;
-            launch_rtile(dev, s, nullptr, nullptr, pl.rt + img.progs[i].off, L);
+            launch_rtile(dev, s, nullptr, nullptr, pl.rt + img.progs[i].off, L, nullptr);
         } else if (steps[i].fused) {
             SegLaunch L = img.metas[i].L;
             L.write_phi = 1;
@@ -1672,7 +1829,7 @@ void enqueue_forward(Device &dev, const State &s, const std::vector<Step> &steps
             L.nj = 0;
             L.trainable = 0;
             L.write_phi = 1;
-            launch_step(dev, s, nullptr, pl.mats + img.singles[i].off, L);
+            launch_step(dev, s, nullptr, pl.mats + img.singles[i].off, L, nullptr);
         } else {
             apply_single(dev, s, steps[i].single.U);
         }
@@ -1680,7 +1837,7 @@ void enqueue_forward(Device &dev, const State &s, const std::vector<Step> &steps
 }
 
 void run_forward(Device &dev, const State &s, const std::vector<Step> &steps) {
-    const PlanImage img = build_image(steps, s);
+    const PlanImage img = build_image(steps, s, 0);
     enqueue_forward(dev, s, steps, img, place_in_arena(dev, img));
     // The host image is read by the stream's copies.
     PLK_HIP(hipStreamSynchronize(dev.stream));
@@ -1844,9 +2001,9 @@ std::vector<Step> forward_plan(const OpsData &ops, int n, int dtype) {
                          ops.matrices[i], n);
         v.push_back(std::move(p));
     }
-    if (use_rtile(n, dtype)) {
-        return plan_tiles(std::move(v), n, rt_register_bits(dtype) + RT_LANE_BITS, low_bits(dtype),
-                          RT_PMAX, false, rt_register_bits(dtype) + 2);
+    if (use_rtile(n, dtype, 0)) {
+        return plan_tiles(std::move(v), n, rt_reg_bits(dtype, 0) + RT_LANE_BITS, low_bits(dtype),
+                          RT_SLOTS_MAX, false);
     }
     const int T = tile_bits_forward(n, dtype);
     if (T > 0) {
@@ -1927,6 +2084,129 @@ struct Hasher {
 // U^dagger on every H lambda) is replaced by fused passes.
 // ---------------------------------------------------------------------------
 
+// One launch of a register-tile pass or of a single-op step: its observables
+// j0 .. j0 + width and where its FP64 partials start.
+struct PartLaunch {
+    size_t j0 = 0;
+    int width = 0;
+    RtLaunch rt{};
+    StepLaunch step{};
+    size_t offset = 0; // doubles from the device's partials buffer
+};
+
+// The launches of a reverse plan and the reductions of their partials. Every
+// pass keeps its partials until a flush, which forms all Jacobian entries
+// since the last one in one launch (a launch per pass costs small circuits
+// as much as the passes themselves).
+struct SweepParts {
+    std::vector<std::vector<PartLaunch>> steps;
+    struct Flush {
+        size_t step;         // after this step
+        size_t first, count; // entries
+    };
+    std::vector<Flush> flushes;
+    size_t doubles = 0;
+};
+
+constexpr size_t kPartialsMax = size_t{1} << 26; // doubles kept between flushes
+
+// Places the partials of every launch and fills img.entries.
+SweepParts place_partials(Device &dev, const std::vector<Step> &steps, PlanImage &img, const State &s,
+                          size_t n_obs, bool alt) {
+    SweepParts sp;
+    sp.steps.resize(steps.size());
+    size_t used = 0, first = 0;
+    auto flush = [&](size_t i) {
+        if (img.entries.size() > first) {
+            sp.flushes.push_back({i, first, img.entries.size() - first});
+            first = img.entries.size();
+        }
+        used = 0;
+    };
+    auto take = [&](size_t i, PartLaunch &pl, size_t doubles) {
+        if (used + doubles > kPartialsMax && i > 0 && used > 0 && sp.steps[i].empty()) {
+            flush(i - 1);
+        }
+        pl.offset = used;
+        used += doubles;
+        sp.doubles = std::max(sp.doubles, used);
+    };
+    auto entry = [](const PartLaunch &pl, int blocks, int col) {
+        RtEntry e{};
+        e.base = pl.offset;
+        e.row[0] = e.row[1] = e.row[2] = -1;
+        e.blocks = blocks;
+        e.col = col;
+        e.j0 = static_cast<int32_t>(pl.j0);
+        e.width = pl.width;
+        return e;
+    };
+    for (size_t i = 0; i < steps.size(); i++) {
+        const Step &st = steps[i];
+        if (st.tiled && st.pass.rt) {
+            // The chunks (balanced: widths nj and nj - 1, wider first) run side
+            // by side in one launch, up to RT_OBS_MAX states, when lambda has a
+            // second buffer.
+            const std::vector<int> sizes = chunk_sizes(n_obs, rtile_chunk(s.dtype, s.n, dev.num_cus));
+            size_t j0 = 0;
+            for (size_t ci = 0; ci < sizes.size();) {
+                PartLaunch pl;
+                RtLaunch &L = pl.rt;
+                L = img.progs[i].L;
+                L.nj = sizes[0];
+                L.nc = 1;
+                L.nbig = sizes[ci] == L.nj ? 1 : 0;
+                pl.width = sizes[ci];
+                while (alt && ci + L.nc < sizes.size() && pl.width + sizes[ci + L.nc] <= RT_OBS_MAX) {
+                    pl.width += sizes[ci + L.nc];
+                    L.nbig += sizes[ci + L.nc] == L.nj ? 1 : 0;
+                    L.nc++;
+                }
+                pl.j0 = j0;
+                L.write_phi = j0 + pl.width == n_obs ? 1 : 0;
+                const int blocks = rtile_blocks(dev, s.dtype, L);
+                take(i, pl, static_cast<size_t>(L.nslots) * pl.width * blocks);
+                for (const RtTerm &t : img.progs[i].terms) {
+                    RtEntry e = entry(pl, blocks, t.col);
+                    for (int k = 0; k < 3; k++) {
+                        e.row[k] = t.slot[k] < 0 ? -1 : t.slot[k] * pl.width;
+                        e.m[k] = t.m[k];
+                    }
+                    img.entries.push_back(e);
+                }
+                j0 += pl.width;
+                ci += L.nc;
+                sp.steps[i].push_back(pl);
+            }
+        } else if (!st.fused && !st.tiled && img.singles[i].ok) {
+            const StepMeta &m = img.singles[i];
+            size_t j0 = 0;
+            for (int nj : chunk_sizes(n_obs, SEG_NJMAX)) {
+                PartLaunch pl;
+                pl.step = m.L;
+                pl.step.nj = nj;
+                pl.j0 = j0;
+                pl.width = nj;
+                pl.step.write_phi = (j0 + nj == n_obs) ? 1 : 0;
+                if (m.L.trainable) {
+                    const int blocks = step_blocks(dev, pl.step);
+                    take(i, pl, static_cast<size_t>(nj) * blocks);
+                    RtEntry e = entry(pl, blocks, m.col);
+                    e.row[0] = 0;
+                    e.m[0] = m.coef;
+                    img.entries.push_back(e);
+                }
+                j0 += nj;
+                sp.steps[i].push_back(pl);
+            }
+        }
+    }
+    if (!steps.empty()) {
+        flush(steps.size() - 1);
+    }
+    return sp;
+}
+
 // Launches reverse step i (a fused segment, register-tile or LDS-tile pass
 // over lambda and every H_j lambda, with its Jacobian reductions); returns
 // false for a single op, which the caller runs.
@@ -1939,7 +2219,7 @@ struct PhiPair {
 
 bool enqueue_reverse_step(Device &dev, PhiPair &phi, void *const *hptr, size_t n_obs,
                           size_t n_tp, const Step &st, const PlanImage &img, size_t i,
-                          const PlanPlace &pl, double *d_jac) {
+                          const PlanPlace &pl, const SweepParts &parts, double *d_jac) {
     const State &lambda = phi.cur;
     if (st.fused) {
         const SegMeta &m = img.metas[i];
@@ -1967,55 +2247,19 @@ bool enqueue_reverse_step(Device &dev, PhiPair &phi, void *const *hptr, size_t n
         return true;
     }
     if (st.tiled && st.pass.rt) {
-        // The chunks (balanced: widths nj and nj - 1, wider first) run side
-        // by side in one launch, up to RT_OBS_MAX states, when lambda has a
-        // second buffer.
-        const std::vector<int> sizes = chunk_sizes(n_obs, rtile_chunk(lambda.dtype, lambda.n, dev.num_cus));
-        size_t j0 = 0, ci = 0;
-        while (ci < sizes.size()) {
-            const int nj = sizes[ci];
-            int nc = 1, nbig = 1;
-            size_t width = static_cast<size_t>(nj);
-            while (phi.alt.d != nullptr && ci + nc < sizes.size() &&
-                   width + static_cast<size_t>(sizes[ci + nc]) <= static_cast<size_t>(RT_OBS_MAX)) {
-                width += static_cast<size_t>(sizes[ci + nc]);
-                nbig += sizes[ci + nc] == nj ? 1 : 0;
-                nc++;
-            }
-            RtLaunch L = img.progs[i].L;
-            L.nj = nj;
-            L.nc = nc;
-            L.nbig = nbig;
-            L.write_phi = (j0 + width == n_obs) ? 1 : 0;
-            const bool swap = L.write_phi && phi.alt.d != nullptr;
-            const int grid = launch_rtile(dev, phi.cur, swap ? &phi.alt : nullptr, hptr + j0,
-                                          pl.rt + img.progs[i].off, L);
-            if (L.nslots > 0) {
-                launch_tile_reduce(dev, grid, L.nslots, static_cast<int>(width), static_cast<int>(j0),
-                                   st.pass.cols.data(), st.pass.coefs.data(), d_jac,
-                                   static_cast<int>(n_tp));
-            }
+        for (const PartLaunch &l : parts.steps[i]) {
+            const bool swap = l.rt.write_phi && phi.alt.d != nullptr;
+            launch_rtile(dev, phi.cur, swap ? &phi.alt : nullptr, hptr + l.j0, pl.rt + img.progs[i].off, l.rt,
+                         dev.parts + l.offset);
             if (swap) {
                 std::swap(phi.cur, phi.alt);
             }
-            j0 += width;
-            ci += nc;
         }
         return true;
     }
     if (!st.fused && !st.tiled && img.singles[i].ok) {
-        const StepMeta &m = img.singles[i];
-        size_t j0 = 0;
-        for (int nj : chunk_sizes(n_obs, SEG_NJMAX)) {
-            StepLaunch L = m.L;
-            L.nj = nj;
-            L.write_phi = (j0 + nj == n_obs) ? 1 : 0;
-            const int grid = launch_step(dev, lambda, hptr + j0, pl.mats + m.off, L);
-            if (L.trainable) {
-                launch_tile_reduce(dev, grid, 1, nj, static_cast<int>(j0), &m.col, &m.coef, d_jac,
-                                   static_cast<int>(n_tp));
-            }
-            j0 += nj;
+        for (const PartLaunch &l : parts.steps[i]) {
+            launch_step(dev, lambda, hptr + l.j0, pl.mats + img.singles[i].off, l.step, dev.parts + l.offset);
         }
         return true;
     }
@@ -2040,6 +2284,17 @@ bool enqueue_reverse_step(Device &dev, PhiPair &phi, void *const *hptr, size_t n
     return false;
 }
 
+// Forms the Jacobian entries whose partials end with step i.
+void enqueue_flush(Device &dev, const SweepParts &parts, const PlanPlace &pl, size_t i, size_t n_obs,
+                   size_t n_tp, double *d_jac) {
+    for (const auto &f : parts.flushes) {
+        if (f.step == i) {
+            launch_rtile_entries(dev, dev.parts, pl.entries + f.first, static_cast<int>(f.count),
+                                 static_cast<int>(n_obs), d_jac, static_cast<int>(n_tp));
+        }
+    }
+}
+
 // A captured sweep: copy of the input state, forward passes, observables,
 // Jacobian zero fill and reverse passes of one circuit structure, replayed
 // with a fresh upload of the plan and Pauli tables (angles and coefficients
@@ -2057,7 +2312,7 @@ struct SweepGraph {
     void *tables = nullptr;
     size_t fwd_bytes = 0, rev_bytes = 0;
     double *jac = nullptr;
-    double *red = nullptr;
+    double *red = nullptr, *parts = nullptr;
     hipGraphExec_t exec = nullptr;
     ~SweepGraph() {
         (void)hipSetDevice(device);
@@ -2188,16 +2443,18 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
     if (n_obs == 0) {
         return;
     }
-    const bool rt = use_rtile(n, ref.dtype);
-    const int T_adj = rt ? rt_register_bits(ref.dtype) + RT_LANE_BITS : tile_bits_adjoint(n, ref.dtype);
+    const int nj = sweep_chunk(ref.dtype, n, n_obs, dev.num_cus);
+    const bool rt = use_rtile(n, ref.dtype, nj);
+    const int T_adj = rt ? rt_reg_bits(ref.dtype, nj) + RT_LANE_BITS : tile_bits_adjoint(n, ref.dtype);
     const std::vector<Step> steps =
-        rt ? plan_tiles(std::move(rev), n, T_adj, low_bits(ref.dtype), RT_PMAX, false,
-                        rt_register_bits(ref.dtype) + 2)
+        rt ? plan_tiles(std::move(rev), n, T_adj, low_bits(ref.dtype), RT_SLOTS_MAX, false)
            : T_adj > 0 ? plan_tiles(std::move(rev), n, T_adj, low_bits(ref.dtype))
                        : plan_steps(std::move(rev));
     const std::vector<Step> fwd = apply_ops ? forward_plan(ops, n, ref.dtype) : std::vector<Step>{};
-    const PlanImage img_f = build_image(fwd, ref);
-    const PlanImage img_r = build_image(steps, ref);
+    const PlanImage img_f = build_image(fwd, ref, 0);
+    PlanImage img_r = build_image(steps, ref, nj);
+    const bool alt = needs_alt(dev, steps, n_obs, ref.dtype, n);
+    const SweepParts parts = place_partials(dev, steps, img_r, ref, n_obs, alt);
     plan_scope.reset();
 
     // Small circuits run as a replayed HIP graph: their sweeps are hundreds
@@ -2248,7 +2505,7 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
             SweepGraph &c = **it;
             const bool same = c.key == key && c.ref == ref.d;
             if (same) {
-                if (c.sig != sig || c.red != dev.red) {
+                if (c.sig != sig || c.red != dev.red || c.parts != dev.parts) {
                     list.erase(it); // stale layout or partials buffer: capture again
                 } else {
                     std::rotate(it, it + 1, list.end()); // most recently used last
@@ -2276,7 +2533,7 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
             ng->ref = ref.d;
             ng->sig = sig;
             ng->lambda = std::make_unique<TmpState>(n, ref.dtype, ref.device);
-            if (needs_alt(dev, steps, n_obs, ref.dtype, n)) {
+            if (alt) {
                 ng->lambda2 = std::make_unique<TmpState>(n, ref.dtype, ref.device);
             }
             for (size_t j = 0; j < n_obs; j++) {
@@ -2290,10 +2547,8 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
             ng->jac = static_cast<double *>(dev_malloc(dev.id, sizeof(double) * n_obs * n_tp, "graph Jacobian"));
             // The launchers grow the partials buffer on demand, which would
             // synchronise inside the capture: size it for any pass first.
-            ensure_red(dev,
-                       static_cast<size_t>(dev.num_cus) * 32 * std::max(TILE_PMAX, RT_PMAX) *
-                           std::max(RT_NJMAX, SEG_NJMAX),
-                       256);
+            ensure_red(dev, static_cast<size_t>(dev.num_cus) * 32 * TILE_PMAX * SEG_NJMAX, 256);
+            ensure_parts(dev, parts.doubles);
             auto *tb = static_cast<unsigned char *>(ng->tables);
             // Addresses only: the tables are copied before every replay.
             const PlanPlace pf = place_addresses(img_f, tb);
@@ -2312,7 +2567,8 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
                 PhiPair phi{lam, ng->lambda2 ? ng->lambda2->s : State{}};
                 for (size_t i = 0; i < steps.size(); i++) {
                     enqueue_reverse_step(dev, phi, ng->hptr.data(), n_obs, n_tp, steps[i], img_r,
-                                         i, pr, ng->jac);
+                                         i, pr, parts, ng->jac);
+                    enqueue_flush(dev, parts, pr, i, n_obs, n_tp, ng->jac);
                 }
                 hipGraph_t graph_def = cap.end();
                 const hipError_t e = hipGraphInstantiate(&ng->exec, graph_def, nullptr, nullptr, 0);
@@ -2320,6 +2576,7 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
                 PLK_HIP(e);
             }
             ng->red = dev.red;
+            ng->parts = dev.parts;
             list.push_back(std::move(ng));
             g = list.back().get();
         }
@@ -2364,14 +2621,16 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
     std::vector<std::pair<size_t, double>> host_entries; // (flat index, value)
 
     const PlanPlace pl = place_in_arena(dev, img_r);
+    ensure_parts(dev, parts.doubles);
     std::unique_ptr<TmpState> mu, lambda2;
-    if (needs_alt(dev, steps, n_obs, ref.dtype, n)) {
+    if (alt) {
         lambda2 = std::make_unique<TmpState>(n, ref.dtype, ref.device);
     }
     PhiPair phi{lambda.s, lambda2 ? lambda2->s : State{}};
     for (size_t i = 0; i < steps.size(); i++) {
         const Step &st = steps[i];
-        if (enqueue_reverse_step(dev, phi, hptr.data(), n_obs, n_tp, st, img_r, i, pl, d_jac)) {
+        if (enqueue_reverse_step(dev, phi, hptr.data(), n_obs, n_tp, st, img_r, i, pl, parts, d_jac)) {
+            enqueue_flush(dev, parts, pl, i, n_obs, n_tp, d_jac);
             continue;
         }
         const PlanOp &p = st.single;
@@ -2394,6 +2653,7 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
         for (size_t j = 0; j < n_obs; j++) {
             apply_single(dev, H[j]->s, p.U);
         }
+        enqueue_flush(dev, parts, pl, i, n_obs, n_tp, d_jac);
     }
     PLK_HIP(hipMemcpyAsync(jac, d_jac, sizeof(double) * n_obs * n_tp, hipMemcpyDeviceToHost,
                            dev.stream));

@@ -3,15 +3,16 @@
 //
 // Each wavefront owns one tile at a time: the 2^(R+6) amplitudes whose index
 // bits outside the pass's tile bits are fixed. Every lane holds 2^R of them
-// per state (R register bits: 3 for complex128, 4 for complex64, so a lane
-// holds 128 bytes of each state); the 6 lane bits select the lane. Which tile
+// per state (R register bits); the 6 lane bits select the lane. Which tile
 // bit sits on which register bit or lane position is the pass's layout,
 // chosen on the host and changed by remaps.
 //
-// A pass program is a list of 32-byte instructions read through the scalar
-// cache. Each instruction first applies up to two remaps -- exchanges of a
-// register bit with lane position 4 or 5, one v_permlane16/32_swap per
-// 32-bit word pair, in place -- then one operation:
+// A pass program is a list of fixed-size instructions read through the scalar
+// cache: a 32-byte header and the eight reals most operations need. The next
+// instruction is fetched while the current one runs, so its latency is off
+// the critical path; only wider payloads are read where they are used. An
+// instruction first applies up to two remaps -- exchanges of a register bit
+// with a lane position, in place -- then one operation:
 //   RT_REG1   one wire on register bit a;
 //   RT_REG2   two wires on register bits a > b;
 //   RT_SEL    mixing register bit a, with the op's other wire on lane position
@@ -22,25 +23,35 @@
 // A selector s0 / s1 of 64 + b names a global index bit b outside the tile
 // instead of a lane: its value is fixed for the whole tile, so an operation
 // whose non-mixing wires (a control, a diagonal factor) lie outside the tile
-// needs no tile bit for them.
+// needs no tile bit for them, and RT_SEL becomes RT_REG1 with one block.
 //
-// Operations write out of place. The NS states (phi and NS - 1 observable
-// states) live in NS + 1 register buffers: each operation writes state s into
-// the buffer that is free at that moment, which leaves the buffer state s
-// occupied free for state s + 1. After one instruction every state has moved
-// one buffer down (state s in buffer (s - rot) mod (NS + 1) after rot
-// instructions), so the instruction loop is unrolled NS + 1 times with the
-// buffer indices as constants: no register copies between instructions and
-// one spare buffer instead of a second copy of every state.
+// Operations work in place on the register tile. A second copy of one state
+// (out-of-place application through a rotating spare buffer) costs a quarter
+// of the registers at four states and unrolls the whole instruction switch
+// once per buffer position: 398 KB of code against a 64 KB instruction cache.
+// In place the four-state kernel has 164 KB, of which a pass runs a part, and
+// 168 VGPRs (three waves per SIMD instead of two).
 //
-// A trainable operation forms G phi in the free buffer and adds the FP64
-// products Im<h_j | G phi> of the lane's amplitudes; the four lanes of each
-// quad are summed by DPP and one lane adds the total into LDS (ds_add_f64,
-// one address per quad, so the order is fixed). After its last tile the
-// wavefront writes per-block partials; a second kernel sums them in a fixed
-// order. No LDS staging of states and no barriers: each wavefront streams its
-// tiles independently, which keeps HBM busy while other wavefronts compute.
-#include <map>
+// Bound (24 qubits complex128, 9 observables, 37 passes of 26 gates): HBM and
+// FP64 issue together, 1.57 ms a pass = 3.4 TB/s of the in-place ceiling of
+// 5.2, vector issue 54 % busy, the waves waiting for memory 41 % of their time;
+// out of place with five mixed bits a pass: 1.74 ms and 50 passes. One state
+// (26-qubit gate stream): 0.52 ms a pass, 4.1 TB/s, 37 passes for 600 gates
+// where the three-register-bit tile took 66 passes of 0.47 ms.
+//
+// The host fuses the one-wire gates that follow each other on a wire into one
+// 2x2 matrix. For trainable gates V_1, V_2, ... of such a run the derivative
+// of the k-th is Im<h| (V_{k-1}...V_1)^dag G_k (V_{k-1}...V_1) |phi> with phi
+// and h as they enter the run, and that operator is a real combination of X,
+// Y and Z of the wire. So the run adds the FP64 sums Im<h_j|X phi>,
+// Im<h_j|Y phi>, Im<h_j|Z phi> once (only those it needs) and the reduction
+// forms every gate's derivative from them.
+//
+// The four lanes of each quad are summed by DPP and one lane adds the total
+// into LDS (ds_add_f64, one address per quad, so the order is fixed). After
+// its last tile the wavefront writes per-block partials; a second kernel sums
+// them in a fixed order. No LDS staging of states and no barriers: each
+// wavefront streams its tiles independently.
 #include <utility>
 
 #include "device_common.hpp"
@@ -51,8 +62,6 @@ namespace {
 
 template <typename T> using CT = const __attribute__((address_space(4))) T;
 
-template <typename T> constexpr int rt_r() { return sizeof(T) == 8 ? 3 : 4; }
-
 __device__ __forceinline__ bool lbit(int lane, int p) { return (lane >> p) & 1; }
 
 // Block selector of RT_SEL / RT_LANE: a lane position (0-5), or 64 + a
@@ -62,253 +71,176 @@ __device__ __forceinline__ bool selbit(int lane, uint64_t tbase, int s) {
     return s < 64 ? lbit(lane, s) : ((tbase >> (s - 64)) & 1);
 }
 
-// Buffer of state s before (in) and after (out) instruction number `ROT`
-// (mod NS + 1) of the rotation.
-template <int NS, int ROT> struct Rot {
-    static constexpr int NB = NS + 1;
-    static constexpr int in(int s) { return ((s - ROT) % NB + NB) % NB; }
-    static constexpr int out(int s) { return s == 0 ? ((NS - ROT) % NB + NB) % NB : in(s - 1); }
-};
-
 // ---------------------------------------------------------------------------
-// Remap: exchange register bit Q with lane position P (4 or 5), in place.
-// Afterwards lanes whose lane bit P is 1 hold the partner's b in a, and lanes
-// whose bit is 0 hold the partner's a in b (v_permlane16_swap swaps the odd
-// 16-lane rows of its first operand with the even rows of its second,
-// v_permlane32_swap the upper half of the first with the lower half of the
-// second).
+// Remap: exchange register bit Q with lane position P, in place. Afterwards
+// lanes whose lane bit P is 1 hold the partner's b in a, and lanes whose bit
+// is 0 hold the partner's a in b. Positions 5 and 4 are one
+// v_permlane32/16_swap per 32-bit word pair; the others take three
+// instructions (DPP within the 16-lane row: rotate by 8 or shift by 4 with
+// the bank mask selecting the lanes written, quad permutations with selects).
+// So any of a tile's bits can be mixed in a pass, 9 to 11 instead of the 5 or
+// 6 that registers and positions 5 and 4 hold.
 // ---------------------------------------------------------------------------
-template <int P> __device__ __forceinline__ void xchg_word(uint32_t &a, uint32_t &b) {
-    static_assert(P == 4 || P == 5, "remaps use lane positions 4 and 5");
+template <int P> __device__ __forceinline__ void xchg_word(uint32_t &a, uint32_t &b, int lane) {
+    const int ia = static_cast<int>(a), ib = static_cast<int>(b);
     if constexpr (P == 5) {
         const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
         a = r[0];
         b = r[1];
-    } else {
+    } else if constexpr (P == 4) {
         const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
         a = r[0];
         b = r[1];
+    } else if constexpr (P == 3) {
+        a = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(ia, ib, 0x128, 0xF, 0xC, false));
+        b = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(ib, ia, 0x128, 0xF, 0x3, false));
+    } else if constexpr (P == 2) {
+        a = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(ia, ib, 0x114, 0xF, 0xA, false));
+        b = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(ib, ia, 0x104, 0xF, 0x5, false));
+    } else {
+        constexpr int ctrl = P == 1 ? 0x4E : 0xB1;
+        const bool hi = lbit(lane, P);
+        const int s = hi ? ia : ib;
+        const int r = __builtin_amdgcn_mov_dpp(s, ctrl, 0xF, 0xF, false);
+        a = static_cast<uint32_t>(hi ? r : ia);
+        b = static_cast<uint32_t>(hi ? ib : r);
     }
 }
 
-template <int P> __device__ __forceinline__ void xchg(double &a, double &b) {
+template <int P> __device__ __forceinline__ void xchg(double &a, double &b, int lane) {
     uint64_t ua = __double_as_longlong(a), ub = __double_as_longlong(b);
     uint32_t a0 = static_cast<uint32_t>(ua), a1 = static_cast<uint32_t>(ua >> 32);
     uint32_t b0 = static_cast<uint32_t>(ub), b1 = static_cast<uint32_t>(ub >> 32);
-    xchg_word<P>(a0, b0);
-    xchg_word<P>(a1, b1);
+    xchg_word<P>(a0, b0, lane);
+    xchg_word<P>(a1, b1, lane);
     a = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(a1) << 32) | a0));
     b = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(b1) << 32) | b0));
 }
 
-template <int P> __device__ __forceinline__ void xchg(float &a, float &b) {
+template <int P> __device__ __forceinline__ void xchg(float &a, float &b, int lane) {
     uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
-    xchg_word<P>(ua, ub);
+    xchg_word<P>(ua, ub, lane);
     a = __uint_as_float(ua);
     b = __uint_as_float(ub);
 }
 
-template <typename T, int A, int Q, int P> __device__ __forceinline__ void remap1(Cx<T> (&v)[A]) {
-#pragma unroll
-    for (int k = 0; k < A; k++) {
-        if (k & (1 << Q)) {
-            continue;
+template <int R, typename F> __device__ __forceinline__ void dispatch_q(int q, F &&f) {
+    if (q == 0) {
+        f(IC<0>{});
+    } else if (q == 1) {
+        f(IC<1>{});
+    } else if (R <= 3 || q == 2) {
+        f(IC<2>{});
+    } else if constexpr (R > 3) {
+        if (R <= 4 || q == 3) {
+            f(IC<3>{});
+        } else if constexpr (R > 4) {
+            f(IC<4>{});
         }
-        xchg<P>(v[k].r, v[k | (1 << Q)].r);
-        xchg<P>(v[k].i, v[k | (1 << Q)].i);
     }
 }
 
-// ---------------------------------------------------------------------------
-// Per-lane selection among uniform blocks: block c = bit s0 + 2 bit s1.
-// ---------------------------------------------------------------------------
-template <typename T, int NV>
-__device__ __forceinline__ void select_block(T (&out)[NV], CT<T> *base, int nb, bool c0, bool c1) {
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-        const T x0 = base[i], x1 = base[NV + i];
-        T lo = c0 ? x1 : x0;
-        if (nb == 4) {
-            const T x2 = base[2 * NV + i], x3 = base[3 * NV + i];
-            const T hi = c0 ? x3 : x2;
-            lo = c1 ? hi : lo;
+// Register bits a > b.
+template <int R, typename F> __device__ __forceinline__ void dispatch_q2(int a, int b, F &&f) {
+    if (a == 1) {
+        f(IC<1>{}, IC<0>{});
+    } else if (R <= 3 || a == 2) {
+        if (b == 0) {
+            f(IC<2>{}, IC<0>{});
+        } else {
+            f(IC<2>{}, IC<1>{});
         }
-        out[i] = lo;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Out-of-place operations on one state: dst = U src.
-// ---------------------------------------------------------------------------
-template <typename T, int A, int Q>
-__device__ __forceinline__ void u1_diag(Cx<T> (&d)[A], const Cx<T> (&s)[A], Cx<T> u0, Cx<T> u1) {
-#pragma unroll
-    for (int k = 0; k < A; k++) {
-        d[k] = cmul((k >> Q) & 1 ? u1 : u0, s[k]);
-    }
-}
-
-template <typename T, int A, int Q>
-__device__ __forceinline__ void u1_real(Cx<T> (&d)[A], const Cx<T> (&s)[A], T m00, T m01, T m10,
-                                        T m11) {
-#pragma unroll
-    for (int k = 0; k < A; k++) {
-        if (k & (1 << Q)) {
-            continue;
-        }
-        const Cx<T> a = s[k], b = s[k | (1 << Q)];
-        d[k] = {fma(m00, a.r, m01 * b.r), fma(m00, a.i, m01 * b.i)};
-        d[k | (1 << Q)] = {fma(m10, a.r, m11 * b.r), fma(m10, a.i, m11 * b.i)};
-    }
-}
-
-template <typename T, int A, int Q>
-__device__ __forceinline__ void u1_dense(Cx<T> (&d)[A], const Cx<T> (&s)[A], Cx<T> u00, Cx<T> u01,
-                                         Cx<T> u10, Cx<T> u11) {
-#pragma unroll
-    for (int k = 0; k < A; k++) {
-        if (k & (1 << Q)) {
-            continue;
-        }
-        const Cx<T> a = s[k], b = s[k | (1 << Q)];
-        d[k] = cmad(u01, b, cmul(u00, a));
-        d[k | (1 << Q)] = cmad(u11, b, cmul(u10, a));
-    }
-}
-
-// The per-lane condition selects between values, never between array
-// elements (a select of two element addresses would put the whole register
-// tile in scratch memory).
-template <typename T, int A, int Q>
-__device__ __forceinline__ void u1_swap(Cx<T> (&d)[A], const Cx<T> (&s)[A], bool on) {
-#pragma unroll
-    for (int k = 0; k < A; k++) {
-        const Cx<T> x = s[k ^ (1 << Q)], y = s[k];
-        d[k] = {on ? x.r : y.r, on ? x.i : y.i};
-    }
-}
-
-template <int QA, int QB> __device__ __forceinline__ constexpr int lidx(int k) {
-    return (((k >> QA) & 1) << 1) | ((k >> QB) & 1);
-}
-
-template <typename T, int A, int QA, int QB>
-__device__ __forceinline__ void u2_dense(Cx<T> (&d)[A], const Cx<T> (&s)[A], CT<T> *U) {
-    constexpr int MQ = (1 << QA) | (1 << QB);
-#pragma unroll
-    for (int k = 0; k < A; k++) {
-        if (k & MQ) {
-            continue;
-        }
-        const int idx[4] = {k, k | (1 << QB), k | (1 << QA), k | MQ};
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            Cx<T> t = cmul(Cx<T>{U[8 * r], U[8 * r + 1]}, s[idx[0]]);
-#pragma unroll
-            for (int c = 1; c < 4; c++) {
-                t = cmad(Cx<T>{U[8 * r + 2 * c], U[8 * r + 2 * c + 1]}, s[idx[c]], t);
+    } else if constexpr (R > 3) {
+        if (R <= 4 || a == 3) {
+            if (b == 0) {
+                f(IC<3>{}, IC<0>{});
+            } else if (b == 1) {
+                f(IC<3>{}, IC<1>{});
+            } else {
+                f(IC<3>{}, IC<2>{});
             }
-            d[idx[r]] = t;
-        }
-    }
-}
-
-template <typename T, int A, int QA, int QB>
-__device__ __forceinline__ void u2_real(Cx<T> (&d)[A], const Cx<T> (&s)[A], CT<T> *U) {
-    constexpr int MQ = (1 << QA) | (1 << QB);
-#pragma unroll
-    for (int k = 0; k < A; k++) {
-        if (k & MQ) {
-            continue;
-        }
-        const int idx[4] = {k, k | (1 << QB), k | (1 << QA), k | MQ};
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            T sr = U[4 * r] * s[idx[0]].r, si = U[4 * r] * s[idx[0]].i;
-#pragma unroll
-            for (int c = 1; c < 4; c++) {
-                sr = fma(U[4 * r + c], s[idx[c]].r, sr);
-                si = fma(U[4 * r + c], s[idx[c]].i, si);
+        } else if constexpr (R > 4) {
+            if (b == 0) {
+                f(IC<4>{}, IC<0>{});
+            } else if (b == 1) {
+                f(IC<4>{}, IC<1>{});
+            } else if (b == 2) {
+                f(IC<4>{}, IC<2>{});
+            } else {
+                f(IC<4>{}, IC<3>{});
             }
-            d[idx[r]] = {sr, si};
         }
     }
 }
 
-template <typename T, int A, int QA, int QB>
-__device__ __forceinline__ void u2_diag(Cx<T> (&d)[A], const Cx<T> (&s)[A], CT<T> *U) {
+template <typename T, int NS, int A, int Q, int P>
+__device__ __forceinline__ void remap_qp(Cx<T> (&v)[NS][A], int lane) {
 #pragma unroll
-    for (int k = 0; k < A; k++) {
-        const int r = lidx<QA, QB>(k);
-        d[k] = cmul(Cx<T>{U[2 * r], U[2 * r + 1]}, s[k]);
+    for (int s = 0; s < NS; s++) {
+#pragma unroll
+        for (int k = 0; k < A; k++) {
+            if (k & (1 << Q)) {
+                continue;
+            }
+            xchg<P>(v[s][k].r, v[s][k | (1 << Q)].r, lane);
+            xchg<P>(v[s][k].i, v[s][k | (1 << Q)].i, lane);
+        }
     }
 }
 
-// Local indices LA and LB exchanged, every other amplitude copied.
-template <typename T, int A, int QA, int QB, int LA, int LB>
-__device__ __forceinline__ void u2_swap(Cx<T> (&d)[A], const Cx<T> (&s)[A]) {
-    constexpr int flip = ((((LA ^ LB) >> 1) & 1) << QA) | (((LA ^ LB) & 1) << QB);
-#pragma unroll
-    for (int k = 0; k < A; k++) {
-        const int r = lidx<QA, QB>(k);
-        d[k] = (r == LA || r == LB) ? s[k ^ flip] : s[k];
-    }
+template <typename T, int NS, int R>
+__device__ __forceinline__ void remap(Cx<T> (&v)[NS][1 << R], int q, int p, int lane) {
+    constexpr int A = 1 << R;
+    dispatch_q<R>(q, [&](auto Qc) {
+        constexpr int Q = decltype(Qc)::value;
+        if (p >= 4) {
+            if (p == 5) {
+                remap_qp<T, NS, A, Q, 5>(v, lane);
+            } else {
+                remap_qp<T, NS, A, Q, 4>(v, lane);
+            }
+        } else if (p >= 2) {
+            if (p == 3) {
+                remap_qp<T, NS, A, Q, 3>(v, lane);
+            } else {
+                remap_qp<T, NS, A, Q, 2>(v, lane);
+            }
+        } else if (p == 1) {
+            remap_qp<T, NS, A, Q, 1>(v, lane);
+        } else {
+            remap_qp<T, NS, A, Q, 0>(v, lane);
+        }
+    });
 }
 
-// gf = G f for a one-register-bit generator.
-template <typename T, int A, int Q>
-__device__ __forceinline__ void gen1(Cx<T> (&gf)[A], const Cx<T> (&f)[A], int gkind, CT<T> *G) {
-    if (gkind == G_Z) {
-#pragma unroll
-        for (int k = 0; k < A; k++) {
-            gf[k] = ((k >> Q) & 1) ? Cx<T>{-f[k].r, -f[k].i} : f[k];
-        }
-    } else if (gkind == G_X) {
-#pragma unroll
-        for (int k = 0; k < A; k++) {
-            gf[k] = f[k ^ (1 << Q)];
-        }
-    } else if (gkind == G_Y) {
-        // Y = [[0, -i], [i, 0]]: (Y f)_0 = -i f_1, (Y f)_1 = i f_0.
-#pragma unroll
-        for (int k = 0; k < A; k++) {
-            const Cx<T> p = f[k ^ (1 << Q)];
-            gf[k] = ((k >> Q) & 1) ? Cx<T>{-p.i, p.r} : Cx<T>{p.i, -p.r};
-        }
-    } else if (gkind == G_DIAG) {
-        const T g0 = G[0], g1 = G[1];
-#pragma unroll
-        for (int k = 0; k < A; k++) {
-            const T g = ((k >> Q) & 1) ? g1 : g0;
-            gf[k] = {g * f[k].r, g * f[k].i};
-        }
-    } else {
-        u1_dense<T, A, Q>(gf, f, {G[0], G[1]}, {G[2], G[3]}, {G[4], G[5]}, {G[6], G[7]});
-    }
-}
+// One instruction in scalar registers.
+template <typename T> struct Ins {
+    int32_t w[8];
+    T u[8];
+};
 
-template <typename T, int A, int QA, int QB>
-__device__ __forceinline__ void gen2(Cx<T> (&gf)[A], const Cx<T> (&f)[A], int gkind, CT<T> *G) {
-    if (gkind == G_Z) {
+template <typename T>
+__device__ __forceinline__ Ins<T> fetch(CT<unsigned char> *prog, int pc) {
+    CT<unsigned char> *p = prog + static_cast<int64_t>(pc) * rt_stride<T>();
+    Ins<T> in;
 #pragma unroll
-        for (int k = 0; k < A; k++) {
-            gf[k] = (__builtin_popcount(lidx<QA, QB>(k)) & 1) ? Cx<T>{-f[k].r, -f[k].i} : f[k];
-        }
-    } else if (gkind == G_DIAG) {
-#pragma unroll
-        for (int k = 0; k < A; k++) {
-            const T g = G[lidx<QA, QB>(k)];
-            gf[k] = {g * f[k].r, g * f[k].i};
-        }
-    } else {
-        u2_dense<T, A, QA, QB>(gf, f, G);
+    for (int k = 0; k < 8; k++) {
+        in.w[k] = reinterpret_cast<CT<int32_t> *>(p)[k];
     }
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        in.u[k] = reinterpret_cast<CT<T> *>(p + 32)[k];
+    }
+    return in;
 }
 
 // ---------------------------------------------------------------------------
-// Inner products of a trainable operation: d_j = scale sum_k Im(conj(h_j[k])
-// gf[k]) in FP64, summed over the quad by DPP and added into LDS by the
-// quad's first lane (address (slot, j, quad)).
+// FP64 sums of a trainable instruction: NV values per lane, summed over the
+// quad by DPP and added into LDS by its lanes (value v at (base + v) * 16 +
+// quad). Lane r of a quad adds values r, r + 4, ... (every lane holds every
+// total); lanes without one add to a dummy slot of their own. No branch on
+// the lane, so the instruction switch around this stays free of divergent
+// control flow.
 // ---------------------------------------------------------------------------
 template <int CTRL> __device__ __forceinline__ double dpp_f64(double v) {
     const uint64_t b = __double_as_longlong(v);
@@ -318,295 +250,531 @@ template <int CTRL> __device__ __forceinline__ double dpp_f64(double v) {
         (static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | static_cast<uint32_t>(lo)));
 }
 
-template <typename T, int NS, int A, int ROT>
-__device__ __forceinline__ void accumulate(const Cx<T> (&B)[NS + 1][A], const Cx<T> (&gf)[A],
-                                           double scale, double *lacc, int slot, int lane) {
-    using RT = Rot<NS, ROT>;
-    constexpr int NJ = NS - 1;
-    double d[NJ > 0 ? NJ : 1];
+template <int NV>
+__device__ __forceinline__ void add_slots(double (&d)[NV], double *lacc, int base, int dummy, int lane) {
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < A; k++) {
-            s += im_conj_mul(B[RT::in(j + 1)][k], gf[k]);
-        }
-        s *= scale;
-        s += dpp_f64<0xB1>(s); // quad_perm [1,0,3,2]
-        s += dpp_f64<0x4E>(s); // quad_perm [2,3,0,1]
-        d[j] = s;
+    for (int v = 0; v < NV; v++) {
+        d[v] += dpp_f64<0xB1>(d[v]); // quad_perm [1,0,3,2]
+        d[v] += dpp_f64<0x4E>(d[v]); // quad_perm [2,3,0,1]
     }
-    // Lane r of a quad adds the totals of observables r and r + 4 (every lane
-    // holds every total); lanes without one add to a dummy slot. No branch on
-    // the lane, so the instruction switch around this stays free of divergent
-    // control flow.
     const int r = lane & 3;
 #pragma unroll
-    for (int j0 = 0; j0 < NJ; j0 += 4) {
-        double v = d[j0];
+    for (int v0 = 0; v0 < NV; v0 += 4) {
+        double x = d[v0];
 #pragma unroll
-        for (int j = j0 + 1; j < j0 + 4 && j < NJ; j++) {
-            v = (r == j - j0) ? d[j] : v;
+        for (int v = v0 + 1; v < v0 + 4 && v < NV; v++) {
+            x = (r == v - v0) ? d[v] : x;
         }
-        const int j = j0 + r;
-        const int idx = j < NJ ? (slot * NJ + j) * 16 + (lane >> 2) : RT_PMAX * NJ * 16 + lane;
-        atomicAdd(&lacc[idx], v);
+        const bool full = v0 + 4 <= NV;
+        const int idx = full || v0 + r < NV ? (base + v0 + r) * 16 + (lane >> 2) : dummy + lane;
+        atomicAdd(&lacc[idx], x);
     }
 }
 
-// ---------------------------------------------------------------------------
-// One instruction at rotation ROT.
-// ---------------------------------------------------------------------------
-template <int R, typename F> __device__ __forceinline__ void dispatch_q(int q, F &&f) {
-    switch (q) {
-    case 0: f(IC<0>{}); break;
-    case 1: f(IC<1>{}); break;
-    case 2: f(IC<2>{}); break;
-    default:
-        if constexpr (R > 3) {
-            f(IC<3>{});
-        }
-        break;
-    }
+template <typename T> struct Dx {
+    double r, i;
+};
+template <typename T> __device__ __forceinline__ Dx<T> wide(const Cx<T> &c) {
+    return {static_cast<double>(c.r), static_cast<double>(c.i)};
+}
+// s + Im(conj(h) g), s + Re(conj(h) g) and their negatives.
+template <typename T> __device__ __forceinline__ double im_add(double s, const Dx<T> &h, const Dx<T> &g) {
+    return fma(h.r, g.i, fma(-h.i, g.r, s));
+}
+template <typename T> __device__ __forceinline__ double im_sub(double s, const Dx<T> &h, const Dx<T> &g) {
+    return fma(-h.r, g.i, fma(h.i, g.r, s));
+}
+template <typename T> __device__ __forceinline__ double re_add(double s, const Dx<T> &h, const Dx<T> &g) {
+    return fma(h.r, g.r, fma(h.i, g.i, s));
+}
+template <typename T> __device__ __forceinline__ double re_sub(double s, const Dx<T> &h, const Dx<T> &g) {
+    return fma(-h.r, g.r, fma(-h.i, g.i, s));
 }
 
-template <int R, typename F> __device__ __forceinline__ void dispatch_q2(int a, int b, F &&f) {
-    switch (a * 4 + b) {
-    case 4: f(IC<1>{}, IC<0>{}); break;
-    case 8: f(IC<2>{}, IC<0>{}); break;
-    case 9: f(IC<2>{}, IC<1>{}); break;
-    default:
-        if constexpr (R > 3) {
-            switch (a * 4 + b) {
-            case 12: f(IC<3>{}, IC<0>{}); break;
-            case 13: f(IC<3>{}, IC<1>{}); break;
-            default: f(IC<3>{}, IC<2>{}); break;
+// Sums over the pairs of register bit Q: Im<h_j|P phi> for P = X (bit 0 of
+// C), Y (bit 1), Z (bit 2), in that order.
+template <typename T, int NS, int A, int Q, int C>
+__device__ __forceinline__ void acc_pauli(const Cx<T> (&v)[NS][A], double *lacc, int slot, int dummy, int lane) {
+    constexpr int NJ = NS - 1;
+    constexpr int NC = (C & 1) + ((C >> 1) & 1) + (C >> 2);
+    constexpr int OY = C & 1, OZ = (C & 1) + ((C >> 1) & 1);
+    double d[NC * NJ];
+#pragma unroll
+    for (int e = 0; e < NC * NJ; e++) {
+        d[e] = 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < A; k++) {
+        if (k & (1 << Q)) {
+            continue;
+        }
+        const Dx<T> f0 = wide(v[0][k]), f1 = wide(v[0][k | (1 << Q)]);
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const Dx<T> h0 = wide(v[j + 1][k]), h1 = wide(v[j + 1][k | (1 << Q)]);
+            if constexpr (C & 1) {
+                d[j] = im_add(im_add(d[j], h0, f1), h1, f0);
+            }
+            if constexpr (C & 2) {
+                // (Y f)_0 = -i f_1, (Y f)_1 = i f_0.
+                d[OY * NJ + j] = re_add(re_sub(d[OY * NJ + j], h0, f1), h1, f0);
+            }
+            if constexpr (C & 4) {
+                d[OZ * NJ + j] = im_sub(im_add(d[OZ * NJ + j], h0, f0), h1, f1);
             }
         }
-        break;
+    }
+    add_slots<NC * NJ>(d, lacc, slot * NJ, dummy, lane);
+}
+
+// Sums Im<h_j|G phi> for a 2x2 generator on register bit Q: real diagonal
+// (g[0], g[1]) or dense (row-major complex).
+template <typename T, int NS, int A, int Q, bool DIAG>
+__device__ __forceinline__ void acc_gen1(const Cx<T> (&v)[NS][A], const T *g, double *lacc, int slot, int dummy,
+                                         int lane) {
+    constexpr int NJ = NS - 1;
+    double d[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        d[j] = 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < A; k++) {
+        if (k & (1 << Q)) {
+            continue;
+        }
+        const Cx<T> f0 = v[0][k], f1 = v[0][k | (1 << Q)];
+        Cx<T> g0, g1;
+        if constexpr (DIAG) {
+            g0 = {g[0] * f0.r, g[0] * f0.i};
+            g1 = {g[1] * f1.r, g[1] * f1.i};
+        } else {
+            g0 = cmad(Cx<T>{g[2], g[3]}, f1, cmul(Cx<T>{g[0], g[1]}, f0));
+            g1 = cmad(Cx<T>{g[6], g[7]}, f1, cmul(Cx<T>{g[4], g[5]}, f0));
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            d[j] = im_add(im_add(d[j], wide(v[j + 1][k]), wide(g0)), wide(v[j + 1][k | (1 << Q)]), wide(g1));
+        }
+    }
+    add_slots<NJ>(d, lacc, slot * NJ, dummy, lane);
+}
+
+template <int QA, int QB> __device__ __forceinline__ constexpr int lidx(int k) {
+    return (((k >> QA) & 1) << 1) | ((k >> QB) & 1);
+}
+
+// Sums Im<h_j|G phi> for a 4x4 generator on register bits QA > QB: KIND
+// G_Z (parity sign), G_DIAG (four reals) or G_DENSE (row-major complex).
+template <typename T, int NS, int A, int QA, int QB, int KIND>
+__device__ __forceinline__ void acc_gen2(const Cx<T> (&v)[NS][A], CT<T> *G, double *lacc, int slot, int dummy,
+                                         int lane) {
+    constexpr int NJ = NS - 1;
+    constexpr int MQ = (1 << QA) | (1 << QB);
+    double d[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        d[j] = 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < A; k++) {
+        if (k & MQ) {
+            continue;
+        }
+        const int idx[4] = {k, k | (1 << QB), k | (1 << QA), k | MQ};
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            Cx<T> t;
+            if constexpr (KIND == G_Z) {
+                const Cx<T> f = v[0][idx[r]];
+                t = (r == 1 || r == 2) ? Cx<T>{-f.r, -f.i} : f;
+            } else if constexpr (KIND == G_DIAG) {
+                const Cx<T> f = v[0][idx[r]];
+                t = {G[r] * f.r, G[r] * f.i};
+            } else {
+                t = cmul(Cx<T>{G[8 * r], G[8 * r + 1]}, v[0][idx[0]]);
+#pragma unroll
+                for (int c = 1; c < 4; c++) {
+                    t = cmad(Cx<T>{G[8 * r + 2 * c], G[8 * r + 2 * c + 1]}, v[0][idx[c]], t);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                d[j] = im_add(d[j], wide(v[j + 1][idx[r]]), wide(t));
+            }
+        }
+    }
+    add_slots<NJ>(d, lacc, slot * NJ, dummy, lane);
+}
+
+// ---------------------------------------------------------------------------
+// In-place operations on every state.
+//
+// Each result is formed as (sum of the other terms) + u x with x the register
+// it replaces, and the last step is written as an instruction whose
+// destination is that register: the compiler's own choice, v_fmac, puts the
+// result into the other terms' register and copies it back (one v_mov_b64 per
+// result, a fifth of the kernel's vector instructions).
+// ---------------------------------------------------------------------------
+// x = u x + t; u uniform (scalar register) or per lane.
+template <bool UNI> __device__ __forceinline__ void fma_ip(double &x, double u, double t) {
+    if constexpr (UNI) {
+        asm("v_fma_f64 %0, %1, %0, %2" : "+v"(x) : "s"(u), "v"(t));
+    } else {
+        asm("v_fma_f64 %0, %1, %0, %2" : "+v"(x) : "v"(u), "v"(t));
+    }
+}
+template <bool UNI> __device__ __forceinline__ void fma_ip(float &x, float u, float t) {
+    if constexpr (UNI) {
+        asm("v_fma_f32 %0, %1, %0, %2" : "+v"(x) : "s"(u), "v"(t));
+    } else {
+        asm("v_fma_f32 %0, %1, %0, %2" : "+v"(x) : "v"(u), "v"(t));
     }
 }
 
-template <typename T, int NS, int A, int R, int ROT>
-__device__ __forceinline__ void remap_all(Cx<T> (&B)[NS + 1][A], int q, int p) {
-    using RT = Rot<NS, ROT>;
-    dispatch_q<R>(q, [&](auto Qc) {
-        constexpr int Q = decltype(Qc)::value;
-        if (p == 5) {
+// x = u x for complex u.
+template <bool UNI, typename T> __device__ __forceinline__ void scale_ip(Cx<T> &x, T ur, T ui) {
+    const T tr = -ui * x.i, ti = ui * x.r;
+    fma_ip<UNI>(x.r, ur, tr);
+    fma_ip<UNI>(x.i, ur, ti);
+}
+
+// Exchange of x and y, on every lane or on the lanes of `mask` (all lanes
+// are active here).
+template <bool ALL> __device__ __forceinline__ void swap_words(uint32_t &x0, uint32_t &y0, uint32_t &x1, uint32_t &y1,
+                                                               uint64_t mask) {
+    if constexpr (ALL) {
+        asm("v_swap_b32 %0, %1\n\tv_swap_b32 %2, %3" : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1));
+    } else {
+        uint64_t saved;
+        asm("s_mov_b64 %4, exec\n\ts_and_b64 exec, exec, %5\n\tv_swap_b32 %0, %1\n\tv_swap_b32 %2, %3\n\t"
+            "s_mov_b64 exec, %4"
+            : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1), "=&s"(saved)
+            : "s"(mask)
+            : "scc");
+    }
+}
+template <bool ALL> __device__ __forceinline__ void swap_ip(double &x, double &y, uint64_t mask) {
+    const uint64_t ux = __double_as_longlong(x), uy = __double_as_longlong(y);
+    uint32_t x0 = static_cast<uint32_t>(ux), x1 = static_cast<uint32_t>(ux >> 32);
+    uint32_t y0 = static_cast<uint32_t>(uy), y1 = static_cast<uint32_t>(uy >> 32);
+    swap_words<ALL>(x0, y0, x1, y1, mask);
+    x = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(x1) << 32) | x0));
+    y = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(y1) << 32) | y0));
+}
+template <bool ALL, typename T> __device__ __forceinline__ void swapc(Cx<T> &x, Cx<T> &y, uint64_t mask) {
+    if constexpr (sizeof(T) == 8) {
+        swap_ip<ALL>(x.r, y.r, mask);
+        swap_ip<ALL>(x.i, y.i, mask);
+    } else {
+        uint32_t x0 = __float_as_uint(x.r), x1 = __float_as_uint(x.i);
+        uint32_t y0 = __float_as_uint(y.r), y1 = __float_as_uint(y.i);
+        swap_words<ALL>(x0, y0, x1, y1, mask);
+        x = {__uint_as_float(x0), __uint_as_float(x1)};
+        y = {__uint_as_float(y0), __uint_as_float(y1)};
+    }
+}
+
+template <typename T, int NS, int A, int Q, typename M>
+__device__ __forceinline__ void each_pair(Cx<T> (&v)[NS][A], M &&m) {
 #pragma unroll
-            for (int s = 0; s < NS; s++) {
-                remap1<T, A, Q, 5>(B[RT::in(s)]);
+    for (int s = 0; s < NS; s++) {
+#pragma unroll
+        for (int k = 0; k < A; k++) {
+            if (!(k & (1 << Q))) {
+                m(v[s][k], v[s][k | (1 << Q)]);
+            }
+        }
+    }
+}
+
+// U on register bit Q; u in scalar registers (UNI) or one block per lane.
+// U_SWAP exchanges on the lanes of `mask`.
+template <typename T, int NS, int A, int Q, bool UNI>
+__device__ __forceinline__ void apply1(Cx<T> (&v)[NS][A], int ukind, const T (&u)[8], uint64_t mask) {
+    if (ukind == U_DENSE) {
+        each_pair<T, NS, A, Q>(v, [&](Cx<T> &a, Cx<T> &b) {
+            T tr = u[2] * b.r, ti = u[2] * b.i, qr = u[4] * a.r, qi = u[4] * a.i;
+            tr = fma(-u[3], b.i, tr);
+            ti = fma(u[3], b.r, ti);
+            qr = fma(-u[5], a.i, qr);
+            qi = fma(u[5], a.r, qi);
+            tr = fma(-u[1], a.i, tr);
+            ti = fma(u[1], a.r, ti);
+            qr = fma(-u[7], b.i, qr);
+            qi = fma(u[7], b.r, qi);
+            fma_ip<UNI>(a.r, u[0], tr);
+            fma_ip<UNI>(a.i, u[0], ti);
+            fma_ip<UNI>(b.r, u[6], qr);
+            fma_ip<UNI>(b.i, u[6], qi);
+        });
+    } else if (ukind == U_REAL) {
+        each_pair<T, NS, A, Q>(v, [&](Cx<T> &a, Cx<T> &b) {
+            const T tr = u[1] * b.r, ti = u[1] * b.i, qr = u[2] * a.r, qi = u[2] * a.i;
+            fma_ip<UNI>(a.r, u[0], tr);
+            fma_ip<UNI>(a.i, u[0], ti);
+            fma_ip<UNI>(b.r, u[3], qr);
+            fma_ip<UNI>(b.i, u[3], qi);
+        });
+    } else if (ukind == U_DIAG) {
+        each_pair<T, NS, A, Q>(v, [&](Cx<T> &a, Cx<T> &b) {
+            scale_ip<UNI>(a, u[0], u[1]);
+            scale_ip<UNI>(b, u[2], u[3]);
+        });
+    } else if (ukind == U_SWAP) {
+        each_pair<T, NS, A, Q>(v, [&](Cx<T> &a, Cx<T> &b) { swapc<UNI>(a, b, mask); });
+    }
+}
+
+template <typename T, int NS, int A, int QA, int QB, typename M>
+__device__ __forceinline__ void each_quad(Cx<T> (&v)[NS][A], M &&m) {
+    constexpr int MQ = (1 << QA) | (1 << QB);
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+#pragma unroll
+        for (int k = 0; k < A; k++) {
+            if (!(k & MQ)) {
+                m(v[s][k], v[s][k | (1 << QB)], v[s][k | (1 << QA)], v[s][k | MQ]);
+            }
+        }
+    }
+}
+
+template <typename T, int NS, int A, int QA, int QB>
+__device__ __forceinline__ void apply2(Cx<T> (&v)[NS][A], int ukind, int swp, const T (&u)[8], CT<T> *U) {
+    using C = Cx<T>;
+    if (ukind == U_DIAG) {
+        each_quad<T, NS, A, QA, QB>(v, [&](C &a, C &b, C &c, C &d) {
+            scale_ip<true>(a, u[0], u[1]);
+            scale_ip<true>(b, u[2], u[3]);
+            scale_ip<true>(c, u[4], u[5]);
+            scale_ip<true>(d, u[6], u[7]);
+        });
+    } else if (ukind == U_SWAP) {
+        if (swp == 11) { // 2 <-> 3: CNOT controlled by a
+            each_quad<T, NS, A, QA, QB>(v, [&](C &, C &, C &c, C &d) { swapc<true>(c, d, 0); });
+        } else if (swp == 7) { // 1 <-> 3: CNOT controlled by b
+            each_quad<T, NS, A, QA, QB>(v, [&](C &, C &b, C &, C &d) { swapc<true>(b, d, 0); });
+        } else if (swp == 6) { // 1 <-> 2: SWAP
+            each_quad<T, NS, A, QA, QB>(v, [&](C &, C &b, C &c, C &) { swapc<true>(b, c, 0); });
+        } else if (swp == 1) {
+            each_quad<T, NS, A, QA, QB>(v, [&](C &a, C &b, C &, C &) { swapc<true>(a, b, 0); });
+        } else if (swp == 2) {
+            each_quad<T, NS, A, QA, QB>(v, [&](C &a, C &, C &c, C &) { swapc<true>(a, c, 0); });
+        } else {
+            each_quad<T, NS, A, QA, QB>(v, [&](C &a, C &, C &, C &d) { swapc<true>(a, d, 0); });
+        }
+    } else if (ukind == U_REAL) {
+        each_quad<T, NS, A, QA, QB>(v, [&](C &a, C &b, C &c, C &d) {
+            C *x[4] = {&a, &b, &c, &d};
+            C t[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int e0 = (r + 1) & 3;
+                t[r] = {U[4 * r + e0] * x[e0]->r, U[4 * r + e0] * x[e0]->i};
+#pragma unroll
+                for (int q = 2; q < 4; q++) {
+                    const int e = (r + q) & 3;
+                    t[r].r = fma(U[4 * r + e], x[e]->r, t[r].r);
+                    t[r].i = fma(U[4 * r + e], x[e]->i, t[r].i);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                fma_ip<true>(x[r]->r, U[5 * r], t[r].r);
+                fma_ip<true>(x[r]->i, U[5 * r], t[r].i);
+            }
+        });
+    } else {
+        each_quad<T, NS, A, QA, QB>(v, [&](C &a, C &b, C &c, C &d) {
+            C *x[4] = {&a, &b, &c, &d};
+            C t[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int e0 = (r + 1) & 3;
+                t[r] = cmul(C{U[2 * (4 * r + e0)], U[2 * (4 * r + e0) + 1]}, *x[e0]);
+#pragma unroll
+                for (int q = 2; q < 4; q++) {
+                    const int e = (r + q) & 3;
+                    t[r] = cmad(C{U[2 * (4 * r + e)], U[2 * (4 * r + e) + 1]}, *x[e], t[r]);
+                }
+                t[r].r = fma(-U[10 * r + 1], x[r]->i, t[r].r);
+                t[r].i = fma(U[10 * r + 1], x[r]->r, t[r].i);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                fma_ip<true>(x[r]->r, U[10 * r], t[r].r);
+                fma_ip<true>(x[r]->i, U[10 * r], t[r].i);
+            }
+        });
+    }
+}
+
+// out = the block of NV reals at base that the lane's (or tile's) bit picks.
+template <typename T, int NV>
+__device__ __forceinline__ void pick(T (&out)[NV], CT<T> *base, bool c) {
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const T x0 = base[i], x1 = base[NV + i];
+        out[i] = c ? x1 : x0;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// One instruction.
+// ---------------------------------------------------------------------------
+template <typename T, int NS, int R>
+__device__ __forceinline__ void step(Cx<T> (&v)[NS][1 << R], Ins<T> &in, CT<unsigned char> *prog,
+                                     double *lacc, int dummy, int lane, uint64_t tbase) {
+    constexpr int A = 1 << R;
+    const int nremap = static_cast<int8_t>(in.w[5]);
+    if (nremap > 0) {
+        remap<T, NS, R>(v, static_cast<int8_t>(in.w[5] >> 8), static_cast<int8_t>(in.w[5] >> 16), lane);
+        if (nremap > 1) {
+            remap<T, NS, R>(v, static_cast<int8_t>(in.w[5] >> 24), static_cast<int8_t>(in.w[6]), lane);
+        }
+    }
+    int code = static_cast<int8_t>(in.w[0]);
+    const int a = static_cast<int8_t>(in.w[0] >> 8);
+    const int b = static_cast<int8_t>(in.w[0] >> 16);
+    const int s0 = static_cast<int8_t>(in.w[0] >> 24);
+    const int s1 = static_cast<int8_t>(in.w[1]);
+    int ukind = static_cast<int8_t>(in.w[1] >> 8);
+    const int gkind = static_cast<int8_t>(in.w[1] >> 16);
+    const int swp = static_cast<int8_t>(in.w[1] >> 24);
+    const int slot = in.w[2];
+    CT<T> *U = reinterpret_cast<CT<T> *>(prog + in.w[3]);
+    CT<T> *G = reinterpret_cast<CT<T> *>(prog + in.w[4]);
+    if (code == RT_SEL && s0 >= 64) {
+        // The selecting bit is fixed for the tile: one block for all lanes.
+        const bool c = (tbase >> (s0 - 64)) & 1;
+        if (ukind == U_SWAP) {
+            ukind = (c ? in.u[1] : in.u[0]) != T(0) ? U_SWAP : U_NONE;
+        } else if (ukind == U_DENSE) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                in.u[e] = U[(c ? 8 : 0) + e];
             }
         } else {
 #pragma unroll
-            for (int s = 0; s < NS; s++) {
-                remap1<T, A, Q, 4>(B[RT::in(s)]);
+            for (int e = 0; e < 4; e++) {
+                in.u[e] = c ? in.u[4 + e] : in.u[e];
             }
         }
-    });
-}
-
-template <typename T, int NS, int A, int R, int ROT>
-__device__ __forceinline__ void step(Cx<T> (&B)[NS + 1][A], CT<unsigned char> *prog, int pc,
-                                     double *lacc, int lane, uint64_t tbase) {
-    using RT = Rot<NS, ROT>;
-    const auto *words = reinterpret_cast<CT<int32_t> *>(prog) + 8 * pc;
-    int32_t w[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-        w[k] = words[k];
-    }
-    const int code = static_cast<int8_t>(w[0]);
-    const int a = static_cast<int8_t>(w[0] >> 8);
-    const int b = static_cast<int8_t>(w[0] >> 16);
-    const int s0 = static_cast<int8_t>(w[0] >> 24);
-    const int s1 = static_cast<int8_t>(w[1]);
-    const int ukind = static_cast<int8_t>(w[1] >> 8);
-    const int gkind = static_cast<int8_t>(w[1] >> 16);
-    const int swp = static_cast<int8_t>(w[1] >> 24);
-    const int slot = w[2];
-    CT<T> *U = reinterpret_cast<CT<T> *>(prog + w[3]);
-    CT<T> *G = reinterpret_cast<CT<T> *>(prog + w[4]);
-    const int nremap = static_cast<int8_t>(w[5]);
-    if (nremap > 0) {
-        remap_all<T, NS, A, R, ROT>(B, static_cast<int8_t>(w[5] >> 8), static_cast<int8_t>(w[5] >> 16));
-        if (nremap > 1) {
-            remap_all<T, NS, A, R, ROT>(B, static_cast<int8_t>(w[5] >> 24), static_cast<int8_t>(w[6]));
+        if (c) {
+            G += gkind == G_DIAG ? 2 : 8;
         }
+        code = RT_REG1;
     }
-    auto &gf = B[RT::out(0)]; // free until state 0 is written
-    const auto &phi = B[RT::in(0)];
     if (code == RT_REG1) {
         dispatch_q<R>(a, [&](auto Qc) {
             constexpr int Q = decltype(Qc)::value;
-            if (slot >= 0) {
-                gen1<T, A, Q>(gf, phi, gkind, G);
-                accumulate<T, NS, A, ROT>(B, gf, 1.0, lacc, slot, lane);
-            }
-            if (ukind == U_DIAG) {
-                const Cx<T> u0{U[0], U[1]}, u1{U[2], U[3]};
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    u1_diag<T, A, Q>(B[RT::out(s)], B[RT::in(s)], u0, u1);
-                }
-            } else if (ukind == U_REAL) {
-                const T m00 = U[0], m01 = U[1], m10 = U[2], m11 = U[3];
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    u1_real<T, A, Q>(B[RT::out(s)], B[RT::in(s)], m00, m01, m10, m11);
-                }
-            } else if (ukind == U_SWAP) {
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    u1_swap<T, A, Q>(B[RT::out(s)], B[RT::in(s)], true);
-                }
-            } else {
-                const Cx<T> u00{U[0], U[1]}, u01{U[2], U[3]}, u10{U[4], U[5]}, u11{U[6], U[7]};
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    u1_dense<T, A, Q>(B[RT::out(s)], B[RT::in(s)], u00, u01, u10, u11);
+            if constexpr (NS > 1) {
+                if (slot >= 0) {
+                    if (gkind == G_XYZ) {
+                        acc_pauli<T, NS, A, Q, 7>(v, lacc, slot, dummy, lane);
+                    } else if (gkind == G_X) {
+                        acc_pauli<T, NS, A, Q, 1>(v, lacc, slot, dummy, lane);
+                    } else if (gkind == G_Y) {
+                        acc_pauli<T, NS, A, Q, 2>(v, lacc, slot, dummy, lane);
+                    } else if (gkind == G_Z) {
+                        acc_pauli<T, NS, A, Q, 4>(v, lacc, slot, dummy, lane);
+                    } else if (gkind == G_DIAG) {
+                        const T g[2] = {G[0], G[1]};
+                        acc_gen1<T, NS, A, Q, true>(v, g, lacc, slot, dummy, lane);
+                    } else {
+                        const T g[8] = {G[0], G[1], G[2], G[3], G[4], G[5], G[6], G[7]};
+                        acc_gen1<T, NS, A, Q, false>(v, g, lacc, slot, dummy, lane);
+                    }
                 }
             }
+            apply1<T, NS, A, Q, true>(v, ukind, in.u, 0);
         });
     } else if (code == RT_REG2) {
         dispatch_q2<R>(a, b, [&](auto QAc, auto QBc) {
             constexpr int QA = decltype(QAc)::value, QB = decltype(QBc)::value;
-            if (slot >= 0) {
-                gen2<T, A, QA, QB>(gf, phi, gkind, G);
-                accumulate<T, NS, A, ROT>(B, gf, 1.0, lacc, slot, lane);
-            }
-            if (ukind == U_DIAG) {
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    u2_diag<T, A, QA, QB>(B[RT::out(s)], B[RT::in(s)], U);
-                }
-            } else if (ukind == U_SWAP) {
-                auto sw = [&](auto LA, auto LB) {
-#pragma unroll
-                    for (int s = 0; s < NS; s++) {
-                        u2_swap<T, A, QA, QB, decltype(LA)::value, decltype(LB)::value>(B[RT::out(s)],
-                                                                                        B[RT::in(s)]);
+            if constexpr (NS > 1) {
+                if (slot >= 0) {
+                    if (gkind == G_Z) {
+                        acc_gen2<T, NS, A, QA, QB, G_Z>(v, G, lacc, slot, dummy, lane);
+                    } else if (gkind == G_DIAG) {
+                        acc_gen2<T, NS, A, QA, QB, G_DIAG>(v, G, lacc, slot, dummy, lane);
+                    } else {
+                        acc_gen2<T, NS, A, QA, QB, G_DENSE>(v, G, lacc, slot, dummy, lane);
                     }
-                };
-                switch (swp) {
-                case 1: sw(IC<0>{}, IC<1>{}); break;
-                case 2: sw(IC<0>{}, IC<2>{}); break;
-                case 3: sw(IC<0>{}, IC<3>{}); break;
-                case 6: sw(IC<1>{}, IC<2>{}); break;
-                case 7: sw(IC<1>{}, IC<3>{}); break;
-                default: sw(IC<2>{}, IC<3>{}); break;
-                }
-            } else if (ukind == U_REAL) {
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    u2_real<T, A, QA, QB>(B[RT::out(s)], B[RT::in(s)], U);
-                }
-            } else {
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    u2_dense<T, A, QA, QB>(B[RT::out(s)], B[RT::in(s)], U);
                 }
             }
+            apply2<T, NS, A, QA, QB>(v, ukind, swp, in.u, U);
         });
     } else if (code == RT_SEL) {
-        const int nb = s1 >= 0 ? 4 : 2;
-        const bool c0 = selbit(lane, tbase, s0);
-        const bool c1 = s1 >= 0 ? selbit(lane, tbase, s1) : false;
+        const bool c0 = lbit(lane, s0);
         dispatch_q<R>(a, [&](auto Qc) {
             constexpr int Q = decltype(Qc)::value;
-            if (slot >= 0) {
-                if (gkind == G_DIAG) {
-                    T g[2];
-                    select_block<T, 2>(g, G, nb, c0, c1);
-#pragma unroll
-                    for (int k = 0; k < A; k++) {
-                        const T x = ((k >> Q) & 1) ? g[1] : g[0];
-                        gf[k] = {x * phi[k].r, x * phi[k].i};
+            if constexpr (NS > 1) {
+                if (slot >= 0) {
+                    if (gkind == G_DIAG) {
+                        T g[2];
+                        pick<T, 2>(g, G, c0);
+                        acc_gen1<T, NS, A, Q, true>(v, g, lacc, slot, dummy, lane);
+                    } else {
+                        T g[8];
+                        pick<T, 8>(g, G, c0);
+                        acc_gen1<T, NS, A, Q, false>(v, g, lacc, slot, dummy, lane);
                     }
-                } else {
-                    T g[8];
-                    select_block<T, 8>(g, G, nb, c0, c1);
-                    u1_dense<T, A, Q>(gf, phi, {g[0], g[1]}, {g[2], g[3]}, {g[4], g[5]}, {g[6], g[7]});
                 }
-                accumulate<T, NS, A, ROT>(B, gf, 1.0, lacc, slot, lane);
             }
-            if (ukind == U_DIAG) {
-                T u[4];
-                select_block<T, 4>(u, U, nb, c0, c1);
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    u1_diag<T, A, Q>(B[RT::out(s)], B[RT::in(s)], {u[0], u[1]}, {u[2], u[3]});
-                }
-            } else if (ukind == U_SWAP) {
-                T fl[1];
-                select_block<T, 1>(fl, U, nb, c0, c1);
-                const bool on = fl[0] != T(0);
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    u1_swap<T, A, Q>(B[RT::out(s)], B[RT::in(s)], on);
-                }
-            } else if (ukind == U_REAL) {
-                T u[4];
-                select_block<T, 4>(u, U, nb, c0, c1);
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    u1_real<T, A, Q>(B[RT::out(s)], B[RT::in(s)], u[0], u[1], u[2], u[3]);
-                }
+            T u[8] = {};
+            uint64_t mask = 0;
+            if (ukind == U_SWAP) {
+                mask = __ballot((c0 ? in.u[1] : in.u[0]) != T(0));
+            } else if (ukind == U_DENSE) {
+                pick<T, 8>(u, U, c0);
             } else {
-                T u[8];
-                select_block<T, 8>(u, U, nb, c0, c1);
 #pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    u1_dense<T, A, Q>(B[RT::out(s)], B[RT::in(s)], {u[0], u[1]}, {u[2], u[3]},
-                                      {u[4], u[5]}, {u[6], u[7]});
+                for (int e = 0; e < 4; e++) {
+                    u[e] = c0 ? in.u[4 + e] : in.u[e];
                 }
             }
+            apply1<T, NS, A, Q, false>(v, ukind, u, mask);
         });
-    } else {
-        // RT_LANE: G phi = g phi on this lane, so the products scale by g.
-        const int nb = s1 >= 0 ? 4 : 2;
+    } else if (code == RT_LANE) {
+        // G phi = g phi on this lane, so the products scale by g.
         const bool c0 = selbit(lane, tbase, s0);
         const bool c1 = s1 >= 0 ? selbit(lane, tbase, s1) : false;
-        if (slot >= 0) {
-            T g[1];
-            select_block<T, 1>(g, G, nb, c0, c1);
-            accumulate<T, NS, A, ROT>(B, phi, static_cast<double>(g[0]), lacc, slot, lane);
+        if constexpr (NS > 1) {
+            if (slot >= 0) {
+                T g = c0 ? G[1] : G[0];
+                if (s1 >= 0) {
+                    const T g1 = c0 ? G[3] : G[2];
+                    g = c1 ? g1 : g;
+                }
+                constexpr int NJ = NS - 1;
+                double d[NJ];
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    double x = 0.0;
+#pragma unroll
+                    for (int k = 0; k < A; k++) {
+                        x = im_add(x, wide(v[j + 1][k]), wide(v[0][k]));
+                    }
+                    d[j] = x * static_cast<double>(g);
+                }
+                add_slots<NJ>(d, lacc, slot * NJ, dummy, lane);
+            }
         }
-        T u[2];
-        select_block<T, 2>(u, U, nb, c0, c1);
-        const Cx<T> f{u[0], u[1]};
+        Cx<T> f{c0 ? in.u[2] : in.u[0], c0 ? in.u[3] : in.u[1]};
+        if (s1 >= 0) {
+            const Cx<T> f1{c0 ? in.u[6] : in.u[4], c0 ? in.u[7] : in.u[5]};
+            f = {c1 ? f1.r : f.r, c1 ? f1.i : f.i};
+        }
 #pragma unroll
         for (int s = 0; s < NS; s++) {
 #pragma unroll
             for (int k = 0; k < A; k++) {
-                B[RT::out(s)][k] = cmul(f, B[RT::in(s)][k]);
+                scale_ip<false>(v[s][k], f.r, f.i);
             }
         }
     }
-}
-
-// Runs the program with the loop unrolled over the NS + 1 rotations; returns
-// the rotation after the last instruction.
-template <typename T, int NS, int A, int R, int... ROTS>
-__device__ __forceinline__ int run_program(Cx<T> (&B)[NS + 1][A], CT<unsigned char> *prog, int ninstr,
-                                           uint64_t tbase,
-                                           double *lacc, int lane,
-                                           std::integer_sequence<int, ROTS...>) {
-    int pc = 0;
-    for (;;) {
-        int end = 0;
-        const bool more = ((pc < ninstr ? (step<T, NS, A, R, ROTS>(B, prog, pc, lacc, lane, tbase), ++pc, true)
-                                        : (end = ROTS, false)) &&
-                           ...);
-        if (!more) {
-            return end;
-        }
-    }
-}
-
-template <typename F, int... RS>
-__device__ __forceinline__ void for_rot(int rot, F &&f, std::integer_sequence<int, RS...>) {
-    ((rot == RS ? (f(IC<RS>{}), 0) : 0), ...);
 }
 
 // Observable-state pointers of one launch: nc chunks of NJ states.
@@ -614,14 +782,24 @@ template <typename T> struct RtPtrs {
     Cx<T> *p[RT_OBS_MAX];
 };
 
-template <typename T, int NJ, typename Off>
-__global__ void __launch_bounds__(64)
+// Byte offset of register slot k: the sum over its set bits q of 2^reg[q].
+template <typename T, int R> __device__ __forceinline__ uint64_t slot_off(const int *reg, int k) {
+    uint64_t o = 0;
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+        if ((k >> q) & 1) {
+            o += uint64_t{sizeof(Cx<T>)} << reg[q];
+        }
+    }
+    return o;
+}
+
+template <typename T, int NJ, int R>
+__global__ void __launch_bounds__(64, (rt_waves<T, NJ>()))
     rtile_kernel(Cx<T> *phi, Cx<T> *phi_out, RtPtrs<T> hp, const unsigned char *__restrict__ prog_g,
                  RtLaunch L, double *__restrict__ partials) {
-    constexpr int R = rt_r<T>();
     constexpr int A = 1 << R;
     constexpr int NS = NJ + 1;
-    constexpr int NA = NJ > 0 ? NJ : 1;
     // Block -> (chunk c, block b of that chunk). Ids are taken in groups of
     // xgroup (consecutive ids land on different XCDs), so the nc blocks that
     // stream the same tiles for different chunks share an XCD and its L2.
@@ -637,11 +815,12 @@ __global__ void __launch_bounds__(64)
     const int njc = c < L.nbig ? NJ : NJ - 1;
     const int jc0 = c < L.nbig ? c * NJ : L.nbig * NJ + (c - L.nbig) * (NJ - 1);
     const int width = L.nbig * NJ + (nc - L.nbig) * (NJ - 1);
-    __shared__ double lacc[NJ > 0 ? RT_PMAX * NA * 16 + 64 : 1]; // + one dummy slot per lane
+    // FP64 sums [slot * NJ + j][quad], then one dummy slot per lane.
+    extern __shared__ double lacc[];
     const int lane = static_cast<int>(__lane_id());
+    const int dummy = L.nslots * NJ * 16;
     if constexpr (NJ > 0) {
-        const int nacc = L.nslots * NA * 16;
-        for (int i = lane; i < nacc; i += 64) {
+        for (int i = lane; i < dummy; i += 64) {
             lacc[i] = 0.0;
         }
     }
@@ -652,70 +831,56 @@ __global__ void __launch_bounds__(64)
     for (int j = 0; j < NJ; j++) {
         sp[j + 1] = j < njc ? hp.p[jc0 + j] : phi;
     }
-    // Per-lane offsets of the load and store layouts (amplitudes; the tile
-    // base is added per tile); register slot k sits at the sum over its set
-    // bits q of 2^reg[q] (uniform).
-    uint64_t lin = 0, lout = 0;
+    // Per-lane byte offsets of the load and store layouts; the tile base and
+    // the register slot's offset are uniform.
+    uint64_t vin = 0, vout = 0;
 #pragma unroll
     for (int p = 0; p < RT_LANE_BITS; p++) {
-        lin |= static_cast<uint64_t>(lbit(lane, p)) << L.lane_in[p];
-        lout |= static_cast<uint64_t>(lbit(lane, p)) << L.lane_out[p];
+        vin |= static_cast<uint64_t>(lbit(lane, p)) << L.lane_in[p];
+        vout |= static_cast<uint64_t>(lbit(lane, p)) << L.lane_out[p];
     }
-    const Off vin = static_cast<Off>(lin * sizeof(Cx<T>));
-    const Off vout = static_cast<Off>(lout * sizeof(Cx<T>));
-    auto roff = [&](const int *reg, int k) {
-        uint64_t o = 0;
-#pragma unroll
-        for (int q = 0; q < R; q++) {
-            if ((k >> q) & 1) {
-                o += uint64_t{1} << reg[q];
-            }
-        }
-        return o;
-    };
+    vin *= sizeof(Cx<T>);
+    vout *= sizeof(Cx<T>);
     const uint64_t ntiles = uint64_t{1} << (L.n - L.T);
+    const Ins<T> first = fetch<T>(prog, 0);
     for (uint64_t g = b; g < ntiles; g += bpc) {
         uint64_t base = g;
         for (int q = 0; q < L.T; q++) {
             base = insert_zero(base, L.tb[q]);
         }
-        Cx<T> B[NS + 1][A];
+        Cx<T> v[NS][A];
 #pragma unroll
         for (int s = 0; s < NS; s++) {
             if (s > njc) {
 #pragma unroll
                 for (int k = 0; k < A; k++) {
-                    B[s][k] = Cx<T>{T(0), T(0)};
+                    v[s][k] = Cx<T>{T(0), T(0)};
                 }
                 continue;
             }
 #pragma unroll
             for (int k = 0; k < A; k++) {
-                B[s][k] = ldo(sp[s], static_cast<Off>((base + roff(L.reg_in, k)) * sizeof(Cx<T>)) + vin);
+                v[s][k] = ldo(sp[s], base * sizeof(Cx<T>) + slot_off<T, R>(L.reg_in, k) + vin);
             }
         }
-        const int rot = run_program<T, NS, A, R>(B, prog, L.ninstr, base, lacc, lane,
-                                                 std::make_integer_sequence<int, NS + 1>{});
-        auto store = [&](auto RC) {
-            using RT = Rot<NS, decltype(RC)::value>;
-            // The store layout's remaps (low index bits back onto lanes).
-            for (int f = 0; f < L.nfin; f++) {
-                remap_all<T, NS, A, R, decltype(RC)::value>(B, L.fin_rq[f], L.fin_rp[f]);
-            }
+        Ins<T> cur = first;
+#pragma unroll 1
+        for (int pc = 0; pc < L.ninstr; pc++) {
+            const Ins<T> nxt = fetch<T>(prog, pc + 1);
+            step<T, NS, R>(v, cur, prog, lacc, dummy, lane, base);
+            cur = nxt;
+        }
 #pragma unroll
-            for (int s = 0; s < NS; s++) {
-                if ((s == 0 && !writes_phi) || s > njc) {
-                    continue;
-                }
-                Cx<T> *dst = s == 0 ? phi_out : sp[s];
-#pragma unroll
-                for (int k = 0; k < A; k++) {
-                    sto(dst, static_cast<Off>((base + roff(L.reg_out, k)) * sizeof(Cx<T>)) + vout,
-                        B[RT::in(s)][k]);
-                }
+        for (int s = 0; s < NS; s++) {
+            if ((s == 0 && !writes_phi) || s > njc) {
+                continue;
             }
-        };
-        for_rot(rot, store, std::make_integer_sequence<int, NS + 1>{});
+            Cx<T> *dst = s == 0 ? phi_out : sp[s];
+#pragma unroll
+            for (int k = 0; k < A; k++) {
+                sto(dst, base * sizeof(Cx<T>) + slot_off<T, R>(L.reg_out, k) + vout, v[s][k]);
+            }
+        }
     }
     if constexpr (NJ > 0) {
         __syncthreads();
@@ -738,58 +903,56 @@ __global__ void __launch_bounds__(64)
 
 } // namespace
 
+// Blocks per chunk of a launch: the chunks share the resident blocks; in
+// groups of 8 (one per XCD) when there are enough.
+template <typename T, int NJ> int rtile_blocks_t(const Device &dev, const RtLaunch &L, int nc) {
+    constexpr int R = rt_reg_bits<T>(NJ);
+    const void *kfn = reinterpret_cast<const void *>(&rtile_kernel<T, NJ, R>);
+    const size_t lds = rt_lds_bytes(NJ, L.nslots);
+    static int per_cu[RT_SLOTS_MAX + 1] = {}; // by slots: the kernel's LDS follows from them
+    int &nb = per_cu[NJ > 0 ? L.nslots : 0];
+    if (nb == 0) {
+        PLK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kfn, 64, lds));
+        nb = std::max(1, std::min(nb, 32));
+    }
+    const uint64_t ntiles = uint64_t{1} << (L.n - L.T);
+    const uint64_t cap = static_cast<uint64_t>(dev.num_cus) * nb;
+    uint64_t bpc = std::max<uint64_t>(1, std::min(ntiles, cap / static_cast<uint64_t>(nc)));
+    if (bpc >= 8) {
+        bpc = bpc / 8 * 8;
+    }
+    return static_cast<int>(bpc);
+}
+
 // Launcher of one (precision, observable chunk) variant. The build compiles
 // this file once per variant with PLK_RT_T and PLK_RT_NJ defined, so the
 // variants compile in parallel.
 template <typename T, int NJ>
-int rtile_launch_t(Device &dev, const State &phi, void *phi_out, void *const *h_ptrs,
-                   const void *d_prog, const RtLaunch &Lin) {
+void rtile_launch_t(Device &dev, const State &phi, void *phi_out, void *const *h_ptrs,
+                    const void *d_prog, const RtLaunch &Lin, int bpc, double *partials) {
+    constexpr int R = rt_reg_bits<T>(NJ);
     RtLaunch L = Lin;
-    L.nc = std::max(1, L.nc);
-    L.nbig = std::min(std::max(L.nbig, NJ > 0 ? 1 : 0), L.nc);
-    if (NJ == 0) {
-        L.nbig = L.nc;
-    }
-    const int width = L.nbig * NJ + (L.nc - L.nbig) * std::max(0, NJ - 1);
+    L.xgroup = bpc >= 8 ? 8 : 1;
+    const int width = rt_width(L);
     RtPtrs<T> hp{};
     for (int j = 0; j < width; j++) {
         hp.p[j] = static_cast<Cx<T> *>(h_ptrs[j]);
     }
-    const void *kfn = reinterpret_cast<const void *>(&rtile_kernel<T, NJ, uint64_t>);
-    static int blocks_per_cu = 0;
-    if (blocks_per_cu == 0) {
-        int nb = 0;
-        PLK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kfn, 64, 0));
-        blocks_per_cu = std::max(1, std::min(nb, 32));
-    }
-    const uint64_t ntiles = uint64_t{1} << (L.n - L.T);
-    const uint64_t cap = static_cast<uint64_t>(dev.num_cus) * blocks_per_cu;
-    // Blocks per chunk: the chunks share the resident blocks; in groups of 8
-    // (one per XCD) when there are enough.
-    uint64_t bpc = std::max<uint64_t>(1, std::min(ntiles, cap / static_cast<uint64_t>(L.nc)));
-    L.xgroup = 1;
-    if (bpc >= 8) {
-        bpc = bpc / 8 * 8;
-        L.xgroup = 8;
-    }
-    const unsigned grid = static_cast<unsigned>(bpc * static_cast<uint64_t>(L.nc));
-    if (NJ > 0 && L.nslots > 0) {
-        ensure_red(dev, static_cast<size_t>(bpc) * L.nslots * width, 0);
-    }
+    const unsigned grid = static_cast<unsigned>(bpc) * static_cast<unsigned>(L.nc);
     // Algorithmic bytes: phi read once and written once, every observable
     // state read and written once.
     const double bytes = (1.0 + L.write_phi + 2.0 * width) * static_cast<double>(phi.bytes());
     ProfScope prof(NJ > 0 ? "adjoint_rtile" : "apply_rtile", bytes, dev.stream);
-    hipLaunchKernelGGL((rtile_kernel<T, NJ, uint64_t>), dim3(grid), dim3(64), 0, dev.stream,
+    hipLaunchKernelGGL((rtile_kernel<T, NJ, R>), dim3(grid), dim3(64), rt_lds_bytes(NJ, L.nslots), dev.stream,
                        static_cast<Cx<T> *>(phi.d), static_cast<Cx<T> *>(phi_out), hp,
-                       static_cast<const unsigned char *>(d_prog), L, dev.red);
+                       static_cast<const unsigned char *>(d_prog), L, partials);
     PLK_HIP(hipGetLastError());
-    return static_cast<int>(bpc);
 }
 
 #if defined(PLK_RT_T) && defined(PLK_RT_NJ)
-template int rtile_launch_t<PLK_RT_T, PLK_RT_NJ>(Device &, const State &, void *, void *const *,
-                                                 const void *, const RtLaunch &);
+template int rtile_blocks_t<PLK_RT_T, PLK_RT_NJ>(const Device &, const RtLaunch &, int);
+template void rtile_launch_t<PLK_RT_T, PLK_RT_NJ>(Device &, const State &, void *, void *const *, const void *,
+                                                  const RtLaunch &, int, double *);
 #endif
 
 } // namespace plk

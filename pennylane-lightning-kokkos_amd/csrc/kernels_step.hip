@@ -22,8 +22,8 @@
 // store.
 //
 // Jacobian sums: per thread in LDS (one slot per observable state), then a
-// fixed-order block sum into dev.red as [j][block]; tile_reduce_kernel adds
-// the blocks in order.
+// fixed-order block sum into the partials as [j][block], which the sweep's
+// reduction adds in order.
 #include "device_common.hpp"
 
 namespace plk {
@@ -189,18 +189,13 @@ __global__ void __launch_bounds__(kStepBlock)
 }
 
 template <typename T>
-int launch_step_t(Device &dev, const State &phi, void *const *h_ptrs, const void *d_mats,
-                  const StepLaunch &L) {
+void launch_step_t(Device &dev, const State &phi, void *const *h_ptrs, const void *d_mats,
+                   const StepLaunch &L, double *partials) {
     SegPtrs<T> hp{};
     for (int j = 0; j < L.nj; j++) {
         hp.p[j] = static_cast<Cx<T> *>(h_ptrs[j]);
     }
-    const uint64_t blocks = (L.groups + kStepBlock - 1) / kStepBlock;
-    const unsigned grid = static_cast<unsigned>(
-        std::max<uint64_t>(1, std::min<uint64_t>(blocks, static_cast<uint64_t>(dev.num_cus) * 8)));
-    if (L.trainable && L.nj > 0) {
-        ensure_red(dev, static_cast<size_t>(grid) * L.nj, 0);
-    }
+    const unsigned grid = static_cast<unsigned>(step_blocks(dev, L));
     const double bytes = (1.0 + L.write_phi + 2.0 * L.nj) * static_cast<double>(phi.bytes());
     ProfScope prof(L.nj > 0 ? "adjoint_step" : "apply_step", bytes, dev.stream);
     auto *p = static_cast<Cx<T> *>(phi.d);
@@ -208,35 +203,40 @@ int launch_step_t(Device &dev, const State &phi, void *const *h_ptrs, const void
     switch (L.m == 0 ? 0 : L.dim) {
     case 0:
         hipLaunchKernelGGL((step_parity_kernel<T>), dim3(grid), dim3(kStepBlock), 0, dev.stream, p,
-                           hp, L, dev.red);
+                           hp, L, partials);
         break;
     case 2:
         hipLaunchKernelGGL((step_dense_kernel<T, 2>), dim3(grid), dim3(kStepBlock), 0, dev.stream,
-                           p, hp, m, L, dev.red);
+                           p, hp, m, L, partials);
         break;
     case 4:
         hipLaunchKernelGGL((step_dense_kernel<T, 4>), dim3(grid), dim3(kStepBlock), 0, dev.stream,
-                           p, hp, m, L, dev.red);
+                           p, hp, m, L, partials);
         break;
     case 8:
         hipLaunchKernelGGL((step_dense_kernel<T, 8>), dim3(grid), dim3(kStepBlock), 0, dev.stream,
-                           p, hp, m, L, dev.red);
+                           p, hp, m, L, partials);
         break;
     case 16:
         hipLaunchKernelGGL((step_dense_kernel<T, 16>), dim3(grid), dim3(kStepBlock), 0, dev.stream,
-                           p, hp, m, L, dev.red);
+                           p, hp, m, L, partials);
         break;
     default:
         raise(PLK_ERR_INVALID, "single-op step kernels take subspaces of 2, 4, 8 or 16 states");
     }
     PLK_HIP(hipGetLastError());
-    return static_cast<int>(grid);
 }
 
 } // namespace
 
-int launch_step(Device &dev, const State &phi, void *const *h_ptrs, const void *d_mats,
-                const StepLaunch &L) {
+int step_blocks(const Device &dev, const StepLaunch &L) {
+    const uint64_t blocks = (L.groups + kStepBlock - 1) / kStepBlock;
+    return static_cast<int>(
+        std::max<uint64_t>(1, std::min<uint64_t>(blocks, static_cast<uint64_t>(dev.num_cus) * 8)));
+}
+
+void launch_step(Device &dev, const State &phi, void *const *h_ptrs, const void *d_mats,
+                 const StepLaunch &L, double *partials) {
     if (L.nj < 0 || L.nj > SEG_NJMAX) {
         raise(PLK_ERR_INVALID, "single-op step: observable chunk out of range");
     }
@@ -250,8 +250,14 @@ int launch_step(Device &dev, const State &phi, void *const *h_ptrs, const void *
     if (L.m == 0 && L.groups != phi.len) {
         raise(PLK_ERR_INVALID, "single-op step: parity step must cover the state");
     }
-    return phi.dtype == PLK_C64 ? launch_step_t<float>(dev, phi, h_ptrs, d_mats, L)
-                                : launch_step_t<double>(dev, phi, h_ptrs, d_mats, L);
+    if (L.trainable && L.nj > 0 && partials == nullptr) {
+        raise(PLK_ERR_INVALID, "single-op step: no buffer for the partial sums");
+    }
+    if (phi.dtype == PLK_C64) {
+        launch_step_t<float>(dev, phi, h_ptrs, d_mats, L, partials);
+    } else {
+        launch_step_t<double>(dev, phi, h_ptrs, d_mats, L, partials);
+    }
 }
 
 } // namespace plk

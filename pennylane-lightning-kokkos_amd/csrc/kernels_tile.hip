@@ -215,7 +215,7 @@ __global__ void __launch_bounds__(TILE_BLOCK)
     }
 }
 
-constexpr int kReduceMax = TILE_PMAX > RT_PMAX ? TILE_PMAX : RT_PMAX;
+constexpr int kReduceMax = TILE_PMAX;
 
 struct TileReduceArgs {
     int grid;

@@ -49,6 +49,8 @@ struct Device {
     size_t red_cap = 0;           // doubles
     double *red_out = nullptr;    // final reduction results
     size_t red_out_cap = 0;
+    double *parts = nullptr;      // partials of a sweep's passes until their reduction
+    size_t parts_cap = 0;         // doubles
     int num_cus = 256;
     void *work = nullptr;         // grow-only device workspace
     size_t work_cap = 0;          // bytes
@@ -80,6 +82,8 @@ std::recursive_mutex &engine_mutex();
 // temporary states is released and the allocation retried once.
 void *dev_malloc(int device, size_t bytes, const char *what);
 void ensure_red(Device &d, size_t partial_doubles, size_t out_doubles);
+// Grows d.parts to at least `doubles` entries (synchronizes when it grows).
+void ensure_parts(Device &d, size_t doubles);
 // Grows d.jac to at least `doubles` entries.
 double *ensure_jac(Device &d, size_t doubles);
 // Grows d.work to at least `bytes` (synchronizes the stream when it grows).
@@ -176,10 +180,11 @@ constexpr int SEG_BLOCK = 256;
 
 // Structure of an operation's matrix, chosen on the host so the kernels skip
 // the multiplications a dense complex product would waste.
-enum SegUKind : int32_t { U_DENSE = 0, U_DIAG = 1, U_REAL = 2, U_SWAP = 3 };
+enum SegUKind : int32_t { U_DENSE = 0, U_DIAG = 1, U_REAL = 2, U_SWAP = 3, U_NONE = 4 };
 // Structure of a generator: dense, real diagonal, (one wire) X or Y, or the
 // parity sign (-1)^popcount of the op-local index (Z, Z(x)Z).
-enum SegGKind : int32_t { G_DENSE = 0, G_DIAG = 1, G_X = 2, G_Y = 3, G_Z = 4 };
+// G_XYZ (register-tile programs): the three Pauli sums of a fused run.
+enum SegGKind : int32_t { G_DENSE = 0, G_DIAG = 1, G_X = 2, G_Y = 3, G_Z = 4, G_XYZ = 5 };
 
 // Host-side description of one fused operation: `cls` selects the
 // compile-time local-position case, m is 1 or 2 wires, U and G are row-major
@@ -265,40 +270,61 @@ void launch_tile_reduce(Device &dev, int grid, int nslots, int nj, int j0, const
 
 // Register-tile passes (kernels_rtile.hip). A wavefront holds a tile of
 // 2^(R+6) amplitudes of phi and nj observable states in VGPRs: R register
-// bits (3 for complex128, 4 for complex64) and 6 lane bits, each holding one
-// tile bit (a global index bit). A pass program is a list of RtInstr
-// followed by the payloads they point to.
+// bits and 6 lane bits, each holding one tile bit (a global index bit). A
+// pass program is a list of instructions followed by the payloads too large
+// for them.
 constexpr int RT_LANE_BITS = 6;
-constexpr int RT_RMAX = 4;
+constexpr int RT_RMAX = 5;
 constexpr int RT_TMAX = RT_RMAX + RT_LANE_BITS;
-constexpr int RT_PMAX = 32; // trainable ops per pass
+constexpr int RT_SLOTS_MAX = 48; // sums per pass (a fused run of two ops takes up to three)
+constexpr int RT_NJMAX = 4;      // observable states per register-tile chunk
+
+// Register bits of a tile by precision and observable chunk: the states of a
+// chunk fill 64 (one or two states) to 160 VGPRs (five).
+template <typename T> constexpr int rt_reg_bits(int nj) {
+    return (nj <= 1 ? 4 : 3) + (sizeof(T) == 4 ? 1 : 0);
+}
+inline int rt_reg_bits(int dtype, int nj) {
+    return dtype == PLK_C64 ? rt_reg_bits<float>(nj) : rt_reg_bits<double>(nj);
+}
+// Waves per SIMD the register allocator is held to.
+template <typename T, int NJ> constexpr int rt_waves() { return NJ == 0 ? 4 : NJ <= 3 && !(NJ == 1 && sizeof(T) == 8) ? 3 : 2; }
 
 enum RtOpCode : int8_t {
+    RT_NOP = 0,   // remaps only
     RT_REG1 = 1,  // one wire on register bit a
     RT_REG2 = 2,  // two wires on register bits a > b (local index 2 bit(a) + bit(b))
-    RT_SEL = 3,   // register bit a mixes; blocks selected per lane by lane bits s0 (, s1)
-    RT_LANE = 4   // diagonal on lane positions s0 (, s1): one factor per lane
+    RT_SEL = 3,   // register bit a mixes; the block is selected by s0
+    RT_LANE = 4   // diagonal on s0 (, s1): one factor per lane
 };
 
-// Payloads (reals of the state's precision, from the program start):
-//   REG1  U: DIAG [u0 u1] complex, REAL [m00 m01 m10 m11], DENSE 2x2 complex,
-//            SWAP none; G: DIAG [g0 g1], DENSE 2x2 complex, X / Y / Z none.
-//   REG2  U: DIAG 4 complex, REAL 4x4, DENSE 4x4 complex, SWAP none (swap =
-//            4 a + b exchanged local indices); G: DIAG 4, DENSE 4x4 complex, Z none.
-//   SEL   nb = 2 (s1 < 0) or 4 blocks, block c = bit(s0) + 2 bit(s1), each
-//            block as REG1 (U SWAP: one real, nonzero = exchange); G: DIAG or DENSE.
-//   LANE  U: nb complex factors; G: nb real factors (same block index).
+// Header of an instruction; the eight reals u[] of the state's precision
+// follow it (stride rt_stride). U_DENSE blocks of SEL and REG2 and U_REAL of
+// REG2 are payloads at uoff, generators payloads at goff (bytes from the
+// program start):
+//   REG1  U: DIAG u = [u0 u1] complex, REAL u = [m00 m01 m10 m11], DENSE u =
+//            2x2 complex, SWAP / NONE nothing; G: DIAG [g0 g1], DENSE 2x2
+//            complex, X / Y / Z / XYZ none.
+//   REG2  U: DIAG u = 4 complex, REAL 4x4 and DENSE 4x4 complex at uoff, SWAP
+//            nothing (swap = 4 a + b exchanged local indices); G: DIAG 4,
+//            DENSE 4x4 complex, Z none.
+//   SEL   two blocks, block c = bit(s0): DIAG u = 2 x 2 complex, REAL u = 2 x 4,
+//            SWAP u[c] nonzero = exchange, DENSE 2 x 8 at uoff; G: DIAG 2 x 2 or
+//            DENSE 2 x 8 at goff.
+//   LANE  U: u = 2 or (s1 >= 0) 4 complex factors, factor c = bit(s0) + 2 bit(s1);
+//            G: as many real factors at goff.
 // Before its operation an instruction applies nremap (0-2) remaps: register
-// bit rq exchanged with lane position rp (4 or 5).
+// bit rq exchanged with lane position rp.
 struct RtInstr {
     int8_t code, a, b, s0, s1, ukind, gkind, swap;
-    int32_t slot; // trainable slot of the pass, -1 otherwise
+    int32_t slot; // first sum of the pass, -1 when not trainable
     int32_t uoff, goff;
     int8_t nremap, rq0, rp0, rq1;
     int8_t rp1, pad8[3];
     int32_t pad;
 };
 static_assert(sizeof(RtInstr) == 32, "RtInstr layout");
+template <typename T> constexpr int rt_stride() { return 32 + 8 * static_cast<int>(sizeof(T)); }
 
 struct RtLaunch {
     int n, T, R;
@@ -312,26 +338,50 @@ struct RtLaunch {
     int tb[RT_TMAX];                   // tile bits, ascending global positions
     int reg_in[RT_RMAX], lane_in[RT_LANE_BITS];   // global bit of each slot at load
     int reg_out[RT_RMAX], lane_out[RT_LANE_BITS]; // and at store
-    int nfin;                          // remaps before the store (0-2):
-    int fin_rq[2], fin_rp[2];          // register bit fin_rq[f] <-> lane position fin_rp[f]
 };
+// Observable states of a launch.
+inline int rt_width(const RtLaunch &L) {
+    return L.nbig * L.nj + (L.nc - L.nbig) * std::max(0, L.nj - 1);
+}
+// LDS of one block: the pass's sums for 16 quads and a dummy slot per lane.
+inline size_t rt_lds_bytes(int nj, int nslots) {
+    return nj > 0 ? (static_cast<size_t>(nslots) * nj * 16 + 64) * sizeof(double) : 0;
+}
 
+constexpr int RT_OBS_MAX = 24; // observable states per register-tile launch
+// Blocks per chunk launch_rtile will use for L (the length of a partials row).
+int rtile_blocks(const Device &dev, int dtype, const RtLaunch &L);
 // Runs one register-tile pass over phi and nc chunks of observable states
 // side by side: nbig chunks of nj states, then nc - nbig chunks of nj - 1
 // (h_ptrs holds their pointers in chunk order). Every chunk
 // reads phi; the last one writes the updated phi to phi_out (nullptr: in
-// place, allowed only with nc == 1). FP64 partials per block go to dev.red
-// as [slot * width + j][block], width = the launch's observable states;
-// returns the blocks per chunk (the reduction's grid).
-constexpr int RT_OBS_MAX = 24; // observable states per register-tile launch
-int launch_rtile(Device &dev, const State &phi, const State *phi_out, void *const *h_ptrs,
-                 const void *d_prog, const RtLaunch &L);
+// place, allowed only with nc == 1). FP64 partials per block go to partials
+// as [slot * width + j][rtile_blocks(L)].
+void launch_rtile(Device &dev, const State &phi, const State *phi_out, void *const *h_ptrs,
+                  const void *d_prog, const RtLaunch &L, double *partials);
+
+// Jacobian entries from the partials of a sweep's launches: entry e's value for
+// observable j0 + j (j < width) is sum_k m[k] (sum of the blocks of row
+// row[k] + j), rows of `blocks` doubles from partials + base.
+struct RtEntry {
+    uint64_t base;    // doubles from the partials buffer
+    int32_t row[3];   // first row (observable 0) of each sum, -1: none
+    int32_t blocks;
+    int32_t col;
+    int32_t j0, width; // observables covered
+    int32_t pad;
+    double m[3];
+};
+static_assert(sizeof(RtEntry) == 64, "RtEntry layout");
+void launch_rtile_entries(Device &dev, const double *partials, const RtEntry *entries, int count, int width,
+                          double *d_jac, int ld);
+
 // Single-operation steps (kernels_step.hip) for operations the fused passes
 // do not hold. One launch applies U to phi (when write_phi) and to nj
 // observable states and, for a trainable op, writes the FP64 block sums of
-// Im<h_j | G phi> (phi before U) to dev.red as [j][block]; d_mats holds U then
-// G restricted to the subspace, D x D FP64 complex matrices (row-major in
-// the order of off). Returns the grid size.
+// Im<h_j | G phi> (phi before U) to partials as [j][step_blocks(L)]; d_mats
+// holds U then G restricted to the subspace, D x D FP64 complex matrices
+// (row-major in the order of off).
 constexpr int STEP_MMAX = 4;
 struct StepLaunch {
     int m;         // 1..4: U (and G) on a subspace of the op's wires; 0: parity phases
@@ -345,15 +395,16 @@ struct StepLaunch {
     uint64_t umask, gmask;         // parity: global bit masks of U's and G's wires
     double ue[2], uo[2];           // parity: U's phase for even / odd parity
 };
-int launch_step(Device &dev, const State &phi, void *const *h_ptrs, const void *d_mats,
-                const StepLaunch &L);
+int step_blocks(const Device &dev, const StepLaunch &L);
+void launch_step(Device &dev, const State &phi, void *const *h_ptrs, const void *d_mats,
+                 const StepLaunch &L, double *partials);
 
-constexpr int RT_NJMAX = 5; // observable states per register-tile launch
 // One variant per precision (float / double) and chunk 0..RT_NJMAX, each
 // compiled from kernels_rtile.hip as an object of its own.
+template <typename T, int NJ> int rtile_blocks_t(const Device &dev, const RtLaunch &L, int nc);
 template <typename T, int NJ>
-int rtile_launch_t(Device &dev, const State &phi, void *phi_out, void *const *h_ptrs,
-                   const void *d_prog, const RtLaunch &L);
+void rtile_launch_t(Device &dev, const State &phi, void *phi_out, void *const *h_ptrs, const void *d_prog,
+                    const RtLaunch &L, int bpc, double *partials);
 
 // Batched circuits (kernels_batch.hip). One workgroup runs one circuit at a
 // time from |0...0>: forward passes, h = H phi and <H>, reverse passes with

@@ -80,6 +80,20 @@ void ensure_red(Device &d, size_t partial_doubles, size_t out_doubles) {
     }
 }
 
+void ensure_parts(Device &d, size_t doubles) {
+    if (doubles > d.parts_cap) {
+        PLK_HIP(hipStreamSynchronize(d.stream));
+        if (d.parts) {
+            PLK_HIP(hipFree(d.parts));
+            d.parts = nullptr;
+            d.parts_cap = 0;
+        }
+        const size_t cap = std::max<size_t>(doubles, size_t{1} << 16);
+        d.parts = static_cast<double *>(dev_malloc(d.id, cap * sizeof(double), "partials"));
+        d.parts_cap = cap;
+    }
+}
+
 namespace {
 uint64_t g_call = 1;
 } // namespace
@@ -358,40 +372,58 @@ std::string profiling_names_impl() {
 namespace plk {
 
 namespace {
-template <typename T>
-int launch_rtile_t(Device &dev, const State &phi, void *out, void *const *h, const void *p,
-                   const RtLaunch &L) {
-    switch (L.nj) {
-    case 0: return rtile_launch_t<T, 0>(dev, phi, out, h, p, L);
-    case 1: return rtile_launch_t<T, 1>(dev, phi, out, h, p, L);
-    case 2: return rtile_launch_t<T, 2>(dev, phi, out, h, p, L);
-    case 3: return rtile_launch_t<T, 3>(dev, phi, out, h, p, L);
-    case 4: return rtile_launch_t<T, 4>(dev, phi, out, h, p, L);
-    case 5: return rtile_launch_t<T, 5>(dev, phi, out, h, p, L);
+// f(variant of the chunk nj).
+template <typename F> void with_chunk(int nj, F &&f) {
+    switch (nj) {
+    case 0: f(std::integral_constant<int, 0>{}); return;
+    case 1: f(std::integral_constant<int, 1>{}); return;
+    case 2: f(std::integral_constant<int, 2>{}); return;
+    case 3: f(std::integral_constant<int, 3>{}); return;
+    case 4: f(std::integral_constant<int, 4>{}); return;
     default: break;
     }
-    raise(PLK_ERR_INVALID, "unsupported register-tile observable chunk " + std::to_string(L.nj));
+    static_assert(RT_NJMAX == 4, "one case per chunk");
+    raise(PLK_ERR_INVALID, "unsupported register-tile observable chunk " + std::to_string(nj));
 }
 } // namespace
 
-int launch_rtile(Device &dev, const State &phi, const State *phi_out, void *const *h_ptrs,
-                 const void *d_prog, const RtLaunch &L) {
-    const int R = phi.dtype == PLK_C64 ? 4 : 3;
-    const int nc = std::max(1, L.nc);
-    if (L.R != R || L.T != R + RT_LANE_BITS || L.T > L.n || L.nslots > RT_PMAX || L.nj < 0 ||
-        nc * std::max(1, L.nj) > RT_OBS_MAX || (nc > 1 && L.nj == 0) || L.nbig > nc ||
-        (L.nj == 1 && L.nbig < nc)) {
+int rtile_blocks(const Device &dev, int dtype, const RtLaunch &L) {
+    int blocks = 0;
+    if (L.nslots < 0 || L.nslots > RT_SLOTS_MAX) {
+        raise(PLK_ERR_INVALID, "register-tile pass with too many sums");
+    }
+    with_chunk(L.nj, [&](auto NJ) {
+        constexpr int nj = decltype(NJ)::value;
+        blocks = dtype == PLK_C64 ? rtile_blocks_t<float, nj>(dev, L, L.nc)
+                                  : rtile_blocks_t<double, nj>(dev, L, L.nc);
+    });
+    return blocks;
+}
+
+void launch_rtile(Device &dev, const State &phi, const State *phi_out, void *const *h_ptrs,
+                  const void *d_prog, const RtLaunch &L, double *partials) {
+    const int R = rt_reg_bits(phi.dtype, L.nj);
+    if (L.R != R || L.T != R + RT_LANE_BITS || L.T > L.n || L.n != phi.n || L.nslots > RT_SLOTS_MAX || L.nj < 0 ||
+        L.nc < 1 || L.nc * std::max(1, L.nj) > RT_OBS_MAX || (L.nc > 1 && L.nj == 0) || L.nbig < 0 ||
+        L.nbig > L.nc || (L.nj == 1 && L.nbig < L.nc) || (L.nslots > 0 && partials == nullptr)) {
         raise(PLK_ERR_INVALID, "register-tile pass does not match the state");
     }
     if (phi_out != nullptr && (phi_out->len != phi.len || phi_out->dtype != phi.dtype)) {
         raise(PLK_ERR_INVALID, "register-tile pass: output state of another shape");
     }
-    if (nc > 1 && L.write_phi && (phi_out == nullptr || phi_out->d == phi.d)) {
+    if (L.nc > 1 && L.write_phi && (phi_out == nullptr || phi_out->d == phi.d)) {
         raise(PLK_ERR_INVALID, "register-tile pass: chunks side by side need a separate output");
     }
     void *out = phi_out ? phi_out->d : phi.d;
-    return phi.dtype == PLK_C64 ? launch_rtile_t<float>(dev, phi, out, h_ptrs, d_prog, L)
-                                : launch_rtile_t<double>(dev, phi, out, h_ptrs, d_prog, L);
+    const int blocks = rtile_blocks(dev, phi.dtype, L);
+    with_chunk(L.nj, [&](auto NJ) {
+        constexpr int nj = decltype(NJ)::value;
+        if (phi.dtype == PLK_C64) {
+            rtile_launch_t<float, nj>(dev, phi, out, h_ptrs, d_prog, L, blocks, partials);
+        } else {
+            rtile_launch_t<double, nj>(dev, phi, out, h_ptrs, d_prog, L, blocks, partials);
+        }
+    });
 }
 
 } // namespace plk
