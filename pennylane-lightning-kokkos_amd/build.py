@@ -34,7 +34,7 @@ HIP_FLAGS = [
 LIB_SOURCES = ["gates.cpp", "runtime.cpp", "capi.cpp", "fuse.cpp", "kernels_apply.hip",
                "kernels_measure.hip", "kernels_tile.hip", "kernels_batch.hip",
                "kernels_sample.hip", "kernels_block.hip", "kernels_dense.hip",
-               "kernels_step.hip", "kernels_reduce.hip"]
+               "kernels_step.hip", "kernels_reduce.hip", "kernels_sweep.hip"]
 
 # The register-tile kernel is compiled once per (precision, observable chunk)
 # variant, each as an object of its own (RT_NJMAX in csrc/plk_internal.hpp).
@@ -82,7 +82,8 @@ def build_lib(verbose=False, incremental=False) -> str:
     work = [("kernels_rtile.hip", [f"PLK_RT_T={t}", f"PLK_RT_NJ={nj}"], f"kernels_rtile_{t}_{nj}",
              ["-mllvm", "-structurizecfg-skip-uniform-regions=true"])
             for t, nj in RTILE_VARIANTS]
-    work += [(s, [], s, []) for s in LIB_SOURCES]
+    work += [(s, [], s, ["-mllvm", "-structurizecfg-skip-uniform-regions=true"] if s == "kernels_sweep.hip" else [])
+             for s in LIB_SOURCES]
     jobs = min(len(work), int(os.environ.get("MAX_JOBS", "8")))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         objs = list(ex.map(lambda j: _compile(j, verbose, incremental), work))

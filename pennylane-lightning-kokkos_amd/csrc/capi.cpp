@@ -11,6 +11,7 @@
 #include <set>
 #include <sstream>
 #include <thread>
+#include <tuple>
 
 #include "plk_internal.hpp"
 
@@ -1666,8 +1667,8 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
 }
 
 // Programs of every register-tile pass of a plan, uploaded as one blob.
-// nj: observable states per chunk (0: forward).
-PlanImage build_image(const std::vector<Step> &steps, const State &s, int nj) {
+// R: register bits of the tile passes.
+PlanImage build_image(const std::vector<Step> &steps, const State &s, int R) {
     PlanImage img;
     if (s.dtype == PLK_C64) {
         build_seg_tables<float>(steps, s.n, img);
@@ -1681,7 +1682,6 @@ PlanImage build_image(const std::vector<Step> &steps, const State &s, int nj) {
         }
     }
     img.progs.resize(steps.size());
-    const int R = rt_reg_bits(s.dtype, nj);
     double norm = 1.0;
     for (size_t i = 0; i < steps.size(); i++) {
         if (steps[i].tiled && steps[i].pass.rt) {
@@ -1837,7 +1837,7 @@ void enqueue_forward(Device &dev, const State &s, const std::vector<Step> &steps
 }
 
 void run_forward(Device &dev, const State &s, const std::vector<Step> &steps) {
-    const PlanImage img = build_image(steps, s, 0);
+    const PlanImage img = build_image(steps, s, rt_reg_bits(s.dtype, 0));
     enqueue_forward(dev, s, steps, img, place_in_arena(dev, img));
     // The host image is read by the stream's copies.
     PLK_HIP(hipStreamSynchronize(dev.stream));
@@ -1992,15 +1992,21 @@ struct OpsData {
     }
 };
 
-// Forward plan of the whole op list (applyOperations, AdjointDiffKokkos.hpp:213-226).
-std::vector<Step> forward_plan(const OpsData &ops, int n, int dtype) {
+// The whole op list, compiled (applyOperations, AdjointDiffKokkos.hpp:213-226).
+std::vector<PlanOp> forward_ops(const OpsData &ops, int n) {
     std::vector<PlanOp> v;
+    v.reserve(ops.names.size());
     for (size_t i = 0; i < ops.names.size(); i++) {
         PlanOp p;
         p.U = compile_op(ops.names[i], ops.wires[i], ops.inverses[i], ops.params[i],
                          ops.matrices[i], n);
         v.push_back(std::move(p));
     }
+    return v;
+}
+
+// Forward plan of the whole op list.
+std::vector<Step> forward_plan(std::vector<PlanOp> &&v, int n, int dtype) {
     if (use_rtile(n, dtype, 0)) {
         return plan_tiles(std::move(v), n, rt_reg_bits(dtype, 0) + RT_LANE_BITS, low_bits(dtype),
                           RT_SLOTS_MAX, false);
@@ -2425,6 +2431,173 @@ bool steps_have_single(const std::vector<Step> &steps, int n) {
     return false;
 }
 
+// ---------------------------------------------------------------------------
+// Whole circuits in one launch (kernels_sweep.hip): one workgroup per
+// observable runs every pass of the circuit.
+// ---------------------------------------------------------------------------
+// Up to 12 qubits the launch beats a launch per pass (12 qubits, 12
+// observables, complex128: 392 against 532 us a Jacobian). PLK_SWEEP=0 turns it off.
+constexpr int kSweepQubits = 12;
+
+bool sweep_serves(const State &s) {
+    return s.n <= kSweepQubits && env_int("PLK_SWEEP", 1) != 0 && env_int("PLK_RTILE", -1) != 0;
+}
+
+// Every op fits a register-tile pass.
+bool sweep_takes(std::vector<PlanOp> &ops) {
+    for (auto &p : ops) {
+        if (p.U.kind == OpKind::Identity && !p.trainable) {
+            continue;
+        }
+        prepare(p);
+        if (!fusable(p)) {
+            return false;
+        }
+    }
+    return true;
+}
+
+// Host tables of a whole-circuit launch.
+struct SweepTables {
+    std::vector<SweepPass> passes;
+    std::vector<SweepEntry> entries;
+    std::vector<SweepTerm> terms;
+    std::vector<unsigned char> blob;
+
+    // Plans ops into passes; returns the first and the number of them.
+    std::pair<int, int> add(std::vector<PlanOp> &&ops, int n, int dtype) {
+        const int R = sweep_reg_bits(dtype), T = R + RT_LANE_BITS;
+        const int first = static_cast<int>(passes.size());
+        double norm = 1.0;
+        // The state stays in L1 and L2, so no low bits are forced into a tile.
+        for (Step &st : plan_tiles(std::move(ops), n, T, 0, RT_SLOTS_MAX, false)) {
+            for (int b = n; static_cast<int>(st.pass.tb.size()) < T; b++) {
+                st.pass.tb.push_back(b); // idle bits of a state smaller than a tile
+            }
+            const RtProgram pr = dtype == PLK_C64 ? build_rt_program<float>(st.pass, n, R, blob, norm)
+                                                  : build_rt_program<double>(st.pass, n, R, blob, norm);
+            SweepPass P{};
+            P.prog = static_cast<int64_t>(pr.off);
+            P.T = T;
+            P.ninstr = pr.L.ninstr;
+            P.nslots = pr.L.nslots;
+            P.entry_first = static_cast<int32_t>(entries.size());
+            P.entry_count = static_cast<int32_t>(pr.terms.size());
+            std::copy(pr.L.tb, pr.L.tb + RT_TMAX, P.tb);
+            std::copy(pr.L.reg_in, pr.L.reg_in + RT_RMAX, P.reg_in);
+            std::copy(pr.L.reg_out, pr.L.reg_out + RT_RMAX, P.reg_out);
+            std::copy(pr.L.lane_in, pr.L.lane_in + RT_LANE_BITS, P.lane_in);
+            std::copy(pr.L.lane_out, pr.L.lane_out + RT_LANE_BITS, P.lane_out);
+            passes.push_back(P);
+            for (const RtTerm &t : pr.terms) {
+                entries.push_back({t.col, {t.slot[0], t.slot[1], t.slot[2]}, {t.m[0], t.m[1], t.m[2]}});
+            }
+        }
+        return {first, static_cast<int>(passes.size()) - first};
+    }
+};
+
+int sweep_waves(int n, int dtype) {
+    const int T = sweep_reg_bits(dtype) + RT_LANE_BITS;
+    return n > T ? std::min(kSweepWaves, 1 << (n - T)) : 1;
+}
+
+// Uploads the tables and the jobs (one copy) and launches; waits for the
+// stream, which has then read the host image.
+void run_sweep(Device &dev, int dtype, int n, const SweepTables &t, const std::vector<SweepJob> &jobs,
+               std::vector<double> *jac, const double *d_jac) {
+    auto up = [](size_t x) { return (x + 255) & ~size_t{255}; };
+    const size_t o_pass = up(jobs.size() * sizeof(SweepJob));
+    const size_t o_ent = o_pass + up(t.passes.size() * sizeof(SweepPass));
+    const size_t o_term = o_ent + up(t.entries.size() * sizeof(SweepEntry));
+    const size_t o_blob = o_term + up(t.terms.size() * sizeof(SweepTerm));
+    std::vector<unsigned char> host(o_blob + up(t.blob.size()));
+    auto put = [&](size_t off, const void *src, size_t bytes) {
+        if (bytes) {
+            std::memcpy(host.data() + off, src, bytes);
+        }
+    };
+    put(0, jobs.data(), jobs.size() * sizeof(SweepJob));
+    put(o_pass, t.passes.data(), t.passes.size() * sizeof(SweepPass));
+    put(o_ent, t.entries.data(), t.entries.size() * sizeof(SweepEntry));
+    put(o_term, t.terms.data(), t.terms.size() * sizeof(SweepTerm));
+    put(o_blob, t.blob.data(), t.blob.size());
+    auto *d = static_cast<unsigned char *>(arena_alloc(dev, host.size()));
+    PLK_HIP(hipMemcpyAsync(d, host.data(), host.size(), hipMemcpyHostToDevice, dev.stream));
+    SweepArgs A;
+    A.jobs = reinterpret_cast<const SweepJob *>(d);
+    A.passes = reinterpret_cast<const SweepPass *>(d + o_pass);
+    A.entries = reinterpret_cast<const SweepEntry *>(d + o_ent);
+    A.terms = reinterpret_cast<const SweepTerm *>(d + o_term);
+    A.blob = d + o_blob;
+    launch_sweep(dev, dtype, A, static_cast<int>(jobs.size()), sweep_waves(n, dtype));
+    if (jac != nullptr && !jac->empty()) {
+        PLK_HIP(hipMemcpyAsync(jac->data(), d_jac, jac->size() * sizeof(double), hipMemcpyDeviceToHost,
+                               dev.stream));
+    }
+    PLK_HIP(hipStreamSynchronize(dev.stream));
+}
+
+void sweep_forward(Device &dev, const State &s, std::vector<PlanOp> &&ops) {
+    SweepTables t;
+    SweepJob J{};
+    J.n = s.n;
+    std::tie(J.fwd_first, J.fwd_count) = t.add(std::move(ops), s.n, s.dtype);
+    J.ref = J.phi = s.d;
+    run_sweep(dev, s.dtype, s.n, t, {J}, nullptr, nullptr);
+}
+
+// The Jacobian by one workgroup per observable; false when an op or an
+// observable needs the general path. rev: the reverse walk's ops.
+bool sweep_jacobian(Device &dev, const State &ref, const std::vector<std::shared_ptr<const ObsNode>> &obs,
+                    const OpsData &ops, std::vector<PlanOp> &rev, size_t n_tp, bool apply_ops, double *jac) {
+    if (!sweep_serves(ref) || !sweep_takes(rev)) {
+        return false;
+    }
+    const int n = ref.n;
+    SweepTables t;
+    std::vector<SweepJob> jobs(obs.size());
+    for (size_t j = 0; j < obs.size(); j++) {
+        std::vector<PauliTerm> terms;
+        if (!to_pauli(*obs[j], n, terms)) {
+            return false;
+        }
+        jobs[j].term_first = static_cast<int32_t>(t.terms.size());
+        jobs[j].term_count = static_cast<int32_t>(terms.size());
+        for (const auto &p : terms) {
+            t.terms.push_back({static_cast<uint32_t>(p.x), static_cast<uint32_t>(p.zy), p.coeff.real(),
+                               p.coeff.imag()});
+        }
+    }
+    std::vector<PlanOp> fwd;
+    if (apply_ops) {
+        fwd = forward_ops(ops, n);
+        if (!sweep_takes(fwd)) {
+            return false;
+        }
+    }
+    const std::pair<int, int> f = t.add(std::move(fwd), n, ref.dtype);
+    const std::pair<int, int> r = t.add(std::move(rev), n, ref.dtype);
+    const size_t bytes = (ref.bytes() + 255) & ~size_t{255};
+    auto *scratch = static_cast<unsigned char *>(arena_alloc(dev, 2 * bytes * obs.size()));
+    double *d_jac = ensure_jac(dev, obs.size() * n_tp);
+    for (size_t j = 0; j < obs.size(); j++) {
+        SweepJob &J = jobs[j];
+        J.n = n;
+        std::tie(J.fwd_first, J.fwd_count) = f;
+        std::tie(J.rev_first, J.rev_count) = r;
+        J.jac_len = static_cast<int32_t>(n_tp);
+        J.ref = ref.d;
+        J.phi = scratch + 2 * j * bytes;
+        J.h = scratch + (2 * j + 1) * bytes;
+        J.jac = d_jac + j * n_tp;
+    }
+    std::vector<double> out(obs.size() * n_tp);
+    run_sweep(dev, ref.dtype, n, t, jobs, &out, d_jac);
+    std::copy(out.begin(), out.end(), jac);
+    return true;
+}
+
 void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const ObsNode>> &obs,
                       const OpsData &ops, const std::vector<size_t> &tp, bool apply_ops,
                       double *jac) {
@@ -2443,6 +2616,9 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
     if (n_obs == 0) {
         return;
     }
+    if (sweep_jacobian(dev, ref, obs, ops, rev, n_tp, apply_ops, jac)) {
+        return;
+    }
     const int nj = sweep_chunk(ref.dtype, n, n_obs, dev.num_cus);
     const bool rt = use_rtile(n, ref.dtype, nj);
     const int T_adj = rt ? rt_reg_bits(ref.dtype, nj) + RT_LANE_BITS : tile_bits_adjoint(n, ref.dtype);
@@ -2450,9 +2626,9 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
         rt ? plan_tiles(std::move(rev), n, T_adj, low_bits(ref.dtype), RT_SLOTS_MAX, false)
            : T_adj > 0 ? plan_tiles(std::move(rev), n, T_adj, low_bits(ref.dtype))
                        : plan_steps(std::move(rev));
-    const std::vector<Step> fwd = apply_ops ? forward_plan(ops, n, ref.dtype) : std::vector<Step>{};
-    const PlanImage img_f = build_image(fwd, ref, 0);
-    PlanImage img_r = build_image(steps, ref, nj);
+    const std::vector<Step> fwd = apply_ops ? forward_plan(forward_ops(ops, n), n, ref.dtype) : std::vector<Step>{};
+    const PlanImage img_f = build_image(fwd, ref, rt_reg_bits(ref.dtype, 0));
+    PlanImage img_r = build_image(steps, ref, rt_reg_bits(ref.dtype, nj));
     const bool alt = needs_alt(dev, steps, n_obs, ref.dtype, n);
     const SweepParts parts = place_partials(dev, steps, img_r, ref, n_obs, alt);
     plan_scope.reset();
@@ -3487,7 +3663,12 @@ int plk_apply_ops(plk_state *sv, const plk_ops *ops) {
             raise(PLK_ERR_INVALID, "null ops handle");
         }
         Device &dev = dev_of(s);
-        run_forward(dev, s, forward_plan(ops->data, s.n, s.dtype));
+        std::vector<PlanOp> v = forward_ops(ops->data, s.n);
+        if (sweep_serves(s) && sweep_takes(v)) {
+            sweep_forward(dev, s, std::move(v));
+        } else {
+            run_forward(dev, s, forward_plan(std::move(v), s.n, s.dtype));
+        }
     })
 }
 

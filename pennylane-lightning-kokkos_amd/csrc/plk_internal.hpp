@@ -376,6 +376,55 @@ static_assert(sizeof(RtEntry) == 64, "RtEntry layout");
 void launch_rtile_entries(Device &dev, const double *partials, const RtEntry *entries, int count, int width,
                           double *d_jac, int ld);
 
+// Whole circuits by one workgroup each (kernels_sweep.hip).
+constexpr int kSweepWaves = 8; // most waves of a workgroup
+// Register bits of a sweep's tiles: the largest state of the dispatch then has
+// one tile per wave (12 qubits, 12 observables, complex128: 223 us a Jacobian;
+// one bit less and 16 waves: 268).
+template <typename T> constexpr int sweep_reg_bits() { return sizeof(T) == 4 ? 4 : 3; }
+inline int sweep_reg_bits(int dtype) { return dtype == PLK_C64 ? 4 : 3; }
+
+struct SweepPass {
+    int64_t prog; // byte offset of the program in the blob
+    int32_t T;    // tile bits (those from n up are idle when n < T)
+    int32_t ninstr, nslots;
+    int32_t entry_first, entry_count;
+    int32_t tb[RT_TMAX];
+    int32_t reg_in[RT_RMAX], lane_in[RT_LANE_BITS];
+    int32_t reg_out[RT_RMAX], lane_out[RT_LANE_BITS];
+};
+// jac[col] = sum_k m[k] * sum slot[k] (-1: none).
+struct SweepEntry {
+    int32_t col;
+    int32_t slot[3];
+    double m[3];
+};
+struct SweepTerm {
+    uint32_t x, zy; // Pauli word: flipped bits, signed bits
+    double cr, ci;  // coefficient, including (-i)^{#Y}
+};
+struct SweepJob {
+    int32_t n;
+    int32_t fwd_first, fwd_count; // passes
+    int32_t rev_first, rev_count;
+    int32_t term_first, term_count;
+    int32_t jac_len; // Jacobian entries (zeroed first)
+    const void *ref; // input state; nullptr: |0...0>; == phi: in place
+    void *phi;
+    void *h;         // nullptr: forward passes only
+    double *jac;
+    double *expval;  // may be nullptr
+};
+struct SweepArgs {
+    const SweepJob *jobs;
+    const SweepPass *passes;
+    const SweepEntry *entries;
+    const SweepTerm *terms;
+    const unsigned char *blob;
+};
+// One workgroup of `waves` waves per job.
+void launch_sweep(Device &dev, int dtype, const SweepArgs &A, int jobs, int waves);
+
 // Single-operation steps (kernels_step.hip) for operations the fused passes
 // do not hold. One launch applies U to phi (when write_phi) and to nj
 // observable states and, for a trainable op, writes the FP64 block sums of
