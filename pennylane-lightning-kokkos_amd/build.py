@@ -82,7 +82,7 @@ def build_lib(verbose=False, incremental=False) -> str:
     work = [("kernels_rtile.hip", [f"PLK_RT_T={t}", f"PLK_RT_NJ={nj}"], f"kernels_rtile_{t}_{nj}",
              ["-mllvm", "-structurizecfg-skip-uniform-regions=true"])
             for t, nj in RTILE_VARIANTS]
-    work += [(s, [], s, ["-mllvm", "-structurizecfg-skip-uniform-regions=true"] if s == "kernels_sweep.hip" else [])
+    work += [(s, [], s, ["-mllvm", "-structurizecfg-skip-uniform-regions=true"] if s in ("kernels_sweep.hip", "kernels_batch.hip") else [])
              for s in LIB_SOURCES]
     jobs = min(len(work), int(os.environ.get("MAX_JOBS", "8")))
     with ThreadPoolExecutor(max_workers=jobs) as ex:

@@ -7,7 +7,6 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
-#include <queue>
 #include <set>
 #include <sstream>
 #include <thread>
@@ -25,6 +24,25 @@ const cd kI{0.0, 1.0};
 
 Device &dev_of(const State &s) { return device(s.device); }
 
+// 64-bit structure hash (multiply-xorshift over 64-bit words).
+struct Hasher {
+    uint64_t h = 0x243F6A8885A308D3ull;
+    void add(uint64_t v) {
+        h ^= v + 0x9E3779B97F4A7C15ull + (h << 6) + (h >> 2);
+        h *= 0xFF51AFD7ED558CCDull;
+        h ^= h >> 32;
+    }
+    void add(double v) {
+        uint64_t b;
+        std::memcpy(&b, &v, sizeof b);
+        add(b);
+    }
+    void add(const std::string &str) {
+        add(static_cast<uint64_t>(str.size()));
+        add(static_cast<uint64_t>(std::hash<std::string>{}(str)));
+    }
+};
+
 // ---------------------------------------------------------------------------
 // Observables (ObservablesKokkos.hpp:19-517).
 // ---------------------------------------------------------------------------
@@ -40,6 +58,7 @@ struct ObsNode {
     std::vector<int32_t> indices32, indptr32;   // int32 matrices (complex64 serialisation)
     bool idx32 = false;
     size_t rows = 0;
+    uint64_t key = 0; // hash of the tree (CSR values left out), set once by obs_key
     // Device copies of the CSR matrix per (device, state dtype), made on first
     // use and kept while the observable lives (entry points hold the engine
     // lock, so the cache needs no lock of its own).
@@ -69,6 +88,31 @@ struct ObsNode {
         return *slot;
     }
 };
+
+// Hash of an observable's tree from its parts; its terms have theirs.
+uint64_t obs_key(const ObsNode &o) {
+    Hasher H;
+    H.add(static_cast<uint64_t>(o.kind));
+    H.add(o.name);
+    H.add(static_cast<uint64_t>(o.wires.size()));
+    for (auto w : o.wires) {
+        H.add(static_cast<uint64_t>(w));
+    }
+    H.add(static_cast<uint64_t>(o.coeffs.size()));
+    for (double c : o.coeffs) {
+        H.add(c);
+    }
+    H.add(static_cast<uint64_t>(o.matrix.size()));
+    for (const cd &m : o.matrix) {
+        H.add(m.real());
+        H.add(m.imag());
+    }
+    H.add(static_cast<uint64_t>(o.terms.size()));
+    for (const auto &t : o.terms) {
+        H.add(t->key);
+    }
+    return H.h;
+}
 
 std::vector<size_t> obs_wires(const ObsNode &o) {
     std::set<size_t> w;
@@ -176,16 +220,21 @@ struct RunTerm {
     double m[3];
 };
 
+// A gate of a run in a batch plan: its patch, or the matrix it always has.
+struct RunGate {
+    BatchGate g{};
+    std::vector<cd> mat; // BPG_CONST
+};
+
 struct PlanOp {
     CompiledOp U;
+    std::vector<RunGate> gates; // batch plans: the gates of a one-wire op, in order
     std::vector<RunTerm> run; // register-tile plans: the trainable gates of a one-wire run
     bool trainable = false;
     CompiledGen G;
     int col = -1;
     double coef = 0.0;
     int32_t src = -1;       // index of the op in its OpsData
-    int32_t param = -1;     // batch plans: global parameter index of a patched op
-    int16_t patch_gate = 0; // batch plans: BatchPatchGate of a patched op
     bool adj = false;       // U was compiled with the inverse flag set
 };
 
@@ -464,6 +513,7 @@ std::vector<PlanOp> fuse_runs(std::vector<PlanOp> &&ops) {
             out.push_back(std::move(p));
         } else {
             PlanOp &o = out[open[w]];
+            o.gates.insert(o.gates.end(), p.gates.begin(), p.gates.end());
             o.U.mat = mul2(p.U.mat, o.U.mat);
         }
     }
@@ -864,23 +914,9 @@ SegMeta build_segment(const Segment &seg, int n, std::vector<unsigned char> &tab
     return meta;
 }
 
-// U payload layout a patched gate keeps for every angle (the structure of
-// the gate at a generic angle, which special angles only refine).
-int32_t patch_ukind(int16_t gate) {
-    switch (gate) {
-    case BPG_RX:
-        return U_DENSE;
-    case BPG_RY:
-        return U_REAL;
-    default:
-        return U_DIAG;
-    }
-}
-
 template <typename T>
 void build_pass(const Pass &ps, int n, std::vector<unsigned char> &table,
-                std::vector<TileBundle> &btab, SegMeta &meta,
-                std::vector<BatchPatch> *patches = nullptr) {
+                std::vector<TileBundle> &btab, SegMeta &meta) {
     TileLaunch &TL = meta.TL;
     TL.n = n;
     TL.T = static_cast<int>(ps.tb.size());
@@ -923,27 +959,11 @@ void build_pass(const Pass &ps, int n, std::vector<unsigned char> &table,
                 d.slot = slot++;
             }
             classify(d, w.size());
-            if (patches != nullptr && p.patch_gate != BPG_NONE) {
-                d.ukind = patch_ukind(p.patch_gate);
-            }
             group.push_back(d);
         }
         const size_t off = pack_ops(table, group.data(), group.size());
         if (off > static_cast<size_t>(INT32_MAX)) {
             raise(PLK_ERR_UNSUPPORTED, "operation table exceeds 2 GiB");
-        }
-        if (patches != nullptr) {
-            for (size_t o = 0; o < b.ops.size(); o++) {
-                const PlanOp &p = b.ops[o];
-                if (p.patch_gate == BPG_NONE) {
-                    continue;
-                }
-                OpHead h;
-                std::memcpy(&h, table.data() + off + o * sizeof(OpHead), sizeof(OpHead));
-                patches->push_back(BatchPatch{static_cast<int64_t>(off) + (h.offs & 0xffff),
-                                              p.param, p.patch_gate,
-                                              static_cast<int16_t>(p.adj ? 1 : 0)});
-            }
         }
         tb.first = static_cast<int32_t>(off);
         slot0 += b.nslots;
@@ -964,8 +984,17 @@ struct RtTerm {
     double m[3]; // coefficients, the gate's own included
 };
 
+// The instruction of an op with patched gates (batch plans).
+struct RtPatch {
+    size_t op;
+    size_t ins;  // byte offset of its reals in the program
+    int term;    // first of its terms, -1: none
+    int16_t ukind, parts;
+};
+
 struct RtProgram {
     RtLaunch L{};
+    std::vector<RtPatch> patches;
     size_t off = 0; // byte offset of the program in the plan blob
     std::vector<RtTerm> terms;
 };
@@ -1321,7 +1350,8 @@ std::vector<double> keep_norm(std::vector<double> u, int dim, double &norm) {
 }
 
 template <typename T>
-RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned char> &blob, double &norm) {
+RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned char> &blob, double &norm,
+                           bool patched = false) {
     RtProgram out;
     RtLaunch &L = out.L;
     L.n = n;
@@ -1478,6 +1508,7 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
         }
         const int m = static_cast<int>(gbits[i].size());
         const std::vector<cd> *G = nullptr;
+        const int term0 = static_cast<int>(out.terms.size());
         if (p.trainable) {
             in.slot = slot;
             if (p.run.empty()) {
@@ -1508,7 +1539,7 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
                 in.code = RT_REG1;
                 in.a = static_cast<int8_t>(r);
                 u = rt_encode_u1(in, p.U.mat);
-                if (sizeof(T) == 4 && !u.empty()) {
+                if (sizeof(T) == 4 && !u.empty() && !patched) {
                     u = keep_norm(std::move(u), 2, norm);
                 }
                 if (G) {
@@ -1525,7 +1556,7 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
                 in.code = RT_LANE;
                 in.s0 = static_cast<int8_t>(sel_of(gbits[i][0]));
                 u = cplx({p.U.mat[0], p.U.mat[3]});
-                if (sizeof(T) == 4) {
+                if (sizeof(T) == 4 && !patched) {
                     u = keep_norm(std::move(u), 2, norm);
                 }
                 if (G) {
@@ -1629,6 +1660,19 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, std::vector<unsigned ch
                     }
                     in.goff = b.put(g);
                 }
+            }
+        }
+        if (patched) {
+            bool any = false;
+            for (const RunGate &g : p.gates) {
+                any = any || g.g.gate != BPG_CONST;
+            }
+            if (any) {
+                const int parts = run_parts(p);
+                out.patches.push_back({i, b.ins.size() * rt_stride<T>() + sizeof(RtInstr),
+                                       p.run.empty() ? -1 : term0,
+                                       static_cast<int16_t>(in.code == RT_LANE ? U_DIAG : in.ukind),
+                                       static_cast<int16_t>(rt_slots(p) == 3 ? 7 : parts)});
             }
         }
         b.add(in, u);
@@ -1983,22 +2027,69 @@ struct OpsData {
     std::vector<std::vector<size_t>> wires;
     std::vector<bool> inverses;
     std::vector<std::vector<cd>> matrices;
-    size_t num_par_ops() const {
-        size_t c = 0;
-        for (auto &p : params) {
-            c += p.empty() ? 0 : 1;
-        }
-        return c;
-    }
+    // Kept as the list is built (plk_ops_create): the first parameter of every
+    // parametric op, and a hash of everything a batch plan depends on (names,
+    // wires, inverse flags, matrices and the parameters of gates whose angles
+    // it does not patch).
+    std::vector<double> angles;
+    uint64_t structure = 0;
+    size_t num_par_ops() const { return angles.size(); }
 };
 
+// Patched gate of an op: one-parameter rotations without an explicit matrix.
+int16_t patch_gate_of(const OpsData &ops, size_t i) {
+    if (ops.params[i].size() != 1 || !ops.matrices[i].empty()) {
+        return BPG_NONE;
+    }
+    const std::string &nm = ops.names[i];
+    if (nm == "RX") {
+        return BPG_RX;
+    }
+    if (nm == "RY") {
+        return BPG_RY;
+    }
+    if (nm == "RZ") {
+        return BPG_RZ;
+    }
+    if (nm == "PhaseShift") {
+        return BPG_PHASE;
+    }
+    return BPG_NONE;
+}
+
+// Adds op i to the list's hash and angles.
+void note_op(OpsData &ops, Hasher &H, size_t i) {
+    H.add(ops.names[i]);
+    H.add(static_cast<uint64_t>(ops.wires[i].size() | (ops.inverses[i] ? size_t{1} << 40 : 0)));
+    for (auto w : ops.wires[i]) {
+        H.add(static_cast<uint64_t>(w));
+    }
+    H.add(static_cast<uint64_t>(ops.params[i].size()));
+    if (patch_gate_of(ops, i) == BPG_NONE) {
+        for (double v : ops.params[i]) {
+            H.add(v);
+        }
+    }
+    H.add(static_cast<uint64_t>(ops.matrices[i].size()));
+    for (const cd &m : ops.matrices[i]) {
+        H.add(m.real());
+        H.add(m.imag());
+    }
+    if (!ops.params[i].empty()) {
+        ops.angles.push_back(ops.params[i][0]);
+    }
+    ops.structure = H.h;
+}
+
+
 // The whole op list, compiled (applyOperations, AdjointDiffKokkos.hpp:213-226).
-std::vector<PlanOp> forward_ops(const OpsData &ops, int n) {
+std::vector<PlanOp> forward_ops(const OpsData &ops, int n,
+                                const std::vector<std::vector<double>> *params = nullptr) {
     std::vector<PlanOp> v;
     v.reserve(ops.names.size());
     for (size_t i = 0; i < ops.names.size(); i++) {
         PlanOp p;
-        p.U = compile_op(ops.names[i], ops.wires[i], ops.inverses[i], ops.params[i],
+        p.U = compile_op(ops.names[i], ops.wires[i], ops.inverses[i], params ? (*params)[i] : ops.params[i],
                          ops.matrices[i], n);
         v.push_back(std::move(p));
     }
@@ -2022,7 +2113,9 @@ std::vector<Step> forward_plan(std::vector<PlanOp> &&v, int n, int dtype) {
 // after the last trainable one, in reverse order, each trainable op carrying
 // its generator, Jacobian column and coefficient -2 s (inverse ? -1 : 1).
 // StatePrep / BasisState are skipped; ops with several parameters abort.
-std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &tp, int n) {
+// params: values used instead of the list's own (batch plans).
+std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &tp, int n,
+                                const std::vector<std::vector<double>> *params = nullptr) {
     const size_t n_tp = tp.size();
     std::vector<PlanOp> rev;
     size_t trainable_number = n_tp - 1;
@@ -2042,7 +2135,7 @@ std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &t
             break;
         }
         PlanOp p;
-        p.U = compile_op(ops.names[o], ops.wires[o], !ops.inverses[o], ops.params[o],
+        p.U = compile_op(ops.names[o], ops.wires[o], !ops.inverses[o], params ? (*params)[o] : ops.params[o],
                          ops.matrices[o], n);
         p.src = static_cast<int32_t>(o);
         p.adj = !ops.inverses[o];
@@ -2061,25 +2154,6 @@ std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &t
     }
     return rev;
 }
-
-// 64-bit structure hash (multiply-xorshift over 64-bit words).
-struct Hasher {
-    uint64_t h = 0x243F6A8885A308D3ull;
-    void add(uint64_t v) {
-        h ^= v + 0x9E3779B97F4A7C15ull + (h << 6) + (h >> 2);
-        h *= 0xFF51AFD7ED558CCDull;
-        h ^= h >> 32;
-    }
-    void add(double v) {
-        uint64_t b;
-        std::memcpy(&b, &v, sizeof b);
-        add(b);
-    }
-    void add(const std::string &str) {
-        add(static_cast<uint64_t>(str.size()));
-        add(static_cast<uint64_t>(std::hash<std::string>{}(str)));
-    }
-};
 
 // ---------------------------------------------------------------------------
 // Adjoint Jacobian (AdjointDiffKokkos.hpp:404-478).
@@ -2464,18 +2538,27 @@ struct SweepTables {
     std::vector<SweepTerm> terms;
     std::vector<unsigned char> blob;
 
-    // Plans ops into passes; returns the first and the number of them.
-    std::pair<int, int> add(std::vector<PlanOp> &&ops, int n, int dtype) {
+    // Batch plans (patched): the runs with angles.
+    std::vector<BatchRun> runs;
+    std::vector<BatchGate> gates;
+    std::vector<double> consts; // 2x2 complex matrices
+
+    // Plans ops into passes whose tiles hold the lowest L bits; returns the
+    // first and the number of them.
+    std::pair<int, int> add(std::vector<PlanOp> &&ops, int n, int dtype, int L = 0, bool patched = false) {
         const int R = sweep_reg_bits(dtype), T = R + RT_LANE_BITS;
         const int first = static_cast<int>(passes.size());
         double norm = 1.0;
-        // The state stays in L1 and L2, so no low bits are forced into a tile.
-        for (Step &st : plan_tiles(std::move(ops), n, T, 0, RT_SLOTS_MAX, false)) {
+        for (Step &st : plan_tiles(std::move(ops), n, T, L, RT_SLOTS_MAX, false)) {
+            if (!st.tiled) {
+                raise(PLK_ERR_UNSUPPORTED,
+                      "batched circuits support dense gates and generators on at most two wires");
+            }
             for (int b = n; static_cast<int>(st.pass.tb.size()) < T; b++) {
                 st.pass.tb.push_back(b); // idle bits of a state smaller than a tile
             }
-            const RtProgram pr = dtype == PLK_C64 ? build_rt_program<float>(st.pass, n, R, blob, norm)
-                                                  : build_rt_program<double>(st.pass, n, R, blob, norm);
+            const RtProgram pr = dtype == PLK_C64 ? build_rt_program<float>(st.pass, n, R, blob, norm, patched)
+                                                  : build_rt_program<double>(st.pass, n, R, blob, norm, patched);
             SweepPass P{};
             P.prog = static_cast<int64_t>(pr.off);
             P.T = T;
@@ -2483,6 +2566,26 @@ struct SweepTables {
             P.nslots = pr.L.nslots;
             P.entry_first = static_cast<int32_t>(entries.size());
             P.entry_count = static_cast<int32_t>(pr.terms.size());
+            for (const RtPatch &pt : pr.patches) {
+                BatchRun r{};
+                r.ins = P.prog + static_cast<int64_t>(pt.ins);
+                r.first = static_cast<int32_t>(gates.size());
+                r.entry = pt.term < 0 ? -1 : P.entry_first + pt.term;
+                r.ukind = pt.ukind;
+                r.parts = pt.parts;
+                for (const RunGate &g : st.pass.ops[pt.op].gates) {
+                    gates.push_back(g.g);
+                    if (g.g.gate == BPG_CONST) {
+                        gates.back().param = static_cast<int32_t>(consts.size() / 8);
+                        for (const cd &m : g.mat) {
+                            consts.push_back(m.real());
+                            consts.push_back(m.imag());
+                        }
+                    }
+                }
+                r.count = static_cast<int32_t>(gates.size()) - r.first;
+                runs.push_back(r);
+            }
             std::copy(pr.L.tb, pr.L.tb + RT_TMAX, P.tb);
             std::copy(pr.L.reg_in, pr.L.reg_in + RT_RMAX, P.reg_in);
             std::copy(pr.L.reg_out, pr.L.reg_out + RT_RMAX, P.reg_out);
@@ -2842,8 +2945,8 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
 
 // ---------------------------------------------------------------------------
 // Batched circuits: independent circuits, each from |0...0> with one
-// observable, planned on the host into LDS tile passes and run by one
-// persistent launch (kernels_batch.hip).
+// observable, planned on the host into register-tile passes
+// (kernels_batch.hip).
 // ---------------------------------------------------------------------------
 struct BatchInput {
     int n = 0;
@@ -2852,168 +2955,97 @@ struct BatchInput {
     std::vector<size_t> tp;
 };
 
-int batch_tile_bits(int dtype) {
-    const int T = env_int("PLK_BATCH_TILE_BITS", dtype == PLK_C64 ? 12 : 11);
-    return std::max(low_bits(dtype) + 2, std::min(T, BATCH_TMAX));
-}
-
-// Host-side batch plan; every table is uploaded as one blob.
-template <typename T> struct BatchPlan {
-    std::vector<BatchCircuit> circuits;
-    std::vector<BatchPass> passes;
-    std::vector<TileBundle> bundles;
-    std::vector<unsigned char> ops; // packed op groups
-    std::vector<BatchTerm> terms;
-    std::vector<int32_t> slot_cols;
-    std::vector<double> slot_coefs;
-    std::vector<double> cost;
-    std::vector<BatchPatch> patches; // offsets into ops
-    int64_t jac_len = 0;
-    int64_t nparams = 0; // parametric ops of the planned circuits
-
-    // Releases dst's memory (a merged part is no longer needed).
-    void swap_into(BatchPlan &dst) {
-        std::swap(*this, dst);
-    }
+// A planned batch circuit: ranges in its part's tables.
+struct BatchPlanned {
+    int n = 0;
+    std::pair<int, int> fwd, rev;
+    int term_first = 0, term_count = 0;
+    int64_t jac = 0;  // first Jacobian entry
+    double cost = 0.0;
+    bool staged = false;
 };
 
-// Patched gate of an op: one-parameter rotations without an explicit matrix.
-int16_t patch_gate_of(const OpsData &ops, size_t i) {
-    if (ops.params[i].size() != 1 || !ops.matrices[i].empty()) {
-        return BPG_NONE;
-    }
-    const std::string &nm = ops.names[i];
-    if (nm == "RX") {
-        return BPG_RX;
-    }
-    if (nm == "RY") {
-        return BPG_RY;
-    }
-    if (nm == "RZ") {
-        return BPG_RZ;
-    }
-    if (nm == "PhaseShift") {
-        return BPG_PHASE;
-    }
-    return BPG_NONE;
+// The circuits one host thread planned.
+struct BatchPart {
+    SweepTables t;
+    std::vector<BatchPlanned> circuits;
+    int64_t nparams = 0;
+    int64_t jac_len = 0;
+};
+
+// Widest circuit that runs whole in one workgroup: eight tiles, one per wave.
+// Wider ones run pass by pass over many workgroups (a 16-qubit, 8-layer
+// circuit takes 32 ms in one workgroup of LDS tiles).
+int batch_whole_qubits(int dtype) {
+    return env_int("PLK_BATCH_WHOLE_QUBITS", sweep_reg_bits(dtype) + RT_LANE_BITS + 3);
 }
 
-template <typename T>
-void plan_batch_passes(BatchPlan<T> &bp, std::vector<Step> &&steps, const BatchCircuit &c,
-                       int Tt, bool forward, int &first, int &count) {
-    first = static_cast<int>(bp.passes.size());
-    if (forward && steps.empty() && !c.resident) {
-        Step s;
-        s.tiled = true;
-        for (int b = 0; b < Tt; b++) {
-            s.pass.tb.push_back(b);
-        }
-        steps.push_back(std::move(s));
-    }
-    for (auto &st : steps) {
-        if (!st.tiled) {
-            raise(PLK_ERR_UNSUPPORTED,
-                  "batched circuits support dense gates and generators on at most two wires");
-        }
-        SegMeta meta;
-        BatchPass P{};
-        P.bundle_first = static_cast<int32_t>(bp.bundles.size());
-        build_pass<T>(st.pass, c.n, bp.ops, bp.bundles, meta, &bp.patches);
-        P.T = meta.TL.T;
-        P.bundle_count = meta.TL.nbundles;
-        P.nslots = st.pass.nslots;
-        P.slot_first = static_cast<int32_t>(bp.slot_cols.size());
-        for (int q = 0; q < P.T; q++) {
-            P.tb[q] = st.pass.tb[q];
-            P.tmask |= 1u << st.pass.tb[q];
-        }
-        for (int k = 0; k < P.nslots; k++) {
-            bp.slot_cols.push_back(st.pass.cols[k]);
-            bp.slot_coefs.push_back(st.pass.coefs[k]);
-        }
-        size_t ops_in_pass = 0;
-        for (const auto &b : st.pass.bundles) {
-            ops_in_pass += b.ops.size();
-        }
-        const double amps = std::ldexp(1.0, c.n);
-        bp.cost.back() += amps * (static_cast<double>(P.bundle_count) + 0.25 * ops_in_pass) *
-                              (forward ? 1.0 : 2.0) +
-                          (c.resident ? 0.0 : 8.0 * amps);
-        bp.passes.push_back(P);
-    }
-    count = static_cast<int>(bp.passes.size()) - first;
-    if (!c.resident && count > 0) {
-        if (forward) {
-            bp.passes[first].flags |= BP_INIT;
-        } else {
-            bp.passes.back().flags |= BP_NO_STORE;
-        }
-    }
-}
-
-template <typename T>
-void plan_batch_circuit(BatchPlan<T> &bp, const BatchInput &in, int tile_bits, int L) {
+void plan_batch_circuit(BatchPart &bp, const BatchInput &in, int dtype) {
     const int n = in.n;
-    BatchCircuit c{};
+    const OpsData &ops = *in.ops;
+    BatchPlanned c;
     c.n = n;
-    c.resident = n <= tile_bits ? 1 : 0;
-    const int Tt = c.resident ? n : tile_bits;
-    const int Lc = c.resident ? 0 : L;
-    c.jac_offset = bp.jac_len;
-    bp.cost.push_back(0.0);
-
+    c.jac = bp.jac_len;
     std::vector<PauliTerm> pt;
     if (!to_pauli(*in.obs, n, pt)) {
         raise(PLK_ERR_UNSUPPORTED,
               "batched circuits support observables that are sums of Pauli words");
     }
-    c.term_first = static_cast<int32_t>(bp.terms.size());
-    c.term_count = static_cast<int32_t>(pt.size());
+    c.term_first = static_cast<int>(bp.t.terms.size());
+    c.term_count = static_cast<int>(pt.size());
     for (const auto &t : pt) {
-        bp.terms.push_back(BatchTerm{t.x, t.zy, t.coeff.real(), t.coeff.imag()});
+        bp.t.terms.push_back({static_cast<uint32_t>(t.x), static_cast<uint32_t>(t.zy), t.coeff.real(),
+                              t.coeff.imag()});
     }
-    bp.cost.back() += std::ldexp(1.0, n) * (1.0 + 0.25 * static_cast<double>(pt.size()));
-
-    const OpsData &ops = *in.ops;
-    std::vector<PlanOp> rev = reverse_ops(ops, in.tp, n);
-    std::vector<PlanOp> fwd;
-    for (size_t i = 0; i < ops.names.size(); i++) {
-        PlanOp p;
-        p.U = compile_op(ops.names[i], ops.wires[i], ops.inverses[i], ops.params[i],
-                         ops.matrices[i], n);
-        fwd.push_back(std::move(p));
-    }
-    // Global parameter index of every parametric op (circuit order), and the
-    // patch gate of the ones whose U payload is rewritten per call.
+    // The plan must hold for every angle of a patched gate, so those are
+    // planned at generic angles: the structure of a run's matrix and of its
+    // Pauli parts is then the one it has for all but special angles.
+    std::vector<std::vector<double>> params = ops.params;
     std::vector<int32_t> pidx(ops.names.size(), -1);
     int64_t np = bp.nparams;
     for (size_t i = 0; i < ops.names.size(); i++) {
         if (!ops.params[i].empty()) {
             pidx[i] = static_cast<int32_t>(np++);
+            if (patch_gate_of(ops, i) != BPG_NONE) {
+                params[i][0] = 0.7 + 0.4 * static_cast<double>(i % 5);
+            }
         }
     }
     if (np > INT32_MAX) {
         raise(PLK_ERR_UNSUPPORTED, "batched parameters exceed 2^31");
     }
-    auto mark = [&](PlanOp &p) {
-        if (p.src >= 0 && pidx[p.src] >= 0) {
-            p.param = pidx[p.src];
-            p.patch_gate = patch_gate_of(ops, static_cast<size_t>(p.src));
-        }
-    };
-    for (size_t i = 0; i < fwd.size(); i++) {
-        fwd[i].src = static_cast<int32_t>(i);
-        fwd[i].adj = ops.inverses[i];
-        mark(fwd[i]);
-    }
-    for (auto &p : rev) {
-        mark(p);
-    }
     bp.nparams = np;
-    plan_batch_passes(bp, plan_tiles(std::move(fwd), n, Tt, Lc, BATCH_PMAX), c, Tt, true,
-                      c.fwd_first, c.fwd_count);
-    plan_batch_passes(bp, plan_tiles(std::move(rev), n, Tt, Lc, BATCH_PMAX), c, Tt, false,
-                      c.bwd_first, c.bwd_count);
+    auto mark = [&](PlanOp &p, size_t i, bool adj) {
+        if (p.U.wires.size() != 1) {
+            return;
+        }
+        RunGate g;
+        const int16_t kind = patch_gate_of(ops, i);
+        g.g.gate = kind == BPG_NONE ? static_cast<int16_t>(BPG_CONST) : kind;
+        g.g.adj = adj ? 1 : 0;
+        g.g.param = pidx[i];
+        g.g.coef = p.trainable ? p.coef : 0.0;
+        if (kind == BPG_NONE) {
+            prepare(p);
+            g.mat = p.U.mat;
+        }
+        p.gates = {std::move(g)};
+    };
+    std::vector<PlanOp> rev = reverse_ops(ops, in.tp, n, &params);
+    for (auto &p : rev) {
+        mark(p, static_cast<size_t>(p.src), p.adj);
+    }
+    std::vector<PlanOp> fwd = forward_ops(ops, n, &params);
+    for (size_t i = 0; i < fwd.size(); i++) {
+        mark(fwd[i], i, ops.inverses[i]);
+    }
+    const int L = n > batch_whole_qubits(dtype) ? low_bits(dtype) : 0;
+    c.fwd = bp.t.add(std::move(fwd), n, dtype, L, true);
+    c.rev = bp.t.add(std::move(rev), n, dtype, L, true);
+    c.staged = L > 0 && c.fwd.second > 0 && n > sweep_reg_bits(dtype) + RT_LANE_BITS;
+    for (int p = c.fwd.first; p < c.rev.first + c.rev.second; p++) {
+        c.cost += bp.t.passes[p].ninstr * (p < c.rev.first ? 1.0 : 2.0) * std::ldexp(1.0, std::max(0, n - 8));
+    }
     bp.jac_len += static_cast<int64_t>(in.tp.size());
     bp.circuits.push_back(c);
 }
@@ -3031,42 +3063,39 @@ struct Blob {
 };
 
 // Appends src's circuits to dst, rebasing every index and offset.
-template <typename T> void merge_plan(BatchPlan<T> &dst, BatchPlan<T> &&src) {
-    const int32_t pass_off = static_cast<int32_t>(dst.passes.size());
-    const int32_t bundle_off = static_cast<int32_t>(dst.bundles.size());
-    const int32_t term_off = static_cast<int32_t>(dst.terms.size());
-    const int32_t slot_off = static_cast<int32_t>(dst.slot_cols.size());
-    dst.ops.resize((dst.ops.size() + 15) & ~size_t{15}, 0);
-    const size_t ops_off = dst.ops.size();
-    if (ops_off + src.ops.size() > static_cast<size_t>(INT32_MAX)) {
-        raise(PLK_ERR_UNSUPPORTED, "operation table exceeds 2 GiB");
+void merge_part(BatchPart &dst, BatchPart &&src) {
+    SweepTables &d = dst.t, &f = src.t;
+    const int pass0 = static_cast<int>(d.passes.size()), entry0 = static_cast<int>(d.entries.size());
+    const int term0 = static_cast<int>(d.terms.size()), gate0 = static_cast<int>(d.gates.size());
+    const int const0 = static_cast<int>(d.consts.size() / 8);
+    d.blob.resize((d.blob.size() + 255) & ~size_t{255}, 0);
+    const int64_t blob0 = static_cast<int64_t>(d.blob.size());
+    for (SweepPass p : f.passes) {
+        p.prog += blob0;
+        p.entry_first += entry0;
+        d.passes.push_back(p);
     }
-    for (auto b : src.bundles) {
-        b.first += static_cast<int32_t>(ops_off);
-        dst.bundles.push_back(b);
+    for (BatchRun r : f.runs) {
+        r.ins += blob0;
+        r.first += gate0;
+        r.entry += r.entry < 0 ? 0 : entry0;
+        d.runs.push_back(r);
     }
-    for (auto p : src.passes) {
-        p.bundle_first += bundle_off;
-        p.slot_first += slot_off;
-        dst.passes.push_back(p);
+    for (BatchGate g : f.gates) {
+        g.param += g.gate == BPG_CONST ? const0 : static_cast<int32_t>(dst.nparams);
+        d.gates.push_back(g);
     }
-    for (auto c : src.circuits) {
-        c.fwd_first += pass_off;
-        c.bwd_first += pass_off;
-        c.term_first += term_off;
-        c.jac_offset += dst.jac_len;
+    for (BatchPlanned c : src.circuits) {
+        c.fwd.first += pass0;
+        c.rev.first += pass0;
+        c.term_first += term0;
+        c.jac += dst.jac_len;
         dst.circuits.push_back(c);
     }
-    dst.ops.insert(dst.ops.end(), src.ops.begin(), src.ops.end());
-    dst.terms.insert(dst.terms.end(), src.terms.begin(), src.terms.end());
-    dst.slot_cols.insert(dst.slot_cols.end(), src.slot_cols.begin(), src.slot_cols.end());
-    dst.slot_coefs.insert(dst.slot_coefs.end(), src.slot_coefs.begin(), src.slot_coefs.end());
-    dst.cost.insert(dst.cost.end(), src.cost.begin(), src.cost.end());
-    for (auto p : src.patches) {
-        p.off += static_cast<int64_t>(ops_off);
-        p.param += static_cast<int32_t>(dst.nparams);
-        dst.patches.push_back(p);
-    }
+    d.blob.insert(d.blob.end(), f.blob.begin(), f.blob.end());
+    d.entries.insert(d.entries.end(), f.entries.begin(), f.entries.end());
+    d.terms.insert(d.terms.end(), f.terms.begin(), f.terms.end());
+    d.consts.insert(d.consts.end(), f.consts.begin(), f.consts.end());
     dst.jac_len += src.jac_len;
     dst.nparams += src.nparams;
 }
@@ -3095,78 +3124,62 @@ size_t plan_threads(size_t count) {
          (count + 31) / 32, size_t{64}});
 }
 
-void hash_obs(Hasher &H, const ObsNode &o) {
-    H.add(static_cast<uint64_t>(o.kind));
-    H.add(o.name);
-    H.add(static_cast<uint64_t>(o.wires.size()));
-    for (auto w : o.wires) {
-        H.add(static_cast<uint64_t>(w));
-    }
-    H.add(static_cast<uint64_t>(o.coeffs.size()));
-    for (double c : o.coeffs) {
-        H.add(c);
-    }
-    H.add(static_cast<uint64_t>(o.matrix.size()));
-    for (const cd &m : o.matrix) {
-        H.add(m.real());
-        H.add(m.imag());
-    }
-    H.add(static_cast<uint64_t>(o.terms.size()));
-    for (const auto &t : o.terms) {
-        hash_obs(H, *t);
-    }
-}
-
 // Everything a batch plan depends on except the angles of patched gates:
 // qubits, op names / wires / inverse flags, the values of every other
 // parameter and matrix, the trainable set and the observable.
 uint64_t circuit_key(const BatchInput &in) {
     Hasher H;
-    const OpsData &ops = *in.ops;
     H.add(static_cast<uint64_t>(in.n));
-    H.add(static_cast<uint64_t>(ops.names.size()));
-    for (size_t i = 0; i < ops.names.size(); i++) {
-        H.add(ops.names[i]);
-        H.add(static_cast<uint64_t>(ops.wires[i].size() | (ops.inverses[i] ? size_t{1} << 40 : 0)));
-        for (auto w : ops.wires[i]) {
-            H.add(static_cast<uint64_t>(w));
-        }
-        H.add(static_cast<uint64_t>(ops.params[i].size()));
-        if (patch_gate_of(ops, i) == BPG_NONE) {
-            for (double v : ops.params[i]) {
-                H.add(v);
-            }
-        }
-        H.add(static_cast<uint64_t>(ops.matrices[i].size()));
-        for (const cd &m : ops.matrices[i]) {
-            H.add(m.real());
-            H.add(m.imag());
-        }
-    }
+    H.add(in.ops->structure);
     H.add(static_cast<uint64_t>(in.tp.size()));
     for (auto t : in.tp) {
         H.add(static_cast<uint64_t>(t));
     }
-    hash_obs(H, *in.obs);
+    H.add(in.obs->key);
     return H.h;
 }
+
+// Circuits whose states fit the scratch together, run by one sequence of
+// launches: the whole circuits' jobs, then the staged ones' launches.
+struct BatchGroup {
+    struct Launch {
+        BatchStage stage;
+        size_t first;
+        int count; // blocks
+    };
+    struct Jobs {
+        size_t first;
+        int count, waves;
+    };
+    std::vector<Jobs> whole;
+    std::vector<Launch> staged;
+    size_t tail_first = 0;
+    int tail_count = 0;
+};
 
 // The last batch plan of one precision, resident on its device: tables,
 // patch list, parameter slots, scratch and result buffers in one allocation.
 // A call whose circuits have the same keys reuses it and uploads only the
 // parameters; any other call replaces it.
-template <typename T> struct BatchCache {
+struct BatchCache {
     bool valid = false;
     int device = -1;
-    int tile_bits = 0;
+    int whole_qubits = 0;
     std::vector<uint64_t> keys;
     std::vector<int64_t> param_base; // first global parameter of each circuit
-    int64_t nparams = 0;
-    int64_t npatches = 0;
+    std::vector<BatchGroup> groups;
+    int64_t nparams = 0, nruns = 0;
+    int64_t jac_len = 0;
     void *dbuf = nullptr;
-    void *ops = nullptr;
-    const BatchPatch *patches = nullptr;
+    unsigned char *blob = nullptr;
+    SweepEntry *entries = nullptr;
+    const BatchRun *runs = nullptr;
+    const BatchGate *gates = nullptr;
+    const double *consts = nullptr;
     double *params = nullptr;
+    const SweepJob *jobs = nullptr;
+    const BatchBlock *blocks = nullptr;
+    const BatchTail *tails = nullptr;
     BatchArgs A{};
 
     void release() {
@@ -3180,25 +3193,27 @@ template <typename T> struct BatchCache {
     hipStream_t device_stream() const { return ::plk::device(device).stream; }
 };
 
-template <typename T> BatchCache<T> &batch_cache() {
-    static BatchCache<T> c; // released with the process
-    return c;
+BatchCache &batch_cache(int dtype) {
+    static BatchCache c64, c128; // released with the process
+    return dtype == PLK_C64 ? c64 : c128;
 }
+
+// Amplitudes of scratch (phi and h of every circuit of a group).
+constexpr int64_t kBatchScratch = int64_t{1} << 29;
+// Blocks of a staged circuit's launches: a wave per tile up to 64.
+constexpr int kBatchBlocks = 64;
 
 // Plans every circuit and makes the result resident in C.
 // Every validation error is raised while planning, before any device call.
-template <typename T>
-void build_batch_cache(BatchCache<T> &C, int device_id, const std::vector<BatchInput> &in,
-                       int tile_bits) {
-    const int dtype = sizeof(T) == 4 ? PLK_C64 : PLK_C128;
+void build_batch_cache(BatchCache &C, int dtype, int device_id, const std::vector<BatchInput> &in) {
     const size_t nthreads = plan_threads(in.size());
     std::unique_ptr<HostScope> phase = std::make_unique<HostScope>("host_batch_plan");
-    std::vector<BatchPlan<T>> parts(nthreads);
+    std::vector<BatchPart> parts(nthreads);
     std::vector<std::pair<size_t, Error>> failures(nthreads, {SIZE_MAX, Error{PLK_OK, ""}});
     parallel_ranges(in.size(), nthreads, [&](size_t t, size_t lo, size_t hi) {
         for (size_t i = lo; i < hi; i++) {
             try {
-                plan_batch_circuit<T>(parts[t], in[i], tile_bits, low_bits(dtype));
+                plan_batch_circuit(parts[t], in[i], dtype);
             } catch (const Error &e) {
                 failures[t] = {i, e};
                 return;
@@ -3214,127 +3229,199 @@ void build_batch_cache(BatchCache<T> &C, int device_id, const std::vector<BatchI
         }
     }
     phase = std::make_unique<HostScope>("host_batch_merge");
-    BatchPlan<T> bp = std::move(parts[0]);
-    {
-        // One allocation per table instead of a regrowth per part.
-        size_t nc = 0, np = 0, nb = 0, no = 0, nt = 0, ns = 0, npt = 0;
-        for (const auto &pt : parts) {
-            nc += pt.circuits.size();
-            np += pt.passes.size();
-            nb += pt.bundles.size();
-            no += pt.ops.size() + 16;
-            nt += pt.terms.size();
-            ns += pt.slot_cols.size();
-            npt += pt.patches.size();
-        }
-        bp.circuits.reserve(nc);
-        bp.cost.reserve(nc);
-        bp.passes.reserve(np);
-        bp.bundles.reserve(nb);
-        bp.ops.reserve(no);
-        bp.terms.reserve(nt);
-        bp.slot_cols.reserve(ns);
-        bp.slot_coefs.reserve(ns);
-        bp.patches.reserve(npt);
-    }
+    BatchPart bp = std::move(parts[0]);
     for (size_t t = 1; t < parts.size(); t++) {
-        merge_plan(bp, std::move(parts[t]));
-        BatchPlan<T>().swap_into(parts[t]);
+        merge_part(bp, std::move(parts[t]));
+        parts[t] = BatchPart{};
     }
     phase = std::make_unique<HostScope>("host_batch_pack");
     Device &dev = device(device_id);
+    SweepTables &T = bp.t;
+    C.release();
+    C.device = dev.id;
+    C.groups.clear();
 
-    // Longest-processing-time-first packing of circuits onto workgroups.
-    const int per_cu = batch_resident_blocks(dtype, tile_bits);
-    const int grid = static_cast<int>(
-        std::min<size_t>(in.size(), static_cast<size_t>(dev.num_cus) * per_cu));
+    // Costliest circuits first, so that a launch ends together.
     std::vector<int32_t> by_cost(in.size());
     for (size_t i = 0; i < in.size(); i++) {
         by_cost[i] = static_cast<int32_t>(i);
     }
     std::stable_sort(by_cost.begin(), by_cost.end(),
-                     [&](int32_t a, int32_t b) { return bp.cost[a] > bp.cost[b]; });
-    using Load = std::pair<double, int>;
-    std::priority_queue<Load, std::vector<Load>, std::greater<Load>> heap;
-    for (int b = 0; b < grid; b++) {
-        heap.push({0.0, b});
-    }
-    std::vector<std::vector<int32_t>> lists(grid);
-    for (int32_t ci : by_cost) {
-        Load l = heap.top();
-        heap.pop();
-        lists[l.second].push_back(ci);
-        l.first += bp.cost[ci];
-        heap.push(l);
-    }
-    std::vector<int32_t> order, block_first{0};
-    std::vector<int64_t> block_scratch;
-    int64_t scratch_amps = 0;
-    for (int b = 0; b < grid; b++) {
-        int64_t need = 0;
-        for (int32_t ci : lists[b]) {
-            order.push_back(ci);
-            if (!bp.circuits[ci].resident) {
-                need = std::max<int64_t>(need, int64_t{2} << bp.circuits[ci].n);
+                     [&](int32_t a, int32_t b) { return bp.circuits[a].cost > bp.circuits[b].cost; });
+    std::vector<SweepJob> jobs;         // pointers are set once the buffer exists
+    std::vector<int32_t> job_circuit;
+    std::vector<std::pair<int64_t, int64_t>> job_state; // phi, h amplitudes
+    std::vector<BatchCircuit> staged;
+    std::vector<BatchBlock> blocks;
+    std::vector<BatchTail> tails;
+    int64_t amps_max = 0, parts_max = 0;
+    const int tile = sweep_reg_bits(dtype) + RT_LANE_BITS;
+    for (size_t at = 0; at < by_cost.size();) {
+        BatchGroup g;
+        int64_t amps = 0, psum = 0;
+        std::vector<int32_t> members;
+        while (at < by_cost.size()) {
+            const int64_t need = int64_t{2} << bp.circuits[by_cost[at]].n;
+            if (!members.empty() && amps + need > kBatchScratch) {
+                break;
+            }
+            members.push_back(by_cost[at++]);
+            amps += need;
+        }
+        amps_max = std::max(amps_max, amps);
+        amps = 0;
+        // Whole circuits, several tiles first; each launch has the waves of its widest.
+        for (const bool wide : {true, false}) {
+            BatchGroup::Jobs l{jobs.size(), 0, 1};
+            for (int32_t ci : members) {
+                const BatchPlanned &c = bp.circuits[ci];
+                if (c.staged || (c.n > tile) != wide) {
+                    continue;
+                }
+                SweepJob J{};
+                J.n = c.n;
+                std::tie(J.fwd_first, J.fwd_count) = c.fwd;
+                std::tie(J.rev_first, J.rev_count) = c.rev;
+                J.term_first = c.term_first;
+                J.term_count = c.term_count;
+                J.jac_len = static_cast<int32_t>(in[ci].tp.size());
+                jobs.push_back(J);
+                job_circuit.push_back(ci);
+                job_state.push_back({amps, amps + (int64_t{1} << c.n)});
+                amps += int64_t{2} << c.n;
+                l.count++;
+                l.waves = std::max(l.waves, sweep_waves(c.n, dtype));
+            }
+            if (l.count > 0) {
+                g.whole.push_back(l);
             }
         }
-        block_first.push_back(static_cast<int32_t>(order.size()));
-        block_scratch.push_back(scratch_amps);
-        scratch_amps += need;
+        // Staged circuits.
+        std::vector<int32_t> ids; // positions in `staged`
+        std::vector<const BatchPlanned *> who;
+        int nfwd = 0, nrev = 0;
+        g.tail_first = tails.size();
+        for (int32_t ci : members) {
+            const BatchPlanned &c = bp.circuits[ci];
+            if (!c.staged) {
+                continue;
+            }
+            BatchCircuit b{};
+            b.phi = amps;
+            b.h = amps + (int64_t{1} << c.n);
+            amps += int64_t{2} << c.n;
+            b.n = c.n;
+            b.blocks = std::min(kBatchBlocks, 1 << (c.n - tile));
+            b.term_first = c.term_first;
+            b.term_count = c.term_count;
+            b.eparts = psum;
+            psum += b.blocks;
+            tails.push_back({b.eparts, ci, -1, b.blocks});
+            for (int p = c.rev.first; p < c.rev.first + c.rev.second; p++) {
+                SweepPass &P = T.passes[p];
+                P.parts = psum;
+                psum += static_cast<int64_t>(P.nslots) * b.blocks;
+                for (int e = 0; e < P.entry_count; e++) {
+                    tails.push_back({P.parts, c.jac, P.entry_first + e, b.blocks});
+                }
+            }
+            nfwd = std::max(nfwd, c.fwd.second);
+            nrev = std::max(nrev, c.rev.second);
+            ids.push_back(static_cast<int32_t>(staged.size()));
+            who.push_back(&c);
+            staged.push_back(b);
+        }
+        auto launch = [&](BatchStage stage, int k) {
+            BatchGroup::Launch l{stage, blocks.size(), 0};
+            for (size_t q = 0; q < ids.size(); q++) {
+                const BatchPlanned &c = *who[q];
+                const std::pair<int, int> r = stage == BATCH_FORWARD ? c.fwd : c.rev;
+                if (stage != BATCH_OBSERVABLE && k >= r.second) {
+                    continue;
+                }
+                for (int x = 0; x < staged[ids[q]].blocks; x++) {
+                    blocks.push_back({ids[q], stage == BATCH_OBSERVABLE ? 0 : r.first + k, x,
+                                      stage == BATCH_FORWARD && k == 0 ? 1 : 0});
+                }
+            }
+            l.count = static_cast<int>(blocks.size() - l.first);
+            g.staged.push_back(l);
+        };
+        if (!ids.empty()) {
+            for (int k = 0; k < nfwd; k++) {
+                launch(BATCH_FORWARD, k);
+            }
+            launch(BATCH_OBSERVABLE, 0);
+            for (int k = 0; k < nrev; k++) {
+                launch(BATCH_REVERSE, k);
+            }
+        }
+        g.tail_count = static_cast<int>(tails.size() - g.tail_first);
+        parts_max = std::max(parts_max, psum);
+        C.groups.push_back(std::move(g));
     }
 
     Blob blob;
-    const size_t o_circ = blob.add(bp.circuits);
-    const size_t o_order = blob.add(order);
-    const size_t o_bfirst = blob.add(block_first);
-    const size_t o_bscr = blob.add(block_scratch);
-    const size_t o_pass = blob.add(bp.passes);
-    const size_t o_bund = blob.add(bp.bundles);
-    const size_t o_ops = blob.add(bp.ops);
-    const size_t o_terms = blob.add(bp.terms);
-    const size_t o_cols = blob.add(bp.slot_cols);
-    const size_t o_coefs = blob.add(bp.slot_coefs);
-    const size_t o_patch = blob.add(bp.patches);
+    const size_t o_jobs = blob.add(jobs); // rewritten below
+    const size_t o_pass = blob.add(T.passes);
+    const size_t o_ent = blob.add(T.entries);
+    const size_t o_terms = blob.add(T.terms);
+    const size_t o_runs = blob.add(T.runs);
+    const size_t o_gates = blob.add(T.gates);
+    const size_t o_consts = blob.add(T.consts);
+    const size_t o_staged = blob.add(staged);
+    const size_t o_blocks = blob.add(blocks);
+    const size_t o_tails = blob.add(tails);
+    const size_t o_prog = blob.add(T.blob);
     auto up = [](size_t x) { return (x + 255) & ~size_t{255}; };
-    const size_t amp = 2 * sizeof(T);
+    const size_t amp = dtype == PLK_C64 ? 8 : 16;
     const size_t o_params = up(blob.bytes.size());
     const size_t o_scratch = o_params + up(static_cast<size_t>(bp.nparams) * sizeof(double));
-    const size_t o_exp = o_scratch + up(static_cast<size_t>(scratch_amps) * amp);
+    const size_t o_parts = o_scratch + up(static_cast<size_t>(amps_max) * amp);
+    const size_t o_exp = o_parts + up(static_cast<size_t>(parts_max) * sizeof(double));
     const size_t o_jac = o_exp + up(in.size() * sizeof(double));
     const size_t total = o_jac + static_cast<size_t>(bp.jac_len) * sizeof(double) + 256;
 
     phase = std::make_unique<HostScope>("host_batch_upload");
-    C.release();
-    C.device = dev.id;
     C.dbuf = dev_malloc(dev.id, total, "batch plan");
     auto *w = static_cast<unsigned char *>(C.dbuf);
+    auto *d_jac = reinterpret_cast<double *>(w + o_jac);
+    auto *d_exp = reinterpret_cast<double *>(w + o_exp);
+    for (size_t j = 0; j < jobs.size(); j++) {
+        SweepJob &J = jobs[j];
+        J.phi = w + o_scratch + static_cast<size_t>(job_state[j].first) * amp;
+        J.h = w + o_scratch + static_cast<size_t>(job_state[j].second) * amp;
+        J.jac = d_jac + bp.circuits[job_circuit[j]].jac;
+        J.expval = d_exp + job_circuit[j];
+    }
+    if (!jobs.empty()) {
+        std::memcpy(blob.bytes.data() + o_jobs, jobs.data(), jobs.size() * sizeof(SweepJob));
+    }
     PLK_HIP(hipMemcpy(w, blob.bytes.data(), blob.bytes.size(), hipMemcpyHostToDevice));
     record_kernel("host_batch_table_bytes", 0.f, static_cast<double>(blob.bytes.size()));
 
     BatchArgs &A = C.A;
-    A = BatchArgs{};
-    A.circuits = reinterpret_cast<const BatchCircuit *>(w + o_circ);
-    A.order = reinterpret_cast<const int32_t *>(w + o_order);
-    A.block_first = reinterpret_cast<const int32_t *>(w + o_bfirst);
-    A.block_scratch = reinterpret_cast<const int64_t *>(w + o_bscr);
-    A.passes = reinterpret_cast<const BatchPass *>(w + o_pass);
-    A.bundles = reinterpret_cast<const TileBundle *>(w + o_bund);
-    A.ops = w + o_ops;
-    A.terms = reinterpret_cast<const BatchTerm *>(w + o_terms);
-    A.slot_cols = reinterpret_cast<const int32_t *>(w + o_cols);
-    A.slot_coefs = reinterpret_cast<const double *>(w + o_coefs);
+    A.circuits = reinterpret_cast<const BatchCircuit *>(w + o_staged);
+    A.passes = reinterpret_cast<const SweepPass *>(w + o_pass);
+    A.entries = reinterpret_cast<const SweepEntry *>(w + o_ent);
+    A.terms = reinterpret_cast<const SweepTerm *>(w + o_terms);
+    A.blob = w + o_prog;
     A.scratch = w + o_scratch;
-    A.expvals = reinterpret_cast<double *>(w + o_exp);
-    A.jac = reinterpret_cast<double *>(w + o_jac);
-    A.jac_len = bp.jac_len;
-    A.tile_bits = tile_bits;
-    A.grid = grid;
-    C.ops = w + o_ops;
-    C.patches = reinterpret_cast<const BatchPatch *>(w + o_patch);
-    C.npatches = static_cast<int64_t>(bp.patches.size());
+    A.parts = reinterpret_cast<double *>(w + o_parts);
+    A.expvals = d_exp;
+    A.jac = d_jac;
+    C.blob = w + o_prog;
+    C.entries = reinterpret_cast<SweepEntry *>(w + o_ent);
+    C.runs = reinterpret_cast<const BatchRun *>(w + o_runs);
+    C.nruns = static_cast<int64_t>(T.runs.size());
+    C.gates = reinterpret_cast<const BatchGate *>(w + o_gates);
+    C.consts = reinterpret_cast<const double *>(w + o_consts);
     C.params = reinterpret_cast<double *>(w + o_params);
+    C.jobs = reinterpret_cast<const SweepJob *>(w + o_jobs);
+    C.blocks = reinterpret_cast<const BatchBlock *>(w + o_blocks);
+    C.tails = reinterpret_cast<const BatchTail *>(w + o_tails);
     C.nparams = bp.nparams;
-    C.tile_bits = tile_bits;
+    C.jac_len = bp.jac_len;
     C.param_base.assign(in.size(), 0);
     int64_t base = 0;
     for (size_t i = 0; i < in.size(); i++) {
@@ -3344,56 +3431,63 @@ void build_batch_cache(BatchCache<T> &C, int device_id, const std::vector<BatchI
     C.valid = true;
 }
 
-template <typename T>
-void adjoint_batched_t(int device_id, const std::vector<BatchInput> &in, double *expvals,
-                       double *jac) {
-    const int dtype = sizeof(T) == 4 ? PLK_C64 : PLK_C128;
-    const int tile_bits = batch_tile_bits(dtype);
+void adjoint_batched_run(int dtype, int device_id, const std::vector<BatchInput> &in, double *expvals,
+                         double *jac) {
     if (in.empty()) {
         return;
     }
-    const size_t nthreads = plan_threads(in.size());
     std::unique_ptr<HostScope> phase = std::make_unique<HostScope>("host_batch_key");
     std::vector<uint64_t> keys(in.size());
-    parallel_ranges(in.size(), nthreads, [&](size_t, size_t lo, size_t hi) {
-        for (size_t i = lo; i < hi; i++) {
-            keys[i] = circuit_key(in[i]);
-        }
-    });
+    for (size_t i = 0; i < in.size(); i++) {
+        keys[i] = circuit_key(in[i]);
+    }
     phase.reset();
-    BatchCache<T> &C = batch_cache<T>();
-    if (!(C.valid && C.device == device_id && C.tile_bits == tile_bits && C.keys == keys)) {
+    BatchCache &C = batch_cache(dtype);
+    const int whole = batch_whole_qubits(dtype);
+    if (!(C.valid && C.device == device_id && C.whole_qubits == whole && C.keys == keys)) {
         C.valid = false;
-        build_batch_cache<T>(C, device_id, in, tile_bits);
+        build_batch_cache(C, dtype, device_id, in);
         C.keys = std::move(keys);
+        C.whole_qubits = whole;
     }
     Device &dev = device(device_id);
 
     // Angles of this call, in the plan's parameter order, then the patch
-    // kernel rewrites every patched U payload on the device.
+    // kernel rewrites every run with angles on the device.
     phase = std::make_unique<HostScope>("host_batch_params");
     std::vector<double> params(static_cast<size_t>(C.nparams));
-    parallel_ranges(in.size(), nthreads, [&](size_t, size_t lo, size_t hi) {
-        for (size_t c = lo; c < hi; c++) {
-            const OpsData &ops = *in[c].ops;
-            int64_t k = C.param_base[c];
-            for (size_t i = 0; i < ops.params.size(); i++) {
-                if (!ops.params[i].empty()) {
-                    params[static_cast<size_t>(k++)] = ops.params[i][0];
-                }
-            }
-        }
-    });
+    for (size_t c = 0; c < in.size(); c++) {
+        const std::vector<double> &a = in[c].ops->angles;
+        std::copy(a.begin(), a.end(), params.begin() + C.param_base[c]);
+    }
     PLK_HIP(hipMemcpyAsync(C.params, params.data(), params.size() * sizeof(double),
                            hipMemcpyHostToDevice, dev.stream));
     phase = std::make_unique<HostScope>("host_batch_launch");
-    launch_batch_patch(dev, dtype, C.ops, C.patches, C.npatches, C.params);
-    launch_batch(dev, dtype, C.A);
+    launch_batch_patch(dev, dtype, C.blob, C.entries, C.runs, C.nruns, C.gates, C.params, C.consts);
+    {
+        ProfScope prof("adjoint_batch", 0.0, dev.stream);
+        launch_fill_zero_doubles(dev, C.A.jac, static_cast<size_t>(C.jac_len));
+        for (const BatchGroup &g : C.groups) {
+            for (const auto &l : g.whole) {
+                SweepArgs S;
+                S.jobs = C.jobs + l.first;
+                S.passes = C.A.passes;
+                S.entries = C.A.entries;
+                S.terms = C.A.terms;
+                S.blob = C.A.blob;
+                launch_sweep(dev, dtype, S, l.count, l.waves);
+            }
+            for (const auto &l : g.staged) {
+                launch_batch_stage(dev, dtype, C.A, C.blocks + l.first, l.count, l.stage);
+            }
+            launch_batch_tails(dev, C.A, C.tails + g.tail_first, g.tail_count);
+        }
+    }
     phase = std::make_unique<HostScope>("host_batch_results");
     PLK_HIP(hipMemcpyAsync(expvals, C.A.expvals, in.size() * sizeof(double),
                            hipMemcpyDeviceToHost, dev.stream));
-    if (C.A.jac_len > 0) {
-        PLK_HIP(hipMemcpyAsync(jac, C.A.jac, static_cast<size_t>(C.A.jac_len) * sizeof(double),
+    if (C.jac_len > 0) {
+        PLK_HIP(hipMemcpyAsync(jac, C.A.jac, static_cast<size_t>(C.jac_len) * sizeof(double),
                                hipMemcpyDeviceToHost, dev.stream));
     }
     // Also keeps `params` alive until its upload has been read.
@@ -3812,6 +3906,7 @@ int plk_obs_named(const char *name, const size_t *wires, size_t num_wires, plk_o
         n->kind = ObsNode::Named;
         n->name = name ? name : "";
         n->wires = to_vec(wires, num_wires);
+        n->key = obs_key(*n);
         *out = new plk_obs{n};
     })
 }
@@ -3824,6 +3919,7 @@ int plk_obs_hermitian(const double *matrix, const size_t *wires, size_t num_wire
         n->wires = to_vec(wires, num_wires);
         const size_t dim = size_t{1} << num_wires;
         n->matrix = to_cvec(matrix, dim * dim);
+        n->key = obs_key(*n);
         *out = new plk_obs{n};
     })
 }
@@ -3842,6 +3938,7 @@ int plk_obs_tensor(const plk_obs *const *factors, size_t num_factors, plk_obs **
             }
             n->terms.push_back(factors[i]->node);
         }
+        n->key = obs_key(*n);
         *out = new plk_obs{n};
     })
 }
@@ -3856,6 +3953,7 @@ int plk_obs_hamiltonian(const double *coeffs, const plk_obs *const *terms, size_
             n->terms.push_back(terms[i]->node);
             n->coeffs.push_back(coeffs[i]);
         }
+        n->key = obs_key(*n);
         *out = new plk_obs{n};
     })
 }
@@ -3871,6 +3969,7 @@ int plk_obs_sparse(const double *data, const int64_t *indices, const int64_t *in
         n->indptr.assign(indptr, indptr + num_rows + 1);
         n->rows = num_rows;
         n->wires = to_vec(wires, num_wires);
+        n->key = obs_key(*n);
         *out = new plk_obs{n};
     })
 }
@@ -3890,6 +3989,7 @@ int plk_obs_sparse_i32(const double *data, const int32_t *indices, const int32_t
         n->indptr32.assign(indptr, indptr + num_rows + 1);
         n->rows = num_rows;
         n->wires = to_vec(wires, num_wires);
+        n->key = obs_key(*n);
         *out = new plk_obs{n};
     })
 }
@@ -3928,6 +4028,7 @@ int plk_ops_create(size_t num_ops, const char *const *names, const double *param
     PLK_TRY({
         auto h = std::make_unique<plk_ops>();
         OpsData &d = h->data;
+        Hasher H;
         for (size_t i = 0; i < num_ops; i++) {
             d.names.emplace_back(names[i]);
             d.params.emplace_back(params + param_offsets[i], params + param_offsets[i + 1]);
@@ -3936,6 +4037,7 @@ int plk_ops_create(size_t num_ops, const char *const *names, const double *param
             const size_t ml = matrix_offsets[i + 1] - matrix_offsets[i];
             d.matrices.push_back(ml ? to_cvec(matrices + 2 * matrix_offsets[i], ml)
                                     : std::vector<cd>{});
+            note_op(d, H, i);
         }
         *out = h.release();
     })
@@ -4018,11 +4120,7 @@ int plk_adjoint_batched(int dtype, int device_id, size_t num_circuits, const int
         if (num_circuits > 0 && !jac) {
             raise(PLK_ERR_INVALID, "null jac buffer");
         }
-        if (dtype == PLK_C64) {
-            adjoint_batched_t<float>(device_id, in, expvals, jac);
-        } else {
-            adjoint_batched_t<double>(device_id, in, expvals, jac);
-        }
+        adjoint_batched_run(dtype, device_id, in, expvals, jac);
     })
 }
 

@@ -28,34 +28,6 @@ namespace plk {
 
 namespace {
 
-// A table entry through the scalar cache (tables are written before the launch).
-template <typename S> __device__ __forceinline__ S load_uniform(const S *p) {
-    static_assert(sizeof(S) % 4 == 0, "whole words");
-    CT<uint32_t> *w = (CT<uint32_t> *)(p);
-    uint32_t buf[sizeof(S) / 4];
-#pragma unroll
-    for (size_t k = 0; k < sizeof(S) / 4; k++) {
-        buf[k] = w[k];
-    }
-    S out;
-    __builtin_memcpy(&out, buf, sizeof(S));
-    return out;
-}
-
-// Loads and stores of a state whose pointer comes from a table: a generic
-// pointer would make them flat instructions, which also count as LDS
-// operations, so that every operation on the tile would wait for the fetch of
-// the next instruction.
-template <typename T> __device__ __forceinline__ Cx<T> ldg(const Cx<T> *p, uint32_t i) {
-    typedef T V __attribute__((ext_vector_type(2)));
-    const V v = ((const __attribute__((address_space(1))) V *)(p))[i];
-    return {v.x, v.y};
-}
-template <typename T> __device__ __forceinline__ void stg(Cx<T> *p, uint32_t i, const Cx<T> &c) {
-    typedef T V __attribute__((ext_vector_type(2)));
-    ((__attribute__((address_space(1))) V *)(p))[i] = V{c.r, c.i};
-}
-
 // Per-wave LDS: the pass's sums for 16 quads and a dummy slot per lane.
 constexpr int kWaveSums = RT_SLOTS_MAX * 16 + 64;
 
@@ -148,16 +120,8 @@ __device__ __forceinline__ void observable(const SweepArgs &A, const SweepJob &J
     const uint32_t len = uint32_t{1} << J.n;
     double e = 0.0;
     for (uint32_t i = threadIdx.x; i < len; i += blockDim.x) {
-        double sr = 0.0, si = 0.0;
-        for (int k = 0; k < J.term_count; k++) {
-            const SweepTerm t = load_uniform(A.terms + J.term_first + k);
-            const Cx<T> p = ldg(phi, i ^ t.x);
-            const double sg = (__popc(i & t.zy) & 1) ? -1.0 : 1.0;
-            const double cr = sg * t.cr, ci = sg * t.ci;
-            const double pr = static_cast<double>(p.r), pi = static_cast<double>(p.i);
-            sr += cr * pr - ci * pi;
-            si += cr * pi + ci * pr;
-        }
+        double sr, si;
+        pauli_sum<T>(A.terms + J.term_first, J.term_count, phi, i, sr, si);
         const Cx<T> a = ldg(phi, i);
         e += static_cast<double>(a.r) * sr + static_cast<double>(a.i) * si;
         stg(h, i, Cx<T>{static_cast<T>(sr), static_cast<T>(si)});

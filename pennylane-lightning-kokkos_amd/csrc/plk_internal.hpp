@@ -389,6 +389,7 @@ struct SweepPass {
     int32_t T;    // tile bits (those from n up are idle when n < T)
     int32_t ninstr, nslots;
     int32_t entry_first, entry_count;
+    int64_t parts; // staged batches: first partial sum (rows of the circuit's blocks)
     int32_t tb[RT_TMAX];
     int32_t reg_in[RT_RMAX], lane_in[RT_LANE_BITS];
     int32_t reg_out[RT_RMAX], lane_out[RT_LANE_BITS];
@@ -455,84 +456,71 @@ template <typename T, int NJ>
 void rtile_launch_t(Device &dev, const State &phi, void *phi_out, void *const *h_ptrs, const void *d_prog,
                     const RtLaunch &L, int bpc, double *partials);
 
-// Batched circuits (kernels_batch.hip). One workgroup runs one circuit at a
-// time from |0...0>: forward passes, h = H phi and <H>, reverse passes with
-// the FP64 Im<h|G phi> of every trainable op. A pass is a set of T tile bits
-// and bundles of ops on <= 2 tile positions. States of n <= tile_bits qubits
-// stay in LDS (resident); larger ones live in a per-workgroup slice of a
-// global buffer and are streamed through LDS one 2^T-amplitude tile at a time.
-constexpr int BATCH_BLOCK = 256;
-constexpr int BATCH_PMAX = 64;  // trainable ops per pass
-constexpr int BATCH_TMAX = 12;  // tile bits
-constexpr int BATCH_NMAX = 20;  // qubits per circuit
+// Batched circuits (kernels_batch.hip): circuits of few tiles run whole, one
+// workgroup each (launch_sweep); the others pass by pass, all of a batch's
+// circuits in one launch per pass.
+constexpr int BATCH_NMAX = 20; // qubits per circuit
 
-enum BatchPassFlags { BP_INIT = 1, BP_NO_STORE = 2 };
-
-struct BatchPass {
-    int32_t T;                 // tile bits (== n for a resident circuit)
-    int32_t flags;             // BatchPassFlags
-    int32_t bundle_first, bundle_count;
-    int32_t nslots;            // trainable ops of the pass
-    int32_t slot_first;        // their Jacobian columns / coefficients
-    uint32_t tmask;            // mask of the tile bits
-    int32_t pad;
-    int32_t tb[BATCH_TMAX];    // ascending global bit of each tile position
-};
-
+// A staged circuit; offsets in amplitudes of the scratch and in partial sums.
 struct BatchCircuit {
+    int64_t phi, h;
+    int64_t eparts; // partial expectation values, one per block
     int32_t n;
-    int32_t resident;
-    int32_t fwd_first, fwd_count; // passes
-    int32_t bwd_first, bwd_count;
+    int32_t blocks; // blocks of each of its launches
     int32_t term_first, term_count;
-    int64_t jac_offset;           // first Jacobian entry of the circuit
-    int64_t pad;
 };
-
-struct BatchTerm {
-    uint64_t x, zy; // Pauli word: flipped bits, signed bits
-    double cr, ci;  // coefficient, including (-i)^{#Y}
+// A block of a staged launch.
+struct BatchBlock {
+    int32_t circuit;
+    int32_t pass;
+    int32_t block; // tiles block, block + blocks, ...
+    int32_t first; // the state is |0...0> and not in memory yet
 };
-
+// A result of a staged circuit: jac[out + col] of an entry, or (entry < 0)
+// the expectation value expvals[out].
+struct BatchTail {
+    int64_t parts;
+    int64_t out;
+    int32_t entry;
+    int32_t blocks;
+};
 struct BatchArgs {
     const BatchCircuit *circuits;
-    const int32_t *order;        // circuit indices, grouped by workgroup
-    const int32_t *block_first;  // grid + 1 offsets into order
-    const int64_t *block_scratch; // amplitude offset of each workgroup's slice
-    const BatchPass *passes;
-    const TileBundle *bundles;
-    const void *ops;             // packed op groups (OpHead)
-    const BatchTerm *terms;
-    const int32_t *slot_cols;
-    const double *slot_coefs;
-    void *scratch;               // Cx<T> amplitudes
+    const SweepPass *passes;
+    const SweepEntry *entries;
+    const SweepTerm *terms;
+    const unsigned char *blob;
+    void *scratch; // Cx<T> amplitudes
+    double *parts;
     double *expvals;
     double *jac;
-    int64_t jac_len;
-    int32_t tile_bits;
-    int32_t grid;
 };
+enum BatchStage { BATCH_FORWARD, BATCH_OBSERVABLE, BATCH_REVERSE };
+void launch_batch_stage(Device &dev, int dtype, const BatchArgs &A, const BatchBlock *blocks, int count,
+                        BatchStage stage);
+void launch_batch_tails(Device &dev, const BatchArgs &A, const BatchTail *tails, int count);
 
-// Parameter patch of a resident batch plan: the U payload of one packed op at
-// byte `off` of the op table is rewritten from params[param] (negated when
-// adj) by the gate's formula, in the payload layout its ukind implies
-// (RX dense, RY real, RZ and PhaseShift diagonal). Circuits whose structure
-// repeats between calls (a training loop) reuse the plan and upload only
-// their parameters.
-enum BatchPatchGate : int32_t { BPG_NONE = 0, BPG_RX = 1, BPG_RY = 2, BPG_RZ = 3, BPG_PHASE = 4 };
-struct BatchPatch {
-    int64_t off;
-    int32_t param;
+// Parameter patch of a resident batch plan. A fused run with angles is a list
+// of gates; its matrix (at byte `ins` of the blob, in the layout of ukind) and
+// the coefficients of its trainable gates' entries (from `entry` on) are
+// formed on the device from params. Circuits whose structure repeats between
+// calls (a training loop) reuse the plan and upload only their parameters.
+enum BatchPatchGate : int16_t { BPG_NONE = 0, BPG_RX = 1, BPG_RY = 2, BPG_RZ = 3, BPG_PHASE = 4, BPG_CONST = 5 };
+struct BatchGate {
     int16_t gate; // BatchPatchGate
     int16_t adj;
+    int32_t param; // BPG_CONST: index of its matrix
+    double coef;   // of its Jacobian entry; 0: not trainable
 };
-void launch_batch_patch(Device &dev, int dtype, void *ops, const BatchPatch *patches,
-                        int64_t count, const double *params);
-
-size_t batch_lds_bytes(int dtype, int tile_bits);
-// Workgroups of the batch kernel resident per CU at this tile width.
-int batch_resident_blocks(int dtype, int tile_bits);
-void launch_batch(Device &dev, int dtype, const BatchArgs &A);
+struct BatchRun {
+    int64_t ins;
+    int32_t first, count; // gates
+    int32_t entry;        // -1: none
+    int16_t ukind;
+    int16_t parts; // Pauli parts its sums hold: 7, or one of 1, 2, 4
+};
+void launch_batch_patch(Device &dev, int dtype, unsigned char *blob, SweepEntry *entries, const BatchRun *runs,
+                        int64_t count, const BatchGate *gates, const double *params, const double *consts);
 
 void launch_dense(Device &dev, const State &s, const CompiledOp &op);
 void launch_dense_matrix(Device &dev, const State &s,

@@ -710,6 +710,51 @@ template <typename T, int R> __device__ __forceinline__ uint64_t slot_off(const 
     return o;
 }
 
+// A table entry through the scalar cache (tables are written before the launch).
+template <typename S> __device__ __forceinline__ S load_uniform(const S *p) {
+    static_assert(sizeof(S) % 4 == 0, "whole words");
+    CT<uint32_t> *w = (CT<uint32_t> *)(p);
+    uint32_t buf[sizeof(S) / 4];
+#pragma unroll
+    for (size_t k = 0; k < sizeof(S) / 4; k++) {
+        buf[k] = w[k];
+    }
+    S out;
+    __builtin_memcpy(&out, buf, sizeof(S));
+    return out;
+}
+
+// Loads and stores of a state whose pointer comes from a table: a generic
+// pointer would make them flat instructions, which also count as LDS
+// operations, so that every operation on the tile would wait for the fetch of
+// the next instruction.
+template <typename T> __device__ __forceinline__ Cx<T> ldg(const Cx<T> *p, uint32_t i) {
+    typedef T V __attribute__((ext_vector_type(2)));
+    const V v = ((const __attribute__((address_space(1))) V *)(p))[i];
+    return {v.x, v.y};
+}
+template <typename T> __device__ __forceinline__ void stg(Cx<T> *p, uint32_t i, const Cx<T> &c) {
+    typedef T V __attribute__((ext_vector_type(2)));
+    ((__attribute__((address_space(1))) V *)(p))[i] = V{c.r, c.i};
+}
+
+// (H phi)_i of a sum of Pauli words.
+template <typename T>
+__device__ __forceinline__ void pauli_sum(const SweepTerm *terms, int count, const Cx<T> *phi, uint32_t i, double &sr,
+                                          double &si) {
+    sr = 0.0;
+    si = 0.0;
+    for (int k = 0; k < count; k++) {
+        const SweepTerm t = load_uniform(terms + k);
+        const Cx<T> p = ldg(phi, i ^ t.x);
+        const double sg = (__popc(i & t.zy) & 1) ? -1.0 : 1.0;
+        const double cr = sg * t.cr, ci = sg * t.ci;
+        const double pr = static_cast<double>(p.r), pi = static_cast<double>(p.i);
+        sr += cr * pr - ci * pi;
+        si += cr * pi + ci * pr;
+    }
+}
+
 // Runs a program on the tile: the next instruction is fetched while the
 // current one runs.
 template <typename T, int NS, int R>
