@@ -187,6 +187,197 @@ __global__ void __launch_bounds__(kBlock)
     }
 }
 
+// Expectation value of the groups whose X masks lie in a set of tile bits: a
+// block holds the 2^kTileBits amplitudes of a tile in LDS (64 KB, two blocks a
+// CU) and each thread its own share in registers, so every group's psi[i ^ x]
+// is an LDS read and the state is read once per set instead of once per two
+// groups. The lowest tile positions are the lowest index bits (whole 128-byte
+// lines), the highest are the thread's register index; a group visits half of
+// the indices (H is Hermitian) when a bit of its mask is a register or a wave
+// position.
+// Bound: the tile loads, 245 us a set (4.4 TB/s of 1 GiB) with few groups, and
+// with many the LDS reads and FP64 products after them. 26 qubits complex128, 64
+// words in 44 groups: five sets, 4.34 -> 1.55 ms (the gathers of the kernel above
+// read (1 + 44/2) S at 5.7 TB/s); complex64 4.14 -> 0.88 ms. Measured and not kept:
+// loading the next tile into registers first (no change in complex128, spills
+// and 1.15 ms in complex64), whole 256-byte lines (the same time per set).
+constexpr int kTileThreads = 512;
+constexpr int kTileThreadBits = 9;
+template <typename T> constexpr int tile_bits() { return sizeof(T) == 8 ? 12 : 13; }
+
+struct TileTerm {
+    uint64_t zy;  // sign mask outside the tile bits (for the tile's base index)
+    double c;     // coefficient (imaginary part when imag), doubled when half the indices are visited
+    uint32_t zl;  // sign mask in tile positions
+    int32_t imag;
+};
+// A group and its first term, in one scalar load.
+struct TileGroup {
+    TileTerm term;
+    uint32_t x;    // X mask in tile positions
+    int32_t half;  // wave position whose set half is skipped, -1: none
+    int32_t kinds; // 1: real coefficients, 2: imaginary ones
+    int32_t more;  // further terms, from terms[first] on
+    int32_t first;
+    int32_t pad[5];
+};
+static_assert(sizeof(TileGroup) == 64, "TileGroup layout");
+struct TileSet {
+    int32_t tb[13]; // global bit of each tile position
+    int32_t ngroups;
+    uint64_t mask;  // of the tile bits
+};
+
+// The real (IMAG: imaginary) terms of a group on the thread's NR amplitudes:
+// XR is the register part of its X mask. With XR != 0 only the r without XR's
+// top bit are visited.
+template <typename T, int NR, int XR, bool IMAG>
+__device__ __forceinline__ double tile_terms(const Cx<T> (&a)[NR], const Cx<T> *at, uint32_t tid, uint64_t base,
+                                             const TileGroup &g, const TileTerm *__restrict__ terms) {
+    constexpr int SKIP = XR == 0 ? 0 : 1 << (31 - __builtin_clz(XR | 1));
+    double p[NR]; // Re(conj(a) b), or Re(conj(a) i b)
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        p[r] = 0.0;
+        if (!(r & SKIP)) {
+            const Cx<T> b = ld(at, static_cast<uint64_t>((r ^ XR) * kTileThreads));
+            const double ar = a[r].r, ai = a[r].i, br = b.r, bi = b.i;
+            p[r] = IMAG ? fma(ai, br, -ar * bi) : fma(ar, br, ai * bi);
+        }
+    }
+    auto term = [&](const TileTerm &w) {
+        // sum over r of (-1)^popcount(r & zr) p[r], a bit of r at a time.
+        const uint32_t zr = w.zl >> kTileThreadBits;
+        double s[NR];
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            s[r] = p[r];
+        }
+#pragma unroll
+        for (int bit = 1; bit < NR; bit *= 2) {
+            if (bit == SKIP) {
+                continue;
+            }
+            const double sg = (zr & static_cast<uint32_t>(bit)) ? -1.0 : 1.0;
+#pragma unroll
+            for (int r = 0; r < NR; r++) {
+                if ((r & (2 * bit - 1)) == 0 && !(r & SKIP)) {
+                    s[r] = fma(sg, s[r | bit], s[r]);
+                }
+            }
+        }
+        const bool odd = ((__popc(tid & w.zl) + __popcll(base & w.zy)) & 1) != 0;
+        return (odd ? -w.c : w.c) * s[0];
+    };
+    double sum = 0.0;
+    if ((g.term.imag != 0) == IMAG) {
+        sum = term(g.term);
+    }
+    for (int k = 0; k < g.more; k++) {
+        const TileTerm w = terms[g.first + k];
+        if ((w.imag != 0) == IMAG) {
+            sum += term(w);
+        }
+    }
+    return sum;
+}
+
+template <typename T, int NR, int XR>
+__device__ __forceinline__ double tile_group(const Cx<T> (&a)[NR], const Cx<T> *tile, uint32_t tid, uint64_t base,
+                                             const TileGroup &g, const TileTerm *__restrict__ terms) {
+    const Cx<T> *at = tile + (tid ^ (g.x & (kTileThreads - 1)));
+    double sum = 0.0;
+    if (g.kinds & 1) {
+        sum = tile_terms<T, NR, XR, false>(a, at, tid, base, g, terms);
+    }
+    if (g.kinds & 2) {
+        sum += tile_terms<T, NR, XR, true>(a, at, tid, base, g, terms);
+    }
+    return sum;
+}
+
+template <typename T, int NR, int XR = 0>
+__device__ __forceinline__ double tile_dispatch(const Cx<T> (&a)[NR], const Cx<T> *tile, uint32_t tid, uint64_t base,
+                                                const TileGroup &g, const TileTerm *__restrict__ terms, int xr) {
+    if constexpr (XR + 1 < NR) {
+        if (xr != XR) {
+            return tile_dispatch<T, NR, XR + 1>(a, tile, tid, base, g, terms, xr);
+        }
+    }
+    return tile_group<T, NR, XR>(a, tile, tid, base, g, terms);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kTileThreads, 4)
+    pauli_tile_kernel(const Cx<T> *__restrict__ psi, int n, TileSet S, const TileGroup *__restrict__ groups,
+                      const TileTerm *__restrict__ terms, double *__restrict__ partials) {
+    constexpr int TB = tile_bits<T>();
+    constexpr int NR = 1 << (TB - kTileThreadBits);
+    extern __shared__ __align__(16) unsigned char tile_mem[];
+    Cx<T> *tile = reinterpret_cast<Cx<T> *>(tile_mem);
+    const uint32_t tid = threadIdx.x;
+    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(tid >> 6)));
+    uint64_t voff = 0;
+#pragma unroll
+    for (int q = 0; q < kTileThreadBits; q++) {
+        voff |= static_cast<uint64_t>((tid >> q) & 1) << S.tb[q];
+    }
+    uint64_t roff[NR];
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        roff[r] = 0;
+#pragma unroll
+        for (int q = 0; q < TB - kTileThreadBits; q++) {
+            roff[r] |= static_cast<uint64_t>((r >> q) & 1) << S.tb[kTileThreadBits + q];
+        }
+    }
+    double acc[1] = {0.0};
+    const uint64_t ntiles = uint64_t{1} << (n - TB);
+    for (uint64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        // The tile's index bits, lowest first, at the positions outside the set.
+        uint64_t base = t;
+        for (uint64_t m = S.mask; m;) {
+            const uint64_t low = m & (~m + 1);
+            base = ((base & ~(low - 1)) << 1) | (base & (low - 1));
+            m &= m - 1;
+        }
+        Cx<T> a[NR];
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            a[r] = ld(psi, base + voff + roff[r]);
+        }
+        __syncthreads(); // the last tile's reads are done
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            st(tile, tid + static_cast<uint32_t>(r) * kTileThreads, a[r]);
+        }
+        __syncthreads();
+        TileGroup next = groups[0];
+        for (int gi = 0; gi < S.ngroups; gi++) {
+            const TileGroup g = next;
+            next = groups[gi + 1 < S.ngroups ? gi + 1 : gi];
+            if (g.half >= 0 && ((wave >> (g.half - 6)) & 1)) {
+                continue;
+            }
+            acc[0] += tile_dispatch<T, NR>(a, tile, tid, base, g, terms, static_cast<int>(g.x >> kTileThreadBits));
+        }
+    }
+    __shared__ double red[kTileThreads / 64];
+    const double v = wave_sum(acc[0]);
+    if ((tid & 63) == 0) {
+        red[tid >> 6] = v;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        double sum = 0.0;
+#pragma unroll
+        for (int w = 0; w < kTileThreads / 64; w++) {
+            sum += red[w];
+        }
+        partials[blockIdx.x] = sum;
+    }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
     pauli_apply_kernel(Cx<T> *__restrict__ out, const Cx<T> *__restrict__ psi,
@@ -479,14 +670,6 @@ void inner_products(Device &dev, const State *const *xs, int nx, const State &y,
     }
 }
 
-PauliDevice::~PauliDevice() {
-    if (blob != nullptr) {
-        (void)hipSetDevice(device);
-        (void)hipStreamSynchronize(stream);
-        (void)hipFree(blob);
-    }
-}
-
 std::unique_ptr<PauliDevice> pauli_upload(Device &dev, const std::vector<PauliTerm> &terms) {
     auto t = std::make_unique<PauliDevice>();
     t->device = dev.id;
@@ -499,6 +682,7 @@ std::unique_ptr<PauliDevice> pauli_upload(Device &dev, const std::vector<PauliTe
     PLK_HIP(hipMemcpy(t->blob, b.bytes.data(), b.bytes.size(), hipMemcpyHostToDevice));
     t->toff = b.toff;
     t->ngroups = b.ngroups;
+    t->terms = terms;
     return t;
 }
 
@@ -516,11 +700,223 @@ PauliTables view_at(const void *blob, size_t toff, int ngroups) {
 
 PauliTables view_of(const PauliDevice &t) { return view_at(t.blob, t.toff, t.ngroups); }
 
+// The sets of a sum's tile plan (see pauli_tile_kernel): repeatedly grow a set
+// from the lowest index bits by the group that adds the fewest bits per
+// group it brings in, until no group fits. Empty when a group alone does not fit.
+struct TilePlan {
+    std::vector<TileSet> sets;
+    std::vector<size_t> first_group, first_term; // of each set
+    std::vector<TileGroup> groups;
+    std::vector<TileTerm> terms;
+};
+
+TilePlan plan_tiles(const std::vector<PauliTerm> &sorted, int n, int tbits, int low) {
+    TilePlan plan;
+    struct Range {
+        uint64_t x;
+        size_t first, count;
+    };
+    std::vector<Range> rem;
+    for (size_t k = 0; k < sorted.size(); k++) {
+        if (rem.empty() || rem.back().x != sorted[k].x) {
+            rem.push_back({sorted[k].x, k, 0});
+        }
+        rem.back().count++;
+    }
+    const uint64_t lows = (uint64_t{1} << low) - 1;
+    for (const Range &g : rem) {
+        if (__builtin_popcountll(g.x | lows) > tbits) {
+            return plan;
+        }
+    }
+    while (!rem.empty()) {
+        uint64_t B = lows;
+        for (;;) {
+            uint64_t best = 0;
+            double score = 0.0;
+            for (const Range &g : rem) {
+                const uint64_t N = B | g.x;
+                const int bits = __builtin_popcountll(N);
+                if (N == B || bits > tbits) {
+                    continue;
+                }
+                int brings = 0;
+                for (const Range &o : rem) {
+                    brings += (o.x | N) == N && (o.x | B) != B ? 1 : 0;
+                }
+                const double sc = static_cast<double>(brings) / (bits - __builtin_popcountll(B));
+                if (best == 0 || sc > score) {
+                    best = N;
+                    score = sc;
+                }
+            }
+            if (best == 0) {
+                break;
+            }
+            B = best;
+        }
+        for (int b = 0; __builtin_popcountll(B) < tbits; b++) {
+            B |= uint64_t{1} << b;
+        }
+        std::vector<Range> in, out;
+        for (const Range &g : rem) {
+            ((g.x | B) == B ? in : out).push_back(g);
+        }
+        // Positions: the low bits, then the others by how many masks hold them, the
+        // most frequent last (register positions).
+        std::vector<int> pos;
+        for (int b = 0; b < low; b++) {
+            pos.push_back(b);
+        }
+        std::vector<std::pair<int, int>> rest; // (masks, bit)
+        for (int b = low; b < n; b++) {
+            if (B >> b & 1) {
+                int c = 0;
+                for (const Range &g : in) {
+                    c += (g.x >> b) & 1;
+                }
+                rest.push_back({c, b});
+            }
+        }
+        std::sort(rest.begin(), rest.end());
+        for (const auto &r : rest) {
+            pos.push_back(r.second);
+        }
+        TileSet S{};
+        S.mask = B;
+        S.ngroups = static_cast<int32_t>(in.size());
+        for (int q = 0; q < tbits; q++) {
+            S.tb[q] = pos[q];
+        }
+        auto local = [&](uint64_t m) {
+            uint32_t l = 0;
+            for (int q = 0; q < tbits; q++) {
+                l |= static_cast<uint32_t>((m >> pos[q]) & 1) << q;
+            }
+            return l;
+        };
+        plan.sets.push_back(S);
+        plan.first_group.push_back(plan.groups.size());
+        plan.first_term.push_back(plan.terms.size());
+        for (const Range &g : in) {
+            TileGroup d{};
+            d.x = local(g.x);
+            // The highest position of the mask: a register or a wave position
+            // halves the indices visited; a lane position would only idle lanes.
+            const int top = d.x ? 31 - __builtin_clz(d.x) : -1;
+            const bool halved = top >= 6;
+            d.half = halved && top < kTileThreadBits ? top : -1;
+            d.first = static_cast<int32_t>(plan.terms.size() - plan.first_term.back());
+            d.more = static_cast<int32_t>(g.count) - 1;
+            for (size_t k = g.first; k < g.first + g.count; k++) {
+                const PauliTerm &t = sorted[k];
+                // A word's coefficient is real or imaginary (by its Y factors).
+                const bool imag = t.coeff.real() == 0.0 && t.coeff.imag() != 0.0;
+                const double c = imag ? t.coeff.imag() : t.coeff.real();
+                const TileTerm w{t.zy & ~B, halved ? 2.0 * c : c, local(t.zy), imag ? 1 : 0};
+                d.kinds |= imag ? 2 : 1;
+                if (k == g.first) {
+                    d.term = w;
+                } else {
+                    plan.terms.push_back(w);
+                }
+            }
+            plan.groups.push_back(d);
+        }
+        rem.swap(out);
+    }
+    return plan;
+}
+
+// Bytes of the device copy of a plan: groups, then terms.
+size_t tile_terms_off(const TilePlan &p) { return (p.groups.size() * sizeof(TileGroup) + 255) / 256 * 256; }
+
+template <typename T>
+double pauli_tile_expval(Device &dev, const State &s, const TilePlan &p, const void *blob) {
+    constexpr int TB = tile_bits<T>();
+    const uint64_t ntiles = uint64_t{1} << (s.n - TB);
+    const unsigned grid = static_cast<unsigned>(std::min<uint64_t>(ntiles, static_cast<uint64_t>(dev.num_cus) * 2));
+    const int total = static_cast<int>(grid * p.sets.size());
+    ensure_red(dev, static_cast<size_t>(total), 1);
+    const auto *b = static_cast<const unsigned char *>(blob);
+    const auto *groups = reinterpret_cast<const TileGroup *>(b);
+    const auto *terms = reinterpret_cast<const TileTerm *>(b + tile_terms_off(p));
+    const size_t lds = sizeof(Cx<T>) << TB;
+    static bool attr = false;
+    if (!attr) {
+        PLK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&pauli_tile_kernel<T>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+        attr = true;
+    }
+    {
+        ProfScope prof("pauli_expval", static_cast<double>(p.sets.size()) * s.bytes(), dev.stream);
+        for (size_t k = 0; k < p.sets.size(); k++) {
+            hipLaunchKernelGGL(pauli_tile_kernel<T>, dim3(grid), dim3(kTileThreads), lds, dev.stream,
+                               static_cast<const Cx<T> *>(s.d), s.n, p.sets[k], groups + p.first_group[k],
+                               terms + p.first_term[k], dev.red + k * grid);
+            PLK_HIP(hipGetLastError());
+        }
+    }
+    double out = 0.0;
+    finish_sums(dev, total, 1, &out);
+    return out;
+}
+
 } // namespace
+
+// Device copy of the tile plan of one precision.
+struct PauliTiles {
+    TilePlan plan;
+    void *blob = nullptr;
+};
+
+void *PauliDevice::tiles_blob(int k) const { return tiles[k] ? tiles[k]->blob : nullptr; }
+
+PauliDevice::~PauliDevice() {
+    void *const bufs[3] = {blob, tiles_blob(0), tiles_blob(1)};
+    for (void *b : bufs) {
+        if (b != nullptr) {
+            (void)hipSetDevice(device);
+            (void)hipStreamSynchronize(stream);
+            (void)hipFree(b);
+        }
+    }
+}
+
+const PauliTiles *PauliDevice::tiles_for(Device &dev, const State &s) const {
+    const int k = s.dtype == PLK_C64 ? 0 : 1;
+    const int tbits = k == 0 ? tile_bits<float>() : tile_bits<double>();
+    if (s.n < kPauliTileQubits + (k == 0 ? 1 : 0) || ngroups < kPauliTileGroups) {
+        return nullptr;
+    }
+    if (!tiles[k]) {
+        auto t = std::make_shared<PauliTiles>();
+        std::vector<PauliTerm> sorted = terms;
+        std::stable_sort(sorted.begin(), sorted.end(),
+                         [](const PauliTerm &a, const PauliTerm &b) { return a.x < b.x; });
+        t->plan = plan_tiles(sorted, s.n, tbits, k == 0 ? 4 : 3);
+        if (!t->plan.sets.empty()) {
+            std::vector<unsigned char> img(tile_terms_off(t->plan) + t->plan.terms.size() * sizeof(TileTerm));
+            std::memcpy(img.data(), t->plan.groups.data(), t->plan.groups.size() * sizeof(TileGroup));
+            std::memcpy(img.data() + tile_terms_off(t->plan), t->plan.terms.data(),
+                        t->plan.terms.size() * sizeof(TileTerm));
+            t->blob = dev_malloc(dev.id, img.size(), "Pauli tile tables");
+            PLK_HIP(hipMemcpy(t->blob, img.data(), img.size(), hipMemcpyHostToDevice));
+        }
+        tiles[k] = t;
+    }
+    // Worth it while the sets read less than the gathers do.
+    const size_t sets = tiles[k]->plan.sets.size();
+    return sets > 0 && 3 * sets <= static_cast<size_t>(ngroups) ? tiles[k].get() : nullptr;
+}
 
 double pauli_expval(Device &dev, const State &s, const PauliDevice &t) {
     if (t.ngroups == 0) {
         return 0.0;
+    }
+    if (const PauliTiles *tp = t.tiles_for(dev, s)) {
+        return s.dtype == PLK_C64 ? pauli_tile_expval<float>(dev, s, tp->plan, tp->blob)
+                                  : pauli_tile_expval<double>(dev, s, tp->plan, tp->blob);
     }
     const unsigned grid = grid_for(dev, s.len);
     ensure_red(dev, grid, 1);
