@@ -670,22 +670,6 @@ void inner_products(Device &dev, const State *const *xs, int nx, const State &y,
     }
 }
 
-std::unique_ptr<PauliDevice> pauli_upload(Device &dev, const std::vector<PauliTerm> &terms) {
-    auto t = std::make_unique<PauliDevice>();
-    t->device = dev.id;
-    t->stream = dev.stream;
-    if (terms.empty()) {
-        return t;
-    }
-    const PauliBlob b = pack_pauli(terms);
-    t->blob = dev_malloc(dev.id, b.bytes.size(), "Pauli tables");
-    PLK_HIP(hipMemcpy(t->blob, b.bytes.data(), b.bytes.size(), hipMemcpyHostToDevice));
-    t->toff = b.toff;
-    t->ngroups = b.ngroups;
-    t->terms = terms;
-    return t;
-}
-
 namespace {
 
 PauliTables view_at(const void *blob, size_t toff, int ngroups) {
@@ -867,20 +851,62 @@ double pauli_tile_expval(Device &dev, const State &s, const TilePlan &p, const v
 // Device copy of the tile plan of one precision.
 struct PauliTiles {
     TilePlan plan;
+    int device = -1;
     void *blob = nullptr;
-};
-
-void *PauliDevice::tiles_blob(int k) const { return tiles[k] ? tiles[k]->blob : nullptr; }
-
-PauliDevice::~PauliDevice() {
-    void *const bufs[3] = {blob, tiles_blob(0), tiles_blob(1)};
-    for (void *b : bufs) {
-        if (b != nullptr) {
-            (void)hipSetDevice(device);
-            (void)hipStreamSynchronize(stream);
-            (void)hipFree(b);
+    size_t bytes = 0;
+    ~PauliTiles() {
+        if (blob != nullptr) {
+            pool_give(device, bytes, blob);
         }
     }
+};
+
+namespace {
+
+// Pool buffers of tables come in powers of two, so that they fit the next
+// observable's.
+size_t table_bytes(size_t need) {
+    size_t b = 4096;
+    while (b < need) {
+        b *= 2;
+    }
+    return b;
+}
+
+// A table image in a pool buffer, written on the device's stream (the image
+// has been read when this returns).
+void *upload_table(Device &dev, const std::vector<unsigned char> &img, size_t &bytes, const char *what) {
+    bytes = table_bytes(img.size());
+    void *d = pool_take(dev.id, bytes, what);
+    const hipError_t e = hipMemcpyAsync(d, img.data(), img.size(), hipMemcpyHostToDevice, dev.stream);
+    const hipError_t w = e == hipSuccess ? hipStreamSynchronize(dev.stream) : e;
+    if (w != hipSuccess) {
+        pool_give(dev.id, bytes, d);
+        check_hip(w, "table upload");
+    }
+    return d;
+}
+
+} // namespace
+
+PauliDevice::~PauliDevice() {
+    if (blob != nullptr) {
+        pool_give(device, bytes, blob);
+    }
+}
+
+std::unique_ptr<PauliDevice> pauli_upload(Device &dev, const std::vector<PauliTerm> &terms) {
+    auto t = std::make_unique<PauliDevice>();
+    t->device = dev.id;
+    if (terms.empty()) {
+        return t;
+    }
+    const PauliBlob b = pack_pauli(terms);
+    t->blob = upload_table(dev, b.bytes, t->bytes, "Pauli tables");
+    t->toff = b.toff;
+    t->ngroups = b.ngroups;
+    t->terms = terms;
+    return t;
 }
 
 const PauliTiles *PauliDevice::tiles_for(Device &dev, const State &s) const {
@@ -900,8 +926,8 @@ const PauliTiles *PauliDevice::tiles_for(Device &dev, const State &s) const {
             std::memcpy(img.data(), t->plan.groups.data(), t->plan.groups.size() * sizeof(TileGroup));
             std::memcpy(img.data() + tile_terms_off(t->plan), t->plan.terms.data(),
                         t->plan.terms.size() * sizeof(TileTerm));
-            t->blob = dev_malloc(dev.id, img.size(), "Pauli tile tables");
-            PLK_HIP(hipMemcpy(t->blob, img.data(), img.size(), hipMemcpyHostToDevice));
+            t->device = dev.id;
+            t->blob = upload_table(dev, img, t->bytes, "Pauli tile tables");
         }
         tiles[k] = t;
     }

@@ -129,6 +129,12 @@ struct State {
     size_t bytes() const { return len * elem_bytes(); }
 };
 
+// Buffers of the device's recycling pool (see TmpPool): pool_take may hand out
+// one that queued work still reads, so it is written on the device's stream
+// only, and returned with the size it was taken with.
+void *pool_take(int device, size_t bytes, const char *what);
+void pool_give(int device, size_t bytes, void *d);
+
 // RAII temporary device state of the same shape.
 struct TmpState {
     State s;
@@ -563,16 +569,15 @@ constexpr int kPauliTileQubits = 20;
 constexpr int kPauliTileGroups = 4;
 struct PauliDevice {
     int device = -1;
-    hipStream_t stream = nullptr;
     void *blob = nullptr;
-    size_t toff = 0; // byte offset of the term table
+    size_t bytes = 0; // of blob, as taken from the pool
+    size_t toff = 0;  // byte offset of the term table
     int ngroups = 0;
     std::vector<PauliTerm> terms;
     // Tile plans of the expectation value per precision (complex64 first), made
     // on first use; entry points hold the engine lock.
     mutable std::shared_ptr<PauliTiles> tiles[2];
     const PauliTiles *tiles_for(Device &dev, const State &s) const;
-    void *tiles_blob(int k) const;
     PauliDevice() = default;
     PauliDevice(const PauliDevice &) = delete;
     PauliDevice &operator=(const PauliDevice &) = delete;

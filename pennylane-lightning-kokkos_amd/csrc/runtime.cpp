@@ -248,12 +248,14 @@ void record_kernel(const char *family, float ms, double bytes) {
     s.bytes += bytes;
 }
 
-// Temporary states are recycled per device instead of being freed: every
-// kernel of the library runs on the device's one stream, so a buffer handed
-// out again is written only after the work that last used it. The pool holds
-// at most kPoolMaxBytes per device; an allocation that fails releases it.
+// Temporary states and observables' tables are recycled per device instead of
+// being freed: every kernel of the library runs on the device's one stream,
+// so a buffer handed out again is written (on that stream) only after the work
+// that last used it. The pool holds at most kPoolMaxBytes per device; an
+// allocation that fails releases it.
 namespace {
 constexpr size_t kPoolMaxBytes = size_t{32} << 30;
+constexpr size_t kPoolMaxBuffers = 4096;
 
 struct TmpPool {
     std::multimap<size_t, void *> free;
@@ -297,43 +299,48 @@ void *dev_malloc(int device, size_t bytes, const char *what) {
     raise(PLK_ERR_OOM, "device allocation of " + std::to_string(bytes) + " bytes failed (" + what + ")");
 }
 
-TmpState::TmpState(int n, int dtype, int dev) {
-    s.n = n;
-    s.dtype = dtype;
-    s.len = size_t{1} << n;
-    s.device = dev;
-    const size_t bytes = s.bytes();
+void *pool_take(int dev, size_t bytes, const char *what) {
     {
         std::lock_guard<std::mutex> lock(g_pool_mutex);
         TmpPool &p = g_pools[dev];
         auto it = p.free.find(bytes);
         if (it != p.free.end()) {
-            s.d = it->second;
+            void *d = it->second;
             p.held -= bytes;
             p.free.erase(it);
-            return;
+            return d;
         }
     }
-    s.d = dev_malloc(dev, bytes, "temporary state");
+    return dev_malloc(dev, bytes, what);
 }
 
-TmpState::~TmpState() {
-    if (!s.d) {
-        return;
-    }
-    const size_t bytes = s.bytes();
+void pool_give(int dev, size_t bytes, void *d) {
     {
         std::lock_guard<std::mutex> lock(g_pool_mutex);
-        TmpPool &p = g_pools[s.device];
-        if (p.held + bytes <= kPoolMaxBytes) {
-            p.free.emplace(bytes, s.d);
+        TmpPool &p = g_pools[dev];
+        if (p.held + bytes <= kPoolMaxBytes && p.free.size() < kPoolMaxBuffers) {
+            p.free.emplace(bytes, d);
             p.held += bytes;
             return;
         }
     }
     // Kernels enqueued on this buffer must finish before it is released.
     (void)hipDeviceSynchronize();
-    (void)hipFree(s.d);
+    (void)hipFree(d);
+}
+
+TmpState::TmpState(int n, int dtype, int dev) {
+    s.n = n;
+    s.dtype = dtype;
+    s.len = size_t{1} << n;
+    s.device = dev;
+    s.d = pool_take(dev, s.bytes(), "temporary state");
+}
+
+TmpState::~TmpState() {
+    if (s.d) {
+        pool_give(s.device, s.bytes(), s.d);
+    }
 }
 
 } // namespace plk

@@ -143,6 +143,24 @@ def _dp(a: np.ndarray):
     return a.ctypes.data_as(_c_double_p)
 
 
+def _plain_wires(x) -> bool:
+    """A list or tuple of non-negative ints: needs no numpy to become a C array."""
+    if type(x) is not list and type(x) is not tuple:
+        return False
+    for w in x:
+        if type(w) is not int or w < 0:
+            return False
+    return True
+
+
+def _wire_array(x):
+    """(C array, length) of a wire list. Small observables are built by the
+    thousand, and a numpy round trip costs several times the C call."""
+    if not _plain_wires(x):
+        x = _sizes(x).tolist()
+    return (ctypes.c_size_t * max(1, len(x)))(*x), len(x)
+
+
 def _cplx_doubles(m) -> np.ndarray:
     return np.ascontiguousarray(np.asarray(m, dtype=np.complex128).reshape(-1)).view(np.float64)
 
@@ -322,9 +340,9 @@ class Obs:
 
     @staticmethod
     def named(name: str, wires: Sequence[int]) -> "Obs":
-        w = _sizes(wires)
+        w, nw = _wire_array(wires)
         h = _vp()
-        check(load().plk_obs_named(name.encode(), _sp(w), w.size, ctypes.byref(h)))
+        check(load().plk_obs_named(name.encode(), w, nw, ctypes.byref(h)))
         return Obs(h)
 
     @staticmethod
@@ -381,28 +399,35 @@ class Ops:
         matrices = matrices if matrices is not None else [[] for _ in range(n)]
         if not (len(params) == len(wires) == len(inverses) == len(matrices) == n):
             raise ValueError("operation lists must have equal lengths")
-        poff = np.zeros(n + 1, dtype=np.uint64)
-        woff = np.zeros(n + 1, dtype=np.uint64)
-        moff = np.zeros(n + 1, dtype=np.uint64)
-        for i in range(n):
-            poff[i + 1] = poff[i] + np.asarray(params[i]).size
-            woff[i + 1] = woff[i] + len(wires[i])
-            moff[i + 1] = moff[i] + np.asarray(matrices[i]).size
-        pflat = np.ascontiguousarray(np.concatenate(
-            [np.asarray(p, dtype=np.float64).reshape(-1) for p in params] + [np.zeros(1)]))
-        wflat = np.ascontiguousarray(np.concatenate(
-            [np.asarray(w, dtype=np.uint64).reshape(-1) for w in wires] + [np.zeros(1, np.uint64)]))
-        mflat = np.ascontiguousarray(np.concatenate(
-            [np.asarray(m, dtype=np.complex128).reshape(-1) for m in matrices]
-            + [np.zeros(1, np.complex128)])).view(np.float64)
+        # Flat lists, op by op; anything but plain lists of numbers goes
+        # through numpy for the conversions it does.
+        pflat, poff, wflat, woff, mflat, moff = [], [0], [], [0], [], [0]
+        for p, w, m in zip(params, wires, matrices):
+            if type(p) is not list or any(type(x) is not float for x in p):
+                p = np.asarray(p, dtype=np.float64).reshape(-1).tolist()
+            pflat += p
+            poff.append(len(pflat))
+            wflat += w if _plain_wires(w) else np.asarray(w, dtype=np.uint64).reshape(-1).tolist()
+            woff.append(len(wflat))
+            count = moff[-1]
+            if type(m) is not list or m:
+                a = np.asarray(m, dtype=np.complex128).reshape(-1)
+                if a.size:
+                    mflat.append(a)
+                    count += a.size
+            moff.append(count)
+        parr = (ctypes.c_double * (len(pflat) + 1))(*pflat)
+        warr = (ctypes.c_size_t * (len(wflat) + 1))(*wflat)
+        marr = np.ascontiguousarray(np.concatenate(mflat + [np.zeros(1, np.complex128)])).view(np.float64)
+        offsets = ctypes.c_size_t * (n + 1)
         cnames = (ctypes.c_char_p * max(1, n))(*[s.encode() for s in names])
-        inv = (ctypes.c_int * max(1, n))(*[int(bool(b)) for b in inverses])
+        inv = (ctypes.c_int * max(1, n))(*[1 if b else 0 for b in inverses])
         h = _vp()
-        check(load().plk_ops_create(n, cnames, _dp(pflat), _sp(poff), _sp(wflat), _sp(woff), inv,
-                                    _dp(mflat), _sp(moff), ctypes.byref(h)))
+        check(load().plk_ops_create(n, cnames, parr, offsets(*poff), warr, offsets(*woff), inv,
+                                    _dp(marr), offsets(*moff), ctypes.byref(h)))
         self.h = h
         self.names = list(names)
-        self._num_par = int(np.count_nonzero(np.diff(poff)))
+        self._num_par = sum(1 for a, b in zip(poff, poff[1:]) if b > a)
 
     def __del__(self):
         try:
