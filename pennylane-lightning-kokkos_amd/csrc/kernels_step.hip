@@ -151,6 +151,97 @@ __global__ void __launch_bounds__(kStepBlock)
     }
 }
 
+// step_dense_kernel for a two-state subspace (DoubleExcitation moves 2 of its 16
+// local states, SingleExcitation 2 of 4, CNOT-like gates 2). Such a step moves
+// so little that latency counts: the amplitudes of phi and of every observable
+// state are loaded before any is used, and the block sums take one barrier
+// (block_total takes two per observable). 20 qubits complex128, five
+// observables: 10.1 us a DoubleExcitation step (25 MB at 16 bytes of every 128-byte
+// line its low wires split, and the launch), 17.4 us a SingleExcitation step (100
+// MB, 5.8 TB/s), 4.2 and 6.1 us forward.
+template <typename T>
+__global__ void __launch_bounds__(kStepBlock)
+    step_pair_kernel(Cx<T> *__restrict__ phi, SegPtrs<T> hp, const double2 *__restrict__ mats, StepLaunch a,
+                     double *__restrict__ partials) {
+    const double2 u0 = mats[0], u1 = mats[1], u2 = mats[2], u3 = mats[3];
+    const double2 g0 = mats[4], g1 = mats[5], g2 = mats[6], g3 = mats[7];
+    const uint64_t o0 = a.off[0], o1 = a.off[1];
+    double acc[SEG_NJMAX];
+#pragma unroll
+    for (int j = 0; j < SEG_NJMAX; j++) {
+        acc[j] = 0.0;
+    }
+    auto store = [&](Cx<T> *p, uint64_t base, const Cx<T> &xa, const Cx<T> &xb) {
+        const double ar = xa.r, ai = xa.i, br = xb.r, bi = xb.i;
+        st(p, base + o0,
+           Cx<T>{static_cast<T>(fma(u1.x, br, fma(-u1.y, bi, fma(u0.x, ar, -u0.y * ai)))),
+                 static_cast<T>(fma(u1.x, bi, fma(u1.y, br, fma(u0.x, ai, u0.y * ar))))});
+        st(p, base + o1,
+           Cx<T>{static_cast<T>(fma(u3.x, br, fma(-u3.y, bi, fma(u2.x, ar, -u2.y * ai)))),
+                 static_cast<T>(fma(u3.x, bi, fma(u3.y, br, fma(u2.x, ai, u2.y * ar))))});
+    };
+    for (uint64_t g = uint64_t{blockIdx.x} * kStepBlock + threadIdx.x; g < a.groups;
+         g += uint64_t{gridDim.x} * kStepBlock) {
+        uint64_t base = g;
+#pragma unroll
+        for (int q = 0; q < STEP_MMAX; q++) {
+            if (q < a.m) {
+                base = insert_zero(base, a.bits[q]);
+            }
+        }
+        const Cx<T> fa = ld(phi, base + o0), fb = ld(phi, base + o1);
+        Cx<T> ha[SEG_NJMAX], hb[SEG_NJMAX];
+#pragma unroll
+        for (int j = 0; j < SEG_NJMAX; j++) {
+            if (j < a.nj) {
+                ha[j] = ld(hp.p[j], base + o0);
+                hb[j] = ld(hp.p[j], base + o1);
+            }
+        }
+        if (a.trainable) {
+            const double ar = fa.r, ai = fa.i, br = fb.r, bi = fb.i;
+            const double xr = fma(g1.x, br, fma(-g1.y, bi, fma(g0.x, ar, -g0.y * ai)));
+            const double xi = fma(g1.x, bi, fma(g1.y, br, fma(g0.x, ai, g0.y * ar)));
+            const double yr = fma(g3.x, br, fma(-g3.y, bi, fma(g2.x, ar, -g2.y * ai)));
+            const double yi = fma(g3.x, bi, fma(g3.y, br, fma(g2.x, ai, g2.y * ar)));
+#pragma unroll
+            for (int j = 0; j < SEG_NJMAX; j++) {
+                if (j < a.nj) {
+                    const double cr = ha[j].r, ci = ha[j].i, dr = hb[j].r, di = hb[j].i;
+                    acc[j] = fma(cr, xi, fma(-ci, xr, fma(dr, yi, fma(-di, yr, acc[j]))));
+                }
+            }
+        }
+        if (a.write_phi) {
+            store(phi, base, fa, fb);
+        }
+#pragma unroll
+        for (int j = 0; j < SEG_NJMAX; j++) {
+            if (j < a.nj) {
+                store(hp.p[j], base, ha[j], hb[j]);
+            }
+        }
+    }
+    if (!a.trainable) {
+        return;
+    }
+    __shared__ double red[SEG_NJMAX][kStepBlock / 64];
+#pragma unroll
+    for (int j = 0; j < SEG_NJMAX; j++) {
+        if (j < a.nj) {
+            const double v = wave_sum(acc[j]);
+            if ((threadIdx.x & 63) == 0) {
+                red[j][threadIdx.x >> 6] = v;
+            }
+        }
+    }
+    __syncthreads();
+    const int j = static_cast<int>(threadIdx.x);
+    if (j < a.nj) {
+        partials[static_cast<uint64_t>(j) * gridDim.x + blockIdx.x] = red[j][0] + red[j][1] + red[j][2] + red[j][3];
+    }
+}
+
 // Parity phases: U multiplies amplitude i by ue or uo by the parity of
 // i & umask; G multiplies it by +1 / -1 by the parity of i & gmask.
 template <typename T>
@@ -206,8 +297,8 @@ void launch_step_t(Device &dev, const State &phi, void *const *h_ptrs, const voi
                            hp, L, partials);
         break;
     case 2:
-        hipLaunchKernelGGL((step_dense_kernel<T, 2>), dim3(grid), dim3(kStepBlock), 0, dev.stream,
-                           p, hp, m, L, partials);
+        hipLaunchKernelGGL(step_pair_kernel<T>, dim3(grid), dim3(kStepBlock), 0, dev.stream, p, hp, m, L,
+                           partials);
         break;
     case 4:
         hipLaunchKernelGGL((step_dense_kernel<T, 4>), dim3(grid), dim3(kStepBlock), 0, dev.stream,
