@@ -3,18 +3,26 @@
 //
 // Marginal probabilities: output bin b collects |psi[i]|^2 over the indices i
 // whose bits at the measured positions spell b (first measured wire = most
-// significant bit of b). One block sums one bin over a contiguous range of
-// the complementary index space, walking it with the masked increment
-// x' = ((x | ~mask) + step) & mask so consecutive threads read consecutive
-// amplitudes whenever the low bits are unmeasured; a second kernel adds the
-// ranges of each bin in a fixed order. With few amplitudes per bin a thread
-// owns a bin instead.
+// significant bit of b). One block sums a contiguous range of the
+// complementary index space for the bins that differ in the lowest measured
+// bits only: those share cache lines, so a thread reads them together. The
+// range is walked with the masked increment x' = ((x | ~mask) + step) & mask, so
+// consecutive threads read consecutive amplitudes whenever the low bits are
+// unmeasured. A second kernel adds the ranges of each bin, a wave per bin, in
+// a fixed order. With few amplitudes per bin a thread owns a bin instead.
+// Bound: HBM reads. 25 qubits complex128, call to return: one wire 414 us with a
+// thread adding 4096 ranges of its bin, 120 us so; the lowest wire 536 us, 116
+// us; the six lowest wires 306 us with a block per bin, 134 us.
 //
-// Sampling: the exclusive FP64 CDF of the full distribution by a three-phase
-// scan (block totals, one-block scan of the totals, block-local scans), then
-// one thread per shot: a SplitMix64 uniform u in (0, 1] (Steele, Lea, Flood
-// 2014; output k of the generator seeded with `seed`) and the reference's
-// binary search for the bin with cdf[k] < u <= cdf[k+1].
+// Sampling: probabilities of 64-amplitude runs and of 4096-amplitude chunks in
+// one pass over the state, an exclusive scan of the chunks, then one wave per
+// shot: a SplitMix64 uniform u in (0, 1] (Steele, Lea, Flood 2014; output k of
+// the generator seeded with `seed`) and the bin with cdf[k] < u <= cdf[k+1] (the
+// reference's binary search, MeasuresFunctors.hpp:74-110), found by a 64-way
+// search of the chunk offsets, then of the chunk's runs, then of the run's
+// amplitudes. No CDF of the whole register is written or read again.
+// Bound: the HBM read of the state. 23 qubits complex128, 2000 shots, call to
+// return: 314 us with a scanned CDF, 73 us so; 25 qubits 1189 us and 157 us.
 #include "device_common.hpp"
 
 namespace plk {
@@ -22,19 +30,29 @@ namespace plk {
 namespace {
 
 constexpr int PB = 256;          // threads per block
-constexpr int MARG_R = 16;       // complement elements per thread
-constexpr int SCAN_R = 16;       // contiguous elements per thread in the scan
-constexpr int SCAN_CHUNK = PB * SCAN_R;
+constexpr int MARG_BLOCKS = 2048; // blocks a marginal aims for
+constexpr int RUN = 64;           // amplitudes of a run: one per lane
+constexpr int CHUNK = 64 * RUN;   // amplitudes of a chunk: a run per lane
 
 struct BinMap {
     int m;        // measured wires
     int g[64];    // global bit of measured wire k (k = 0 most significant)
+    int p[64];    // bin bit of measured wire k
 };
 
 __device__ __forceinline__ uint64_t bin_bits(const BinMap &bm, uint64_t b) {
     uint64_t v = 0;
     for (int k = 0; k < bm.m; k++) {
         v |= ((b >> (bm.m - 1 - k)) & 1ull) << bm.g[k];
+    }
+    return v;
+}
+
+// The bin bits of group b of the map's wires.
+__device__ __forceinline__ uint64_t bin_base(const BinMap &bm, uint64_t b) {
+    uint64_t v = 0;
+    for (int k = 0; k < bm.m; k++) {
+        v |= ((b >> (bm.m - 1 - k)) & 1ull) << bm.p[k];
     }
     return v;
 }
@@ -57,58 +75,78 @@ template <typename T> __device__ __forceinline__ double prob_of(const Cx<T> &a) 
     return r * r + i * i;
 }
 
-__device__ __forceinline__ double block_sum(double v, double *lds) {
-    v = wave_sum(v);
-    if ((threadIdx.x & 63) == 0) {
-        lds[threadIdx.x >> 6] = v;
-    }
-    __syncthreads();
-    double t = 0.0;
-    if (threadIdx.x == 0) {
-        for (int w = 0; w < PB / 64; w++) {
-            t += lds[w];
-        }
-    }
-    return t;
-}
-
-// One block per (bin, range of MARG_R * PB complement indices).
-template <typename T>
+// One block per (group of 2^K bins, range of `per` complement indices); the
+// bins of a group differ in the K lowest measured bits, at offsets off[].
+template <int K> struct LowBins {
+    uint64_t off[1 << K]; // index bits of the group's bins
+    uint32_t bin[1 << K]; // their bin bits
+};
+template <typename T, int K>
 __global__ void __launch_bounds__(PB)
-    marg_block_kernel(const Cx<T> *__restrict__ psi, BinMap bm, uint64_t cmask, uint64_t step,
-                      uint64_t count, uint64_t chunks, double *__restrict__ partial) {
-    __shared__ double lds[PB / 64];
+    marg_block_kernel(const Cx<T> *__restrict__ psi, BinMap high, LowBins<K> low, uint64_t cmask, uint64_t step,
+                      uint64_t per, uint64_t chunks, double *__restrict__ partial) {
+    constexpr int NB = 1 << K;
+    __shared__ double lds[NB][PB / 64];
     const uint64_t b = blockIdx.x / chunks;
     const uint64_t chunk = blockIdx.x % chunks;
-    const uint64_t base = bin_bits(bm, b);
-    const uint64_t c0 = chunk * (uint64_t{MARG_R} * PB) + threadIdx.x;
-    uint64_t x = pdep(c0, cmask);
-    double acc = 0.0;
-    for (int r = 0; r < MARG_R; r++) {
-        if (c0 + static_cast<uint64_t>(r) * PB >= count) {
-            break;
-        }
-        acc += prob_of(psi[base | x]);
-        x = ((x | ~cmask) + step) & cmask;
+    const uint64_t base = bin_bits(high, b);
+    uint64_t x = pdep(chunk * per + threadIdx.x, cmask);
+    double acc[NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+        acc[i] = 0.0;
     }
-    const double t = block_sum(acc, lds);
-    if (threadIdx.x == 0) {
-        partial[blockIdx.x] = t;
+    constexpr int U = K >= 3 ? 1 : 4 >> K; // loads in flight per thread
+    for (uint64_t r = threadIdx.x; r < per; r += uint64_t{U} * PB) {
+        Cx<T> a[U][NB];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const bool on = r + static_cast<uint64_t>(u) * PB < per;
+#pragma unroll
+            for (int i = 0; i < NB; i++) {
+                a[u][i] = on ? psi[base | x | low.off[i]] : Cx<T>{T(0), T(0)};
+            }
+            x = ((x | ~cmask) + step) & cmask;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+#pragma unroll
+            for (int i = 0; i < NB; i++) {
+                acc[i] += prob_of(a[u][i]);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+        const double v = wave_sum(acc[i]);
+        if ((threadIdx.x & 63) == 0) {
+            lds[i][threadIdx.x >> 6] = v;
+        }
+    }
+    __syncthreads();
+    const int i = static_cast<int>(threadIdx.x);
+    if (i < NB) {
+        partial[(bin_base(high, b) | low.bin[i]) * chunks + chunk] = lds[i][0] + lds[i][1] + lds[i][2] + lds[i][3];
     }
 }
 
+// One wave per bin.
 __global__ void __launch_bounds__(PB)
     marg_finish_kernel(const double *__restrict__ partial, uint64_t bins, uint64_t chunks,
                        double *__restrict__ out) {
-    const uint64_t b = uint64_t{blockIdx.x} * PB + threadIdx.x;
+    const uint64_t b = uint64_t{blockIdx.x} * (PB / 64) + (threadIdx.x >> 6);
     if (b >= bins) {
         return;
     }
     double s = 0.0;
-    for (uint64_t c = 0; c < chunks; c++) {
+#pragma unroll 8
+    for (uint64_t c = threadIdx.x & 63; c < chunks; c += 64) {
         s += partial[b * chunks + c];
     }
-    out[b] = s;
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) {
+        out[b] = s;
+    }
 }
 
 // One thread per bin (few amplitudes per bin).
@@ -130,85 +168,76 @@ __global__ void __launch_bounds__(PB)
     out[b] = s;
 }
 
-// Phase 1 of the CDF: total probability of each SCAN_CHUNK-element block.
+// Probability of every run and chunk: a block per chunk, a wave per 16 runs.
 template <typename T>
 __global__ void __launch_bounds__(PB)
-    scan_totals_kernel(const Cx<T> *__restrict__ psi, uint64_t len, double *__restrict__ totals) {
-    __shared__ double lds[PB / 64];
-    const uint64_t first = uint64_t{blockIdx.x} * SCAN_CHUNK + uint64_t{threadIdx.x} * SCAN_R;
-    double s = 0.0;
-    for (int r = 0; r < SCAN_R; r++) {
-        if (first + r < len) {
-            s += prob_of(psi[first + r]);
-        }
+    run_totals_kernel(const Cx<T> *__restrict__ psi, uint64_t len, double *__restrict__ runs,
+                      double *__restrict__ chunks) {
+    constexpr int PER = CHUNK / PB; // runs of a wave
+    __shared__ double lds[64];
+    const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
+    const uint64_t first = uint64_t{blockIdx.x} * CHUNK + static_cast<uint64_t>(wave * PER * RUN + lane);
+    Cx<T> a[PER];
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const uint64_t i = first + static_cast<uint64_t>(r) * RUN;
+        a[r] = i < len ? psi[i] : Cx<T>{T(0), T(0)};
     }
-    const double t = block_sum(s, lds);
-    if (threadIdx.x == 0) {
-        totals[blockIdx.x] = t;
+    double mine = 0.0; // lane r keeps run r
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const double t = wave_sum(prob_of(a[r])); // DPP; halving exchanges through LDS take longer
+        mine = lane == r ? t : mine;
+    }
+    if (lane < PER) {
+        lds[wave * PER + lane] = mine;
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const double t = lds[threadIdx.x];
+        runs[uint64_t{blockIdx.x} * 64 + threadIdx.x] = t;
+        const double s = wave_sum(t);
+        if (threadIdx.x == 0) {
+            chunks[blockIdx.x] = s;
+        }
     }
 }
 
-// Phase 2: exclusive scan of the block totals by one block.
-__global__ void __launch_bounds__(PB) scan_top_kernel(double *__restrict__ totals, uint64_t nb) {
-    __shared__ double seg[PB];
-    const uint64_t per = (nb + PB - 1) / PB;
-    const uint64_t lo = threadIdx.x * per;
-    const uint64_t hi = lo + per < nb ? lo + per : nb;
-    double s = 0.0;
-    for (uint64_t i = lo; i < hi; i++) {
-        s += totals[i];
+// Inclusive prefix sum over the wave.
+__device__ __forceinline__ double wave_scan(double v, int lane) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const double o = __shfl_up(v, off, 64);
+        v = lane >= off ? v + o : v;
     }
-    seg[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double run = 0.0;
-        for (int t = 0; t < PB; t++) {
-            const double v = seg[t];
-            seg[t] = run;
-            run += v;
-        }
-    }
-    __syncthreads();
-    double run = seg[threadIdx.x];
-    for (uint64_t i = lo; i < hi; i++) {
-        const double v = totals[i];
-        totals[i] = run;
-        run += v;
-    }
+    return v;
 }
 
-// Phase 3: cdf[k] = sum_{i<k} |psi_i|^2.
-template <typename T>
-__global__ void __launch_bounds__(PB)
-    scan_final_kernel(const Cx<T> *__restrict__ psi, uint64_t len,
-                      const double *__restrict__ offsets, double *__restrict__ cdf) {
-    __shared__ double seg[PB];
-    const uint64_t first = uint64_t{blockIdx.x} * SCAN_CHUNK + uint64_t{threadIdx.x} * SCAN_R;
-    double p[SCAN_R];
-    double s = 0.0;
-#pragma unroll
-    for (int r = 0; r < SCAN_R; r++) {
-        p[r] = first + r < len ? prob_of(psi[first + r]) : 0.0;
-        s += p[r];
-    }
-    seg[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double run = offsets[blockIdx.x];
-        for (int t = 0; t < PB; t++) {
-            const double v = seg[t];
-            seg[t] = run;
-            run += v;
+// In-place exclusive scan of the chunk totals by one block, SCAN at a time.
+constexpr int SCAN = 1024;
+__global__ void __launch_bounds__(SCAN) scan_top_kernel(double *__restrict__ totals, uint64_t nb) {
+    __shared__ double part[SCAN / 64];
+    const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
+    double carry = 0.0;
+    for (uint64_t at = 0; at < nb; at += SCAN) {
+        const uint64_t i = at + threadIdx.x;
+        const double v = i < nb ? totals[i] : 0.0;
+        const double inc = wave_scan(v, lane);
+        if (lane == 63) {
+            part[wave] = inc;
         }
-    }
-    __syncthreads();
-    double run = seg[threadIdx.x];
-#pragma unroll
-    for (int r = 0; r < SCAN_R; r++) {
-        if (first + r < len) {
-            cdf[first + r] = run;
+        __syncthreads();
+        double before = carry, all = carry;
+        for (int w = 0; w < SCAN / 64; w++) {
+            before += w < wave ? part[w] : 0.0;
+            all += part[w];
         }
-        run += p[r];
+        const double exc = __shfl_up(inc, 1, 64);
+        if (i < nb) {
+            totals[i] = before + (lane == 0 ? 0.0 : exc);
+        }
+        carry = all;
+        __syncthreads();
     }
 }
 
@@ -218,36 +247,87 @@ __device__ __forceinline__ uint64_t splitmix64(uint64_t z) {
     return z ^ (z >> 31);
 }
 
-// MeasuresFunctors.hpp:74-110: bin of u in the exclusive CDF, bits of the
-// bin written most significant (wire 0) first.
+// The last lane whose value lies below u (lane 0's always does).
+__device__ __forceinline__ int last_below(double v, double u) {
+    const uint64_t m = __ballot(v < u);
+    return m == 0 ? 0 : 63 - __clzll(static_cast<long long>(m));
+}
+
+// One wave per shot: the last k with cdf[k] < u; bits of the bin written most
+// significant (wire 0) first.
+template <typename T>
 __global__ void __launch_bounds__(PB)
-    sample_kernel(const double *__restrict__ cdf, uint64_t len, int n, uint64_t shots,
-                  uint64_t seed, uint64_t *__restrict__ out) {
-    const uint64_t s = uint64_t{blockIdx.x} * PB + threadIdx.x;
+    sample_kernel(const Cx<T> *__restrict__ psi, uint64_t len, const double *__restrict__ runs,
+                  const double *__restrict__ chunks, uint64_t nb, int n, uint64_t shots, uint64_t seed,
+                  uint64_t *__restrict__ out) {
+    const uint64_t s = uint64_t{blockIdx.x} * (PB / 64) + (threadIdx.x >> 6);
     if (s >= shots) {
         return;
     }
+    const int lane = static_cast<int>(threadIdx.x) & 63;
     const uint64_t z = splitmix64(seed + (s + 1) * 0x9E3779B97F4A7C15ull);
     const double u = static_cast<double>((z >> 11) + 1) * 0x1.0p-53;
-    uint64_t index;
-    if (u <= cdf[1]) {
-        index = 0;
-    } else {
-        uint64_t low = 1, high = len;
-        while (high - low > 1) {
-            const uint64_t mid = high - ((high - low) >> 1);
-            const double c = mid == len ? 1.0 : cdf[mid];
-            if (c < u) {
-                low = mid;
-            } else {
-                high = mid;
+    // Chunk: the last whose offset lies below u, 64 candidates at a time.
+    uint64_t lo = 0, count = nb;
+    while (count > 1) {
+        const uint64_t step = (count + 63) / 64;
+        const uint64_t at = static_cast<uint64_t>(lane) * step;
+        const double v = at < count ? chunks[lo + at] : 2.0;
+        const uint64_t k = static_cast<uint64_t>(last_below(v, u)) * step;
+        lo += k;
+        count = count - k < step ? count - k : step;
+    }
+    double below = chunks[lo];
+    // Run of the chunk, then amplitude of the run.
+    double t = runs[lo * 64 + static_cast<uint64_t>(lane)];
+    double exc = __shfl_up(wave_scan(t, lane), 1, 64);
+    exc = lane == 0 ? below : below + exc;
+    const uint64_t first_run = lo * CHUNK + static_cast<uint64_t>(lane) * RUN;
+    const int run = last_below(first_run < len ? exc : 2.0, u);
+    below = __shfl(exc, run, 64);
+    const uint64_t i = lo * CHUNK + static_cast<uint64_t>(run * RUN + lane);
+    t = i < len ? prob_of(psi[i]) : 0.0;
+    exc = __shfl_up(wave_scan(t, lane), 1, 64);
+    exc = lane == 0 ? below : below + exc;
+    const uint64_t index = lo * CHUNK + static_cast<uint64_t>(run * RUN + last_below(i < len ? exc : 2.0, u));
+    for (int j = lane; j < n; j += 64) {
+        out[s * static_cast<uint64_t>(n) + static_cast<uint64_t>(j)] = (index >> (n - 1 - j)) & 1ull;
+    }
+}
+
+template <typename T, int K>
+void launch_marg(Device &dev, const Cx<T> *psi, const BinMap &bm, uint64_t cmask, uint64_t step, uint64_t per,
+                 uint64_t chunks, double *partial) {
+    BinMap high{};
+    LowBins<K> low{};
+    // The K measured wires on the lowest bits leave the map.
+    std::vector<int> order;
+    for (int k = 0; k < bm.m; k++) {
+        order.push_back(k);
+    }
+    std::sort(order.begin(), order.end(), [&](int a, int b) { return bm.g[a] < bm.g[b]; });
+    for (int i = 0; i < (1 << K); i++) {
+        for (int q = 0; q < K; q++) {
+            if ((i >> q) & 1) {
+                low.off[i] |= uint64_t{1} << bm.g[order[q]];
+                low.bin[i] |= uint32_t{1} << (bm.m - 1 - order[q]);
             }
         }
-        index = high - 1;
     }
-    for (int j = 0; j < n; j++) {
-        out[s * n + (n - 1 - j)] = (index >> j) & 1ull;
+    for (int k = 0; k < bm.m; k++) {
+        if (std::find(order.begin(), order.begin() + K, k) == order.begin() + K) {
+            high.g[high.m] = bm.g[k];
+            high.p[high.m] = bm.m - 1 - k;
+            high.m++;
+        }
     }
+    const uint64_t grid = (uint64_t{1} << high.m) * chunks;
+    if (grid > (uint64_t{1} << 31)) {
+        raise(PLK_ERR_UNSUPPORTED, "probability grid too large");
+    }
+    hipLaunchKernelGGL((marg_block_kernel<T, K>), dim3(static_cast<unsigned>(grid)), dim3(PB), 0, dev.stream, psi,
+                       high, low, cmask, step, per, chunks, partial);
+    PLK_HIP(hipGetLastError());
 }
 
 template <typename T>
@@ -275,11 +355,20 @@ void probs_t(Device &dev, const State &s, const std::vector<int> &gbits, double 
         PLK_HIP(hipMemcpyAsync(host_out, out, bins * sizeof(double), hipMemcpyDeviceToHost,
                                dev.stream));
     } else {
-        const uint64_t per_block = uint64_t{MARG_R} * PB;
-        const uint64_t chunks = (count + per_block - 1) / per_block;
-        if (bins * chunks > (uint64_t{1} << 31)) {
-            raise(PLK_ERR_UNSUPPORTED, "probability grid too large");
+        // Measured bits inside a 128-byte line: their bins are summed together.
+        const int line = sizeof(T) == 8 ? 3 : 4;
+        int K = 0;
+        for (int k = 0; k < m; k++) {
+            K += gbits[k] < line ? 1 : 0;
         }
+        K = std::min(K, 3);
+        // A power of two of ranges per bin: enough blocks to fill the device, of at
+        // least 1024 amplitudes a bin.
+        uint64_t chunks = 1;
+        while ((bins >> K) * chunks < MARG_BLOCKS && count / (2 * chunks) >= 1024) {
+            chunks *= 2;
+        }
+        const uint64_t per = count / chunks;
         double *partial = static_cast<double *>(
             ensure_work(dev, (bins * chunks + bins) * sizeof(double)));
         double *out = partial + bins * chunks;
@@ -295,10 +384,13 @@ void probs_t(Device &dev, const State &s, const std::vector<int> &gbits, double 
             }
             return v;
         }();
-        hipLaunchKernelGGL((marg_block_kernel<T>), dim3(static_cast<unsigned>(bins * chunks)),
-                           dim3(PB), 0, dev.stream, psi, bm, cmask, step, count, chunks, partial);
-        PLK_HIP(hipGetLastError());
-        hipLaunchKernelGGL(marg_finish_kernel, dim3(static_cast<unsigned>((bins + PB - 1) / PB)),
+        switch (K) {
+        case 0: launch_marg<T, 0>(dev, psi, bm, cmask, step, per, chunks, partial); break;
+        case 1: launch_marg<T, 1>(dev, psi, bm, cmask, step, per, chunks, partial); break;
+        case 2: launch_marg<T, 2>(dev, psi, bm, cmask, step, per, chunks, partial); break;
+        default: launch_marg<T, 3>(dev, psi, bm, cmask, step, per, chunks, partial); break;
+        }
+        hipLaunchKernelGGL(marg_finish_kernel, dim3(static_cast<unsigned>((bins + PB / 64 - 1) / (PB / 64))),
                            dim3(PB), 0, dev.stream, partial, bins, chunks, out);
         PLK_HIP(hipGetLastError());
         PLK_HIP(hipMemcpyAsync(host_out, out, bins * sizeof(double), hipMemcpyDeviceToHost,
@@ -310,30 +402,25 @@ void probs_t(Device &dev, const State &s, const std::vector<int> &gbits, double 
 template <typename T>
 void sample_t(Device &dev, const State &s, size_t shots, uint64_t seed, size_t *host_out) {
     const uint64_t len = s.len;
-    const uint64_t nb = (len + SCAN_CHUNK - 1) / SCAN_CHUNK;
-    const size_t cdf_bytes = len * sizeof(double);
+    const uint64_t nb = (len + CHUNK - 1) / CHUNK;
+    const size_t run_bytes = nb * 64 * sizeof(double);
     const size_t tot_bytes = ((nb * sizeof(double)) + 255) & ~size_t{255};
     const size_t out_bytes = static_cast<size_t>(shots) * s.n * sizeof(uint64_t);
-    unsigned char *w = static_cast<unsigned char *>(
-        ensure_work(dev, ((cdf_bytes + 255) & ~size_t{255}) + tot_bytes + out_bytes));
-    double *cdf = reinterpret_cast<double *>(w);
-    double *totals = reinterpret_cast<double *>(w + ((cdf_bytes + 255) & ~size_t{255}));
-    uint64_t *out = reinterpret_cast<uint64_t *>(reinterpret_cast<unsigned char *>(totals) +
-                                                 tot_bytes);
+    unsigned char *w = static_cast<unsigned char *>(ensure_work(dev, run_bytes + tot_bytes + out_bytes));
+    double *runs = reinterpret_cast<double *>(w);
+    double *totals = reinterpret_cast<double *>(w + run_bytes);
+    uint64_t *out = reinterpret_cast<uint64_t *>(w + run_bytes + tot_bytes);
     const auto *psi = static_cast<const Cx<T> *>(s.d);
-    ProfScope prof("sample", 3.0 * static_cast<double>(s.bytes()), dev.stream);
-    hipLaunchKernelGGL((scan_totals_kernel<T>), dim3(static_cast<unsigned>(nb)), dim3(PB), 0,
-                       dev.stream, psi, len, totals);
-    PLK_HIP(hipGetLastError());
-    hipLaunchKernelGGL(scan_top_kernel, dim3(1), dim3(PB), 0, dev.stream, totals, nb);
-    PLK_HIP(hipGetLastError());
-    hipLaunchKernelGGL((scan_final_kernel<T>), dim3(static_cast<unsigned>(nb)), dim3(PB), 0,
-                       dev.stream, psi, len, totals, cdf);
-    PLK_HIP(hipGetLastError());
     if (shots > 0) {
-        hipLaunchKernelGGL(sample_kernel, dim3(static_cast<unsigned>((shots + PB - 1) / PB)),
-                           dim3(PB), 0, dev.stream, cdf, len, s.n, static_cast<uint64_t>(shots),
-                           seed, out);
+        ProfScope prof("sample", static_cast<double>(s.bytes()), dev.stream);
+        hipLaunchKernelGGL((run_totals_kernel<T>), dim3(static_cast<unsigned>(nb)), dim3(PB), 0,
+                           dev.stream, psi, len, runs, totals);
+        PLK_HIP(hipGetLastError());
+        hipLaunchKernelGGL(scan_top_kernel, dim3(1), dim3(SCAN), 0, dev.stream, totals, nb);
+        PLK_HIP(hipGetLastError());
+        hipLaunchKernelGGL((sample_kernel<T>), dim3(static_cast<unsigned>((shots + PB / 64 - 1) / (PB / 64))),
+                           dim3(PB), 0, dev.stream, psi, len, runs, totals, nb, s.n,
+                           static_cast<uint64_t>(shots), seed, out);
         PLK_HIP(hipGetLastError());
         PLK_HIP(hipMemcpyAsync(host_out, out, out_bytes, hipMemcpyDeviceToHost, dev.stream));
     }
