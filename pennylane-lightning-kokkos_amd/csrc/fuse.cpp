@@ -2,8 +2,8 @@
 // (kernels_block.hip). The reference applies every gate as its own kernel
 // (StateVectorKokkos.hpp:585-676) and dense matrices through
 // multiQubitOpFunctor (GateFunctors.hpp:195-300); here runs of gates on at
-// most five wires are multiplied into one 32x32 matrix on the host and each
-// block is one pass over the state.
+// most five wires are multiplied into one 32x32 matrix on the host; large
+// states take two blocks a pass, others one.
 #include <set>
 
 #include "plk_internal.hpp"
@@ -175,8 +175,14 @@ void apply_blocks_t(Device &dev, const State &s, const std::vector<FusedBlock> &
     auto *d = static_cast<T *>(ensure_work(dev, all.size() * sizeof(T)));
     PLK_HIP(hipMemcpyAsync(d, all.data(), all.size() * sizeof(T), hipMemcpyHostToDevice,
                            dev.stream));
+    const bool pairs = block_pairs(dev, s);
     for (size_t b = 0; b < blocks.size(); b++) {
-        launch_block5(dev, s, blocks[b].bits, d + b * 4096);
+        if (pairs && b + 1 < blocks.size()) {
+            launch_block_pair(dev, s, blocks[b].bits, blocks[b + 1].bits, d + b * 4096);
+            b++;
+        } else {
+            launch_block5(dev, s, blocks[b].bits, d + b * 4096);
+        }
     }
     // The host buffer stays alive until its upload has been read.
     PLK_HIP(hipStreamSynchronize(dev.stream));

@@ -667,6 +667,10 @@ int block5_lane_pack(const std::vector<cd> &M, std::vector<float> &out);
 int block5_lane_pack(const std::vector<cd> &M, std::vector<double> &out);
 // One block pass (n >= 9); d_apack = block5_lane_pack in the state's precision.
 void launch_block5(Device &dev, const State &s, const int *bits, const void *d_apack);
+// Whether two blocks of s share one pass, and that pass: the lane packs of both
+// follow each other at d_apack.
+bool block_pairs(const Device &dev, const State &s);
+void launch_block_pair(Device &dev, const State &s, const int *bits0, const int *bits1, const void *d_apack);
 // Uploads the lane packs of every block (one copy) and applies them in order.
 void apply_blocks(Device &dev, const State &s, const std::vector<FusedBlock> &blocks);
 
