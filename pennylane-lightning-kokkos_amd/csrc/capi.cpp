@@ -542,10 +542,16 @@ uint64_t mixing_mask(const PlanOp &p, int n) {
 // lowest L bits. Operations on disjoint wires commute, so an operation may be
 // taken ahead of skipped ones it shares no wire with; an unfusable operation
 // is a barrier and runs on its own. With bundled == false (register-tile
-// passes) one-wire runs are fused first, and a pass needs in its tile only
-// the bits its operations mix.
+// passes) one-wire runs are fused first, a pass needs in its tile only the
+// bits its operations mix, and operations that share only wires which neither
+// mixes commute as well.
+//
+// A pass's tile starts as the bits of the first operations that fit. With
+// `exchange` each of them is then exchanged for the outside bit with which the
+// pass takes most operations, if any takes more. A trial walks the operations
+// until every wire is blocked.
 std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
-                             int pmax = TILE_PMAX, bool bundled = true) {
+                             int pmax = TILE_PMAX, bool bundled = true, bool exchange = false) {
     std::vector<PlanOp> all;
     if (bundled) {
         for (auto &p : ops_in) {
@@ -558,67 +564,113 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
     } else {
         all = fuse_runs(std::move(ops_in));
     }
-    // Wire and state-bit masks (wires and bits < 64).
-    std::vector<uint64_t> wmask(all.size()), bmask(all.size());
-    std::vector<char> fus(all.size());
-    std::vector<int> rem(all.size());
+    // State bits (< 64) an op acts on, and of these the ones its pass needs in
+    // the tile.
+    struct Item {
+        uint64_t on, mix;
+        int index, sums;
+        bool fus;
+    };
+    std::vector<Item> rem(all.size()), rest;
+    uint64_t every = 0;
     for (size_t i = 0; i < all.size(); i++) {
+        Item &it = rem[i];
+        it.index = static_cast<int>(i);
+        it.on = 0;
         for (auto w : all[i].U.wires) {
-            wmask[i] |= uint64_t{1} << w;
-            bmask[i] |= uint64_t{1} << (n - 1 - static_cast<int>(w));
+            it.on |= uint64_t{1} << (n - 1 - static_cast<int>(w));
         }
-        fus[i] = fusable(all[i]) ? 1 : 0;
-        rem[i] = static_cast<int>(i);
+        every |= it.on;
+        it.fus = fusable(all[i]);
+        it.mix = bundled || !it.fus ? it.on : mixing_mask(all[i], n);
+        it.sums = bundled ? (all[i].trainable ? 1 : 0) : rt_slots(all[i]);
     }
-    std::vector<uint64_t> mmask(all.size(), 0);
-    if (!bundled) {
-        for (size_t i = 0; i < all.size(); i++) {
-            if (fus[i]) {
-                mmask[i] = mixing_mask(all[i], n);
+    // Skipped operations so far: the bits they mix, and the bits they only
+    // select by, which stop an operation that mixes them.
+    struct Blocked {
+        uint64_t mixed = 0, selected = 0;
+        bool stops(const Item &it) const { return ((mixed & it.on) | (selected & it.mix)) != 0; }
+        void add(const Item &it) {
+            mixed |= it.mix;
+            selected |= it.on;
+        }
+    };
+    // Operations of rem that a pass over these bits takes.
+    auto count = [&](uint64_t bits) {
+        Blocked blocked;
+        size_t taken = 0;
+        int sums = 0;
+        const size_t end = std::min(rem.size(), kLookahead);
+        for (size_t k = 0; k < end && rem[k].fus && (blocked.mixed & every) != every; k++) {
+            const Item &it = rem[k];
+            if ((it.mix & ~bits) == 0 && !blocked.stops(it) && taken < kPassMaxOps && sums + it.sums <= pmax) {
+                taken++;
+                sums += it.sums;
+            } else {
+                blocked.add(it);
             }
         }
-    }
+        return taken;
+    };
+    const uint64_t low = L > 0 ? (uint64_t{1} << L) - 1 : 0;
     std::vector<Step> steps;
-    std::vector<int> taken, rest;
+    std::vector<int> taken;
     while (!rem.empty()) {
-        if (!fus[rem[0]]) {
+        if (!rem[0].fus) {
             Step s;
-            s.single = std::move(all[rem[0]]);
+            s.single = std::move(all[rem[0].index]);
             steps.push_back(std::move(s));
             rem.erase(rem.begin());
             continue;
         }
-        uint64_t bits = L > 0 ? (uint64_t{1} << L) - 1 : 0;
-        uint64_t blocked = 0;
-        taken.clear();
-        rest.clear();
+        // Bits of the first operations that fit, then the lowest unused ones.
+        uint64_t bits = low;
+        auto pad = [&] {
+            for (int b = 0; __builtin_popcountll(bits) < T && b < n; b++) {
+                bits |= uint64_t{1} << b;
+            }
+        };
         int nslots = 0;
-        size_t k = 0;
-        for (; k < rem.size(); k++) {
-            const int i = rem[k];
-            if (!fus[i] || k >= kLookahead) {
-                break;
+        auto take = [&](bool grow) {
+            Blocked blocked;
+            taken.clear();
+            rest.clear();
+            nslots = 0;
+            size_t k = 0;
+            for (; k < rem.size() && rem[k].fus && k < kLookahead; k++) {
+                const Item &it = rem[k];
+                const uint64_t nb = bits | it.mix;
+                if ((grow ? __builtin_popcountll(nb) <= T : nb == bits) && !blocked.stops(it) &&
+                    taken.size() < kPassMaxOps && nslots + it.sums <= pmax) {
+                    bits = nb;
+                    nslots += it.sums;
+                    taken.push_back(it.index);
+                } else {
+                    blocked.add(it);
+                    rest.push_back(it);
+                }
             }
-            const int sums = bundled ? (all[i].trainable ? 1 : 0) : rt_slots(all[i]);
-            // Register-tile passes need only the bits an op mixes in the
-            // tile: its other bits may lie outside, where they are fixed per
-            // tile and select the op's block.
-            const uint64_t nb = bits | (bundled ? bmask[i] : mmask[i]);
-            const bool ok = taken.size() < kPassMaxOps && nslots + sums <= pmax &&
-                            !(blocked & wmask[i]) && __builtin_popcountll(nb) <= T;
-            if (ok) {
-                bits = nb;
-                nslots += sums;
-                taken.push_back(i);
-            } else {
-                blocked |= wmask[i];
-                rest.push_back(i);
+            rest.insert(rest.end(), rem.begin() + static_cast<long>(k), rem.end());
+        };
+        take(true);
+        pad();
+        if (exchange && !rest.empty() && rest[0].fus) {
+            const uint64_t before = bits;
+            size_t best = count(bits);
+            for (uint64_t outs = bits & ~low; outs != 0; outs &= outs - 1) {
+                const uint64_t others = bits & ~(outs & (~outs + 1));
+                for (uint64_t ins = every & ~bits; ins != 0; ins &= ins - 1) {
+                    const uint64_t trial = others | (ins & (~ins + 1));
+                    const size_t c = count(trial);
+                    if (c > best) {
+                        best = c;
+                        bits = trial;
+                    }
+                }
             }
-        }
-        rest.insert(rest.end(), rem.begin() + static_cast<long>(k), rem.end());
-        // Pad the tile with the lowest unused bits.
-        for (int b = 0; __builtin_popcountll(bits) < T && b < n; b++) {
-            bits |= uint64_t{1} << b;
+            if (bits != before || best > taken.size()) {
+                take(false);
+            }
         }
         Step s;
         s.tiled = true;
@@ -650,6 +702,16 @@ int low_bits(int dtype) { return dtype == PLK_C64 ? 4 : 3; }
 int env_int(const char *name, int dflt) {
     const char *v = std::getenv(name);
     return v && *v ? std::atoi(v) : dflt;
+}
+
+// Whether a register-tile plan for this many states exchanges tile bits: the
+// trials take 20 to 30 us of host time a pass and save a fifth to a quarter of
+// the passes, which pays from 1 GiB moved a pass on (25-qubit complex128 gate
+// stream, 1 GiB: 6.3 ms without and 5.6 with; 24 qubits 2.67 and 2.84; 24-qubit
+// complex128 Jacobian of 9 observables, 5 GiB: 37 passes and 60.4 ms without,
+// 29 and 54.3 with).
+bool plan_exchange(int n, int dtype, size_t states) {
+    return 2.0 * static_cast<double>(states) * std::ldexp(dtype == PLK_C64 ? 8.0 : 16.0, n) >= 1073741824.0;
 }
 
 // Tile width of backward (adjoint) passes; 0 selects register segments.
@@ -2148,7 +2210,7 @@ std::vector<PlanOp> forward_ops(const OpsData &ops, int n,
 std::vector<Step> forward_plan(std::vector<PlanOp> &&v, int n, int dtype) {
     if (use_rtile(n, dtype, 0)) {
         std::vector<Step> steps = plan_tiles(std::move(v), n, rt_reg_bits(dtype, 0) + RT_LANE_BITS,
-                                             low_bits(dtype), RT_SLOTS_MAX, false);
+                                             low_bits(dtype), RT_SLOTS_MAX, false, plan_exchange(n, dtype, 1));
         split_sparse_passes(steps, n);
         return steps;
     }
@@ -2778,7 +2840,8 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
     const bool rt = use_rtile(n, ref.dtype, nj);
     const int T_adj = rt ? rt_reg_bits(ref.dtype, nj) + RT_LANE_BITS : tile_bits_adjoint(n, ref.dtype);
     std::vector<Step> steps =
-        rt ? plan_tiles(std::move(rev), n, T_adj, low_bits(ref.dtype), RT_SLOTS_MAX, false)
+        rt ? plan_tiles(std::move(rev), n, T_adj, low_bits(ref.dtype), RT_SLOTS_MAX, false,
+                        plan_exchange(n, ref.dtype, n_obs + 1))
            : T_adj > 0 ? plan_tiles(std::move(rev), n, T_adj, low_bits(ref.dtype))
                        : plan_steps(std::move(rev));
     if (rt) {

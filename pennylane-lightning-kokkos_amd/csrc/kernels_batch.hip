@@ -12,7 +12,7 @@
 // each launch bound by the vector issue and latency of two waves of tiles per
 // SIMD (states stay in the 256 MB last-level cache).
 //
-// Jacobian sums are FP64 and in a fixed order: quads by DPP, LDS per quad, the
+// Jacobian sums are FP64 and in a fixed order: row halves by DPP, LDS per half, the
 // blocks of a pass in order.
 #include "rtile_device.hpp"
 
@@ -24,12 +24,12 @@ template <typename T, int NS, int R>
 __global__ void __launch_bounds__(64, 4) stage_kernel(BatchArgs A, const BatchBlock *__restrict__ blocks) {
     constexpr int NA = 1 << R;
     constexpr int TB = R + RT_LANE_BITS;
-    __shared__ double lacc[NS > 1 ? RT_SLOTS_MAX * 16 + 64 : 1];
+    __shared__ double lacc[NS > 1 ? RT_SLOTS_MAX * RT_CELLS + 64 : 1];
     const BatchBlock b = load_uniform(blocks + blockIdx.x);
     const BatchCircuit c = load_uniform(A.circuits + b.circuit);
     const SweepPass P = load_uniform(A.passes + b.pass);
     const int lane = static_cast<int>(__lane_id());
-    const int dummy = P.nslots * 16;
+    const int dummy = P.nslots * RT_CELLS;
     if constexpr (NS > 1) {
         for (int i = lane; i < dummy; i += 64) {
             lacc[i] = 0.0;
@@ -78,8 +78,8 @@ __global__ void __launch_bounds__(64, 4) stage_kernel(BatchArgs A, const BatchBl
         for (int i = lane; i < P.nslots; i += 64) {
             double s = 0.0;
 #pragma unroll
-            for (int q = 0; q < 16; q++) {
-                s += lacc[i * 16 + q];
+            for (int q = 0; q < RT_CELLS; q++) {
+                s += lacc[i * RT_CELLS + q];
             }
             A.parts[P.parts + static_cast<int64_t>(i) * c.blocks + b.block] = s;
         }

@@ -47,8 +47,8 @@
 // Im<h_j|Y phi>, Im<h_j|Z phi> once (only those it needs) and the reduction
 // forms every gate's derivative from them.
 //
-// The four lanes of each quad are summed by DPP and one lane adds the total
-// into LDS (ds_add_f64, one address per quad, so the order is fixed). After
+// The lanes of two quads are summed by DPP and one lane adds the total into
+// LDS (ds_add_f64, one address per two quads, so the order is fixed). After
 // its last tile the wavefront writes per-block partials; a second kernel sums
 // them in a fixed order. No LDS staging of states and no barriers: each
 // wavefront streams its tiles independently.
@@ -84,10 +84,10 @@ __global__ void __launch_bounds__(64, (rt_waves<T, NJ>()))
     const int njc = c < L.nbig ? NJ : NJ - 1;
     const int jc0 = c < L.nbig ? c * NJ : L.nbig * NJ + (c - L.nbig) * (NJ - 1);
     const int width = L.nbig * NJ + (nc - L.nbig) * (NJ - 1);
-    // FP64 sums [slot * NJ + j][quad], then one dummy slot per lane.
+    // FP64 sums [slot * NJ + j][cell], then one dummy slot per lane.
     extern __shared__ double lacc[];
     const int lane = static_cast<int>(__lane_id());
-    const int dummy = L.nslots * NJ * 16;
+    const int dummy = L.nslots * NJ * RT_CELLS;
     if constexpr (NJ > 0) {
         for (int i = lane; i < dummy; i += 64) {
             lacc[i] = 0.0;
@@ -151,8 +151,8 @@ __global__ void __launch_bounds__(64, (rt_waves<T, NJ>()))
         for (int i = lane; i < per; i += 64) {
             double s = 0.0;
 #pragma unroll
-            for (int q = 0; q < 16; q++) {
-                s += lacc[i * 16 + q];
+            for (int q = 0; q < RT_CELLS; q++) {
+                s += lacc[i * RT_CELLS + q];
             }
             // Local (slot, j) -> launch-wide (slot, jc0 + j).
             const int slot = i / NJ, j = i % NJ;

@@ -20,16 +20,16 @@
 // us in the kernel and 392 us a call, against 532 us a call with one launch per
 // pass replayed from a HIP graph.
 //
-// Jacobian sums are FP64 and in a fixed order: quads by DPP, LDS per quad and
-// wave, then quads and waves in order.
+// Jacobian sums are FP64 and in a fixed order: row halves by DPP, LDS per half and
+// wave, then halves and waves in order.
 #include "rtile_device.hpp"
 
 namespace plk {
 
 namespace {
 
-// Per-wave LDS: the pass's sums for 16 quads and a dummy slot per lane.
-constexpr int kWaveSums = RT_SLOTS_MAX * 16 + 64;
+// Per-wave LDS: the pass's sums and a dummy slot per lane.
+constexpr int kWaveSums = RT_SLOTS_MAX * RT_CELLS + 64;
 
 template <typename T, int NS, int R>
 __device__ __forceinline__ void run_pass(const SweepArgs &A, const SweepPass &P, int n, Cx<T> *phi, Cx<T> *h,
@@ -39,7 +39,7 @@ __device__ __forceinline__ void run_pass(const SweepArgs &A, const SweepPass &P,
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
     const int nwaves = static_cast<int>(blockDim.x) >> 6;
     double *lacc = sums + wave * kWaveSums;
-    const int dummy = P.nslots * 16;
+    const int dummy = P.nslots * RT_CELLS;
     if constexpr (NS > 1) {
         for (int i = lane; i < dummy; i += 64) {
             lacc[i] = 0.0;
@@ -91,8 +91,8 @@ __device__ __forceinline__ void run_pass(const SweepArgs &A, const SweepPass &P,
             for (int i = static_cast<int>(threadIdx.x); i < P.nslots; i += static_cast<int>(blockDim.x)) {
                 double s = 0.0;
                 for (int w = 0; w < nwaves; w++) {
-                    for (int q = 0; q < 16; q++) {
-                        s += sums[w * kWaveSums + i * 16 + q];
+                    for (int q = 0; q < RT_CELLS; q++) {
+                        s += sums[w * kWaveSums + i * RT_CELLS + q];
                     }
                 }
                 totals[i] = s;

@@ -349,9 +349,11 @@ struct RtLaunch {
 inline int rt_width(const RtLaunch &L) {
     return L.nbig * L.nj + (L.nc - L.nbig) * std::max(0, L.nj - 1);
 }
-// LDS of one block: the pass's sums for 16 quads and a dummy slot per lane.
+// LDS cells of a sum: two per 16-lane row.
+constexpr int RT_CELLS = 8;
+// LDS of one block: the pass's sums and a dummy slot per lane.
 inline size_t rt_lds_bytes(int nj, int nslots) {
-    return nj > 0 ? (static_cast<size_t>(nslots) * nj * 16 + 64) * sizeof(double) : 0;
+    return nj > 0 ? (static_cast<size_t>(nslots) * nj * RT_CELLS + 64) * sizeof(double) : 0;
 }
 
 constexpr int RT_OBS_MAX = 24; // observable states per register-tile launch

@@ -156,12 +156,15 @@ __device__ __forceinline__ Ins<T> fetch(CT<unsigned char> *prog, int pc) {
 }
 
 // ---------------------------------------------------------------------------
-// FP64 sums of a trainable instruction: NV values per lane, summed over the
-// quad by DPP and added into LDS by its lanes (value v at (base + v) * 16 +
-// quad). Lane r of a quad adds values r, r + 4, ... (every lane holds every
-// total); lanes without one add to a dummy slot of their own. No branch on
-// the lane, so the instruction switch around this stays free of divergent
-// control flow.
+// FP64 sums of a trainable instruction: NV values per lane, summed by DPP over
+// the quad, then over two quads of the 16-lane row (lane r of a quad for values
+// r, r + 4, ...: every lane holds every total of its quad), and added into one
+// of the value's RT_CELLS cells in LDS; lanes without a value or cell add to a
+// dummy slot of their own. No branch on the lane, so the instruction switch
+// around this stays free of divergent control flow. A cell per quad instead
+// took twice the LDS: passes of more than 30 sums of three states then fitted
+// fewer than the three wavefronts per SIMD that their registers allow, and ran
+// in two rounds (24 qubits complex128, 33 sums: 2.5 to 2.9 ms, now 1.9 to 2.2).
 // ---------------------------------------------------------------------------
 template <int CTRL> __device__ __forceinline__ double dpp_f64(double v) {
     const uint64_t b = __double_as_longlong(v);
@@ -179,6 +182,7 @@ __device__ __forceinline__ void add_slots(double (&d)[NV], double *lacc, int bas
         d[v] += dpp_f64<0x4E>(d[v]); // quad_perm [2,3,0,1]
     }
     const int r = lane & 3;
+    const int cell = ((lane >> 4) << 1) | ((lane >> 2) & 1);
 #pragma unroll
     for (int v0 = 0; v0 < NV; v0 += 4) {
         double x = d[v0];
@@ -187,7 +191,9 @@ __device__ __forceinline__ void add_slots(double (&d)[NV], double *lacc, int bas
             x = (r == v - v0) ? d[v] : x;
         }
         const bool full = v0 + 4 <= NV;
-        const int idx = full || v0 + r < NV ? (base + v0 + r) * 16 + (lane >> 2) : dummy + lane;
+        x += dpp_f64<0x128>(x); // row_ror:8
+        const bool mine = (lane & 8) == 0 && (full || v0 + r < NV);
+        const int idx = mine ? (base + v0 + r) * RT_CELLS + cell : dummy + lane;
         atomicAdd(&lacc[idx], x);
     }
 }
