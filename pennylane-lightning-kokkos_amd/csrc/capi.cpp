@@ -2619,6 +2619,33 @@ bool steps_have_single(const std::vector<Step> &steps, int n) {
     return false;
 }
 
+// The launches of a reverse plan and where their partials lie: the entries
+// that a replay copies have to match the launches it replays.
+void append_signature(const SweepParts &parts, std::vector<unsigned char> &sig) {
+    auto put = [&](uint64_t v) {
+        const auto *b = reinterpret_cast<const unsigned char *>(&v);
+        sig.insert(sig.end(), b, b + sizeof v);
+    };
+    for (const auto &step : parts.steps) {
+        put(step.size());
+        for (const PartLaunch &l : step) {
+            for (const uint64_t v : {static_cast<uint64_t>(l.j0), static_cast<uint64_t>(l.width),
+                                     static_cast<uint64_t>(l.offset), static_cast<uint64_t>(l.rt.nj),
+                                     static_cast<uint64_t>(l.rt.nc), static_cast<uint64_t>(l.rt.nbig),
+                                     static_cast<uint64_t>(l.rt.write_phi), static_cast<uint64_t>(l.step.nj),
+                                     static_cast<uint64_t>(l.step.write_phi)}) {
+                put(v);
+            }
+        }
+    }
+    for (const auto &f : parts.flushes) {
+        put(f.step);
+        put(f.first);
+        put(f.count);
+    }
+    put(parts.doubles);
+}
+
 // ---------------------------------------------------------------------------
 // Whole circuits in one launch (kernels_sweep.hip): one workgroup per
 // observable runs every pass of the circuit.
@@ -2889,6 +2916,7 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
         std::vector<unsigned char> sig;
         append_signature(img_f, sig);
         append_signature(img_r, sig);
+        append_signature(parts, sig);
         size_t pauli_bytes = 0;
         for (const auto &pi : pimg) {
             const uint64_t f[3] = {pi.bytes.size(), pi.toff, static_cast<uint64_t>(pi.ngroups)};
