@@ -1822,7 +1822,7 @@ void split_sparse_passes(std::vector<Step> &steps, int n) {
 
 // Programs of every register-tile pass of a plan, uploaded as one blob.
 // R: register bits of the tile passes.
-PlanImage build_image(const std::vector<Step> &steps, const State &s, int R) {
+PlanImage build_image(const std::vector<Step> &steps, const State &s) {
     PlanImage img;
     if (s.dtype == PLK_C64) {
         build_seg_tables<float>(steps, s.n, img);
@@ -1839,6 +1839,7 @@ PlanImage build_image(const std::vector<Step> &steps, const State &s, int R) {
     double norm = 1.0;
     for (size_t i = 0; i < steps.size(); i++) {
         if (steps[i].tiled && steps[i].pass.rt) {
+            const int R = static_cast<int>(steps[i].pass.tb.size()) - RT_LANE_BITS;
             img.progs[i] = s.dtype == PLK_C64 ? build_rt_program<float>(steps[i].pass, s.n, R, img.rt, norm)
                                               : build_rt_program<double>(steps[i].pass, s.n, R, img.rt, norm);
         }
@@ -1933,7 +1934,7 @@ int rtile_chunk(int dtype, int n, int num_cus) {
     if (e > 0) {
         return std::min(RT_NJMAX, e);
     }
-    const int T = rt_reg_bits(dtype, 3) + RT_LANE_BITS;
+    const int T = rt_reg_max(dtype, 3) + RT_LANE_BITS;
     const bool few_tiles = n - T < 30 && (int64_t{1} << std::max(0, n - T)) < num_cus;
     return few_tiles ? 1 : 3;
 }
@@ -1949,7 +1950,26 @@ int sweep_chunk(int dtype, int n, size_t n_obs, int num_cus) {
 // (6-layer adjoint, 9 observables, complex128: 0.70 vs 2.52 ms at 10 qubits,
 // 1.32 vs 2.12 at 16, 8.35 vs 11.26 at 21). PLK_RTILE=0 turns them off.
 bool use_rtile(int n, int dtype, int nj) {
-    return env_int("PLK_RTILE", -1) != 0 && n >= rt_reg_bits(dtype, nj) + RT_LANE_BITS;
+    return env_int("PLK_RTILE", -1) != 0 && n >= rt_reg_min(dtype, nj) + RT_LANE_BITS;
+}
+
+// Register bits of a plan's tiles. Wider tiles take fewer passes, narrower ones
+// spread a pass over more wavefronts that each walk less: a pass of a few tiles
+// takes as long as one wavefront needs for its program. Measured, forward
+// (400-gate stream, R = 3 / 4 / 5): 15 qubits complex128 553 / 590 / 661 us, 20
+// qubits 757 / 763 / 838, 22 qubits 1139 / 976 / 1023, 24 qubits 3133 / 2701 /
+// 2635; 20 qubits complex64 630 / 612 / 680, 24 qubits 2407 / 1914 / 1728. One
+// observable a chunk (R = 3 / 4): 17 qubits complex64, 5 observables 742 / 766 us
+// (R = 5: 897); 16 qubits complex128, 9 observables 636 / 675; one observable,
+// 20 qubits complex128 3208 / 3320, 21 qubits 3828 / 3673.
+int plan_reg_bits(int n, int dtype, int nj, size_t chunks, int num_cus) {
+    const int lo = rt_reg_min(dtype, nj);
+    int R = std::min(rt_reg_max(dtype, nj), n - RT_LANE_BITS);
+    auto tiles_per_cu = [&] { return std::ldexp(static_cast<double>(chunks), n - R - RT_LANE_BITS) / num_cus; };
+    while (R > lo && tiles_per_cu() < (R == 5 ? 32.0 : nj == 1 ? 8.0 : 2.0)) {
+        R--;
+    }
+    return R;
 }
 
 void apply_single(Device &dev, const State &s, const CompiledOp &op);
@@ -1991,7 +2011,7 @@ void enqueue_forward(Device &dev, const State &s, const std::vector<Step> &steps
 }
 
 void run_forward(Device &dev, const State &s, const std::vector<Step> &steps) {
-    const PlanImage img = build_image(steps, s, rt_reg_bits(s.dtype, 0));
+    const PlanImage img = build_image(steps, s);
     enqueue_forward(dev, s, steps, img, place_in_arena(dev, img));
     // The host image is read by the stream's copies.
     PLK_HIP(hipStreamSynchronize(dev.stream));
@@ -2207,9 +2227,9 @@ std::vector<PlanOp> forward_ops(const OpsData &ops, int n,
 }
 
 // Forward plan of the whole op list.
-std::vector<Step> forward_plan(std::vector<PlanOp> &&v, int n, int dtype) {
+std::vector<Step> forward_plan(const Device &dev, std::vector<PlanOp> &&v, int n, int dtype) {
     if (use_rtile(n, dtype, 0)) {
-        std::vector<Step> steps = plan_tiles(std::move(v), n, rt_reg_bits(dtype, 0) + RT_LANE_BITS,
+        std::vector<Step> steps = plan_tiles(std::move(v), n, plan_reg_bits(n, dtype, 0, 1, dev.num_cus) + RT_LANE_BITS,
                                              low_bits(dtype), RT_SLOTS_MAX, false, plan_exchange(n, dtype, 1));
         split_sparse_passes(steps, n);
         return steps;
@@ -2865,7 +2885,7 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
     }
     const int nj = sweep_chunk(ref.dtype, n, n_obs, dev.num_cus);
     const bool rt = use_rtile(n, ref.dtype, nj);
-    const int T_adj = rt ? rt_reg_bits(ref.dtype, nj) + RT_LANE_BITS : tile_bits_adjoint(n, ref.dtype);
+    const int T_adj = rt ? plan_reg_bits(n, ref.dtype, nj, chunk_sizes(n_obs, nj).size(), dev.num_cus) + RT_LANE_BITS : tile_bits_adjoint(n, ref.dtype);
     std::vector<Step> steps =
         rt ? plan_tiles(std::move(rev), n, T_adj, low_bits(ref.dtype), RT_SLOTS_MAX, false,
                         plan_exchange(n, ref.dtype, n_obs + 1))
@@ -2874,9 +2894,9 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
     if (rt) {
         split_sparse_passes(steps, n);
     }
-    const std::vector<Step> fwd = apply_ops ? forward_plan(forward_ops(ops, n), n, ref.dtype) : std::vector<Step>{};
-    const PlanImage img_f = build_image(fwd, ref, rt_reg_bits(ref.dtype, 0));
-    PlanImage img_r = build_image(steps, ref, rt_reg_bits(ref.dtype, nj));
+    const std::vector<Step> fwd = apply_ops ? forward_plan(dev, forward_ops(ops, n), n, ref.dtype) : std::vector<Step>{};
+    const PlanImage img_f = build_image(fwd, ref);
+    PlanImage img_r = build_image(steps, ref);
     const bool alt = needs_alt(dev, steps, n_obs, ref.dtype, n);
     const SweepParts parts = place_partials(dev, steps, img_r, ref, n_obs, alt);
     plan_scope.reset();
@@ -3907,7 +3927,7 @@ int plk_apply_ops(plk_state *sv, const plk_ops *ops) {
         if (sweep_serves(s) && sweep_takes(v)) {
             sweep_forward(dev, s, std::move(v));
         } else {
-            run_forward(dev, s, forward_plan(std::move(v), s.n, s.dtype));
+            run_forward(dev, s, forward_plan(dev, std::move(v), s.n, s.dtype));
         }
     })
 }

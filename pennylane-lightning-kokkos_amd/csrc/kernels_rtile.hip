@@ -64,7 +64,7 @@ template <typename T> struct RtPtrs {
 };
 
 template <typename T, int NJ, int R>
-__global__ void __launch_bounds__(64, (rt_waves<T, NJ>()))
+__global__ void __launch_bounds__(64, (rt_waves<T, NJ, R>()))
     rtile_kernel(Cx<T> *phi, Cx<T> *phi_out, RtPtrs<T> hp, const unsigned char *__restrict__ prog_g,
                  RtLaunch L, double *__restrict__ partials) {
     constexpr int A = 1 << R;
@@ -166,10 +166,18 @@ __global__ void __launch_bounds__(64, (rt_waves<T, NJ>()))
 
 } // namespace
 
-// Blocks per chunk of a launch: the chunks share the resident blocks; in
-// groups of 8 (one per XCD) when there are enough.
-template <typename T, int NJ> int rtile_blocks_t(const Device &dev, const RtLaunch &L, int nc) {
-    constexpr int R = rt_reg_bits<T>(NJ);
+// f(R) for the launch's register bits.
+template <typename T, int NJ, int R = rt_reg_min<T>(NJ), typename F> void with_reg(int r, F &&f) {
+    if constexpr (R < rt_reg_max<T>(NJ)) {
+        if (r != R) {
+            with_reg<T, NJ, R + 1>(r, f);
+            return;
+        }
+    }
+    f(IC<R>{});
+}
+
+template <typename T, int NJ, int R> int blocks_per_chunk(const Device &dev, const RtLaunch &L, int nc) {
     const void *kfn = reinterpret_cast<const void *>(&rtile_kernel<T, NJ, R>);
     const size_t lds = rt_lds_bytes(NJ, L.nslots);
     static int per_cu[RT_SLOTS_MAX + 1] = {}; // by slots: the kernel's LDS follows from them
@@ -187,13 +195,20 @@ template <typename T, int NJ> int rtile_blocks_t(const Device &dev, const RtLaun
     return static_cast<int>(bpc);
 }
 
+// Blocks per chunk of a launch: the chunks share the resident blocks; in
+// groups of 8 (one per XCD) when there are enough.
+template <typename T, int NJ> int rtile_blocks_t(const Device &dev, const RtLaunch &L, int nc) {
+    int blocks = 0;
+    with_reg<T, NJ>(L.R, [&](auto R) { blocks = blocks_per_chunk<T, NJ, decltype(R)::value>(dev, L, nc); });
+    return blocks;
+}
+
 // Launcher of one (precision, observable chunk) variant. The build compiles
 // this file once per variant with PLK_RT_T and PLK_RT_NJ defined, so the
 // variants compile in parallel.
 template <typename T, int NJ>
 void rtile_launch_t(Device &dev, const State &phi, void *phi_out, void *const *h_ptrs,
                     const void *d_prog, const RtLaunch &Lin, int bpc, double *partials) {
-    constexpr int R = rt_reg_bits<T>(NJ);
     RtLaunch L = Lin;
     L.xgroup = bpc >= 8 ? 8 : 1;
     const int width = rt_width(L);
@@ -206,9 +221,12 @@ void rtile_launch_t(Device &dev, const State &phi, void *phi_out, void *const *h
     // state read and written once.
     const double bytes = (1.0 + L.write_phi + 2.0 * width) * static_cast<double>(phi.bytes());
     ProfScope prof(NJ > 0 ? "adjoint_rtile" : "apply_rtile", bytes, dev.stream);
-    hipLaunchKernelGGL((rtile_kernel<T, NJ, R>), dim3(grid), dim3(64), rt_lds_bytes(NJ, L.nslots), dev.stream,
-                       static_cast<Cx<T> *>(phi.d), static_cast<Cx<T> *>(phi_out), hp,
-                       static_cast<const unsigned char *>(d_prog), L, partials);
+    with_reg<T, NJ>(L.R, [&](auto R) {
+        hipLaunchKernelGGL((rtile_kernel<T, NJ, decltype(R)::value>), dim3(grid), dim3(64),
+                           rt_lds_bytes(NJ, L.nslots), dev.stream, static_cast<Cx<T> *>(phi.d),
+                           static_cast<Cx<T> *>(phi_out), hp, static_cast<const unsigned char *>(d_prog), L,
+                           partials);
+    });
     PLK_HIP(hipGetLastError());
 }
 

@@ -285,16 +285,23 @@ constexpr int RT_TMAX = RT_RMAX + RT_LANE_BITS;
 constexpr int RT_SLOTS_MAX = 48; // sums per pass (a fused run of two ops takes up to three)
 constexpr int RT_NJMAX = 4;      // observable states per register-tile chunk
 
-// Register bits of a tile by precision and observable chunk: the states of a
-// chunk fill 64 (one or two states) to 160 VGPRs (five).
-template <typename T> constexpr int rt_reg_bits(int nj) {
-    return (nj <= 1 ? 4 : 3) + (sizeof(T) == 4 ? 1 : 0);
+// Register bits of a tile by precision and observable chunk: from rt_reg_min to
+// rt_reg_max, where the states of a chunk fill 64 (one or two states of
+// complex64) to 160 VGPRs (five states). Larger chunks have one width.
+template <typename T> constexpr int rt_reg_max(int nj) {
+    return nj == 0 ? 5 : nj == 1 || sizeof(T) == 4 ? 4 : 3;
 }
-inline int rt_reg_bits(int dtype, int nj) {
-    return dtype == PLK_C64 ? rt_reg_bits<float>(nj) : rt_reg_bits<double>(nj);
+template <typename T> constexpr int rt_reg_min(int nj) { return nj <= 1 ? 3 : rt_reg_max<T>(nj); }
+inline int rt_reg_max(int dtype, int nj) {
+    return dtype == PLK_C64 ? rt_reg_max<float>(nj) : rt_reg_max<double>(nj);
+}
+inline int rt_reg_min(int dtype, int nj) {
+    return dtype == PLK_C64 ? rt_reg_min<float>(nj) : rt_reg_min<double>(nj);
 }
 // Waves per SIMD the register allocator is held to.
-template <typename T, int NJ> constexpr int rt_waves() { return NJ == 0 ? 4 : NJ <= 3 && !(NJ == 1 && sizeof(T) == 8) ? 3 : 2; }
+template <typename T, int NJ, int R> constexpr int rt_waves() {
+    return NJ == 0 ? (R == 5 && sizeof(T) == 8 ? 3 : 4) : NJ <= 3 && !(NJ == 1 && R == 4 && sizeof(T) == 8) ? 3 : 2;
+}
 
 enum RtOpCode : int8_t {
     RT_NOP = 0,   // remaps only
