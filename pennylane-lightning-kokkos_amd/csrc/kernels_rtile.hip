@@ -189,6 +189,14 @@ template <typename T, int NJ, int R> int blocks_per_chunk(const Device &dev, con
     const uint64_t ntiles = uint64_t{1} << (L.n - L.T);
     const uint64_t cap = static_cast<uint64_t>(dev.num_cus) * nb;
     uint64_t bpc = std::max<uint64_t>(1, std::min(ntiles, cap / static_cast<uint64_t>(nc)));
+    // Without sums a block costs nothing to start: a block a tile lets the
+    // hardware even out the wavefronts' speeds (resident blocks end between 70 %
+    // and 100 % of a pass). 26-qubit stream: complex128 14.9 -> 14.0 ms, complex64
+    // 6.0 -> 5.5; with two tiles a block 14.3. From four rounds on: with 2.7 (24
+    // qubits complex128) the last round is too empty, 2.40 -> 2.47 ms.
+    if (NJ == 0 && ntiles >= 4 * cap) {
+        bpc = ntiles;
+    }
     if (bpc >= 8) {
         bpc = bpc / 8 * 8;
     }
