@@ -1074,7 +1074,15 @@ struct StepMeta {
     double coef = 0.0;
 };
 
+// Steps first .. first + count - 1 of a plan, taken in one launch.
+struct SlabGroup {
+    size_t first = 0, count = 0;
+    size_t off = 0; // their SlabSteps in PlanImage::mats
+    SlabLaunch L{};
+};
+
 struct PlanImage {
+    std::vector<SlabGroup> slabs;
     std::vector<unsigned char> ops;
     std::vector<TileBundle> bundles;
     std::vector<SegMeta> metas;
@@ -1851,6 +1859,74 @@ void split_sparse_passes(std::vector<Step> &steps, int n) {
 
 // Programs of every register-tile pass of a plan, uploaded as one blob.
 // R: register bits of the tile passes.
+// Groups consecutive two-state steps whose wires fit kSlabBits bits together
+// with the lowest ones (whole cache lines).
+void build_slabs(PlanImage &img, int n, int dtype) {
+    const int S = std::min(n, kSlabBits);
+    const uint64_t low = (uint64_t{1} << std::min(n, low_bits(dtype))) - 1;
+    // The partials of a launch lie side by side: at most 2^26 doubles for SEG_NJMAX observables.
+    const size_t most = std::min<size_t>(64, std::max<size_t>(2, (size_t{1} << 26) >> std::min(63, n - S + 3)));
+    auto takes = [&](size_t i) { return img.singles[i].ok && img.singles[i].L.m > 0 && img.singles[i].L.dim == 2; };
+    for (size_t i = 0; i < img.singles.size();) {
+        uint64_t bits = low;
+        size_t end = i;
+        for (; end < img.singles.size() && end - i < most && takes(end); end++) {
+            uint64_t with = bits;
+            for (int q = 0; q < img.singles[end].L.m; q++) {
+                with |= uint64_t{1} << img.singles[end].L.bits[q];
+            }
+            if (__builtin_popcountll(with) > S) {
+                break;
+            }
+            bits = with;
+        }
+        if (end - i < 2) {
+            i = std::max(end, i + 1);
+            continue;
+        }
+        for (int b = 0; __builtin_popcountll(bits) < S; b++) {
+            bits |= uint64_t{1} << b;
+        }
+        SlabGroup g;
+        g.first = i;
+        g.count = end - i;
+        g.L.n = n;
+        g.L.S = S;
+        g.L.nsteps = static_cast<int>(g.count);
+        for (int b = 0, q = 0; b < n; b++) {
+            if (bits >> b & 1) {
+                g.L.sb[q++] = b;
+            }
+        }
+        img.mats.resize((img.mats.size() + 255) & ~size_t{255}, 0);
+        g.off = img.mats.size();
+        for (; i < end; i++) {
+            const StepMeta &m = img.singles[i];
+            SlabStep p{};
+            p.off0 = m.L.off[0];
+            p.off1 = m.L.off[1];
+            p.mats = m.off;
+            p.m = m.L.m;
+            for (int q = 0; q < m.L.m; q++) {
+                p.lb[q] = static_cast<int32_t>(std::find(g.L.sb, g.L.sb + S, m.L.bits[q]) - g.L.sb);
+            }
+            p.trainable = m.L.trainable;
+            const auto *b = reinterpret_cast<const unsigned char *>(&p);
+            img.mats.insert(img.mats.end(), b, b + sizeof p);
+        }
+        img.slabs.push_back(g);
+    }
+}
+
+const SlabGroup *slab_of(const PlanImage &img, size_t i) {
+    for (const SlabGroup &g : img.slabs) {
+        if (i >= g.first && i < g.first + g.count) {
+            return &g;
+        }
+    }
+    return nullptr;
+}
+
 PlanImage build_image(const std::vector<Step> &steps, const State &s) {
     PlanImage img;
     if (s.dtype == PLK_C64) {
@@ -1864,6 +1940,7 @@ PlanImage build_image(const std::vector<Step> &steps, const State &s) {
             build_step(steps[i].single, s.n, img.mats, img.singles[i]);
         }
     }
+    build_slabs(img, s.n, s.dtype);
     img.progs.resize(steps.size());
     double norm = 1.0;
     for (size_t i = 0; i < steps.size(); i++) {
@@ -1932,6 +2009,12 @@ void append_signature(const PlanImage &img, std::vector<unsigned char> &sig) {
     const uint64_t sizes[5] = {img.ops.size(), img.bundles.size(), img.rt.size(), img.mats.size(),
                                img.entries.size()};
     put(sizes, sizeof sizes);
+    for (const SlabGroup &g : img.slabs) {
+        put(&g.first, sizeof g.first);
+        put(&g.count, sizeof g.count);
+        put(&g.off, sizeof g.off);
+        put(&g.L, sizeof g.L);
+    }
     for (const StepMeta &m : img.singles) {
         put(&m.ok, sizeof m.ok);
         put(&m.L, sizeof m.L);
@@ -2007,7 +2090,14 @@ void apply_single(Device &dev, const State &s, const CompiledOp &op);
 // unless a step is a single op outside the fused kernels).
 void enqueue_forward(Device &dev, const State &s, const std::vector<Step> &steps,
                      const PlanImage &img, const PlanPlace &pl) {
+    size_t next_slab = 0;
     for (size_t i = 0; i < steps.size(); i++) {
+        if (next_slab < img.slabs.size() && img.slabs[next_slab].first == i) {
+            const SlabGroup &g = img.slabs[next_slab++];
+            launch_slab_steps(dev, s, nullptr, pl.mats, pl.mats + g.off, g.L, nullptr);
+            i += g.count - 1;
+            continue;
+        }
         if (steps[i].tiled && steps[i].pass.rt) {
             RtLaunch L = img.progs[i].L;
             L.nj = 0;
@@ -2356,6 +2446,9 @@ SweepParts place_partials(Device &dev, const std::vector<Step> &steps, PlanImage
                           size_t n_obs, bool alt) {
     SweepParts sp;
     sp.steps.resize(steps.size());
+    if (n_obs > static_cast<size_t>(SEG_NJMAX)) {
+        img.slabs.clear(); // several chunks read phi before the last one writes it
+    }
     size_t used = 0, first = 0;
     auto flush = [&](size_t i) {
         if (img.entries.size() > first) {
@@ -2419,6 +2512,30 @@ SweepParts place_partials(Device &dev, const std::vector<Step> &steps, PlanImage
                 ci += L.nc;
                 sp.steps[i].push_back(pl);
             }
+        } else if (const SlabGroup *g = slab_of(img, i)) {
+            // All steps of the launch keep their partials until it has run.
+            const StepMeta &m = img.singles[i];
+            const size_t slabs = size_t{1} << (g->L.n - g->L.S);
+            if (i == g->first && used + g->count * n_obs * slabs > kPartialsMax && used > 0) {
+                flush(i - 1);
+            }
+            PartLaunch pl;
+            pl.step = m.L;
+            pl.step.nj = static_cast<int>(n_obs);
+            pl.width = static_cast<int>(n_obs);
+            if (m.L.trainable) {
+                pl.offset = used;
+                used += n_obs * slabs;
+                sp.doubles = std::max(sp.doubles, used);
+                const uint64_t part = pl.offset;
+                std::memcpy(img.mats.data() + g->off + (i - g->first) * sizeof(SlabStep) + offsetof(SlabStep, part),
+                            &part, sizeof part);
+                RtEntry e = entry(pl, static_cast<int>(slabs), m.col);
+                e.row[0] = 0;
+                e.m[0] = m.coef;
+                img.entries.push_back(e);
+            }
+            sp.steps[i].push_back(pl);
         } else if (!st.fused && !st.tiled && img.singles[i].ok) {
             const StepMeta &m = img.singles[i];
             size_t j0 = 0;
@@ -2462,6 +2579,14 @@ bool enqueue_reverse_step(Device &dev, PhiPair &phi, void *const *hptr, size_t n
                           size_t n_tp, const Step &st, const PlanImage &img, size_t i,
                           const PlanPlace &pl, const SweepParts &parts, double *d_jac) {
     const State &lambda = phi.cur;
+    if (const SlabGroup *g = slab_of(img, i)) {
+        if (g->first == i) {
+            SlabLaunch L = g->L;
+            L.nj = static_cast<int>(n_obs);
+            launch_slab_steps(dev, lambda, hptr, pl.mats, pl.mats + g->off, L, dev.parts);
+        }
+        return true;
+    }
     if (st.fused) {
         const SegMeta &m = img.metas[i];
         const int njmax = std::min(SEG_NJMAX, seg_max_nj(lambda.dtype, m.L.K));

@@ -464,6 +464,25 @@ int step_blocks(const Device &dev, const StepLaunch &L);
 void launch_step(Device &dev, const State &phi, void *const *h_ptrs, const void *d_mats,
                  const StepLaunch &L, double *partials);
 
+// Consecutive two-state steps in one launch (see slab_steps_kernel).
+constexpr int kSlabBits = 12;
+struct SlabStep {
+    uint64_t off0, off1; // state offsets of the step's two states
+    uint64_t mats;       // U and G, bytes from the matrices' start
+    uint64_t part;       // its partials [nj][slabs], doubles from the partials' start
+    int32_t m;           // wires
+    int32_t lb[STEP_MMAX]; // their slab positions, ascending
+    int32_t trainable;
+    int32_t pad[2];
+};
+static_assert(sizeof(SlabStep) == 64, "SlabStep layout");
+struct SlabLaunch {
+    int n, S, nj, nsteps;
+    int sb[kSlabBits]; // the slab's state bits, ascending
+};
+void launch_slab_steps(Device &dev, const State &phi, void *const *h_ptrs, const unsigned char *d_mats,
+                       const unsigned char *d_steps, const SlabLaunch &L, double *partials);
+
 // One variant per precision (float / double) and chunk 0..RT_NJMAX, each
 // compiled from kernels_rtile.hip as an object of its own.
 template <typename T, int NJ> int rtile_blocks_t(const Device &dev, const RtLaunch &L, int nc);
