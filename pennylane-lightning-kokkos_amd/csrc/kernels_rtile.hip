@@ -63,8 +63,9 @@ template <typename T> struct RtPtrs {
     Cx<T> *p[RT_OBS_MAX];
 };
 
-template <typename T, int NJ, int R>
-__global__ void __launch_bounds__(64, (rt_waves<T, NJ, R>()))
+// C: precision of the program and of the registers.
+template <typename T, int NJ, int R, typename C>
+__global__ void __launch_bounds__(64, (rt_waves<C, NJ, R>()))
     rtile_kernel(Cx<T> *phi, Cx<T> *phi_out, RtPtrs<T> hp, const unsigned char *__restrict__ prog_g,
                  RtLaunch L, double *__restrict__ partials) {
     constexpr int A = 1 << R;
@@ -111,28 +112,29 @@ __global__ void __launch_bounds__(64, (rt_waves<T, NJ, R>()))
     vin *= sizeof(Cx<T>);
     vout *= sizeof(Cx<T>);
     const uint64_t ntiles = uint64_t{1} << (L.n - L.T);
-    const Ins<T> first = fetch<T>(prog, 0);
+    const Ins<C> first = fetch<C>(prog, 0);
     for (uint64_t g = b; g < ntiles; g += bpc) {
         uint64_t base = g;
         for (int q = 0; q < L.T; q++) {
             base = insert_zero(base, L.tb[q]);
         }
-        Cx<T> v[NS][A];
+        Cx<C> v[NS][A];
 #pragma unroll
         for (int s = 0; s < NS; s++) {
             if (s > njc) {
 #pragma unroll
                 for (int k = 0; k < A; k++) {
-                    v[s][k] = Cx<T>{T(0), T(0)};
+                    v[s][k] = Cx<C>{C(0), C(0)};
                 }
                 continue;
             }
 #pragma unroll
             for (int k = 0; k < A; k++) {
-                v[s][k] = ldo(sp[s], base * sizeof(Cx<T>) + slot_off<T, R>(L.reg_in, k) + vin);
+                const Cx<T> x = ldo(sp[s], base * sizeof(Cx<T>) + slot_off<T, R>(L.reg_in, k) + vin);
+                v[s][k] = Cx<C>{static_cast<C>(x.r), static_cast<C>(x.i)};
             }
         }
-        run_program<T, NS, R>(v, first, prog, L.ninstr, lacc, dummy, lane, base);
+        run_program<C, NS, R>(v, first, prog, L.ninstr, lacc, dummy, lane, base);
 #pragma unroll
         for (int s = 0; s < NS; s++) {
             if ((s == 0 && !writes_phi) || s > njc) {
@@ -141,7 +143,8 @@ __global__ void __launch_bounds__(64, (rt_waves<T, NJ, R>()))
             Cx<T> *dst = s == 0 ? phi_out : sp[s];
 #pragma unroll
             for (int k = 0; k < A; k++) {
-                sto(dst, base * sizeof(Cx<T>) + slot_off<T, R>(L.reg_out, k) + vout, v[s][k]);
+                sto(dst, base * sizeof(Cx<T>) + slot_off<T, R>(L.reg_out, k) + vout,
+                    Cx<T>{static_cast<T>(v[s][k].r), static_cast<T>(v[s][k].i)});
             }
         }
     }
@@ -166,19 +169,25 @@ __global__ void __launch_bounds__(64, (rt_waves<T, NJ, R>()))
 
 } // namespace
 
-// f(R) for the launch's register bits.
-template <typename T, int NJ, int R = rt_reg_min<T>(NJ), typename F> void with_reg(int r, F &&f) {
+// f(R, C) for the launch's register bits and its program's precision.
+template <typename T, int NJ, int R = rt_reg_min<T>(NJ), typename F> void with_reg(const RtLaunch &L, F &&f) {
     if constexpr (R < rt_reg_max<T>(NJ)) {
-        if (r != R) {
-            with_reg<T, NJ, R + 1>(r, f);
+        if (L.R != R) {
+            with_reg<T, NJ, R + 1>(L, f);
             return;
         }
     }
-    f(IC<R>{});
+    if constexpr (NJ == 0) {
+        if (L.wide) {
+            f(IC<R>{}, double{});
+            return;
+        }
+    }
+    f(IC<R>{}, T{});
 }
 
-template <typename T, int NJ, int R> int blocks_per_chunk(const Device &dev, const RtLaunch &L, int nc) {
-    const void *kfn = reinterpret_cast<const void *>(&rtile_kernel<T, NJ, R>);
+template <typename T, int NJ, int R, typename C> int blocks_per_chunk(const Device &dev, const RtLaunch &L, int nc) {
+    const void *kfn = reinterpret_cast<const void *>(&rtile_kernel<T, NJ, R, C>);
     const size_t lds = rt_lds_bytes(NJ, L.nslots);
     static int per_cu[RT_SLOTS_MAX + 1] = {}; // by slots: the kernel's LDS follows from them
     int &nb = per_cu[NJ > 0 ? L.nslots : 0];
@@ -207,7 +216,9 @@ template <typename T, int NJ, int R> int blocks_per_chunk(const Device &dev, con
 // groups of 8 (one per XCD) when there are enough.
 template <typename T, int NJ> int rtile_blocks_t(const Device &dev, const RtLaunch &L, int nc) {
     int blocks = 0;
-    with_reg<T, NJ>(L.R, [&](auto R) { blocks = blocks_per_chunk<T, NJ, decltype(R)::value>(dev, L, nc); });
+    with_reg<T, NJ>(L, [&](auto R, auto C) {
+        blocks = blocks_per_chunk<T, NJ, decltype(R)::value, decltype(C)>(dev, L, nc);
+    });
     return blocks;
 }
 
@@ -229,8 +240,8 @@ void rtile_launch_t(Device &dev, const State &phi, void *phi_out, void *const *h
     // state read and written once.
     const double bytes = (1.0 + L.write_phi + 2.0 * width) * static_cast<double>(phi.bytes());
     ProfScope prof(NJ > 0 ? "adjoint_rtile" : "apply_rtile", bytes, dev.stream);
-    with_reg<T, NJ>(L.R, [&](auto R) {
-        hipLaunchKernelGGL((rtile_kernel<T, NJ, decltype(R)::value>), dim3(grid), dim3(64),
+    with_reg<T, NJ>(L, [&](auto R, auto C) {
+        hipLaunchKernelGGL((rtile_kernel<T, NJ, decltype(R)::value, decltype(C)>), dim3(grid), dim3(64),
                            rt_lds_bytes(NJ, L.nslots), dev.stream, static_cast<Cx<T> *>(phi.d),
                            static_cast<Cx<T> *>(phi_out), hp, static_cast<const unsigned char *>(d_prog), L,
                            partials);

@@ -347,6 +347,7 @@ struct RtLaunch {
     int write_phi; // the last chunk writes the updated phi (to phi_out)
     int nc;        // observable chunks run side by side in this launch (>= 1)
     int nbig;      // the first nbig chunks hold nj states, the others nj - 1
+    int wide;      // the program is FP64 (a forward pass over a complex64 state may be)
     int xgroup;    // block ids taken in groups of xgroup (8: one per XCD) when mapping to chunks
     int tb[RT_TMAX];                   // tile bits, ascending global positions
     int reg_in[RT_RMAX], lane_in[RT_LANE_BITS];   // global bit of each slot at load

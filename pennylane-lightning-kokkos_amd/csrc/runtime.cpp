@@ -409,6 +409,9 @@ int rtile_blocks(const Device &dev, int dtype, const RtLaunch &L) {
 
 void launch_rtile(Device &dev, const State &phi, const State *phi_out, void *const *h_ptrs,
                   const void *d_prog, const RtLaunch &L, double *partials) {
+    if (L.wide != (phi.dtype == PLK_C128 ? 1 : 0) && !(L.wide == 1 && L.nj == 0)) {
+        raise(PLK_ERR_INVALID, "register-tile pass of another precision than the state's");
+    }
     if (L.R < rt_reg_min(phi.dtype, L.nj) || L.R > rt_reg_max(phi.dtype, L.nj) || L.T != L.R + RT_LANE_BITS || L.T > L.n || L.n != phi.n || L.nslots > RT_SLOTS_MAX || L.nj < 0 ||
         L.nc < 1 || L.nc * std::max(1, L.nj) > RT_OBS_MAX || (L.nc > 1 && L.nj == 0) || L.nbig < 0 ||
         L.nbig > L.nc || (L.nj == 1 && L.nbig < L.nc) || (L.nslots > 0 && partials == nullptr)) {
