@@ -32,12 +32,13 @@
 // In place the four-state kernel has 164 KB, of which a pass runs a part, and
 // 168 VGPRs (three waves per SIMD instead of two).
 //
-// Bound (24 qubits complex128, 9 observables, 37 passes of 26 gates): HBM and
-// FP64 issue together, 1.57 ms a pass = 3.4 TB/s of the in-place ceiling of
-// 5.2, vector issue 54 % busy, the waves waiting for memory 41 % of their time;
-// out of place with five mixed bits a pass: 1.74 ms and 50 passes. One state
-// (26-qubit gate stream): 0.52 ms a pass, 4.1 TB/s, 37 passes for 600 gates
-// where the three-register-bit tile took 66 passes of 0.47 ms.
+// Bound (24 qubits complex128, 9 observables, 29 passes of 33 gates, 1.61 ms a
+// pass = 3.3 TB/s of the in-place ceiling of 5.2): FP64 issue, busy 65 to 73 % at
+// the 2.0 GHz the card holds under this load, and memory, for which the waves
+// wait 30 % of their time; out of place with five mixed bits a pass it was 50
+// passes of 1.74 ms. One state (26-qubit stream of 600 gates, 32 amplitudes a
+// lane): 25 passes of 0.53 ms, 4.1 TB/s; with 16 amplitudes 29 passes of 0.53,
+// with 8 and no exchange below position 4, 66 of 0.47.
 //
 // The host fuses the one-wire gates that follow each other on a wire into one
 // 2x2 matrix. For trainable gates V_1, V_2, ... of such a run the derivative
