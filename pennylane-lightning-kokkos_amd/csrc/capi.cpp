@@ -236,6 +236,9 @@ struct PlanOp {
     double coef = 0.0;
     int32_t src = -1;       // index of the op in its OpsData
     bool adj = false;       // U was compiled with the inverse flag set
+    // Batch plans, runs with patched gates: the U kind and the Pauli parts that
+    // hold for every angle (see fix_form); -1: as the matrices are.
+    int ukind = -1, parts = -1;
 };
 
 // Parity ops/generators on <= 2 wires become dense diagonals so they fuse.
@@ -444,6 +447,9 @@ bool mixes_bit(const std::vector<cd> &M, int dim, int lb) {
 
 // Pauli parts the gates of a run need: bit 0 X, bit 1 Y, bit 2 Z.
 int run_parts(const PlanOp &p) {
+    if (p.parts >= 0) {
+        return p.parts;
+    }
     int parts = 0;
     for (const auto &t : p.run) {
         for (int k = 0; k < 3; k++) {
@@ -520,13 +526,83 @@ std::vector<PlanOp> fuse_runs(std::vector<PlanOp> &&ops) {
     return out;
 }
 
+// Whether a gate of a batch run is diagonal, whether it is real, and for each
+// Pauli P (X, Y, Z) the parts that M^dag P M may have, M the gate's matrix at
+// any angle.
+struct GateForm {
+    bool diag, real;
+    int reach[3];
+};
+
+GateForm gate_form(const RunGate &g) {
+    switch (g.g.gate) {
+    case BPG_RX:
+        return {false, false, {1, 6, 6}};
+    case BPG_RY:
+        return {false, true, {5, 2, 5}};
+    case BPG_RZ:
+    case BPG_PHASE:
+        return {true, false, {3, 3, 4}};
+    default:
+        break;
+    }
+    const std::vector<cd> &M = g.mat;
+    const std::vector<cd> Md = {std::conj(M[0]), std::conj(M[2]), std::conj(M[1]), std::conj(M[3])};
+    const std::vector<cd> P[3] = {{0.0, 1.0, 1.0, 0.0}, {0.0, -kI, kI, 0.0}, {1.0, 0.0, 0.0, -1.0}};
+    const cd none(0.0, 0.0);
+    GateForm f{M[1] == none && M[2] == none, true, {0, 0, 0}};
+    for (const cd &m : M) {
+        f.real = f.real && m.imag() == 0.0;
+    }
+    for (int k = 0; k < 3; k++) {
+        const std::vector<cd> W = mul2(Md, mul2(P[k], M));
+        f.reach[k] = (W[1] + W[2] != none ? 1 : 0) | (W[1] != W[2] ? 2 : 0) | (W[0] != W[3] ? 4 : 0);
+    }
+    return f;
+}
+
+// The kind of a batch run's matrix and its Pauli parts, from the kinds of its
+// gates. A plan serves every angle of its patched gates, so neither may come
+// from the product at some angles: RX(a) Z RX(b) is diagonal at a = b only, and
+// RY(a) RY(b)^dag the identity.
+void fix_form(PlanOp &p) {
+    bool patched = false;
+    for (const RunGate &g : p.gates) {
+        patched = patched || g.g.gate != BPG_CONST;
+    }
+    if (!patched) {
+        return;
+    }
+    bool diag = true, real = true;
+    int parts = 0;
+    int reach[3] = {1, 2, 4}; // of V^dag P V, V the gates so far
+    for (const RunGate &g : p.gates) {
+        const GateForm f = gate_form(g);
+        if (g.g.coef != 0.0) { // its generator: X, Y, else Z
+            parts |= reach[g.g.gate == BPG_RX ? 0 : g.g.gate == BPG_RY ? 1 : 2];
+        }
+        int next[3] = {0, 0, 0};
+        for (int k = 0; k < 3; k++) {
+            for (int q = 0; q < 3; q++) {
+                next[k] |= (f.reach[k] >> q & 1) ? reach[q] : 0;
+            }
+        }
+        std::copy(next, next + 3, reach);
+        diag = diag && f.diag;
+        real = real && f.real;
+    }
+    p.ukind = diag ? U_DIAG : real ? U_REAL : U_DENSE;
+    p.parts = p.run.empty() ? -1 : parts;
+}
+
 // Global state bits an op mixes (its U or, when trainable, its generator has
 // an entry between indices that differ in the bit).
 uint64_t mixing_mask(const PlanOp &p, int n) {
     const int m = static_cast<int>(p.U.wires.size());
     uint64_t mask = 0;
-    if (!p.run.empty()) {
-        const bool mixes = mixes_bit(p.U.mat, 2, 0) || run_parts(p) != 4;
+    if (!p.run.empty() || p.ukind >= 0) {
+        const bool mixes = (p.ukind >= 0 ? p.ukind != U_DIAG : mixes_bit(p.U.mat, 2, 0)) ||
+                           (!p.run.empty() && run_parts(p) != 4);
         return mixes ? uint64_t{1} << (n - 1 - static_cast<int>(p.U.wires[0])) : 0;
     }
     for (int k = 0; k < m; k++) {
@@ -575,6 +651,9 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
         }
     } else {
         all = fuse_runs(std::move(ops_in));
+        for (PlanOp &p : all) {
+            fix_form(p);
+        }
     }
     // State bits (< 64) an op acts on, and of these the ones its pass needs in
     // the tile.
@@ -1382,26 +1461,23 @@ bool is_x2(const std::vector<cd> &B) {
     return B[0] == cd(0, 0) && B[3] == cd(0, 0) && B[1] == cd(1, 0) && B[2] == cd(1, 0);
 }
 
-// Encodes the U part of a one-register-bit op; returns its reals.
-std::vector<double> rt_encode_u1(RtInstr &in, const std::vector<cd> &U) {
-    if (is_ident2(U)) {
-        in.ukind = U_NONE;
-        return {};
+// Encodes the U part of a one-register-bit op; returns its reals. ukind: the
+// kind of a batch run (its reals are patched), -1: the matrix's.
+std::vector<double> rt_encode_u1(RtInstr &in, const std::vector<cd> &U, int ukind) {
+    if (ukind < 0) {
+        ukind = is_ident2(U) ? U_NONE : is_diag2(U) ? U_DIAG : is_x2(U) ? U_SWAP : is_real(U) ? U_REAL : U_DENSE;
     }
-    if (is_diag2(U)) {
-        in.ukind = U_DIAG;
+    in.ukind = static_cast<int8_t>(ukind);
+    switch (ukind) {
+    case U_DIAG:
         return cplx({U[0], U[3]});
-    }
-    if (is_x2(U)) {
-        in.ukind = U_SWAP;
+    case U_REAL:
+        return {U[0].real(), U[1].real(), U[2].real(), U[3].real()};
+    case U_DENSE:
+        return cplx(U);
+    default:
         return {};
     }
-    if (is_real(U)) {
-        in.ukind = U_REAL;
-        return {U[0].real(), U[1].real(), U[2].real(), U[3].real()};
-    }
-    in.ukind = U_DENSE;
-    return cplx(U);
 }
 
 // complex64 programs round every matrix to FP32, which changes the norm of
@@ -1639,7 +1715,7 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, int keep, std::vector<u
             if (r >= 0) {
                 in.code = RT_REG1;
                 in.a = static_cast<int8_t>(r);
-                u = rt_encode_u1(in, p.U.mat);
+                u = rt_encode_u1(in, p.U.mat, p.ukind);
                 if (sizeof(T) == 4 && !u.empty() && !patched) {
                     u = keep_norm(std::move(u), 2, norm);
                 }
@@ -2343,13 +2419,12 @@ void note_op(OpsData &ops, Hasher &H, size_t i) {
 
 
 // The whole op list, compiled (applyOperations, AdjointDiffKokkos.hpp:213-226).
-std::vector<PlanOp> forward_ops(const OpsData &ops, int n,
-                                const std::vector<std::vector<double>> *params = nullptr) {
+std::vector<PlanOp> forward_ops(const OpsData &ops, int n) {
     std::vector<PlanOp> v;
     v.reserve(ops.names.size());
     for (size_t i = 0; i < ops.names.size(); i++) {
         PlanOp p;
-        p.U = compile_op(ops.names[i], ops.wires[i], ops.inverses[i], params ? (*params)[i] : ops.params[i],
+        p.U = compile_op(ops.names[i], ops.wires[i], ops.inverses[i], ops.params[i],
                          ops.matrices[i], n);
         v.push_back(std::move(p));
     }
@@ -2375,9 +2450,7 @@ std::vector<Step> forward_plan(const Device &dev, std::vector<PlanOp> &&v, int n
 // after the last trainable one, in reverse order, each trainable op carrying
 // its generator, Jacobian column and coefficient -2 s (inverse ? -1 : 1).
 // StatePrep / BasisState are skipped; ops with several parameters abort.
-// params: values used instead of the list's own (batch plans).
-std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &tp, int n,
-                                const std::vector<std::vector<double>> *params = nullptr) {
+std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &tp, int n) {
     const size_t n_tp = tp.size();
     std::vector<PlanOp> rev;
     size_t trainable_number = n_tp - 1;
@@ -2397,7 +2470,7 @@ std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &t
             break;
         }
         PlanOp p;
-        p.U = compile_op(ops.names[o], ops.wires[o], !ops.inverses[o], params ? (*params)[o] : ops.params[o],
+        p.U = compile_op(ops.names[o], ops.wires[o], !ops.inverses[o], ops.params[o],
                          ops.matrices[o], n);
         p.src = static_cast<int32_t>(o);
         p.adj = !ops.inverses[o];
@@ -3328,18 +3401,11 @@ void plan_batch_circuit(BatchPart &bp, const BatchInput &in, int dtype) {
         bp.t.terms.push_back({static_cast<uint32_t>(t.x), static_cast<uint32_t>(t.zy), t.coeff.real(),
                               t.coeff.imag()});
     }
-    // The plan must hold for every angle of a patched gate, so those are
-    // planned at generic angles: the structure of a run's matrix and of its
-    // Pauli parts is then the one it has for all but special angles.
-    std::vector<std::vector<double>> params = ops.params;
     std::vector<int32_t> pidx(ops.names.size(), -1);
     int64_t np = bp.nparams;
     for (size_t i = 0; i < ops.names.size(); i++) {
         if (!ops.params[i].empty()) {
             pidx[i] = static_cast<int32_t>(np++);
-            if (patch_gate_of(ops, i) != BPG_NONE) {
-                params[i][0] = 0.7 + 0.4 * static_cast<double>(i % 5);
-            }
         }
     }
     if (np > INT32_MAX) {
@@ -3362,11 +3428,11 @@ void plan_batch_circuit(BatchPart &bp, const BatchInput &in, int dtype) {
         }
         p.gates = {std::move(g)};
     };
-    std::vector<PlanOp> rev = reverse_ops(ops, in.tp, n, &params);
+    std::vector<PlanOp> rev = reverse_ops(ops, in.tp, n);
     for (auto &p : rev) {
         mark(p, static_cast<size_t>(p.src), p.adj);
     }
-    std::vector<PlanOp> fwd = forward_ops(ops, n, &params);
+    std::vector<PlanOp> fwd = forward_ops(ops, n);
     for (size_t i = 0; i < fwd.size(); i++) {
         mark(fwd[i], i, ops.inverses[i]);
     }
