@@ -1484,17 +1484,25 @@ std::vector<double> rt_encode_u1(RtInstr &in, const std::vector<cd> &U, int ukin
 // the whole state by a few 1e-8 per gate: the one rounding error that does not
 // average out over the amplitudes (its random walk over a circuit's gates is
 // the bulk of an FP32 expectation value's error). `norm` is the product of
-// these factors so far; a one-wire matrix is divided by it before it is
-// rounded, so the product stays within one rounding of 1.
-std::vector<double> keep_norm(std::vector<double> u, int dim, double &norm) {
-    double sum = 0.0;
-    for (double &x : u) {
-        x /= norm;
-        const double r = static_cast<double>(static_cast<float>(x));
-        sum += r * r;
+// these factors so far, the norms of the rounded matrices by those of the given
+// ones (which need not be unitary); a one-wire matrix is divided by it before it
+// is rounded, so the product stays within one rounding of 1. A matrix of zeros or
+// of numbers that FP32 does not hold is left as it is.
+std::vector<double> keep_norm(const std::vector<double> &u, double &norm) {
+    std::vector<double> v = u;
+    double given = 0.0, rounded = 0.0;
+    for (size_t k = 0; k < u.size(); k++) {
+        v[k] = u[k] / norm;
+        const double r = static_cast<double>(static_cast<float>(v[k]));
+        given += u[k] * u[k];
+        rounded += r * r;
     }
-    norm *= std::sqrt(sum / dim);
-    return u;
+    const double next = norm * std::sqrt(rounded / given);
+    if (!(std::abs(next - 1.0) < 1e-6)) {
+        return u;
+    }
+    norm = next;
+    return v;
 }
 
 // Index bits that sit on lanes at load and store (complex128: bit 0, complex64:
@@ -1717,7 +1725,7 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, int keep, std::vector<u
                 in.a = static_cast<int8_t>(r);
                 u = rt_encode_u1(in, p.U.mat, p.ukind);
                 if (sizeof(T) == 4 && !u.empty() && !patched) {
-                    u = keep_norm(std::move(u), 2, norm);
+                    u = keep_norm(u, norm);
                 }
                 if (G) {
                     const auto &g = *G;
@@ -1734,7 +1742,7 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, int keep, std::vector<u
                 in.s0 = static_cast<int8_t>(sel_of(gbits[i][0]));
                 u = cplx({p.U.mat[0], p.U.mat[3]});
                 if (sizeof(T) == 4 && !patched) {
-                    u = keep_norm(std::move(u), 2, norm);
+                    u = keep_norm(u, norm);
                 }
                 if (G) {
                     in.goff = b.put({(*G)[0].real(), (*G)[3].real()});
