@@ -236,6 +236,7 @@ struct PlanOp {
     double coef = 0.0;
     int32_t src = -1;       // index of the op in its OpsData
     bool adj = false;       // U was compiled with the inverse flag set
+    bool skew = false;      // reverse sweeps: U is not unitary (see Blocked)
     // Batch plans, runs with patched gates: the U kind and the Pauli parts that
     // hold for every angle (see fix_form); -1: as the matrices are.
     int ukind = -1, parts = -1;
@@ -379,7 +380,7 @@ void make_bundles(Pass &ps, std::vector<PlanOp> &&ops, int n) {
     std::vector<int> rem(all.size());
     for (size_t i = 0; i < all.size(); i++) {
         uint32_t ob = 0;
-        uint64_t wm = 0;
+        uint64_t wm = all[i].skew ? ~uint64_t{0} : 0;
         for (auto w : all[i].U.wires) {
             ob |= 1u << pos[n - 1 - static_cast<int>(w)];
             wm |= uint64_t{1} << w;
@@ -477,7 +478,9 @@ std::vector<cd> mul2(const std::vector<cd> &A, const std::vector<cd> &B) {
 // Fuses the one-wire ops that follow each other on a wire into one 2x2
 // matrix, at the place of the first (ops on other wires commute with them).
 // Trainable ops join when their generator is traceless (X, Y, Z and real
-// combinations of them); anything else on the wire ends the run.
+// combinations of them); anything else on the wire ends the run. A skew op of a
+// reverse sweep ends every run, and no trainable op joins the one it begins
+// (V^dag G V would have a trace).
 std::vector<PlanOp> fuse_runs(std::vector<PlanOp> &&ops) {
     std::vector<PlanOp> out;
     out.reserve(ops.size());
@@ -492,6 +495,9 @@ std::vector<PlanOp> fuse_runs(std::vector<PlanOp> &&ops) {
             one = p.G.kind == OpKind::Dense && p.G.wires == p.U.wires && p.G.mat[0] + p.G.mat[3] == cd(0.0, 0.0);
         }
         if (!one) {
+            if (p.skew) {
+                std::fill(open.begin(), open.end(), -1);
+            }
             for (auto w : p.U.wires) {
                 open[w] = -1;
             }
@@ -499,7 +505,10 @@ std::vector<PlanOp> fuse_runs(std::vector<PlanOp> &&ops) {
             continue;
         }
         const size_t w = p.U.wires[0];
-        const bool first = open[w] < 0;
+        if (p.skew) {
+            std::fill(open.begin(), open.end(), -1);
+        }
+        const bool first = open[w] < 0 || (p.trainable && out[open[w]].skew);
         if (p.trainable) {
             std::vector<cd> g = p.G.mat;
             if (!first) {
@@ -614,15 +623,29 @@ uint64_t mixing_mask(const PlanOp &p, int n) {
     return mask;
 }
 
+// The state bits an operation acts on and those it mixes; whether it leaves a
+// derivative, and whether it is a matrix that is not unitary.
+struct Place {
+    uint64_t on = 0, mix = 0;
+    bool trainable = false, skew = false;
+};
+
 // Operations skipped so far: the bits they mix, and the bits they act on,
 // which stop an operation that mixes them. Operations that share only bits
-// neither mixes commute.
+// neither mixes commute. A trainable and a skew operation never change places:
+// the derivative Im<h|G phi> is the same before and after a unitary on other
+// wires, but not a matrix A, which makes it Im<h|A^dag A G phi>.
 struct Blocked {
     uint64_t mixed = 0, selected = 0;
-    bool stops(uint64_t on, uint64_t mix) const { return ((mixed & on) | (selected & mix)) != 0; }
-    void add(uint64_t on, uint64_t mix) {
-        mixed |= mix;
-        selected |= on;
+    bool trainable = false, skew = false;
+    bool stops(const Place &p) const {
+        return ((mixed & p.on) | (selected & p.mix)) != 0 || (trainable && p.skew) || (skew && p.trainable);
+    }
+    void add(const Place &p) {
+        mixed |= p.mix;
+        selected |= p.on;
+        trainable = trainable || p.trainable;
+        skew = skew || p.skew;
     }
 };
 
@@ -657,8 +680,7 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
     }
     // State bits (< 64) an op acts on, and of these the ones its pass needs in
     // the tile.
-    struct Item {
-        uint64_t on, mix;
+    struct Item : Place {
         int index, sums;
         bool fus;
     };
@@ -667,7 +689,8 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
     for (size_t i = 0; i < all.size(); i++) {
         Item &it = rem[i];
         it.index = static_cast<int>(i);
-        it.on = 0;
+        it.trainable = all[i].trainable;
+        it.skew = all[i].skew;
         for (auto w : all[i].U.wires) {
             it.on |= uint64_t{1} << (n - 1 - static_cast<int>(w));
         }
@@ -684,11 +707,11 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
         const size_t end = std::min(rem.size(), kLookahead);
         for (size_t k = 0; k < end && rem[k].fus && (blocked.mixed & every) != every; k++) {
             const Item &it = rem[k];
-            if ((it.mix & ~bits) == 0 && !blocked.stops(it.on, it.mix) && taken < kPassMaxOps && sums + it.sums <= pmax) {
+            if ((it.mix & ~bits) == 0 && !blocked.stops(it) && taken < kPassMaxOps && sums + it.sums <= pmax) {
                 taken++;
                 sums += it.sums;
             } else {
-                blocked.add(it.on, it.mix);
+                blocked.add(it);
             }
         }
         return taken;
@@ -721,13 +744,13 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
             for (; k < rem.size() && rem[k].fus && k < kLookahead; k++) {
                 const Item &it = rem[k];
                 const uint64_t nb = bits | it.mix;
-                if ((grow ? __builtin_popcountll(nb) <= T : nb == bits) && !blocked.stops(it.on, it.mix) &&
+                if ((grow ? __builtin_popcountll(nb) <= T : nb == bits) && !blocked.stops(it) &&
                     taken.size() < kPassMaxOps && nslots + it.sums <= pmax) {
                     bits = nb;
                     nslots += it.sums;
                     taken.push_back(it.index);
                 } else {
-                    blocked.add(it.on, it.mix);
+                    blocked.add(it);
                     rest.push_back(it);
                 }
             }
@@ -1530,14 +1553,16 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, int keep, std::vector<u
     }
     const size_t nops = ps.ops.size();
     std::vector<std::vector<int>> gbits(nops), mix(nops);
-    std::vector<uint64_t> on(nops, 0), mixes(nops);
+    std::vector<Place> place(nops);
     for (size_t i = 0; i < nops; i++) {
         const PlanOp &p = ps.ops[i];
-        const uint64_t mm = mixes[i] = mixing_mask(p, n);
+        const uint64_t mm = place[i].mix = mixing_mask(p, n);
+        place[i].trainable = p.trainable;
+        place[i].skew = p.skew;
         for (auto w : p.U.wires) {
             const int gb = n - 1 - static_cast<int>(w);
             gbits[i].push_back(gb);
-            on[i] |= uint64_t{1} << gb;
+            place[i].on |= uint64_t{1} << gb;
             if (mm >> gb & 1) {
                 mix[i].push_back(gb);
             }
@@ -1651,12 +1676,12 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, int keep, std::vector<u
         size_t at = 0;
         for (; scan < left.size(); scan++) {
             const size_t k = left[scan];
-            if (!blocked.stops(on[k], mixes[k]) &&
+            if (!blocked.stops(place[k]) &&
                 std::all_of(mix[k].begin(), mix[k].end(), [&](int q) { return reg_of(q) >= 0; })) {
                 at = scan;
                 break;
             }
-            blocked.add(on[k], mixes[k]);
+            blocked.add(place[k]);
         }
         const bool stuck = scan == left.size();
         const size_t i = left[at];
@@ -1681,7 +1706,7 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, int keep, std::vector<u
                     continue;
                 }
                 size_t use = 0;
-                while (use < left.size() && !(mixes[left[use]] >> reg[r] & 1)) {
+                while (use < left.size() && !(place[left[use]].mix >> reg[r] & 1)) {
                     use++;
                 }
                 if (victim < 0 || use > far) {
@@ -2454,11 +2479,30 @@ std::vector<Step> forward_plan(const Device &dev, std::vector<PlanOp> &&v, int n
     return plan_steps(std::move(v));
 }
 
+bool is_unitary(const std::vector<cd> &M, double tol) {
+    const size_t dim = M.size() == 4 ? 2 : 4;
+    for (size_t a = 0; a < dim; a++) {
+        for (size_t b = 0; b <= a; b++) {
+            cd s = a == b ? -1.0 : 0.0;
+            for (size_t r = 0; r < dim; r++) {
+                s += std::conj(M[r * dim + a]) * M[r * dim + b];
+            }
+            if (!(std::abs(s) <= tol)) {
+                return false;
+            }
+        }
+    }
+    return true;
+}
+
 // The reverse walk of AdjointDiffKokkos.hpp:432-470: U^dagger of every op
 // after the last trainable one, in reverse order, each trainable op carrying
 // its generator, Jacobian column and coefficient -2 s (inverse ? -1 : 1).
 // StatePrep / BasisState are skipped; ops with several parameters abort.
-std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &tp, int n) {
+// unitary: largest entry of U^dag U - 1 at which an explicit matrix still counts
+// as unitary (a matrix that a complex64 program gives in its own precision).
+std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &tp, int n, int dtype) {
+    const double unitary = dtype == PLK_C64 ? 1e-6 : 1e-12;
     const size_t n_tp = tp.size();
     std::vector<PlanOp> rev;
     size_t trainable_number = n_tp - 1;
@@ -2482,6 +2526,8 @@ std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &t
                          ops.matrices[o], n);
         p.src = static_cast<int32_t>(o);
         p.adj = !ops.inverses[o];
+        p.skew = !is_named_gate(ops.names[o]) && p.U.kind == OpKind::Dense && p.U.wires.size() <= 2 &&
+                 !is_unitary(p.U.mat, unitary);
         if (!ops.params[o].empty()) {
             if (current_param_idx == *tp_it) {
                 p.trainable = true;
@@ -3122,7 +3168,7 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
 
     // Reverse plan first: it validates the op list before any device work.
     std::unique_ptr<HostScope> plan_scope = std::make_unique<HostScope>("host_adjoint_plan");
-    std::vector<PlanOp> rev = reverse_ops(ops, tp, n);
+    std::vector<PlanOp> rev = reverse_ops(ops, tp, n, ref.dtype);
     if (n_obs == 0) {
         return;
     }
@@ -3436,7 +3482,7 @@ void plan_batch_circuit(BatchPart &bp, const BatchInput &in, int dtype) {
         }
         p.gates = {std::move(g)};
     };
-    std::vector<PlanOp> rev = reverse_ops(ops, in.tp, n);
+    std::vector<PlanOp> rev = reverse_ops(ops, in.tp, n, dtype);
     for (auto &p : rev) {
         mark(p, static_cast<size_t>(p.src), p.adj);
     }
