@@ -2405,9 +2405,10 @@ struct OpsData {
     size_t num_par_ops() const { return angles.size(); }
 };
 
-// Patched gate of an op: one-parameter rotations without an explicit matrix.
+// Patched gate of an op: the one-wire rotations and PhaseShift (a named gate
+// ignores an explicit matrix).
 int16_t patch_gate_of(const OpsData &ops, size_t i) {
-    if (ops.params[i].size() != 1 || !ops.matrices[i].empty()) {
+    if (ops.params[i].size() != 1) {
         return BPG_NONE;
     }
     const std::string &nm = ops.names[i];

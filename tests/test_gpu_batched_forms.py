@@ -60,3 +60,25 @@ def test_run_forms_hold_for_every_angle(capi, monkeypatch, kind, n, whole, dtype
             np.testing.assert_allclose(v, O.expval(psi, to_oracle(obs)), rtol=rtol, atol=atol)
             ref = O.adjoint_jacobian(O.zero_state(n), [to_oracle(obs)], o, tp, True)[0]
             np.testing.assert_allclose(row, ref, rtol=rtol, atol=atol)
+
+
+@pytest.mark.parametrize("dtype,rtol,atol", [(np.complex128, 1e-10, 1e-12), (np.complex64, 0.0, 1e-5)])
+@pytest.mark.parametrize("gate", ["RX", "RY", "RZ", "PhaseShift"])
+def test_named_gate_with_matrix(capi, gate, dtype, rtol, atol):
+    """A named gate is the gate whatever matrix its op carries, in a run with
+    other rotations too; two calls with other angles."""
+    n, rng = 4, np.random.default_rng(12)
+    names = ["Hadamard", gate, "RZ", "CNOT", "RY", gate]
+    wires = [[0], [0], [0], [0, 1], [1], [1]]
+    mats = [[], np.array([0, 1, 1, 0], dtype=np.complex128), [], [], [], np.array([1, 0, 0, 2], dtype=np.complex128)]
+    obs = ("ham", [0.7, 0.2], [("named", "PauliY", [0]), ("named", "PauliX", [1])])
+    for _ in range(2):
+        params = [[], [float(rng.uniform(0, 6))], [float(rng.uniform(0, 6))], [], [float(rng.uniform(0, 6))],
+                  [float(rng.uniform(0, 6))]]
+        ops = (names, params, wires, [False, True, False, False, False, False], mats)
+        values, rows = capi.adjoint_batched([n], [capi.Ops(*ops)], [to_capi(capi, obs)], [[0, 1, 2, 3]], dtype=dtype)
+        o = O.Ops(*ops)
+        np.testing.assert_allclose(values[0], O.expval(O.apply_ops(O.zero_state(n), o), to_oracle(obs)), rtol=rtol,
+                                   atol=atol)
+        np.testing.assert_allclose(rows[0], O.adjoint_jacobian(O.zero_state(n), [to_oracle(obs)], o, [0, 1, 2, 3], True)[0],
+                                   rtol=rtol, atol=atol)
