@@ -3515,55 +3515,71 @@ void plan_batch_circuit(BatchPart &bp, const BatchInput &in, int dtype) {
     bp.circuits.push_back(c);
 }
 
-struct Blob {
-    std::vector<unsigned char> bytes;
-    template <typename V> size_t add(const std::vector<V> &v) {
-        const size_t off = (bytes.size() + 255) & ~size_t{255};
-        bytes.resize(off + v.size() * sizeof(V));
-        if (!v.empty()) {
-            std::memcpy(bytes.data() + off, v.data(), v.size() * sizeof(V));
-        }
-        return off;
-    }
+// Where a part's tables begin among the batch's.
+struct BatchBase {
+    int32_t pass = 0, entry = 0, term = 0, run = 0, gate = 0, mat = 0, param = 0;
+    int64_t prog = 0, jac = 0;
 };
 
-// Appends src's circuits to dst, rebasing every index and offset.
-void merge_part(BatchPart &dst, BatchPart &&src) {
-    SweepTables &d = dst.t, &f = src.t;
-    const int pass0 = static_cast<int>(d.passes.size()), entry0 = static_cast<int>(d.entries.size());
-    const int term0 = static_cast<int>(d.terms.size()), gate0 = static_cast<int>(d.gates.size());
-    const int const0 = static_cast<int>(d.consts.size() / 8);
-    d.blob.resize((d.blob.size() + 255) & ~size_t{255}, 0);
-    const int64_t blob0 = static_cast<int64_t>(d.blob.size());
-    for (SweepPass p : f.passes) {
-        p.prog += blob0;
-        p.entry_first += entry0;
-        d.passes.push_back(p);
-    }
-    for (BatchRun r : f.runs) {
-        r.ins += blob0;
-        r.first += gate0;
-        r.entry += r.entry < 0 ? 0 : entry0;
-        d.runs.push_back(r);
-    }
-    for (BatchGate g : f.gates) {
-        g.param += g.gate == BPG_CONST ? const0 : static_cast<int32_t>(dst.nparams);
-        d.gates.push_back(g);
-    }
-    for (BatchPlanned c : src.circuits) {
-        c.fwd.first += pass0;
-        c.rev.first += pass0;
-        c.term_first += term0;
-        c.jac += dst.jac_len;
-        dst.circuits.push_back(c);
-    }
-    d.blob.insert(d.blob.end(), f.blob.begin(), f.blob.end());
-    d.entries.insert(d.entries.end(), f.entries.begin(), f.entries.end());
-    d.terms.insert(d.terms.end(), f.terms.begin(), f.terms.end());
-    d.consts.insert(d.consts.end(), f.consts.begin(), f.consts.end());
-    dst.jac_len += src.jac_len;
-    dst.nparams += src.nparams;
+BatchBase after(const BatchBase &b, const BatchPart &p) {
+    auto sum = [](int32_t x, int64_t y) {
+        if (x + y > INT32_MAX) {
+            raise(PLK_ERR_UNSUPPORTED, "batch tables exceed 2^31 rows");
+        }
+        return static_cast<int32_t>(x + y);
+    };
+    BatchBase n;
+    n.pass = sum(b.pass, static_cast<int64_t>(p.t.passes.size()));
+    n.entry = sum(b.entry, static_cast<int64_t>(p.t.entries.size()));
+    n.term = sum(b.term, static_cast<int64_t>(p.t.terms.size()));
+    n.run = sum(b.run, static_cast<int64_t>(p.t.runs.size()));
+    n.gate = sum(b.gate, static_cast<int64_t>(p.t.gates.size()));
+    n.mat = sum(b.mat, static_cast<int64_t>(p.t.consts.size() / 8));
+    n.param = sum(b.param, p.nparams);
+    n.prog = (b.prog + static_cast<int64_t>(p.t.blob.size()) + 255) & ~int64_t{255};
+    n.jac = b.jac + p.jac_len;
+    return n;
 }
+
+// The batch's tables in one image, each part's written where it belongs with
+// its indices rebased.
+struct BatchImage {
+    size_t passes, entries, terms, runs, gates, consts, prog; // bytes from the image's start
+
+    void put(unsigned char *img, const BatchPart &part, const BatchBase &b) const {
+        const SweepTables &t = part.t;
+        auto *P = reinterpret_cast<SweepPass *>(img + passes) + b.pass;
+        for (SweepPass p : t.passes) {
+            p.prog += b.prog;
+            p.entry_first += b.entry;
+            *P++ = p;
+        }
+        auto *R = reinterpret_cast<BatchRun *>(img + runs) + b.run;
+        for (BatchRun r : t.runs) {
+            r.ins += b.prog;
+            r.first += b.gate;
+            r.entry += r.entry < 0 ? 0 : b.entry;
+            *R++ = r;
+        }
+        auto *G = reinterpret_cast<BatchGate *>(img + gates) + b.gate;
+        for (BatchGate g : t.gates) {
+            g.param += g.gate == BPG_CONST ? b.mat : b.param;
+            *G++ = g;
+        }
+        auto copy = [&](size_t at, const void *src, size_t bytes) {
+            if (bytes > 0) {
+                std::memcpy(img + at, src, bytes);
+            }
+        };
+        copy(entries + static_cast<size_t>(b.entry) * sizeof(SweepEntry), t.entries.data(),
+             t.entries.size() * sizeof(SweepEntry));
+        copy(terms + static_cast<size_t>(b.term) * sizeof(SweepTerm), t.terms.data(),
+             t.terms.size() * sizeof(SweepTerm));
+        copy(consts + static_cast<size_t>(b.mat) * 8 * sizeof(double), t.consts.data(),
+             t.consts.size() * sizeof(double));
+        copy(prog + static_cast<size_t>(b.prog), t.blob.data(), t.blob.size());
+    }
+};
 
 // Runs fn(t, lo, hi) for nthreads contiguous ranges of [0, count) on host
 // threads (inline when there is one).
@@ -3693,15 +3709,24 @@ void build_batch_cache(BatchCache &C, int dtype, int device_id, const std::vecto
             raise(f.second.code, "circuit " + std::to_string(f.first) + ": " + f.second.msg);
         }
     }
-    phase = std::make_unique<HostScope>("host_batch_merge");
-    BatchPart bp = std::move(parts[0]);
-    for (size_t t = 1; t < parts.size(); t++) {
-        merge_part(bp, std::move(parts[t]));
-        parts[t] = BatchPart{};
-    }
     phase = std::make_unique<HostScope>("host_batch_pack");
+    std::vector<BatchBase> base(parts.size() + 1);
+    std::vector<BatchPlanned> circuits; // ranges within their part's tables
+    std::vector<int32_t> part_of;
+    circuits.reserve(in.size());
+    for (size_t t = 0; t < parts.size(); t++) {
+        base[t + 1] = after(base[t], parts[t]);
+        for (const BatchPlanned &c : parts[t].circuits) {
+            circuits.push_back(c);
+            circuits.back().jac += base[t].jac;
+            part_of.push_back(static_cast<int32_t>(t));
+        }
+    }
+    const BatchBase &all = base.back();
+    auto passes = [&](int32_t ci, const std::pair<int, int> &r) { // in the batch's table
+        return std::pair<int, int>{r.first + base[part_of[ci]].pass, r.second};
+    };
     Device &dev = device(device_id);
-    SweepTables &T = bp.t;
     C.release();
     C.device = dev.id;
     C.groups.clear();
@@ -3712,21 +3737,35 @@ void build_batch_cache(BatchCache &C, int dtype, int device_id, const std::vecto
         by_cost[i] = static_cast<int32_t>(i);
     }
     std::stable_sort(by_cost.begin(), by_cost.end(),
-                     [&](int32_t a, int32_t b) { return bp.circuits[a].cost > bp.circuits[b].cost; });
+                     [&](int32_t a, int32_t b) { return circuits[a].cost > circuits[b].cost; });
     std::vector<SweepJob> jobs;         // pointers are set once the buffer exists
     std::vector<int32_t> job_circuit;
     std::vector<std::pair<int64_t, int64_t>> job_state; // phi, h amplitudes
     std::vector<BatchCircuit> staged;
     std::vector<BatchBlock> blocks;
     std::vector<BatchTail> tails;
-    int64_t amps_max = 0, parts_max = 0;
     const int tile = sweep_reg_bits(dtype) + RT_LANE_BITS;
+    {
+        size_t nblocks = 0, ntails = 0;
+        for (size_t i = 0; i < circuits.size(); i++) {
+            const BatchPlanned &c = circuits[i];
+            if (!c.staged) {
+                continue;
+            }
+            nblocks += static_cast<size_t>(c.fwd.second + c.rev.second + 1) *
+                       static_cast<size_t>(std::min(kBatchBlocks, 1 << (c.n - tile)));
+            ntails += 1 + in[i].tp.size();
+        }
+        blocks.reserve(nblocks);
+        tails.reserve(ntails);
+    }
+    int64_t amps_max = 0, parts_max = 0;
     for (size_t at = 0; at < by_cost.size();) {
         BatchGroup g;
         int64_t amps = 0, psum = 0;
         std::vector<int32_t> members;
         while (at < by_cost.size()) {
-            const int64_t need = int64_t{2} << bp.circuits[by_cost[at]].n;
+            const int64_t need = int64_t{2} << circuits[by_cost[at]].n;
             if (!members.empty() && amps + need > kBatchScratch) {
                 break;
             }
@@ -3739,15 +3778,15 @@ void build_batch_cache(BatchCache &C, int dtype, int device_id, const std::vecto
         for (const bool wide : {true, false}) {
             BatchGroup::Jobs l{jobs.size(), 0, 1};
             for (int32_t ci : members) {
-                const BatchPlanned &c = bp.circuits[ci];
+                const BatchPlanned &c = circuits[ci];
                 if (c.staged || (c.n > tile) != wide) {
                     continue;
                 }
                 SweepJob J{};
                 J.n = c.n;
-                std::tie(J.fwd_first, J.fwd_count) = c.fwd;
-                std::tie(J.rev_first, J.rev_count) = c.rev;
-                J.term_first = c.term_first;
+                std::tie(J.fwd_first, J.fwd_count) = passes(ci, c.fwd);
+                std::tie(J.rev_first, J.rev_count) = passes(ci, c.rev);
+                J.term_first = c.term_first + base[part_of[ci]].term;
                 J.term_count = c.term_count;
                 J.jac_len = static_cast<int32_t>(in[ci].tp.size());
                 jobs.push_back(J);
@@ -3763,11 +3802,11 @@ void build_batch_cache(BatchCache &C, int dtype, int device_id, const std::vecto
         }
         // Staged circuits.
         std::vector<int32_t> ids; // positions in `staged`
-        std::vector<const BatchPlanned *> who;
+        std::vector<int32_t> who;         // and the circuits there
         int nfwd = 0, nrev = 0;
         g.tail_first = tails.size();
         for (int32_t ci : members) {
-            const BatchPlanned &c = bp.circuits[ci];
+            const BatchPlanned &c = circuits[ci];
             if (!c.staged) {
                 continue;
             }
@@ -3777,30 +3816,30 @@ void build_batch_cache(BatchCache &C, int dtype, int device_id, const std::vecto
             amps += int64_t{2} << c.n;
             b.n = c.n;
             b.blocks = std::min(kBatchBlocks, 1 << (c.n - tile));
-            b.term_first = c.term_first;
+            b.term_first = c.term_first + base[part_of[ci]].term;
             b.term_count = c.term_count;
             b.eparts = psum;
             psum += b.blocks;
             tails.push_back({b.eparts, ci, -1, b.blocks});
             for (int p = c.rev.first; p < c.rev.first + c.rev.second; p++) {
-                SweepPass &P = T.passes[p];
+                SweepPass &P = parts[part_of[ci]].t.passes[p];
                 P.parts = psum;
                 psum += static_cast<int64_t>(P.nslots) * b.blocks;
                 for (int e = 0; e < P.entry_count; e++) {
-                    tails.push_back({P.parts, c.jac, P.entry_first + e, b.blocks});
+                    tails.push_back({P.parts, c.jac, base[part_of[ci]].entry + P.entry_first + e, b.blocks});
                 }
             }
             nfwd = std::max(nfwd, c.fwd.second);
             nrev = std::max(nrev, c.rev.second);
             ids.push_back(static_cast<int32_t>(staged.size()));
-            who.push_back(&c);
+            who.push_back(ci);
             staged.push_back(b);
         }
         auto launch = [&](BatchStage stage, int k) {
             BatchGroup::Launch l{stage, blocks.size(), 0};
             for (size_t q = 0; q < ids.size(); q++) {
-                const BatchPlanned &c = *who[q];
-                const std::pair<int, int> r = stage == BATCH_FORWARD ? c.fwd : c.rev;
+                const BatchPlanned &c = circuits[who[q]];
+                const std::pair<int, int> r = passes(who[q], stage == BATCH_FORWARD ? c.fwd : c.rev);
                 if (stage != BATCH_OBSERVABLE && k >= r.second) {
                     continue;
                 }
@@ -3826,26 +3865,49 @@ void build_batch_cache(BatchCache &C, int dtype, int device_id, const std::vecto
         C.groups.push_back(std::move(g));
     }
 
-    Blob blob;
-    const size_t o_jobs = blob.add(jobs); // rewritten below
-    const size_t o_pass = blob.add(T.passes);
-    const size_t o_ent = blob.add(T.entries);
-    const size_t o_terms = blob.add(T.terms);
-    const size_t o_runs = blob.add(T.runs);
-    const size_t o_gates = blob.add(T.gates);
-    const size_t o_consts = blob.add(T.consts);
-    const size_t o_staged = blob.add(staged);
-    const size_t o_blocks = blob.add(blocks);
-    const size_t o_tails = blob.add(tails);
-    const size_t o_prog = blob.add(T.blob);
+    // The image: the parts' tables, written side by side by several threads, and
+    // the schedule. Not a vector, whose zeroes would be written first.
+    size_t bytes = 0;
+    auto table = [&](size_t count, size_t size) {
+        const size_t at = bytes;
+        bytes = (bytes + count * size + 255) & ~size_t{255};
+        return at;
+    };
+    BatchImage img;
+    const size_t o_jobs = table(jobs.size(), sizeof(SweepJob));
+    img.passes = table(static_cast<size_t>(all.pass), sizeof(SweepPass));
+    img.entries = table(static_cast<size_t>(all.entry), sizeof(SweepEntry));
+    img.terms = table(static_cast<size_t>(all.term), sizeof(SweepTerm));
+    img.runs = table(static_cast<size_t>(all.run), sizeof(BatchRun));
+    img.gates = table(static_cast<size_t>(all.gate), sizeof(BatchGate));
+    img.consts = table(static_cast<size_t>(all.mat) * 8, sizeof(double));
+    const size_t o_staged = table(staged.size(), sizeof(BatchCircuit));
+    const size_t o_blocks = table(blocks.size(), sizeof(BatchBlock));
+    const size_t o_tails = table(tails.size(), sizeof(BatchTail));
+    img.prog = table(static_cast<size_t>(all.prog), 1);
+    std::unique_ptr<unsigned char[]> host(new unsigned char[bytes]);
+    parallel_ranges(parts.size(), parts.size(), [&](size_t, size_t lo, size_t hi) {
+        for (size_t t = lo; t < hi; t++) {
+            img.put(host.get(), parts[t], base[t]);
+            parts[t] = BatchPart{};
+        }
+    });
+    auto put = [&](size_t at, const auto &v) {
+        if (!v.empty()) {
+            std::memcpy(host.get() + at, v.data(), v.size() * sizeof(v[0]));
+        }
+    };
+    put(o_staged, staged);
+    put(o_blocks, blocks);
+    put(o_tails, tails);
     auto up = [](size_t x) { return (x + 255) & ~size_t{255}; };
     const size_t amp = dtype == PLK_C64 ? 8 : 16;
-    const size_t o_params = up(blob.bytes.size());
-    const size_t o_scratch = o_params + up(static_cast<size_t>(bp.nparams) * sizeof(double));
+    const size_t o_params = bytes;
+    const size_t o_scratch = o_params + up(static_cast<size_t>(all.param) * sizeof(double));
     const size_t o_parts = o_scratch + up(static_cast<size_t>(amps_max) * amp);
     const size_t o_exp = o_parts + up(static_cast<size_t>(parts_max) * sizeof(double));
     const size_t o_jac = o_exp + up(in.size() * sizeof(double));
-    const size_t total = o_jac + static_cast<size_t>(bp.jac_len) * sizeof(double) + 256;
+    const size_t total = o_jac + static_cast<size_t>(all.jac) * sizeof(double) + 256;
 
     phase = std::make_unique<HostScope>("host_batch_upload");
     C.dbuf = dev_malloc(dev.id, total, "batch plan");
@@ -3856,42 +3918,40 @@ void build_batch_cache(BatchCache &C, int dtype, int device_id, const std::vecto
         SweepJob &J = jobs[j];
         J.phi = w + o_scratch + static_cast<size_t>(job_state[j].first) * amp;
         J.h = w + o_scratch + static_cast<size_t>(job_state[j].second) * amp;
-        J.jac = d_jac + bp.circuits[job_circuit[j]].jac;
+        J.jac = d_jac + circuits[job_circuit[j]].jac;
         J.expval = d_exp + job_circuit[j];
     }
-    if (!jobs.empty()) {
-        std::memcpy(blob.bytes.data() + o_jobs, jobs.data(), jobs.size() * sizeof(SweepJob));
-    }
-    PLK_HIP(hipMemcpy(w, blob.bytes.data(), blob.bytes.size(), hipMemcpyHostToDevice));
-    record_kernel("host_batch_table_bytes", 0.f, static_cast<double>(blob.bytes.size()));
+    put(o_jobs, jobs);
+    PLK_HIP(hipMemcpy(w, host.get(), bytes, hipMemcpyHostToDevice));
+    record_kernel("host_batch_table_bytes", 0.f, static_cast<double>(bytes));
 
     BatchArgs &A = C.A;
     A.circuits = reinterpret_cast<const BatchCircuit *>(w + o_staged);
-    A.passes = reinterpret_cast<const SweepPass *>(w + o_pass);
-    A.entries = reinterpret_cast<const SweepEntry *>(w + o_ent);
-    A.terms = reinterpret_cast<const SweepTerm *>(w + o_terms);
-    A.blob = w + o_prog;
+    A.passes = reinterpret_cast<const SweepPass *>(w + img.passes);
+    A.entries = reinterpret_cast<const SweepEntry *>(w + img.entries);
+    A.terms = reinterpret_cast<const SweepTerm *>(w + img.terms);
+    A.blob = w + img.prog;
     A.scratch = w + o_scratch;
     A.parts = reinterpret_cast<double *>(w + o_parts);
     A.expvals = d_exp;
     A.jac = d_jac;
-    C.blob = w + o_prog;
-    C.entries = reinterpret_cast<SweepEntry *>(w + o_ent);
-    C.runs = reinterpret_cast<const BatchRun *>(w + o_runs);
-    C.nruns = static_cast<int64_t>(T.runs.size());
-    C.gates = reinterpret_cast<const BatchGate *>(w + o_gates);
-    C.consts = reinterpret_cast<const double *>(w + o_consts);
+    C.blob = w + img.prog;
+    C.entries = reinterpret_cast<SweepEntry *>(w + img.entries);
+    C.runs = reinterpret_cast<const BatchRun *>(w + img.runs);
+    C.nruns = all.run;
+    C.gates = reinterpret_cast<const BatchGate *>(w + img.gates);
+    C.consts = reinterpret_cast<const double *>(w + img.consts);
     C.params = reinterpret_cast<double *>(w + o_params);
     C.jobs = reinterpret_cast<const SweepJob *>(w + o_jobs);
     C.blocks = reinterpret_cast<const BatchBlock *>(w + o_blocks);
     C.tails = reinterpret_cast<const BatchTail *>(w + o_tails);
-    C.nparams = bp.nparams;
-    C.jac_len = bp.jac_len;
+    C.nparams = all.param;
+    C.jac_len = all.jac;
     C.param_base.assign(in.size(), 0);
-    int64_t base = 0;
+    int64_t param = 0;
     for (size_t i = 0; i < in.size(); i++) {
-        C.param_base[i] = base;
-        base += static_cast<int64_t>(in[i].ops->num_par_ops());
+        C.param_base[i] = param;
+        param += static_cast<int64_t>(in[i].ops->num_par_ops());
     }
     C.valid = true;
 }
