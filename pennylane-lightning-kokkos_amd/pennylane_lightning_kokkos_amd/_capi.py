@@ -144,11 +144,12 @@ def _dp(a: np.ndarray):
 
 
 def _plain_wires(x) -> bool:
-    """A list or tuple of non-negative ints: needs no numpy to become a C array."""
+    """A list or tuple of ints that a size_t holds: needs no numpy to become a C
+    array (ctypes would wrap larger ones)."""
     if type(x) is not list and type(x) is not tuple:
         return False
     for w in x:
-        if type(w) is not int or w < 0:
+        if type(w) is not int or not 0 <= w < 1 << 64:
             return False
     return True
 
@@ -407,7 +408,10 @@ class Ops:
                 p = np.asarray(p, dtype=np.float64).reshape(-1).tolist()
             pflat += p
             poff.append(len(pflat))
-            wflat += w if _plain_wires(w) else np.asarray(w, dtype=np.uint64).reshape(-1).tolist()
+            if not _plain_wires(w):
+                len(w)  # a list of wires: a bare number raises
+                w = np.asarray(w, dtype=np.uint64).reshape(-1).tolist()
+            wflat += w
             woff.append(len(wflat))
             count = moff[-1]
             if type(m) is not list or m:
