@@ -247,6 +247,7 @@ struct PlanOp {
     int32_t src = -1;       // index of the op in its OpsData
     bool adj = false;       // U was compiled with the inverse flag set
     bool skew = false;      // reverse sweeps: U is not unitary (see Blocked)
+    uint64_t mix = 0;       // register-tile plans: the state bits it mixes
     // Batch plans, runs with patched gates: the U kind and the Pauli parts that
     // hold for every angle (see fix_form); -1: as the matrices are.
     int ukind = -1, parts = -1;
@@ -707,6 +708,7 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
         every |= it.on;
         it.fus = fusable(all[i]);
         it.mix = bundled || !it.fus ? it.on : mixing_mask(all[i], n);
+        all[i].mix = it.mix;
         it.sums = bundled ? (all[i].trainable ? 1 : 0) : rt_slots(all[i]);
     }
     // Operations of rem that a pass over these bits takes.
@@ -1411,7 +1413,7 @@ template <typename T> struct RtBuilder {
     std::vector<Slot> ins;
     std::vector<unsigned char> pay;
 
-    explicit RtBuilder(std::vector<unsigned char> &b) : blob(b) {}
+    RtBuilder(std::vector<unsigned char> &b, size_t ops) : blob(b) { ins.reserve(ops + 2); }
 
     void add(const RtInstr &h, const std::vector<double> &u) {
         Slot s{};
@@ -1456,6 +1458,7 @@ template <typename T> struct RtBuilder {
 
 std::vector<double> cplx(const std::vector<cd> &v) {
     std::vector<double> out;
+    out.reserve(2 * v.size());
     for (auto &x : v) {
         out.push_back(x.real());
         out.push_back(x.imag());
@@ -1546,6 +1549,17 @@ std::vector<double> keep_norm(const std::vector<double> &u, double &norm) {
 // a register when an op needs it.
 int keep_bits(int dtype) { return dtype == PLK_C64 ? 2 : 1; }
 
+// The state bits of an op of at most two wires.
+struct BitList {
+    int bit[2];
+    int count = 0;
+    void push_back(int b) { bit[count++] = b; }
+    const int *begin() const { return bit; }
+    const int *end() const { return bit + count; }
+    int size() const { return count; }
+    int operator[](int k) const { return bit[k]; }
+};
+
 template <typename T>
 RtProgram build_rt_program(const Pass &ps, int n, int R, int keep, std::vector<unsigned char> &blob, double &norm,
                            bool patched = false) {
@@ -1562,11 +1576,11 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, int keep, std::vector<u
         L.tb[q] = ps.tb[q];
     }
     const size_t nops = ps.ops.size();
-    std::vector<std::vector<int>> gbits(nops), mix(nops);
+    std::vector<BitList> gbits(nops), mix(nops);
     std::vector<Place> place(nops);
     for (size_t i = 0; i < nops; i++) {
         const PlanOp &p = ps.ops[i];
-        const uint64_t mm = place[i].mix = mixing_mask(p, n);
+        const uint64_t mm = place[i].mix = p.mix;
         place[i].trainable = p.trainable;
         place[i].skew = p.skew;
         for (auto w : p.U.wires) {
@@ -1624,7 +1638,7 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, int keep, std::vector<u
         L.lane_in[p] = lane[p];
     }
 
-    RtBuilder<T> b(blob);
+    RtBuilder<T> b(blob, nops);
     auto reg_of = [&](int q) {
         for (int r = 0; r < R; r++) {
             if (reg[r] == q) {
@@ -1726,7 +1740,7 @@ RtProgram build_rt_program(const Pass &ps, int n, int R, int keep, std::vector<u
             }
             add_remap(in, victim, lane_of(q));
         }
-        const int m = static_cast<int>(gbits[i].size());
+        const int m = gbits[i].size();
         const std::vector<cd> *G = nullptr;
         const int term0 = static_cast<int>(out.terms.size());
         if (p.trainable) {
