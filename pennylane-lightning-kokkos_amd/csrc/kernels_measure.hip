@@ -856,7 +856,7 @@ struct PauliTiles {
     size_t bytes = 0;
     ~PauliTiles() {
         if (blob != nullptr) {
-            pool_give(device, bytes, blob);
+            pool_give(Pool::Tables, device, bytes, blob);
         }
     }
 };
@@ -877,11 +877,11 @@ size_t table_bytes(size_t need) {
 // has been read when this returns).
 void *upload_table(Device &dev, const std::vector<unsigned char> &img, size_t &bytes, const char *what) {
     bytes = table_bytes(img.size());
-    void *d = pool_take(dev.id, bytes, what);
+    void *d = pool_take(Pool::Tables, dev.id, bytes, what);
     const hipError_t e = hipMemcpyAsync(d, img.data(), img.size(), hipMemcpyHostToDevice, dev.stream);
     const hipError_t w = e == hipSuccess ? hipStreamSynchronize(dev.stream) : e;
     if (w != hipSuccess) {
-        pool_give(dev.id, bytes, d);
+        pool_give(Pool::Tables, dev.id, bytes, d);
         check_hip(w, "table upload");
     }
     return d;
@@ -891,7 +891,7 @@ void *upload_table(Device &dev, const std::vector<unsigned char> &img, size_t &b
 
 PauliDevice::~PauliDevice() {
     if (blob != nullptr) {
-        pool_give(device, bytes, blob);
+        pool_give(Pool::Tables, device, bytes, blob);
     }
 }
 

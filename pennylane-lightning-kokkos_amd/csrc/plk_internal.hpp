@@ -129,11 +129,12 @@ struct State {
     size_t bytes() const { return len * elem_bytes(); }
 };
 
-// Buffers of the device's recycling pool (see TmpPool): pool_take may hand out
+// Buffers of the device's recycling pools (see TmpPool): pool_take may hand out
 // one that queued work still reads, so it is written on the device's stream
 // only, and returned with the size it was taken with.
-void *pool_take(int device, size_t bytes, const char *what);
-void pool_give(int device, size_t bytes, void *d);
+enum class Pool { States, Tables };
+void *pool_take(Pool kind, int device, size_t bytes, const char *what);
+void pool_give(Pool kind, int device, size_t bytes, void *d);
 
 // RAII temporary device state of the same shape.
 struct TmpState {

@@ -251,30 +251,37 @@ void record_kernel(const char *family, float ms, double bytes) {
 // Temporary states and observables' tables are recycled per device instead of
 // being freed: every kernel of the library runs on the device's one stream,
 // so a buffer handed out again is written (on that stream) only after the work
-// that last used it. The pool holds at most kPoolMaxBytes per device; an
-// allocation that fails releases it.
+// that last used it. States and tables have a pool each, so that the tables of
+// many observables do not keep states out; an allocation that fails releases
+// both.
 namespace {
-constexpr size_t kPoolMaxBytes = size_t{32} << 30;
-constexpr size_t kPoolMaxBuffers = 4096;
-
 struct TmpPool {
     std::multimap<size_t, void *> free;
     size_t held = 0;
 };
 
+// What a device's pool holds at most.
+struct PoolLimit {
+    size_t bytes, buffers;
+};
+constexpr PoolLimit kPoolLimit[] = {{size_t{32} << 30, SIZE_MAX}, // Pool::States
+                                    {size_t{1} << 30, 4096}};     // Pool::Tables
+
 std::mutex g_pool_mutex;
-std::map<int, TmpPool> g_pools;
+std::map<int, TmpPool> g_pools[2];
 
 void release_pool(int dev) {
     std::vector<void *> bufs;
     {
         std::lock_guard<std::mutex> lock(g_pool_mutex);
-        TmpPool &p = g_pools[dev];
-        for (auto &kv : p.free) {
-            bufs.push_back(kv.second);
+        for (auto &pools : g_pools) {
+            TmpPool &p = pools[dev];
+            for (auto &kv : p.free) {
+                bufs.push_back(kv.second);
+            }
+            p.free.clear();
+            p.held = 0;
         }
-        p.free.clear();
-        p.held = 0;
     }
     if (!bufs.empty()) {
         (void)hipDeviceSynchronize();
@@ -287,22 +294,26 @@ void release_pool(int dev) {
 
 void *dev_malloc(int device, size_t bytes, const char *what) {
     void *p = nullptr;
-    if (hipMalloc(&p, bytes) == hipSuccess) {
-        return p;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        release_pool(device);
+        e = hipMalloc(&p, bytes);
     }
-    (void)hipGetLastError();
-    release_pool(device);
-    if (hipMalloc(&p, bytes) == hipSuccess) {
+    if (e == hipSuccess) {
+        if (g_prof_on) {
+            record_kernel("device_alloc", 0.f, static_cast<double>(bytes));
+        }
         return p;
     }
     (void)hipGetLastError();
     raise(PLK_ERR_OOM, "device allocation of " + std::to_string(bytes) + " bytes failed (" + what + ")");
 }
 
-void *pool_take(int dev, size_t bytes, const char *what) {
+void *pool_take(Pool kind, int dev, size_t bytes, const char *what) {
     {
         std::lock_guard<std::mutex> lock(g_pool_mutex);
-        TmpPool &p = g_pools[dev];
+        TmpPool &p = g_pools[static_cast<int>(kind)][dev];
         auto it = p.free.find(bytes);
         if (it != p.free.end()) {
             void *d = it->second;
@@ -314,11 +325,12 @@ void *pool_take(int dev, size_t bytes, const char *what) {
     return dev_malloc(dev, bytes, what);
 }
 
-void pool_give(int dev, size_t bytes, void *d) {
+void pool_give(Pool kind, int dev, size_t bytes, void *d) {
     {
         std::lock_guard<std::mutex> lock(g_pool_mutex);
-        TmpPool &p = g_pools[dev];
-        if (p.held + bytes <= kPoolMaxBytes && p.free.size() < kPoolMaxBuffers) {
+        TmpPool &p = g_pools[static_cast<int>(kind)][dev];
+        const PoolLimit &most = kPoolLimit[static_cast<int>(kind)];
+        if (p.held + bytes <= most.bytes && p.free.size() < most.buffers) {
             p.free.emplace(bytes, d);
             p.held += bytes;
             return;
@@ -334,12 +346,12 @@ TmpState::TmpState(int n, int dtype, int dev) {
     s.dtype = dtype;
     s.len = size_t{1} << n;
     s.device = dev;
-    s.d = pool_take(dev, s.bytes(), "temporary state");
+    s.d = pool_take(Pool::States, dev, s.bytes(), "temporary state");
 }
 
 TmpState::~TmpState() {
     if (s.d) {
-        pool_give(s.device, s.bytes(), s.d);
+        pool_give(Pool::States, s.device, s.bytes(), s.d);
     }
 }
 
