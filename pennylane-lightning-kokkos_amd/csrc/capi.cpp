@@ -3131,14 +3131,41 @@ void sweep_forward(Device &dev, const State &s, std::vector<PlanOp> &&ops) {
     run_sweep(dev, s.dtype, s.n, t, {J}, nullptr, nullptr);
 }
 
+// Pauli words of an observable, at least, without expanding it.
+size_t least_words(const ObsNode &o) {
+    return o.kind == ObsNode::Hamiltonian ? o.terms.size() : 1;
+}
+
+// Whether the whole-circuit launch forms H lambda fast enough: there one
+// workgroup walks every word of an observable for each of its amplitudes (0.036
+// us a word and amplitude of a thread more than the general path, whose launch
+// has the whole chip), where the general path has a launch and an upload for each
+// observable (6 us and 0.2 to 0.3 us a word). One observable, one layer, whole / general:
+// 12 qubits complex128 64 words 154 / 159 us, 128 words 191 / 189, 600 words
+// 547 / 420; 12 qubits complex64 32 words 140 / 137, 600 words 743 / 425; 10 qubits
+// complex64 64 words 144 / 148, 128 words 196 / 181. Four observables of 600 words
+// each, 12 qubits complex128: 889 / 1291. Below nine qubits the general path has no
+// register-tile passes: 8 qubits complex128, 600 words 361 / 410, 1500 words 821 / 763.
+bool sweep_takes_words(const std::vector<std::shared_ptr<const ObsNode>> &obs, int n, int dtype) {
+    const size_t threads = static_cast<size_t>(64) * sweep_waves(n, dtype);
+    const size_t each = std::max<size_t>(1, (size_t{1} << n) / threads);
+    size_t most = 0, all = 0;
+    for (const auto &o : obs) {
+        const size_t words = least_words(*o);
+        most = std::max(most, words);
+        all += 6 * words + 165;
+    }
+    return most * each <= (n < 9 ? 2500 : 800) + all - (6 * most + 165);
+}
+
 // The Jacobian by one workgroup per observable; false when an op or an
 // observable needs the general path. rev: the reverse walk's ops.
 bool sweep_jacobian(Device &dev, const State &ref, const std::vector<std::shared_ptr<const ObsNode>> &obs,
                     const OpsData &ops, std::vector<PlanOp> &rev, size_t n_tp, bool apply_ops, double *jac) {
-    if (!sweep_serves(ref) || !sweep_takes(rev)) {
+    const int n = ref.n;
+    if (!sweep_serves(ref) || !sweep_takes_words(obs, n, ref.dtype) || !sweep_takes(rev)) {
         return false;
     }
-    const int n = ref.n;
     SweepTables t;
     std::vector<SweepJob> jobs(obs.size());
     for (size_t j = 0; j < obs.size(); j++) {

@@ -95,15 +95,9 @@ __global__ void __launch_bounds__(256) stage_observable_kernel(BatchArgs A, cons
     const Cx<T> *phi = static_cast<const Cx<T> *>(A.scratch) + c.phi;
     Cx<T> *h = static_cast<Cx<T> *>(A.scratch) + c.h;
     const uint32_t len = uint32_t{1} << c.n;
-    double e = 0.0;
-    for (uint32_t i = static_cast<uint32_t>(b.block) * 256 + threadIdx.x; i < len;
-         i += static_cast<uint32_t>(c.blocks) * 256) {
-        double sr, si;
-        pauli_sum<T>(A.terms + c.term_first, c.term_count, phi, i, sr, si);
-        const Cx<T> a = ldg(phi, i);
-        e += static_cast<double>(a.r) * sr + static_cast<double>(a.i) * si;
-        stg(h, i, Cx<T>{static_cast<T>(sr), static_cast<T>(si)});
-    }
+    double e = pauli_share<T>(A.terms + c.term_first, c.term_count, phi, h,
+                              static_cast<uint32_t>(b.block) * 256 + threadIdx.x,
+                              static_cast<uint32_t>(c.blocks) * 256, len);
     e = wave_sum(e);
     if ((threadIdx.x & 63) == 0) {
         red[threadIdx.x >> 6] = e;

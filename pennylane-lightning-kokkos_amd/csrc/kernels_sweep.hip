@@ -118,14 +118,7 @@ template <typename T>
 __device__ __forceinline__ void observable(const SweepArgs &A, const SweepJob &J, const Cx<T> *phi, Cx<T> *h,
                                            double *red) {
     const uint32_t len = uint32_t{1} << J.n;
-    double e = 0.0;
-    for (uint32_t i = threadIdx.x; i < len; i += blockDim.x) {
-        double sr, si;
-        pauli_sum<T>(A.terms + J.term_first, J.term_count, phi, i, sr, si);
-        const Cx<T> a = ldg(phi, i);
-        e += static_cast<double>(a.r) * sr + static_cast<double>(a.i) * si;
-        stg(h, i, Cx<T>{static_cast<T>(sr), static_cast<T>(si)});
-    }
+    double e = pauli_share<T>(A.terms + J.term_first, J.term_count, phi, h, threadIdx.x, blockDim.x, len);
     e = wave_sum(e);
     if ((threadIdx.x & 63) == 0) {
         red[threadIdx.x >> 6] = e;
