@@ -66,8 +66,15 @@ void left_multiply(std::vector<cd> &M, const std::vector<cd> &U, const std::vect
                 continue;
             }
             const int s = spread(uc, rest);
-            for (int c = 0; c < 32; c++) {
-                out[static_cast<size_t>(r) * 32 + c] += u * M[static_cast<size_t>(s) * 32 + c];
+            // Written out in reals: std::complex's product tests each result for NaN, a
+            // loop so dense in branches that where the linker put it decided between
+            // 163 and 188 us for 105 gates on 12 wires; now 122 wherever it lies.
+            const double ur = u.real(), ui = u.imag();
+            const auto *m = reinterpret_cast<const double *>(M.data() + static_cast<size_t>(s) * 32);
+            auto *o = reinterpret_cast<double *>(out.data() + static_cast<size_t>(r) * 32);
+            for (int c = 0; c < 64; c += 2) {
+                o[c] += ur * m[c] - ui * m[c + 1];
+                o[c + 1] += ur * m[c + 1] + ui * m[c];
             }
         }
     }
