@@ -2217,12 +2217,17 @@ bool use_rtile(int n, int dtype, int nj) {
 // 2635; 20 qubits complex64 630 / 612 / 680, 24 qubits 2407 / 1914 / 1728. One
 // observable a chunk (R = 3 / 4): 17 qubits complex64, 5 observables 742 / 766 us
 // (R = 5: 897); 16 qubits complex128, 9 observables 636 / 675; one observable,
-// 20 qubits complex128 3208 / 3320, 21 qubits 3828 / 3673.
-int plan_reg_bits(int n, int dtype, int nj, size_t chunks, int num_cus) {
+// 20 qubits complex128 3208 / 3320, 21 qubits 3828 / 3673. The complex64 figures are
+// those of FP32 programs. A wide one (see build_image) is bound by its FP64
+// exchanges before memory, and R = 5 has fewest of them: it pays from eight tiles
+// a CU on (streams of 200 gates, R = 4 / 5: 21 qubits 374 / 427 us, 22 qubits 454 /
+// 448, 23 qubits 690 / 629, 24 qubits 1168 / 1062).
+int plan_reg_bits(int n, int dtype, int nj, size_t chunks, int num_cus, bool wide) {
     const int lo = rt_reg_min(dtype, nj);
     int R = std::min(rt_reg_max(dtype, nj), n - RT_LANE_BITS);
     auto tiles_per_cu = [&] { return std::ldexp(static_cast<double>(chunks), n - R - RT_LANE_BITS) / num_cus; };
-    while (R > lo && tiles_per_cu() < (R == 5 ? 32.0 : nj == 1 ? 8.0 : 2.0)) {
+    const double widest = wide && dtype == PLK_C64 ? 8.0 : 32.0;
+    while (R > lo && tiles_per_cu() < (R == 5 ? widest : nj == 1 ? 8.0 : 2.0)) {
         R--;
     }
     return R;
@@ -2492,10 +2497,10 @@ std::vector<PlanOp> forward_ops(const OpsData &ops, int n) {
     return v;
 }
 
-// Forward plan of the whole op list.
-std::vector<Step> forward_plan(const Device &dev, std::vector<PlanOp> &&v, int n, int dtype) {
+// Forward plan of the whole op list. wide: as its image is built.
+std::vector<Step> forward_plan(const Device &dev, std::vector<PlanOp> &&v, int n, int dtype, bool wide) {
     if (use_rtile(n, dtype, 0)) {
-        std::vector<Step> steps = plan_tiles(std::move(v), n, plan_reg_bits(n, dtype, 0, 1, dev.num_cus) + RT_LANE_BITS,
+        std::vector<Step> steps = plan_tiles(std::move(v), n, plan_reg_bits(n, dtype, 0, 1, dev.num_cus, wide) + RT_LANE_BITS,
                                              low_bits(dtype), RT_SLOTS_MAX, false, plan_exchange(n, dtype, 1));
         split_sparse_passes(steps, n);
         return steps;
@@ -3232,7 +3237,7 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
     }
     const int nj = sweep_chunk(ref.dtype, n, n_obs, dev.num_cus);
     const bool rt = use_rtile(n, ref.dtype, nj);
-    const int T_adj = rt ? plan_reg_bits(n, ref.dtype, nj, chunk_sizes(n_obs, nj).size(), dev.num_cus) + RT_LANE_BITS : tile_bits_adjoint(n, ref.dtype);
+    const int T_adj = rt ? plan_reg_bits(n, ref.dtype, nj, chunk_sizes(n_obs, nj).size(), dev.num_cus, false) + RT_LANE_BITS : tile_bits_adjoint(n, ref.dtype);
     std::vector<Step> steps =
         rt ? plan_tiles(std::move(rev), n, T_adj, low_bits(ref.dtype), RT_SLOTS_MAX, false,
                         plan_exchange(n, ref.dtype, n_obs + 1))
@@ -3241,7 +3246,7 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
     if (rt) {
         split_sparse_passes(steps, n);
     }
-    const std::vector<Step> fwd = apply_ops ? forward_plan(dev, forward_ops(ops, n), n, ref.dtype) : std::vector<Step>{};
+    const std::vector<Step> fwd = apply_ops ? forward_plan(dev, forward_ops(ops, n), n, ref.dtype, false) : std::vector<Step>{};
     const PlanImage img_f = build_image(fwd, ref, false);
     PlanImage img_r = build_image(steps, ref, false);
     const bool alt = needs_alt(dev, steps, n_obs, ref.dtype, n);
@@ -4342,7 +4347,7 @@ int plk_apply_ops(plk_state *sv, const plk_ops *ops) {
         if (sweep_serves(s) && sweep_takes(v)) {
             sweep_forward(dev, s, std::move(v));
         } else {
-            run_forward(dev, s, forward_plan(dev, std::move(v), s.n, s.dtype));
+            run_forward(dev, s, forward_plan(dev, std::move(v), s.n, s.dtype, true));
         }
     })
 }
