@@ -24,12 +24,13 @@ def taken_path(request, capi, monkeypatch):
     if "batched" in request.node.name:
         yield
         return
+    name = request.node.originalname
     monkeypatch.setenv("PLK_SWEEP", "0")
+    monkeypatch.setenv("PLK_GRAPH", "1" if "graph" in name else "0")
     capi.profiling_enable(True)
     yield
     names = capi.profiling_names()
     capi.profiling_enable(False)
-    name = request.node.originalname
     assert "circuit_sweep" not in names
     assert ("host_adjoint_graph" if "graph" in name else "apply_rtile" if "forward" in name else "adjoint_rtile") in names
 
