@@ -826,12 +826,9 @@ double pauli_tile_expval(Device &dev, const State &s, const TilePlan &p, const v
     const auto *groups = reinterpret_cast<const TileGroup *>(b);
     const auto *terms = reinterpret_cast<const TileTerm *>(b + tile_terms_off(p));
     const size_t lds = sizeof(Cx<T>) << TB;
-    static bool attr = false;
-    if (!attr) {
-        PLK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&pauli_tile_kernel<T>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        attr = true;
-    }
+    // On every call: the attribute belongs to the function on the current device.
+    PLK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&pauli_tile_kernel<T>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
     {
         ProfScope prof("pauli_expval", static_cast<double>(p.sets.size()) * s.bytes(), dev.stream);
         for (size_t k = 0; k < p.sets.size(); k++) {
