@@ -59,7 +59,11 @@ struct ObsNode {
     std::vector<int32_t> indices32, indptr32;   // int32 matrices (complex64 serialisation)
     bool idx32 = false;
     size_t rows = 0;
-    mutable uint64_t key = 0; // hash of the tree, once a batched call has asked (obs_key)
+    // Hash of the tree (CSR values left out) without its matrices, whether it has
+    // any, and the hash with them once a batched call has asked (see obs_key).
+    uint64_t key = 0;
+    bool dense = false;
+    mutable uint64_t full_key = 0;
     mutable bool keyed = false;
     // Device copies of the CSR matrix per (device, state dtype), made on first
     // use and kept while the observable lives (entry points hold the engine
@@ -91,14 +95,31 @@ struct ObsNode {
     }
 };
 
-// Hash of an observable's tree (CSR values left out). Only batched calls need it,
-// so it is formed by the first one (under the engine lock) and not with the
-// observable: hashing a matrix takes several times as long as copying it (10
-// wires: 2.8 ms to make the observable, 10.9 with the hash).
+// Hash of an observable's tree, for batched calls. All but the matrices is hashed
+// with the observable (note_obs); hashing a matrix takes several times as long as
+// copying it (10 wires: 2.8 ms to make the observable, 10.9 with the hash), so that
+// is left to the first call that asks (under the engine lock).
 uint64_t obs_key(const ObsNode &o) {
-    if (o.keyed) {
+    if (!o.dense) {
         return o.key;
     }
+    if (!o.keyed) {
+        Hasher H;
+        H.add(o.key);
+        for (const cd &m : o.matrix) {
+            H.add(m.real());
+            H.add(m.imag());
+        }
+        for (const auto &t : o.terms) {
+            H.add(obs_key(*t));
+        }
+        o.full_key = H.h;
+        o.keyed = true;
+    }
+    return o.full_key;
+}
+
+void note_obs(ObsNode &o) {
     Hasher H;
     H.add(static_cast<uint64_t>(o.kind));
     H.add(o.name);
@@ -111,17 +132,13 @@ uint64_t obs_key(const ObsNode &o) {
         H.add(c);
     }
     H.add(static_cast<uint64_t>(o.matrix.size()));
-    for (const cd &m : o.matrix) {
-        H.add(m.real());
-        H.add(m.imag());
-    }
     H.add(static_cast<uint64_t>(o.terms.size()));
+    o.dense = !o.matrix.empty();
     for (const auto &t : o.terms) {
-        H.add(obs_key(*t));
+        H.add(t->key);
+        o.dense = o.dense || t->dense;
     }
     o.key = H.h;
-    o.keyed = true;
-    return o.key;
 }
 
 std::vector<size_t> obs_wires(const ObsNode &o) {
@@ -2437,7 +2454,9 @@ struct OpsData {
     std::vector<bool> inverses;
     std::vector<std::vector<cd>> matrices;
     std::vector<double> angles; // the first parameter of every parametric op
-    mutable uint64_t key = 0;   // once a batched call has asked (ops_key)
+    uint64_t key = 0; // hash without the matrices; full_key: with them, see ops_key
+    bool dense = false;
+    mutable uint64_t full_key = 0;
     mutable bool keyed = false;
     size_t num_par_ops() const { return angles.size(); }
 };
@@ -2465,34 +2484,46 @@ int16_t patch_gate_of(const OpsData &ops, size_t i) {
 }
 
 // Hash of everything a batch plan depends on: names, wires, inverse flags,
-// matrices and the parameters of gates whose angles it does not patch. Formed by
-// the first batched call, like obs_key.
+// matrices and the parameters of gates whose angles it does not patch; the
+// matrices when a batched call asks, like obs_key.
 uint64_t ops_key(const OpsData &ops) {
-    if (ops.keyed) {
+    if (!ops.dense) {
         return ops.key;
     }
-    Hasher H;
-    for (size_t i = 0; i < ops.names.size(); i++) {
-        H.add(ops.names[i]);
-        H.add(static_cast<uint64_t>(ops.wires[i].size() | (ops.inverses[i] ? size_t{1} << 40 : 0)));
-        for (auto w : ops.wires[i]) {
-            H.add(static_cast<uint64_t>(w));
-        }
-        H.add(static_cast<uint64_t>(ops.params[i].size()));
-        if (patch_gate_of(ops, i) == BPG_NONE) {
-            for (double v : ops.params[i]) {
-                H.add(v);
+    if (!ops.keyed) {
+        Hasher H;
+        H.add(ops.key);
+        for (const auto &matrix : ops.matrices) {
+            for (const cd &m : matrix) {
+                H.add(m.real());
+                H.add(m.imag());
             }
         }
-        H.add(static_cast<uint64_t>(ops.matrices[i].size()));
-        for (const cd &m : ops.matrices[i]) {
-            H.add(m.real());
-            H.add(m.imag());
+        ops.full_key = H.h;
+        ops.keyed = true;
+    }
+    return ops.full_key;
+}
+
+// Adds op i to the list's hash and angles.
+void note_op(OpsData &ops, Hasher &H, size_t i) {
+    H.add(ops.names[i]);
+    H.add(static_cast<uint64_t>(ops.wires[i].size() | (ops.inverses[i] ? size_t{1} << 40 : 0)));
+    for (auto w : ops.wires[i]) {
+        H.add(static_cast<uint64_t>(w));
+    }
+    H.add(static_cast<uint64_t>(ops.params[i].size()));
+    if (patch_gate_of(ops, i) == BPG_NONE) {
+        for (double v : ops.params[i]) {
+            H.add(v);
         }
     }
+    H.add(static_cast<uint64_t>(ops.matrices[i].size()));
+    ops.dense = ops.dense || !ops.matrices[i].empty();
+    if (!ops.params[i].empty()) {
+        ops.angles.push_back(ops.params[i][0]);
+    }
     ops.key = H.h;
-    ops.keyed = true;
-    return ops.key;
 }
 
 // The whole op list, compiled (applyOperations, AdjointDiffKokkos.hpp:213-226).
@@ -4019,11 +4050,11 @@ void adjoint_batched_run(int dtype, int device_id, const std::vector<BatchInput>
         return;
     }
     std::unique_ptr<HostScope> phase = std::make_unique<HostScope>("host_batch_key");
-    // New op lists are hashed by several threads, each list by one (circuits may
-    // share it).
+    // New matrices are hashed by several threads, each list's by one (circuits
+    // may share it).
     std::vector<const OpsData *> fresh;
     for (const BatchInput &c : in) {
-        if (!c.ops->keyed) {
+        if (c.ops->dense && !c.ops->keyed) {
             fresh.push_back(c.ops);
         }
     }
@@ -4503,6 +4534,7 @@ int plk_obs_named(const char *name, const size_t *wires, size_t num_wires, plk_o
         n->kind = ObsNode::Named;
         n->name = name ? name : "";
         n->wires = to_vec(wires, num_wires);
+        note_obs(*n);
         *out = new plk_obs{n};
     })
 }
@@ -4515,6 +4547,7 @@ int plk_obs_hermitian(const double *matrix, const size_t *wires, size_t num_wire
         n->wires = to_vec(wires, num_wires);
         const size_t dim = size_t{1} << num_wires;
         n->matrix = to_cvec(matrix, dim * dim);
+        note_obs(*n);
         *out = new plk_obs{n};
     })
 }
@@ -4533,6 +4566,7 @@ int plk_obs_tensor(const plk_obs *const *factors, size_t num_factors, plk_obs **
             }
             n->terms.push_back(factors[i]->node);
         }
+        note_obs(*n);
         *out = new plk_obs{n};
     })
 }
@@ -4547,6 +4581,7 @@ int plk_obs_hamiltonian(const double *coeffs, const plk_obs *const *terms, size_
             n->terms.push_back(terms[i]->node);
             n->coeffs.push_back(coeffs[i]);
         }
+        note_obs(*n);
         *out = new plk_obs{n};
     })
 }
@@ -4562,6 +4597,7 @@ int plk_obs_sparse(const double *data, const int64_t *indices, const int64_t *in
         n->indptr.assign(indptr, indptr + num_rows + 1);
         n->rows = num_rows;
         n->wires = to_vec(wires, num_wires);
+        note_obs(*n);
         *out = new plk_obs{n};
     })
 }
@@ -4581,6 +4617,7 @@ int plk_obs_sparse_i32(const double *data, const int32_t *indices, const int32_t
         n->indptr32.assign(indptr, indptr + num_rows + 1);
         n->rows = num_rows;
         n->wires = to_vec(wires, num_wires);
+        note_obs(*n);
         *out = new plk_obs{n};
     })
 }
@@ -4619,6 +4656,7 @@ int plk_ops_create(size_t num_ops, const char *const *names, const double *param
     PLK_TRY({
         auto h = std::make_unique<plk_ops>();
         OpsData &d = h->data;
+        Hasher H;
         for (size_t i = 0; i < num_ops; i++) {
             d.names.emplace_back(names[i]);
             d.params.emplace_back(params + param_offsets[i], params + param_offsets[i + 1]);
@@ -4627,9 +4665,7 @@ int plk_ops_create(size_t num_ops, const char *const *names, const double *param
             const size_t ml = matrix_offsets[i + 1] - matrix_offsets[i];
             d.matrices.push_back(ml ? to_cvec(matrices + 2 * matrix_offsets[i], ml)
                                     : std::vector<cd>{});
-            if (!d.params.back().empty()) {
-                d.angles.push_back(d.params.back()[0]);
-            }
+            note_op(d, H, i);
         }
         *out = h.release();
     })
