@@ -2357,7 +2357,7 @@ const PauliDevice *ObsNode::pauli_on(Device &dev, int n) const {
         return nullptr;
     }
     auto &slot = pauli_dev[{dev.id, n}];
-    slot = pauli_upload(dev, terms);
+    slot = pauli_device(dev, terms);
     return slot.get();
 }
 

@@ -588,9 +588,10 @@ void launch_pauli_apply(Device &dev, const State &out, const State &in,
                         const std::vector<PauliTerm> &terms);
 double pauli_expval(Device &dev, const State &s,
                     const std::vector<PauliTerm> &terms);
-// Device copy of a Pauli-word sum's grouped term tables. Observables keep one
-// per (device, qubit count) for their life, so repeated expectation values
-// and adjoint sweeps upload nothing.
+// A Pauli-word sum on a device: its grouped term tables and tile plans, each
+// uploaded by the first call that reads it. Observables keep one per (device,
+// qubit count) for their life, so repeated expectation values and adjoint sweeps
+// upload nothing.
 struct PauliTiles;
 // Smallest complex128 state (one qubit more in complex64) and number of groups
 // that use tiles: below, the gathers hit the caches (20 qubits complex128, 6 to
@@ -599,11 +600,12 @@ constexpr int kPauliTileQubits = 20;
 constexpr int kPauliTileGroups = 4;
 struct PauliDevice {
     int device = -1;
-    void *blob = nullptr;
-    size_t bytes = 0; // of blob, as taken from the pool
-    size_t toff = 0;  // byte offset of the term table
+    mutable void *blob = nullptr; // see tables()
+    mutable size_t bytes = 0;     // of blob, as taken from the pool
+    mutable size_t toff = 0;      // byte offset of the term table
     int ngroups = 0;
-    std::vector<PauliTerm> terms;
+    std::vector<PauliTerm> terms; // by X mask
+    const void *tables(Device &dev) const;
     // Tile plans of the expectation value per precision (complex64 first), made
     // on first use; entry points hold the engine lock.
     mutable std::shared_ptr<PauliTiles> tiles[2];
@@ -613,7 +615,7 @@ struct PauliDevice {
     PauliDevice &operator=(const PauliDevice &) = delete;
     ~PauliDevice();
 };
-std::unique_ptr<PauliDevice> pauli_upload(Device &dev, const std::vector<PauliTerm> &terms);
+std::unique_ptr<PauliDevice> pauli_device(Device &dev, const std::vector<PauliTerm> &terms);
 double pauli_expval(Device &dev, const State &s, const PauliDevice &t);
 void launch_pauli_apply(Device &dev, const State &out, const State &in, const PauliDevice &t);
 // Host image of a Pauli-word sum's tables (the layout PauliDevice holds on
