@@ -712,10 +712,10 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
         int index, sums;
         bool fus;
     };
-    std::vector<Item> rem(all.size()), rest;
+    std::vector<Item> items(all.size());
     uint64_t every = 0;
     for (size_t i = 0; i < all.size(); i++) {
-        Item &it = rem[i];
+        Item &it = items[i];
         it.index = static_cast<int>(i);
         it.trainable = all[i].trainable;
         it.skew = all[i].skew;
@@ -728,13 +728,21 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
         all[i].mix = it.mix;
         it.sums = bundled ? (all[i].trainable ? 1 : 0) : rt_slots(all[i]);
     }
+    // The first kLookahead operations left, all that a pass looks at: those that
+    // earlier passes skipped, then items from `next` on.
+    std::vector<Item> rem, rest;
+    size_t next = 0;
+    auto refill = [&] {
+        const size_t add = std::min(kLookahead - rem.size(), items.size() - next);
+        rem.insert(rem.end(), items.begin() + static_cast<long>(next), items.begin() + static_cast<long>(next + add));
+        next += add;
+    };
     // Operations of rem that a pass over these bits takes.
     auto count = [&](uint64_t bits) {
         Blocked blocked;
         size_t taken = 0;
         int sums = 0;
-        const size_t end = std::min(rem.size(), kLookahead);
-        for (size_t k = 0; k < end && rem[k].fus && (blocked.mixed & every) != every; k++) {
+        for (size_t k = 0; k < rem.size() && rem[k].fus && (blocked.mixed & every) != every; k++) {
             const Item &it = rem[k];
             if ((it.mix & ~bits) == 0 && !blocked.stops(it) && taken < kPassMaxOps && sums + it.sums <= pmax) {
                 taken++;
@@ -748,7 +756,7 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
     const uint64_t low = L > 0 ? (uint64_t{1} << L) - 1 : 0;
     std::vector<Step> steps;
     std::vector<int> taken;
-    while (!rem.empty()) {
+    for (refill(); !rem.empty(); refill()) {
         if (!rem[0].fus) {
             Step s;
             s.single = std::move(all[rem[0].index]);
@@ -770,7 +778,7 @@ std::vector<Step> plan_tiles(std::vector<PlanOp> &&ops_in, int n, int T, int L,
             rest.clear();
             nslots = 0;
             size_t k = 0;
-            for (; k < rem.size() && rem[k].fus && k < kLookahead; k++) {
+            for (; k < rem.size() && rem[k].fus; k++) {
                 const Item &it = rem[k];
                 const uint64_t nb = bits | it.mix;
                 if ((grow ? __builtin_popcountll(nb) <= T : nb == bits) && !blocked.stops(it) &&
