@@ -2090,12 +2090,12 @@ void build_slabs(PlanImage &img, int n, int dtype) {
 }
 
 const SlabGroup *slab_of(const PlanImage &img, size_t i) {
-    for (const SlabGroup &g : img.slabs) {
-        if (i >= g.first && i < g.first + g.count) {
-            return &g;
-        }
+    auto g = std::upper_bound(img.slabs.begin(), img.slabs.end(), i,
+                              [](size_t at, const SlabGroup &x) { return at < x.first; });
+    if (g == img.slabs.begin() || i >= std::prev(g)->first + std::prev(g)->count) {
+        return nullptr;
     }
-    return nullptr;
+    return &*std::prev(g);
 }
 
 // wide: register-tile programs in FP64 for complex64 states too, which are then
