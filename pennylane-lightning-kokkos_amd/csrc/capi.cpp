@@ -3177,6 +3177,15 @@ void run_sweep(Device &dev, int dtype, int n, const SweepTables &t, const std::v
     PLK_HIP(hipStreamSynchronize(dev.stream));
 }
 
+// Op lists that run whole in one launch. A handful of operations is one or two
+// launches in the general path too, with less to plan and upload (general /
+// whole: 5 qubits complex128 1 op 14.7 / 16.9 us, 4 ops 18.2 / 18.4, 8 ops 21 / 19;
+// complex64 4 ops 17.9 / 19.3, 8 one-wire ops 22.1 / 21.4; states of at most three
+// wires, one register segment: 8 ops 18.0 / 18.9).
+bool sweep_pays_forward(const State &s, size_t ops) {
+    return ops > (s.n <= SEG_KMAX ? 8u : s.dtype == PLK_C64 ? 6u : 4u);
+}
+
 void sweep_forward(Device &dev, const State &s, std::vector<PlanOp> &&ops) {
     SweepTables t;
     SweepJob J{};
@@ -4394,7 +4403,7 @@ int plk_apply_ops(plk_state *sv, const plk_ops *ops) {
         }
         Device &dev = dev_of(s);
         std::vector<PlanOp> v = forward_ops(ops->data, s.n);
-        if (sweep_serves(s) && sweep_takes(v)) {
+        if (sweep_serves(s) && sweep_pays_forward(s, v.size()) && sweep_takes(v)) {
             sweep_forward(dev, s, std::move(v));
         } else {
             run_forward(dev, s, forward_plan(dev, std::move(v), s.n, s.dtype, true));
