@@ -361,17 +361,23 @@ void probs_t(Device &dev, const State &s, const std::vector<int> &gbits, double 
         for (int k = 0; k < m; k++) {
             K += gbits[k] < line ? 1 : 0;
         }
-        K = std::min(K, 3);
+        // A state of at most 4 MiB stays in the L2s, where bins apart cost nothing and
+        // more blocks hide more latency (16 qubits complex128, the five lowest wires: 31
+        // us together, 28 apart; 20 qubits complex64, the lowest wire: 29 and 39).
+        K = s.bytes() <= (size_t{4} << 20) ? 0 : std::min(K, 3);
         // A power of two of ranges per bin: enough blocks to fill the device, of at
-        // least 1024 amplitudes a bin.
+        // least 1024 amplitudes a bin, or a block a CU of at least one a thread.
         uint64_t chunks = 1;
         while ((bins >> K) * chunks < MARG_BLOCKS && count / (2 * chunks) >= 1024) {
+            chunks *= 2;
+        }
+        while ((bins >> K) * chunks < static_cast<uint64_t>(dev.num_cus) && count / (2 * chunks) >= PB) {
             chunks *= 2;
         }
         const uint64_t per = count / chunks;
         double *partial = static_cast<double *>(
             ensure_work(dev, (bins * chunks + bins) * sizeof(double)));
-        double *out = partial + bins * chunks;
+        double *out = chunks == 1 ? partial : partial + bins * chunks;
         const uint64_t step = [&] {
             uint64_t v = 0, c = PB, mk = cmask;
             while (mk) {
@@ -390,9 +396,11 @@ void probs_t(Device &dev, const State &s, const std::vector<int> &gbits, double 
         case 2: launch_marg<T, 2>(dev, psi, bm, cmask, step, per, chunks, partial); break;
         default: launch_marg<T, 3>(dev, psi, bm, cmask, step, per, chunks, partial); break;
         }
-        hipLaunchKernelGGL(marg_finish_kernel, dim3(static_cast<unsigned>((bins + PB / 64 - 1) / (PB / 64))),
-                           dim3(PB), 0, dev.stream, partial, bins, chunks, out);
-        PLK_HIP(hipGetLastError());
+        if (chunks > 1) {
+            hipLaunchKernelGGL(marg_finish_kernel, dim3(static_cast<unsigned>((bins + PB / 64 - 1) / (PB / 64))),
+                               dim3(PB), 0, dev.stream, partial, bins, chunks, out);
+            PLK_HIP(hipGetLastError());
+        }
         PLK_HIP(hipMemcpyAsync(host_out, out, bins * sizeof(double), hipMemcpyDeviceToHost,
                                dev.stream));
     }
