@@ -295,6 +295,54 @@ __global__ void __launch_bounds__(PB)
     }
 }
 
+// The same for a state of one chunk and many shots, a thread a shot: every block
+// forms the offsets of all amplitudes in LDS (as sample_kernel does for the run
+// it needs, in the same order) and its threads search those. With 64 times as many
+// threads as shots 300000 shots of 1 qubit took 286 us, of 6 qubits 1100, so 191
+// and 990; 10000 shots of 10 qubits 73 and 70, of 12 qubits 81 and 85: used from
+// four shots an amplitude on.
+template <typename T>
+__global__ void __launch_bounds__(PB)
+    sample_chunk_kernel(const Cx<T> *__restrict__ psi, uint32_t len, const double *__restrict__ runs, int n,
+                        uint64_t shots, uint64_t seed, uint64_t *__restrict__ out) {
+    __shared__ double offset[CHUNK];
+    __shared__ double run_offset[64];
+    const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
+    const uint32_t nruns = (len + RUN - 1) / RUN;
+    const double t = runs[lane];
+    const double exc = __shfl_up(wave_scan(t, lane), 1, 64);
+    const double mine = lane == 0 ? 0.0 : exc; // of run `lane`
+    if (wave == 0) {
+        run_offset[lane] = mine;
+    }
+    for (uint32_t r = static_cast<uint32_t>(wave); r < nruns; r += PB / 64) {
+        const uint32_t i = r * RUN + static_cast<uint32_t>(lane);
+        const double p = i < len ? prob_of(psi[i]) : 0.0;
+        const double below = __shfl(mine, static_cast<int>(r), 64);
+        const double e = __shfl_up(wave_scan(p, lane), 1, 64);
+        offset[i] = lane == 0 ? below : below + e;
+    }
+    __syncthreads();
+    // The last of `count` (a power of two) ascending offsets that lies below u, or the first.
+    auto last = [](const double *v, uint32_t count, double u) {
+        uint32_t at = 0;
+        for (uint32_t step = count / 2; step > 0; step /= 2) {
+            at += v[at + step] < u ? step : 0;
+        }
+        return at;
+    };
+    const uint32_t per = len < RUN ? len : RUN;
+    for (uint64_t s = uint64_t{blockIdx.x} * PB + threadIdx.x; s < shots; s += uint64_t{gridDim.x} * PB) {
+        const uint64_t z = splitmix64(seed + (s + 1) * 0x9E3779B97F4A7C15ull);
+        const double u = static_cast<double>((z >> 11) + 1) * 0x1.0p-53;
+        const uint32_t r = last(run_offset, nruns, u);
+        const uint32_t index = r * RUN + last(offset + r * RUN, per, u);
+        for (int j = 0; j < n; j++) {
+            out[s * static_cast<uint64_t>(n) + static_cast<uint64_t>(j)] = (index >> (n - 1 - j)) & 1u;
+        }
+    }
+}
+
 template <typename T, int K>
 void launch_marg(Device &dev, const Cx<T> *psi, const BinMap &bm, uint64_t cmask, uint64_t step, uint64_t per,
                  uint64_t chunks, double *partial) {
@@ -426,9 +474,15 @@ void sample_t(Device &dev, const State &s, size_t shots, uint64_t seed, size_t *
         PLK_HIP(hipGetLastError());
         hipLaunchKernelGGL(scan_top_kernel, dim3(1), dim3(SCAN), 0, dev.stream, totals, nb);
         PLK_HIP(hipGetLastError());
-        hipLaunchKernelGGL((sample_kernel<T>), dim3(static_cast<unsigned>((shots + PB / 64 - 1) / (PB / 64))),
-                           dim3(PB), 0, dev.stream, psi, len, runs, totals, nb, s.n,
-                           static_cast<uint64_t>(shots), seed, out);
+        if (nb == 1 && shots >= std::max<size_t>(8192, 4 * static_cast<size_t>(len))) {
+            const uint64_t blocks = std::min<uint64_t>((shots + PB - 1) / PB, static_cast<uint64_t>(dev.num_cus) * 4);
+            hipLaunchKernelGGL((sample_chunk_kernel<T>), dim3(static_cast<unsigned>(blocks)), dim3(PB), 0, dev.stream,
+                               psi, static_cast<uint32_t>(len), runs, s.n, static_cast<uint64_t>(shots), seed, out);
+        } else {
+            hipLaunchKernelGGL((sample_kernel<T>), dim3(static_cast<unsigned>((shots + PB / 64 - 1) / (PB / 64))),
+                               dim3(PB), 0, dev.stream, psi, len, runs, totals, nb, s.n,
+                               static_cast<uint64_t>(shots), seed, out);
+        }
         PLK_HIP(hipGetLastError());
         PLK_HIP(hipMemcpyAsync(host_out, out, out_bytes, hipMemcpyDeviceToHost, dev.stream));
     }
