@@ -2100,11 +2100,12 @@ const SlabGroup *slab_of(const PlanImage &img, size_t i) {
 
 // wide: register-tile programs in FP64 for complex64 states too, which are then
 // rounded once a pass instead of at every operation (forward passes only). A
-// program whose result is the state takes it: an expectation value of a 22-qubit,
-// 4-layer circuit is a third as far from 64 bits as with a rounding per
+// pass-by-pass program whose result is the state takes it: an expectation value of
+// a 22-qubit, 4-layer circuit is a third as far from 64 bits as with a rounding per
 // operation (3.4e-7 against 8.6e-7 relative). 400 gates complex64: 22 qubits 0.82
-// -> 0.93 ms, 26 qubits 5.5 -> 7.2 ms. The forward run of a Jacobian, whose reverse
-// sweep rounds anyway, stays in FP32.
+// -> 0.92 ms, 26 qubits 5.5 -> 7.2 ms. The forward run of a Jacobian, whose reverse
+// sweep rounds anyway, stays in FP32, and so do states that run whole in one launch
+// (at most 12 qubits), which round at every operation.
 PlanImage build_image(const std::vector<Step> &steps, const State &s, bool wide) {
     PlanImage img;
     if (s.dtype == PLK_C64) {
@@ -3046,7 +3047,9 @@ void append_signature(const SweepParts &parts, std::vector<unsigned char> &sig) 
 // observable runs every pass of the circuit.
 // ---------------------------------------------------------------------------
 // Up to 12 qubits the launch beats a launch per pass (12 qubits, 12
-// observables, complex128: 392 against 532 us a Jacobian). PLK_SWEEP=0 turns it off.
+// observables, complex128: 0.36 against 0.53 ms a Jacobian), but for observables of
+// many words and lists of a few operations (sweep_takes_words, sweep_pays_forward).
+// PLK_SWEEP=0 turns it off.
 constexpr int kSweepQubits = 12;
 
 bool sweep_serves(const State &s) {

@@ -201,9 +201,9 @@ template <typename T, int NJ, int R, typename C> int blocks_per_chunk(const Devi
     uint64_t bpc = std::max<uint64_t>(1, std::min(ntiles, cap / static_cast<uint64_t>(nc)));
     // Without sums a block costs nothing to start: a block a tile lets the
     // hardware even out the wavefronts' speeds (resident blocks end between 70 %
-    // and 100 % of a pass). 26-qubit stream: complex128 14.9 -> 14.0 ms, complex64
-    // 6.0 -> 5.5; with two tiles a block 14.3. From four rounds on: with 2.7 (24
-    // qubits complex128) the last round is too empty, 2.40 -> 2.47 ms.
+    // and 100 % of a pass). 26-qubit stream of 400 gates: complex128 10.4 -> 9.7 ms,
+    // complex64 (an FP64 program) 7.7 -> 7.2. From four rounds on: with 2 to 2.7 (24
+    // qubits) the last round is too empty, 2.49 -> 2.60 and 1.97 -> 2.06 ms.
     if (NJ == 0 && ntiles >= 4 * cap) {
         bpc = ntiles;
     }
