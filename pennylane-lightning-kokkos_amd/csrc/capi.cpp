@@ -3327,6 +3327,7 @@ void adjoint_jacobian(const State &ref, const std::vector<std::shared_ptr<const 
     };
     std::vector<PauliImg> pimg;
     bool graph = n <= kGraphMaxQubits && env_int("PLK_GRAPH", 1) != 0 &&
+                 (2 + n_obs) * ref.bytes() <= kGraphBytesPerDevice && // one graph alone stays in the bound
                  !steps_have_single(steps, n) && !steps_have_single(fwd, n);
     for (size_t j = 0; graph && j < n_obs; j++) {
         std::vector<PauliTerm> terms;
