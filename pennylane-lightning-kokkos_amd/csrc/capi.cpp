@@ -263,7 +263,7 @@ struct PlanOp {
     double coef = 0.0;
     int32_t src = -1;       // index of the op in its OpsData
     bool adj = false;       // U was compiled with the inverse flag set
-    bool skew = false;      // reverse sweeps: U is not unitary (see Blocked)
+    bool skew = false;      // reverse sweeps: U is not unitary, or may not be (see Blocked)
     uint64_t mix = 0;       // register-tile plans: the state bits it mixes
     // Batch plans, runs with patched gates: the U kind and the Pauli parts that
     // hold for every angle (see fix_form); -1: as the matrices are.
@@ -2563,8 +2563,7 @@ std::vector<Step> forward_plan(const Device &dev, std::vector<PlanOp> &&v, int n
     return plan_steps(std::move(v));
 }
 
-bool is_unitary(const std::vector<cd> &M, double tol) {
-    const size_t dim = M.size() == 4 ? 2 : 4;
+bool is_unitary(const std::vector<cd> &M, size_t dim, double tol) {
     for (size_t a = 0; a < dim; a++) {
         for (size_t b = 0; b <= a; b++) {
             cd s = a == b ? -1.0 : 0.0;
@@ -2584,7 +2583,9 @@ bool is_unitary(const std::vector<cd> &M, double tol) {
 // its generator, Jacobian column and coefficient -2 s (inverse ? -1 : 1).
 // StatePrep / BasisState are skipped; ops with several parameters abort.
 // unitary: largest entry of U^dag U - 1 at which an explicit matrix still counts
-// as unitary (a matrix that a complex64 program gives in its own precision).
+// as unitary (a matrix that a complex64 program gives in its own precision). One
+// on five wires or more counts as skew unseen: the look takes 8^m products, and
+// all that it would save is that runs of gates end there.
 std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &tp, int n, int dtype) {
     const double unitary = dtype == PLK_C64 ? 1e-6 : 1e-12;
     const size_t n_tp = tp.size();
@@ -2610,8 +2611,8 @@ std::vector<PlanOp> reverse_ops(const OpsData &ops, const std::vector<size_t> &t
                          ops.matrices[o], n);
         p.src = static_cast<int32_t>(o);
         p.adj = !ops.inverses[o];
-        p.skew = !is_named_gate(ops.names[o]) && p.U.kind == OpKind::Dense && p.U.wires.size() <= 2 &&
-                 !is_unitary(p.U.mat, unitary);
+        p.skew = !is_named_gate(ops.names[o]) && p.U.kind == OpKind::Dense &&
+                 (p.U.wires.size() > 4 || !is_unitary(p.U.mat, size_t{1} << p.U.wires.size(), unitary));
         if (!ops.params[o].empty()) {
             if (current_param_idx == *tp_it) {
                 p.trainable = true;
